@@ -11,7 +11,7 @@ import sys
 
 import torch
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "moye.jl_amd"))
+sys.path.insert(0, os.path.join(os.getcwd(), "moye.jl_amd"))  # the package of the working folder, whose root this runs in
 
 import moye_hip as mh  # noqa: E402
 from moye_hip import _lib  # noqa: E402
