@@ -21,6 +21,7 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-
 SOURCES = {
     "capi.hip": [],
     "copy_kernels.hip": [],
+    "copy_transpose.hip": [],
     # the epilogue's alpha * acc + beta * c is two products and a sum, each rounded (the oracle composes it from axpby!):
     # never contracted into fused operations
     "gemm_mfma.hip": ["-ffp-contract=off"],

@@ -2,528 +2,19 @@
 //
 // Takes over the element loop of the reference's `copyto!`
 // (src/algorithm/copy.jl:4-12,42-64 and :106-130): logical element i of src goes to logical
-// element i of dst through both layouts.  Three kernels:
-//   transpose_lds   rank-2, the unit-stride mode differs between src and dst: 128-bit global
-//                   loads, 4x4 register transpose, XOR-swizzled LDS tile, 128-bit stores
+// element i of dst through both layouts.  Three kinds of kernel:
+//   transpose_blocks (copy_transpose.hip)  the unit-stride mode differs between src and dst
 //   copy_flat       both sides contiguous in the same order: 128-bit streaming copy
-//   copy_generic    anything else: per-element gather/scatter with optional conversion
+//   copy_generic, copy_groups    anything else: gather/scatter with optional conversion
 #include <algorithm>
 
+#include "copy_convert.hpp"
+#include "copy_transpose.hpp"
 #include "kernels.hpp"
 
 namespace moye {
 
-// ------------------------------------------------------------------------------------------
-// transpose through a 64x64 LDS tile
-// ------------------------------------------------------------------------------------------
-// src(i, j) at i + j*lds   (i is the contiguous index),  dst(i, j) at i*ldd + j.
-// One workgroup of 256 threads moves one 64x64 tile of 4-byte elements.
-//
-// LDS tile T[64 rows = i][16 chunks of 4 = j]; the chunk index is XORed with (row>>2)&15 so
-// that the 16 lanes which write one float4 each to 16 different rows, and the 16 lanes which
-// read 16 different chunks of one row, both touch all 64 banks exactly once.
-
-constexpr int kTile = 64;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // one 128-bit access
-
-template <bool kSwizzle>
-__device__ __forceinline__ int lds_chunk(int row, int chunk) {
-    return kSwizzle ? (chunk ^ ((row >> 2) & 15)) : chunk;
-}
-
-// tile index -> (ti, tj): tiles are visited in square super-blocks of `sb` x `sb` tiles so
-// that the workgroups in flight read and write runs of sb*256 contiguous bytes per row on
-// BOTH sides (a plain row-major order makes one side hop a full leading dimension per tile).
-__device__ __forceinline__ void tile_coords(int64_t t, int tiles_i, int tiles_j, int sb,
-                                            int* ti, int* tj) {
-    const int64_t per_band = (int64_t)sb * tiles_i;       // a band = sb tile-columns (j), all i
-    const int band = (int)(t / per_band);
-    const int64_t r = t - (int64_t)band * per_band;
-    const int band_w = min(sb, tiles_j - band * sb);      // last band may be narrower
-    const int blk = (int)(r / ((int64_t)sb * band_w));    // block of sb tiles along i
-    const int64_t q = r - (int64_t)blk * sb * band_w;
-    const int blk_h = min(sb, tiles_i - blk * sb);
-    // inside a block: i fastest
-    *ti = blk * sb + (int)(q % blk_h);
-    *tj = band * sb + (int)(q / blk_h);
-}
-
-// One workgroup moves GI tiles that are neighbours along the source's contiguous index: every
-// source row it touches is then a run of GI*256 bytes, which is what keeps DRAM pages open on the
-// read side; all 4*GI loads of a thread are in flight before the first LDS write.
-template <bool kSwizzle, int GI>
-__global__ __launch_bounds__(256) void transpose_lds_b32(const uint32_t* __restrict__ src,
-                                                         uint32_t* __restrict__ dst, int64_t lds_,
-                                                         int64_t ldd, int groups_i, int tiles_j,
-                                                         int sb, int64_t bs_src, int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    extern __shared__ u32x4 tile[];  // GI tiles of 64 x 16 chunks
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;  // blockIdx.y counts the matrices of a batch
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    int gi, tj;
-    tile_coords(blockIdx.x, groups_i, tiles_j, sb, &gi, &tj);
-
-    const int lane16 = threadIdx.x & 15;  // chunk of 4 along the contiguous index
-    const int grp = threadIdx.x >> 4;     // 0..15
-
-    // ---- load: rows j = 4*grp+q, columns i = 4*lane16 .. +3 of each tile ----
-    const uint32_t* s = src + ((int64_t)tj * kTile + 4 * grp) * lds_ + (int64_t)gi * GI * kTile + 4 * lane16;
-    u32x4 v[GI][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int a = 0; a < GI; ++a)
-            v[a][q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + q * lds_ + a * kTile));
-
-    // ---- 4x4 register transpose, store float4 over j into row i of the LDS tile ----
-#pragma unroll
-    for (int a = 0; a < GI; ++a)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = 4 * lane16 + e;  // i within the tile
-            tile[a * 1024 + row * 16 + lds_chunk<kSwizzle>(row, grp)] = u32x4{v[a][0][e], v[a][1][e], v[a][2][e], v[a][3][e]};
-        }
-    __syncthreads();
-
-    // ---- store: rows i = grp + 16*p, columns j = 4*lane16 .. +3 ----
-    uint32_t* d = dst + ((int64_t)gi * GI * kTile + grp) * ldd + (int64_t)tj * kTile + 4 * lane16;
-#pragma unroll
-    for (int a = 0; a < GI; ++a)
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const int row = grp + 16 * p;
-            const u32x4 w = tile[a * 1024 + row * 16 + lds_chunk<kSwizzle>(row, lane16)];
-            __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(d + (int64_t)(a * kTile + 16 * p) * ldd));
-        }
-}
-
-template <bool kSwizzle, int GI>
-static int32_t launch_transpose(const uint32_t* s, uint32_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st, int64_t bs_src = 0,
-                              int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b32<kSwizzle, GI>;
-    constexpr int kLds = GI * kTile * kTile * 4;
-    if (kLds > 48 * 1024) {
-        static LdsCap cap;
-        if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    }
-    const int64_t groups = (int64_t)(ti / GI) * tj;
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    // groups are walked with the source-contiguous index fastest in bands of 64 tile columns: the
-    // workgroups in flight read whole source rows and write runs of several KiB per destination row
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 256, kLds, st>>>(s, d, lds_, ldd, ti / GI, tj, 64, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-// The form for large matrices: a workgroup moves GJ tiles that are neighbours along the DESTINATION's contiguous index
-// (64 destination rows of GJ * 256 bytes each) and workgroups are numbered along that index first, so consecutive
-// workgroups complete whole destination rows: 64 x ldd elements of contiguous memory per tj / GJ workgroups.  On this
-// part writes are the side that needs the locality (measured on 16384^2, one side at a time with the other left out:
-// reads of 256-byte pieces a pitch apart run at 6.9 TB/s whatever the order; writes run at 6.6-6.9 TB/s in this order
-// against 5.1 with the source-contiguous index first), and fewer workgroups in flight do better than more: one per CU
-// (6.25 TB/s) against two (6.15) or five (5.85), hence the LDS request above what the tiles need.
-// 512 lanes, eight 16-byte loads each (same box, alternating runs, 16384^2: 256 lanes with sixteen loads each 6226-6252 GB/s,
-// 512 with eight 6263-6300, 1024 with four 6236; two such workgroups per CU 6254; workgroups of 32 x 512, 128 x 256 or
-// 64 x 512 elements 5.9-6.2; ordinary stores, or half of each row stored the ordinary way, 5.89; ordinary loads 5.90).
-template <int GJ>
-__global__ __launch_bounds__(512) void transpose_lds_b32_rows(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
-                                                              int64_t lds_, int64_t ldd, int groups_j, int64_t bs_src,
-                                                              int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    constexpr int TJ = GJ * kTile, JC = TJ / 4;  // the group's extent along j, in elements and in 16-byte chunks
-    constexpr int NG = 512 / 16, NB = JC / NG;   // lanes come as 16 chunks along i x NG row quads along j
-    static_assert(JC % NG == 0 && 512 % JC == 0, "group shape");
-    extern __shared__ u32x4 tile[];  // 64 rows (i) of JC chunks (j), the chunk index XORed with (row / 4) % 8
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    const int gj = blockIdx.x % groups_j, ti = blockIdx.x / groups_j;
-    const int ic = threadIdx.x & 15;  // chunk of 4 along i
-    const int jr = threadIdx.x >> 4;  // 0..31: source rows 4 (jr + NG b) + q
-
-    const uint32_t* s = src + ((int64_t)gj * TJ) * lds_ + (int64_t)ti * kTile + 4 * ic;
-    u32x4 v[NB][4];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            v[b][q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(4 * (jr + NG * b) + q) * lds_));
-    // 4 x 4 register transpose: eight consecutive lanes write eight different rows-of-four, hence eight different bank groups
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = 4 * ic + e, c = jr + NG * b;
-            tile[row * JC + (c ^ ((row >> 2) & 7))] = u32x4{v[b][0][e], v[b][1][e], v[b][2][e], v[b][3][e]};
-        }
-    __syncthreads();
-    // ---- store: JC consecutive lanes write one destination row of the group (GJ * 256 bytes), 512 / JC rows per pass ----
-    constexpr int RPP = 512 / JC;
-    const int jc = threadIdx.x % JC, r0 = threadIdx.x / JC;
-    uint32_t* d = dst + ((int64_t)ti * kTile + r0) * ldd + (int64_t)gj * TJ + 4 * jc;
-#pragma unroll
-    for (int p = 0; p < kTile / RPP; ++p) {
-        const int row = r0 + RPP * p;
-        const u32x4 w = tile[row * JC + (jc ^ ((row >> 2) & 7))];
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(d + (int64_t)(RPP * p) * ldd));
-    }
-}
-
-template <int GJ>
-static int32_t launch_transpose_rows(const uint32_t* s, uint32_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st,
-                                     int64_t bs_src = 0, int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b32_rows<GJ>;
-    constexpr int kLds = 96 * 1024;  // the tiles need GJ * 16 KiB; more than half of a CU's 160 KiB keeps it to one workgroup per CU
-    static_assert(GJ * kTile * kTile * 4 <= kLds, "tiles fit");
-    static LdsCap cap;
-    if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    const int64_t groups = (int64_t)ti * (tj / GJ);
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 512)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 512, kLds, st>>>(s, d, lds_, ldd, tj / GJ, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-// ------------------------------------------------------------------------------------------
-// the same for 8-byte elements (Float64 / Int64 matrices), destination rows first
-// ------------------------------------------------------------------------------------------
-// A workgroup moves 64 (i) x 128 (j) elements, 64 KiB like the 4-byte form: a source row's piece is 512 bytes (32 lanes of
-// two elements), a destination row's 1 KiB (64 lanes of two elements).  A lane loads two elements along i from each of two
-// neighbouring source rows, turns the 2 x 2 block in registers and writes two elements along j into each of two LDS rows;
-// the chunk index of an LDS row is XORed with (row / 2) % 8.
-constexpr int kTileJ64 = 128;
-__global__ __launch_bounds__(512) void transpose_lds_b64_rows(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst, int64_t lds_,
-                                                              int64_t ldd, int groups_j, int64_t bs_src, int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    constexpr int JC = kTileJ64 / 2;            // 16-byte chunks (two elements) per LDS row
-    constexpr int NG = 512 / 32, NB = JC / NG;  // lanes come as 32 chunks along i x NG row pairs along j
-    extern __shared__ u32x4 tile[];             // 64 rows (i) of JC chunks (j)
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    const int gj = blockIdx.x % groups_j, ti = blockIdx.x / groups_j;
-    const int ic = threadIdx.x & 31;  // chunk of 2 along i
-    const int jr = threadIdx.x >> 5;  // 0..15: source rows 2 (jr + NG b) + q
-    const uint64_t* s = src + ((int64_t)gj * kTileJ64) * lds_ + (int64_t)ti * kTile + 2 * ic;
-    u32x4 v[NB][2];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            v[b][q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(2 * (jr + NG * b) + q) * lds_));
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int row = 2 * ic + e, c = jr + NG * b;
-            tile[row * JC + (c ^ ((row >> 1) & 7))] = u32x4{v[b][0][2 * e], v[b][0][2 * e + 1], v[b][1][2 * e], v[b][1][2 * e + 1]};
-        }
-    __syncthreads();
-    // ---- store: JC consecutive lanes write one destination row of the group (1 KiB), 512 / JC rows per pass ----
-    constexpr int RPP = 512 / JC;
-    const int jc = threadIdx.x % JC, r0 = threadIdx.x / JC;
-    uint64_t* d = dst + ((int64_t)ti * kTile + r0) * ldd + (int64_t)gj * kTileJ64 + 2 * jc;
-#pragma unroll
-    for (int p = 0; p < kTile / RPP; ++p) {
-        const int row = r0 + RPP * p;
-        const u32x4 w = tile[row * JC + (jc ^ ((row >> 1) & 7))];
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(d + (int64_t)(RPP * p) * ldd));
-    }
-}
-
-static int32_t launch_transpose64_rows(const uint64_t* s, uint64_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st,
-                                       int64_t bs_src = 0, int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b64_rows;
-    constexpr int kLds = 96 * 1024;  // the tile needs 64 KiB; the request keeps it to one workgroup per CU
-    static LdsCap cap;
-    if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    const int64_t groups = (int64_t)ti * tj;
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 512)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 512, kLds, st>>>(s, d, lds_, ldd, tj, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-// ------------------------------------------------------------------------------------------
-// the same for 2-byte elements (fp16 / bf16 matrices)
-// ------------------------------------------------------------------------------------------
-// A 64 x 64 tile is 64 source rows (j) of 128 bytes.  Rows go to LDS as they come, 16 bytes per lane,
-// with the 16-byte chunk index XORed with j / 8; a lane then gathers the 8 values S[8c .. 8c+7][i]
-// with 2-byte LDS reads (for a wave: 8 values of i, 8 values of c -> 32 different banks) and stores them
-// as one 16-byte piece of destination row i, 8 lanes per 128-byte run.
-template <int GI>
-__global__ __launch_bounds__(256) void transpose_lds_b16(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                         int64_t lds_, int64_t ldd, int groups_i, int tiles_j, int sb,
-                                                         int64_t bs_src, int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    extern __shared__ u32x4 tile[];  // GI tiles of 64 rows x 8 chunks
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    int gi, tj;
-    tile_coords(blockIdx.x, groups_i, tiles_j, sb, &gi, &tj);
-    const int v = threadIdx.x & 7;   // 16-byte chunk inside a 128-byte run
-    const int r = threadIdx.x >> 3;  // 0..31
-
-    // ---- load: rows j = r and r + 32, elements i = 8v .. 8v+7 of each tile ----
-    const uint16_t* s = src + ((int64_t)tj * kTile + r) * lds_ + (int64_t)gi * GI * kTile + 8 * v;
-    u32x4 x[GI][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int a = 0; a < GI; ++a)
-            x[a][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(32 * h) * lds_ + a * kTile));
-#pragma unroll
-    for (int a = 0; a < GI; ++a)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int j = r + 32 * h;
-            tile[a * 512 + j * 8 + (v ^ (j >> 3))] = x[a][h];
-        }
-    __syncthreads();
-
-    // ---- store: destination rows i = r and r + 32, elements j = 8v .. 8v+7 ----
-    const uint16_t* lds16 = reinterpret_cast<const uint16_t*>(tile);
-    uint16_t* d = dst + ((int64_t)gi * GI * kTile + r) * ldd + (int64_t)tj * kTile + 8 * v;
-#pragma unroll
-    for (int a = 0; a < GI; ++a)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int i = r + 32 * h;
-            uint16_t w[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int j = 8 * v + q;  // j / 8 == v
-                w[q] = lds16[a * 4096 + j * 64 + ((((i >> 3) ^ v) << 3) | (i & 7))];
-            }
-            u32x4 o;
-            o.x = w[0] | ((uint32_t)w[1] << 16);
-            o.y = w[2] | ((uint32_t)w[3] << 16);
-            o.z = w[4] | ((uint32_t)w[5] << 16);
-            o.w = w[6] | ((uint32_t)w[7] << 16);
-            __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(d + (int64_t)(a * kTile + 32 * h) * ldd));
-        }
-}
-
-template <int GI>
-static int32_t launch_transpose16(const uint16_t* s, uint16_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st, int64_t bs_src = 0,
-                              int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b16<GI>;
-    constexpr int kLds = GI * kTile * kTile * 2;
-    if (kLds > 48 * 1024) {
-        static LdsCap cap;
-        if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    }
-    const int64_t groups = (int64_t)(ti / GI) * tj;
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 256, kLds, st>>>(s, d, lds_, ldd, ti / GI, tj, 64, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-// The same with destination rows first (see transpose_lds_b32_rows): a workgroup moves GJ tiles that are neighbours
-// along the destination's contiguous index, 64 destination rows of GJ * 128 bytes, and workgroups are numbered along that
-// index first; one workgroup per CU.
-template <int GJ>
-__global__ __launch_bounds__(256) void transpose_lds_b16_rows(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                              int64_t lds_, int64_t ldd, int groups_j, int64_t bs_src,
-                                                              int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    extern __shared__ u32x4 tile[];  // GJ tiles of 64 rows x 8 chunks
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    const int gj = blockIdx.x % groups_j, ti = blockIdx.x / groups_j;
-    const int v = threadIdx.x & 7;   // 16-byte chunk inside a 128-byte run
-    const int r = threadIdx.x >> 3;  // 0..31
-    const uint16_t* s = src + ((int64_t)gj * GJ * kTile + r) * lds_ + (int64_t)ti * kTile + 8 * v;
-    u32x4 x[GJ][2];
-#pragma unroll
-    for (int b = 0; b < GJ; ++b)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            x[b][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(b * kTile + 32 * h) * lds_));
-#pragma unroll
-    for (int b = 0; b < GJ; ++b)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int j = r + 32 * h;
-            tile[b * 512 + j * 8 + (v ^ (j >> 3))] = x[b][h];
-        }
-    __syncthreads();
-    const uint16_t* lds16 = reinterpret_cast<const uint16_t*>(tile);
-    uint16_t* d = dst + ((int64_t)ti * kTile + r) * ldd + (int64_t)gj * GJ * kTile + 8 * v;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int b = 0; b < GJ; ++b) {
-            const int i = r + 32 * h;
-            uint16_t w[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int j = 8 * v + q;  // j / 8 == v
-                w[q] = lds16[b * 4096 + j * 64 + ((((i >> 3) ^ v) << 3) | (i & 7))];
-            }
-            u32x4 o;
-            o.x = w[0] | ((uint32_t)w[1] << 16);
-            o.y = w[2] | ((uint32_t)w[3] << 16);
-            o.z = w[4] | ((uint32_t)w[5] << 16);
-            o.w = w[6] | ((uint32_t)w[7] << 16);
-            __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(d + (int64_t)(32 * h) * ldd + b * kTile));
-        }
-}
-
-template <int GJ>
-static int32_t launch_transpose16_rows(const uint16_t* s, uint16_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st,
-                                       int64_t bs_src = 0, int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b16_rows<GJ>;
-    constexpr int kLds = 96 * 1024;  // the tiles need GJ * 8 KiB; the request keeps it to one workgroup per CU
-    static_assert(GJ * kTile * kTile * 2 <= kLds, "tiles fit");
-    static LdsCap cap;
-    if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    const int64_t groups = (int64_t)ti * (tj / GJ);
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 256, kLds, st>>>(s, d, lds_, ldd, tj / GJ, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-// ------------------------------------------------------------------------------------------
-// the same for 1-byte elements (fp8 matrices, bytes)
-// ------------------------------------------------------------------------------------------
-// A sub-tile is 256 source rows (j) of 64 bytes (i); a workgroup moves GI of them that are neighbours along i.  Rows go
-// to LDS as they come, 16 bytes per lane.  A lane then owns a block of 4 (i) x 16 (j) bytes: it reads the 16 rows'
-// dwords, transposes the bytes in registers and stores four 16-byte pieces, one to each of four consecutive
-// destination rows.  A 64-byte LDS row spans 16 of the 64 banks, so rows that are a multiple of four apart share
-// banks; the lanes of a wave read rows 16 apart, hence rows are stored with their two low index bits XORed with
-// bits 4-5: the four rows a wave reads at once then lie in four different bank groups.
-constexpr int kTileJ8 = 256;
-__device__ __forceinline__ int lds_row_b8(int j) { return (j & ~3) | ((j & 3) ^ ((j >> 4) & 3)); }
-
-template <int GI>
-__global__ __launch_bounds__(256) void transpose_lds_b8(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t lds_,
-                                                        int64_t ldd, int groups_i, int tiles_j, int sb, int64_t bs_src,
-                                                        int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    extern __shared__ u32x4 tile[];  // GI sub-tiles of 256 rows x 4 chunks
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    int gi, tj;
-    tile_coords(blockIdx.x, groups_i, tiles_j, sb, &gi, &tj);
-    const int v = threadIdx.x & 3;   // 16-byte chunk of a 64-byte row
-    const int r = threadIdx.x >> 2;  // 0..63
-
-    // ---- load: rows j = r + 64 h, bytes i = 16 v .. 16 v + 15 of each sub-tile ----
-    const uint8_t* s = src + ((int64_t)tj * kTileJ8 + r) * lds_ + (int64_t)gi * GI * kTile + 16 * v;
-    u32x4 x[GI][4];
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-        for (int a = 0; a < GI; ++a)
-            x[a][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(64 * h) * lds_ + a * kTile));
-#pragma unroll
-    for (int a = 0; a < GI; ++a)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) tile[a * 1024 + lds_row_b8(r + 64 * h) * 4 + v] = x[a][h];
-    __syncthreads();
-
-    // ---- store: destination rows i = 4 ib .. 4 ib + 3, bytes j = 16 c .. 16 c + 15 ----
-    const uint32_t* lds32 = reinterpret_cast<const uint32_t*>(tile);
-    const int ib = threadIdx.x & 15, c = threadIdx.x >> 4;
-    uint8_t* d = dst + ((int64_t)gi * GI * kTile + 4 * ib) * ldd + (int64_t)tj * kTileJ8 + 16 * c;
-#pragma unroll
-    for (int a = 0; a < GI; ++a) {
-        uint32_t w[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = lds32[a * 4096 + lds_row_b8(16 * c + q) * 16 + ib];  // S[16 c + q][4 ib .. 4 ib + 3]
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            u32x4 o;
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                o[g] = ((w[4 * g] >> (8 * e)) & 0xffu) | (((w[4 * g + 1] >> (8 * e)) & 0xffu) << 8) |
-                       (((w[4 * g + 2] >> (8 * e)) & 0xffu) << 16) | (((w[4 * g + 3] >> (8 * e)) & 0xffu) << 24);
-            __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(d + (int64_t)(a * kTile + e) * ldd));
-        }
-    }
-}
-
-// The same for matrices whose source rows come in whole runs of 256 bytes: a workgroup moves a tile of 256 x 256 bytes,
-// four of the sub-tiles above side by side along i, and both sides move whole 256-byte runs per instruction: a load
-// instruction reads four source rows of 256 bytes (sixteen lanes each), a store instruction writes four destination rows
-// of 256 bytes.  (The kernel above reads and writes 64-byte pieces of sixteen rows per instruction: half lines, which the
-// address path takes several times slower, and four waves complete a destination row's run between them.)  A lane of the
-// store phase owns 4 (i) x 16 (j) bytes of each sub-tile as above; the sixteen lanes of a run read LDS rows 16 apart and
-// the four runs of a wave four neighbouring dwords, so besides the row swizzle above the dword position of a row is
-// XORed with 4 ((j / 64) % 4): the 64 dwords a wave reads at once then lie in 64 banks.  The 4 x 4 byte blocks are
-// transposed with v_perm_b32, eight per block.
-// Workgroups are numbered along the destination's contiguous index first (see transpose_lds_b32_rows), one per CU.
-__device__ __forceinline__ void transpose_bytes_4x4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3, uint32_t (&o)[4]) {
-    const uint32_t t0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), t1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-    const uint32_t t2 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), t3 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-    o[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-    o[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-    o[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-    o[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
-
-__global__ __launch_bounds__(256) void transpose_lds_b8_wide(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t lds_,
-                                                             int64_t ldd, int tiles_j, int64_t bs_src, int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    extern __shared__ u32x4 tile[];  // four sub-tiles of 256 rows x 4 chunks
-    src += (int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src;
-    dst += (int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst;
-    const int tj = blockIdx.x % tiles_j, gi = blockIdx.x / tiles_j;
-    // ---- load: rows j = r + 16 h, bytes i = 64 a + 16 v .. + 15: a row's sixteen lanes read 256 contiguous bytes ----
-    const int v = threadIdx.x & 3, a = (threadIdx.x >> 2) & 3, r = threadIdx.x >> 4;
-    const uint8_t* s = src + ((int64_t)tj * kTileJ8 + r) * lds_ + (int64_t)gi * 4 * kTile + 64 * a + 16 * v;
-    u32x4 x[16];
-#pragma unroll
-    for (int h = 0; h < 16; ++h) x[h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(16 * h) * lds_));
-#pragma unroll
-    for (int h = 0; h < 16; ++h) {
-        const int j = r + 16 * h;
-        tile[a * 1024 + lds_row_b8(j) * 4 + (v ^ ((j >> 6) & 3))] = x[h];
-    }
-    __syncthreads();
-
-    // ---- store: destination rows i = 64 a + 4 ib .. + 3, bytes j = 16 c .. 16 c + 15: sixteen lanes write 256 contiguous bytes ----
-    const uint32_t* lds32 = reinterpret_cast<const uint32_t*>(tile);
-    const int c = threadIdx.x & 15, ib = threadIdx.x >> 4;
-    uint8_t* d = dst + ((int64_t)gi * 4 * kTile + 4 * ib) * ldd + (int64_t)tj * kTileJ8 + 16 * c;
-    const int pos = ib ^ ((c >> 2) << 2);  // (16 c + q) / 64 == c / 4
-#pragma unroll
-    for (int a2 = 0; a2 < 4; ++a2) {
-        uint32_t w[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = lds32[a2 * 4096 + lds_row_b8(16 * c + q) * 16 + pos];  // S[16 c + q][64 a2 + 4 ib .. + 3]
-        uint32_t o[4][4];  // [g][e]
-#pragma unroll
-        for (int g = 0; g < 4; ++g) transpose_bytes_4x4(w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3], o[g]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            __builtin_nontemporal_store(u32x4{o[0][e], o[1][e], o[2][e], o[3][e]}, reinterpret_cast<u32x4*>(d + (int64_t)(a2 * kTile + e) * ldd));
-    }
-}
-
-static int32_t launch_transpose8_wide(const uint8_t* s, uint8_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st, int64_t bs_src = 0,
-                                      int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b8_wide;
-    constexpr int kLds = 96 * 1024;  // the tile needs 64 KiB; the request keeps it to one workgroup per CU (+2-3 % on large matrices)
-    static_assert(4 * kTileJ8 * kTile <= kLds, "the tile fits");
-    static LdsCap cap;
-    if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    const int64_t groups = (int64_t)(ti / 4) * tj;
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 256, kLds, st>>>(s, d, lds_, ldd, tj, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-
-template <int GI>
-static int32_t launch_transpose8(const uint8_t* s, uint8_t* d, int64_t lds_, int64_t ldd, int ti, int tj, hipStream_t st, int64_t bs_src = 0,
-                              int64_t bs_dst = 0, int batch = 1, int64_t bz_src = 0, int64_t bz_dst = 0, int batch2 = 1) {
-    auto kern = transpose_lds_b8<GI>;
-    constexpr int kLds = GI * kTileJ8 * kTile;
-    if (kLds > 48 * 1024) {
-        static LdsCap cap;
-        if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    }
-    const int64_t groups = (int64_t)(ti / GI) * tj;
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    kern<<<dim3((unsigned)groups, (unsigned)batch, (unsigned)batch2), 256, kLds, st>>>(s, d, lds_, ldd, ti / GI, tj, 64, bs_src, bs_dst, bz_src, bz_dst);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
 
 // ------------------------------------------------------------------------------------------
 // contiguous streaming copy, 16 bytes per lane per step
@@ -563,45 +54,6 @@ __device__ __forceinline__ int64_t layout_offset(const FlatLayout& l, int64_t i)
         i = q;
     }
     return off;
-}
-
-__device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
-// round to nearest even, a NaN made quiet: v_cvt_pk_bf16_f32 (the same bits as the integer form for all 2^32 inputs)
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
-
-// OCP e4m3fn <-> fp32 through v_cvt_f32_fp8 / v_cvt_pk_fp8_f32.  Narrowing rounds to nearest even and turns NaN, infinities
-// and everything beyond the last tie (|x| > 464) into NaN, as the integer form these replaced did: a one-off kernel compared
-// the two over all 2^32 inputs (and all 256 the other way) on the hardware.  They differ in one thing only, the sign of a NaN:
-// the instructions make every NaN negative, here a NaN keeps the sign it came with.
-__device__ __forceinline__ float f8e4m3_to_f32(uint8_t b) {
-    return b == 0x7f ? __uint_as_float(0x7fc00000u) : __builtin_amdgcn_cvt_f32_fp8((int)b, 0);
-}
-__device__ __forceinline__ uint8_t f32_to_f8e4m3(float f) {
-    const uint8_t h = (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(f, f, 0, false) & 0xff);
-    return f != f ? (uint8_t)(((__float_as_uint(f) >> 24) & 0x80) | 0x7f) : h;
-}
-
-template <int kDt>
-__device__ __forceinline__ double load_as_f64(const char* p) {
-    if constexpr (kDt == MOYE_F32) return (double)*reinterpret_cast<const float*>(p);
-    else if constexpr (kDt == MOYE_F16) return (double)(float)*reinterpret_cast<const _Float16*>(p);
-    else if constexpr (kDt == MOYE_BF16) return (double)bf16_to_f32(*reinterpret_cast<const uint16_t*>(p));
-    else if constexpr (kDt == MOYE_F8E4M3) return (double)f8e4m3_to_f32(*reinterpret_cast<const uint8_t*>(p));
-    else return *reinterpret_cast<const double*>(p);
-}
-
-// Every narrower float format here embeds exactly in fp32 and fp32 in fp64, so one rounding
-// step per conversion happens below (f64 -> f16/bf16/f8 goes through f32 only when the source
-// was at most f32, which is then exact).
-template <int kDt>
-__device__ __forceinline__ void store_from(char* p, double v, bool src_is_f64) {
-    if constexpr (kDt == MOYE_F64) *reinterpret_cast<double*>(p) = v;
-    else if constexpr (kDt == MOYE_F32) *reinterpret_cast<float*>(p) = (float)v;
-    else if constexpr (kDt == MOYE_F16)
-        *reinterpret_cast<_Float16*>(p) = src_is_f64 ? (_Float16)v : (_Float16)(float)v;
-    else if constexpr (kDt == MOYE_BF16) *reinterpret_cast<uint16_t*>(p) = f32_to_bf16((float)v);
-    else *reinterpret_cast<uint8_t*>(p) = f32_to_f8e4m3((float)v);
 }
 
 // copyto_if! (src/algorithm/copy.jl:4-16): element i moves only where the mask's logical element i is nonzero
@@ -926,100 +378,6 @@ static int64_t launch_cvt_dense(int32_t sd, int32_t dd, const char* s, char* d, 
     }
 }
 
-// ------------------------------------------------------------------------------------------
-// a transpose that converts on the way (copyto! between arrays of different element types whose unit strides lie on
-// different modes: src/algorithm/copy.jl:38-43 with the layouts of a transpose)
-// ------------------------------------------------------------------------------------------
-// A tile is TI elements along the source's contiguous index i (at least 128 bytes of a source row) by TJ along the
-// destination's (at least 256 bytes of a destination row).  A lane loads 16-byte pieces of source rows, converts their
-// elements and writes them one by one into an LDS tile of destination elements, [i][j]; a lane then reads 16 bytes of an
-// LDS row and stores them as 16 bytes of a destination row.  Workgroups are numbered along j first, as in the other
-// destination-order kernels.  An LDS row is 16 bytes longer than its data, which spreads the rows over the banks.
-template <int kSrc, int kDst, int SB, int DB>
-__global__ __launch_bounds__(256) void transpose_cvt_lds(const char* __restrict__ src, char* __restrict__ dst, int64_t lds_, int64_t ldd, int tiles_j,
-                                                         int64_t bs_src, int64_t bs_dst, int64_t bz_src, int64_t bz_dst) {
-    constexpr int TI = SB == 1 ? 128 : 64, TJ = DB == 1 ? 256 : 128;
-    constexpr int ES = 16 / SB, ED = 16 / DB;  // elements per 16-byte piece
-    constexpr int PI = TI / ES, RJ = 256 / PI, NL = TJ / RJ;  // pieces per source row of the tile, source rows per pass, passes
-    constexpr int PITCH = TJ * DB + 16;
-    extern __shared__ char cvt_tile[];  // TI rows of PITCH bytes
-    src += ((int64_t)blockIdx.y * bs_src + (int64_t)blockIdx.z * bz_src) * SB;  // (a batch of matrices: their indices in the grid)
-    dst += ((int64_t)blockIdx.y * bs_dst + (int64_t)blockIdx.z * bz_dst) * DB;
-    const int tj = blockIdx.x % tiles_j, ti = blockIdx.x / tiles_j;
-    const int pi = threadIdx.x % PI, jr = threadIdx.x / PI;
-    const char* s = src + (((int64_t)tj * TJ + jr) * lds_ + (int64_t)ti * TI + ES * pi) * SB;
-    constexpr int CH = NL < 8 ? NL : 8;  // loads in flight per lane
-#pragma unroll 1
-    for (int h0 = 0; h0 < NL; h0 += CH) {
-        u32x4 x[CH];
-#pragma unroll
-        for (int h = 0; h < CH; ++h) x[h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + (int64_t)(RJ * (h0 + h)) * lds_ * SB));
-#pragma unroll
-        for (int h = 0; h < CH; ++h) {
-            const int j = jr + RJ * (h0 + h);
-#pragma unroll
-            for (int e = 0; e < ES; ++e) {
-                char e_in[SB];
-                __builtin_memcpy(e_in, reinterpret_cast<const char*>(&x[h]) + e * SB, SB);
-                store_from<kDst>(cvt_tile + (ES * pi + e) * PITCH + j * DB, load_as_f64<kSrc>(e_in), kSrc == MOYE_F64);
-            }
-        }
-    }
-    __syncthreads();
-    constexpr int PJ = TJ / ED, RP = 256 / PJ;  // pieces per destination row of the tile, destination rows per pass
-    const int pj = threadIdx.x % PJ, r0 = threadIdx.x / PJ;
-    char* d = dst + (((int64_t)ti * TI + r0) * ldd + (int64_t)tj * TJ + ED * pj) * DB;
-#pragma unroll
-    for (int p = 0; p < TI / RP; ++p) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(cvt_tile + (r0 + RP * p) * PITCH + pj * 16);
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(d + (int64_t)(RP * p) * ldd * DB));
-    }
-}
-
-// tile extents of transpose_cvt_lds for elements of sb and db bytes
-static int cvt_tile_i(int sb) { return sb == 1 ? 128 : 64; }
-static int cvt_tile_j(int db) { return db == 1 ? 256 : 128; }
-
-template <int kSrc, int kDst, int SB, int DB>
-static int32_t launch_transpose_cvt_pair(const char* s, char* d, int64_t lds_, int64_t ldd, int64_t ni, int64_t nj, hipStream_t st, const int64_t (&bt)[6]) {
-    auto kern = transpose_cvt_lds<kSrc, kDst, SB, DB>;
-    constexpr int TI = SB == 1 ? 128 : 64, TJ = DB == 1 ? 256 : 128, kLds = TI * (TJ * DB + 16);
-    if (kLds > 48 * 1024) {
-        static LdsCap cap;
-        if (int32_t e = raise_lds_cap(cap, reinterpret_cast<const void*>(kern), kLds)) return e;
-    }
-    const int64_t groups = (ni / TI) * (nj / TJ);
-    if (groups >= (1 << 24)) return fail(MOYE_ERR_SHAPE, "copyto!: too many tiles for one launch (2^24 workgroups of 256)");
-    kern<<<dim3((unsigned)groups, (unsigned)bt[4], (unsigned)bt[5]), 256, kLds, st>>>(s, d, lds_, ldd, (int)(nj / TJ), bt[0], bt[1], bt[2], bt[3]);
-    MOYE_HIP_CHECK(hipGetLastError());
-    return MOYE_OK;
-}
-template <int kSrc, int SB>
-static int32_t launch_transpose_cvt_dst(int32_t dd, const char* s, char* d, int64_t lds_, int64_t ldd, int64_t ni, int64_t nj, hipStream_t st, const int64_t (&bt)[6]) {
-    switch (dd) {
-        case MOYE_F32: if constexpr (kSrc != MOYE_F32) return launch_transpose_cvt_pair<kSrc, MOYE_F32, SB, 4>(s, d, lds_, ldd, ni, nj, st, bt); break;
-        case MOYE_F16: if constexpr (kSrc != MOYE_F16) return launch_transpose_cvt_pair<kSrc, MOYE_F16, SB, 2>(s, d, lds_, ldd, ni, nj, st, bt); break;
-        case MOYE_BF16: if constexpr (kSrc != MOYE_BF16) return launch_transpose_cvt_pair<kSrc, MOYE_BF16, SB, 2>(s, d, lds_, ldd, ni, nj, st, bt); break;
-        case MOYE_F8E4M3: if constexpr (kSrc != MOYE_F8E4M3) return launch_transpose_cvt_pair<kSrc, MOYE_F8E4M3, SB, 1>(s, d, lds_, ldd, ni, nj, st, bt); break;
-        case MOYE_F64: if constexpr (kSrc != MOYE_F64) return launch_transpose_cvt_pair<kSrc, MOYE_F64, SB, 8>(s, d, lds_, ldd, ni, nj, st, bt); break;
-        default: break;
-    }
-    return fail(MOYE_ERR_UNSUPPORTED, "copyto!: no conversion between these element types");
-}
-// bt: the strides (in elements) of one or two modes that count matrices, source and destination, and their extents
-// {bs_src, bs_dst, bz_src, bz_dst, batch, batch2}; {0, 0, 0, 0, 1, 1} for one matrix
-static int32_t launch_transpose_cvt(int32_t sd, int32_t dd, const char* s, char* d, int64_t lds_, int64_t ldd, int64_t ni, int64_t nj, hipStream_t st,
-                                    const int64_t (&bt)[6]) {
-    switch (sd) {
-        case MOYE_F32: return launch_transpose_cvt_dst<MOYE_F32, 4>(dd, s, d, lds_, ldd, ni, nj, st, bt);
-        case MOYE_F16: return launch_transpose_cvt_dst<MOYE_F16, 2>(dd, s, d, lds_, ldd, ni, nj, st, bt);
-        case MOYE_BF16: return launch_transpose_cvt_dst<MOYE_BF16, 2>(dd, s, d, lds_, ldd, ni, nj, st, bt);
-        case MOYE_F8E4M3: return launch_transpose_cvt_dst<MOYE_F8E4M3, 1>(dd, s, d, lds_, ldd, ni, nj, st, bt);
-        case MOYE_F64: return launch_transpose_cvt_dst<MOYE_F64, 8>(dd, s, d, lds_, ldd, ni, nj, st, bt);
-        default: return fail(MOYE_ERR_UNSUPPORTED, "copyto!: no conversion between these element types");
-    }
-}
-
 template <int kSrc>
 static bool launch_cvt_dst(int32_t dd, dim3 g, hipStream_t st, const char* s, char* d, FlatLayout ls,
                            FlatLayout ld, int64_t n, int sb, int db, const Mask& mk) {
@@ -1192,238 +550,32 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
             MOYE_HIP_CHECK(hipGetLastError());
             return MOYE_OK;
         }
-        // whole tiles of an aligned matrix (or of `batch` such matrices bs / bd elements apart) through the LDS kernels
-        auto tiled_launch = [&](const char* s_, char* d_, int64_t ni, int64_t nj, int64_t lds_, int64_t ldd, int64_t bs, int64_t bd,
-                                int batch, int64_t bs2 = 0, int64_t bd2 = 0, int batch2 = 1) -> int32_t {
-            const int tile_j = sb == 1 ? kTileJ8 : sb == 8 ? kTileJ64 : kTile;
-            const int ti = (int)(ni / kTile), tj = (int)(nj / tile_j);
-            if (sb == 8)
-                return launch_transpose64_rows(reinterpret_cast<const uint64_t*>(s_), reinterpret_cast<uint64_t*>(d_), lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            if (sb == 1) {
-                const uint8_t* s8 = reinterpret_cast<const uint8_t*>(s_);
-                uint8_t* d8 = reinterpret_cast<uint8_t*>(d_);
-                // whole 256-byte runs on both sides, destination rows first (measured, TB/s, the 64-byte-piece kernel in
-                // super-block order / this one: 16384^2 2.91 / 4.82, 32768^2 3.20 / 5.89, 8192^2 3.29 / 4.94, 32768 x 4096
-                // 3.32 / 5.70, 4096 x 32768 3.46 / 4.99, 65536 x 16384 3.09 / 6.12; this one in super-block order 4.35-5.05)
-                if (ti % 4 == 0) return launch_transpose8_wide(s8, d8, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                if (ti % 2 == 0) return launch_transpose8<2>(s8, d8, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                return launch_transpose8<1>(s8, d8, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            }
-            if (sb == 2) {
-                const uint16_t* s16 = reinterpret_cast<const uint16_t*>(s_);
-                uint16_t* d16 = reinterpret_cast<uint16_t*>(d_);
-                // measured, TB/s, source-first / destination-first: 16384^2 5.32 / 5.75, 4096^2 x 16 6.25 / 6.47, 32768 x 4096
-                // 4.07 / 6.10; 2048^2 x 64 5.83 / 5.18, 4096 x 32768 5.65 / 4.46
-                if (tj % 8 == 0 && ni >= nj && ni >= 3072)
-                    return launch_transpose16_rows<8>(s16, d16, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                if (ti % 8 == 0) return launch_transpose16<8>(s16, d16, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                if (ti % 4 == 0) return launch_transpose16<4>(s16, d16, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                if (ti % 2 == 0) return launch_transpose16<2>(s16, d16, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-                return launch_transpose16<1>(s16, d16, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            }
-            const uint32_t* s32 = reinterpret_cast<const uint32_t*>(s_);
-            uint32_t* d32 = reinterpret_cast<uint32_t*>(d_);
-            if (tc && (tc->flags & MOYE_GEMM_NO_LDS_SWIZZLE)) return launch_transpose<false, 1>(s32, d32, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            // Destination rows first (transpose_lds_b32_rows) when the source's contiguous extent is at least the destination's
-            // and 2048 or more; measured, TB/s, source-first / destination-first order: 16384^2 5.68 / 6.25, 12288^2 5.20 / 5.94,
-            // 4096^2 x 16 5.81 / 6.02, 2048^2 x 64 6.30 / 6.48, 32768 x 4096 4.33 / 6.39; the other way round 4096 x 32768
-            // 5.58 / 5.08, 2048 x 65536 5.77 / 4.52, 1024^2 x 128 6.03 / 5.86.
-            if (tj % 4 == 0 && ni >= nj && ni >= 2048)
-                return launch_transpose_rows<4>(s32, d32, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            if (ti % 4 == 0) return launch_transpose<true, 4>(s32, d32, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            if (ti % 2 == 0) return launch_transpose<true, 2>(s32, d32, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-            return launch_transpose<true, 1>(s32, d32, lds_, ldd, ti, tj, st, bs, bd, batch, bs2, bd2, batch2);
-        };
-        // (2) rank-2 transpose of 1-, 2- and 4-byte elements through LDS patches
-        bool lds_pair = false;  // a rank-2 pair with the unit strides on different modes: what the LDS-tiled op is for
+        // (2) the unit strides on different modes: a transpose, or a batch of them.
         // The tiler of the descriptor (tiler_MN of make_tiled_copy, src/atom/copy.jl:249-258; 32 x 32 in the reference's own
         // transpose kernel, test/host/copy_async.jl:51-76) must divide the array, as zipped_divide asserts; how the kernels
-        // group elements into LDS patches (64 x 64, several per workgroup) is their own business and changes no result.
+        // group elements into LDS tiles is their own business and changes no result.
         if (tc && tc->op == MOYE_COPY_LDS_TILED && src->rank >= 2) {
             for (int m = 0; m < 2; ++m)
                 if (tc->tiler_mn[m] < 0 || (tc->tiler_mn[m] > 0 && src->shape[m] % tc->tiler_mn[m]))
                     return fail(MOYE_ERR_SHAPE, "copyto!: tiler extent %d does not divide mode %d of size %lld", tc->tiler_mn[m], m + 1,
                                 (long long)src->shape[m]);
         }
-        if ((sb == 8 || sb == 4 || sb == 2 || sb == 1) && src->rank == 2 && dst->rank == 2 && src->shape[0] == dst->shape[0] &&
-            src->shape[1] == dst->shape[1]) {
-            const moye_tensor *a = src, *b = dst;
-            bool ok = false, swap = false;
-            if (a->stride[0] == 1 && b->stride[1] == 1) ok = true;
-            else if (a->stride[1] == 1 && b->stride[0] == 1) ok = swap = true;
-            lds_pair = ok;
-            if (ok) {
-                // normalise to: i = contiguous index of src, j = contiguous index of dst
-                const int mi = swap ? 1 : 0, mj = swap ? 0 : 1;
-                const int64_t ni = a->shape[mi], nj = a->shape[mj];
-                const int64_t lds_ = a->stride[mj], ldd = b->stride[mi];
-                const int per16 = 16 / sb;  // elements per 16-byte access
-                const int tile_j = sb == 1 ? kTileJ8 : sb == 8 ? kTileJ64 : kTile;  // extent of a tile along the destination's contiguous index
-                const bool aligned = ni % kTile == 0 && nj % tile_j == 0 && lds_ % per16 == 0 && ldd % per16 == 0 &&
-                                     lds_ >= ni && ldd >= nj &&
-                                     (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0;
-                if (aligned) return tiled_launch(s, d, ni, nj, lds_, ldd, 0, 0, 1);
-                // Sizes that are not multiples of the tile (everything else in order): the interior goes through the
-                // LDS tiles, the two strips that are left through the general kernel.  Three launches, disjoint parts.  (A strip
-                // touches one page per row of the other side, so it costs far more per byte than the interior: 16400 x 16392
-                // fp32 runs at 3.3 TB/s against 5.6 for 16384 x 16384; whole tiles pushed against the edge cost the same.)
-                const int64_t ni0 = ni / kTile * kTile, nj0 = nj / tile_j * tile_j;
-                if (ni0 > 0 && nj0 > 0 && lds_ % per16 == 0 && ldd % per16 == 0 &&
-                    lds_ >= ni && ldd >= nj && (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0) {
-                    // sub-array [i0, i0 + ci) x [j0, j0 + cj) of both sides
-                    auto part = [&](int64_t i0, int64_t ci, int64_t j0, int64_t cj) -> int32_t {
-                        if (ci == 0 || cj == 0) return MOYE_OK;
-                        moye_tensor ps = *src, pd = *dst;
-                        for (moye_tensor* t : {&ps, &pd}) {
-                            t->ptr = static_cast<char*>(t->ptr) + (i0 * t->stride[mi] + j0 * t->stride[mj]) * sb;
-                            t->shape[mi] = ci;
-                            t->shape[mj] = cj;
-                        }
-                        // the strips are not whole patches: they go through the general kernel whatever the descriptor says
-                        const bool interior = i0 == 0 && j0 == 0 && ci == ni0 && cj == nj0;
-                        return copy_if_dispatch(interior ? tc : nullptr, &pd, &ps, nullptr, st);
-                    };
-                    if (int32_t e = part(0, ni0, 0, nj0)) return e;
-                    if (int32_t e = part(ni0, ni - ni0, 0, nj)) return e;
-                    return part(0, ni0, nj0, nj - nj0);
-                }
-            }
-        }
-        // (2b) a batch of such transposes: arrays of one shape, rank above two, the unit strides of the two sides on
-        // different modes of 64 and more; every other mode counts matrices.  One launch with the matrix index in the
-        // grid when there are one or two such modes and the matrices are whole aligned tiles; else one rank-2 call per matrix while
-        // the matrices are large enough to fill the chip on their own and few enough for the launches not to matter
-        // (64 fp32 matrices of 2048 x 2048: 1.5 TB/s through the general kernel, which reads one side in single
-        // elements a pitch apart).
-        if ((sb == 8 || sb == 4 || sb == 2 || sb == 1) && src->rank == dst->rank && src->rank > 2) {
-            const int r = src->rank;
-            bool same = true;
-            int mi = -1, mj = -1;
-            for (int m = 0; m < r; ++m) {
-                same = same && src->shape[m] == dst->shape[m];
-                if (src->shape[m] > 1 && src->stride[m] == 1 && mi < 0) mi = m;
-                if (dst->shape[m] > 1 && dst->stride[m] == 1 && mj < 0) mj = m;
-            }
-            if (same && mi >= 0 && mj >= 0 && mi != mj && src->shape[mi] >= kTile && src->shape[mj] >= kTile) {
-                const int64_t per = src->shape[mi] * src->shape[mj], batch = n / per;
-                // one or two batch modes, whole aligned tiles: one launch, the matrix indices in the grid
-                // (fp16 [16, 2048, 32, 128] -> [16, 32, 128, 2048], 512 matrices in two modes: 1645 us as 512 launches)
-                int bm[2] = {-1, -1}, nbatch_modes = 0;
-                for (int m = 0; m < r; ++m)
-                    if (m != mi && m != mj && src->shape[m] > 1) {
-                        if (nbatch_modes < 2) bm[nbatch_modes] = m;
-                        ++nbatch_modes;
-                    }
-                if (nbatch_modes == 1 || nbatch_modes == 2) {
-                    const int64_t ni = src->shape[mi], nj = src->shape[mj], lds_ = src->stride[mj], ldd = dst->stride[mi];
-                    const int per16 = 16 / sb, tile_j = sb == 1 ? kTileJ8 : sb == 8 ? kTileJ64 : kTile;
-                    bool fits = ni % kTile == 0 && nj % tile_j == 0 && lds_ % per16 == 0 && ldd % per16 == 0 && lds_ >= ni && ldd >= nj &&
-                                (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0;
-                    for (int b = 0; b < nbatch_modes; ++b)
-                        fits = fits && src->shape[bm[b]] <= 65535 && src->stride[bm[b]] % per16 == 0 && dst->stride[bm[b]] % per16 == 0;
-                    if (fits) {
-                        const bool two = nbatch_modes == 2;
-                        return tiled_launch(s, d, ni, nj, lds_, ldd, src->stride[bm[0]], dst->stride[bm[0]], (int)src->shape[bm[0]],
-                                            two ? src->stride[bm[1]] : 0, two ? dst->stride[bm[1]] : 0, two ? (int)src->shape[bm[1]] : 1);
-                    }
-                }
-                if (batch <= 4096 && per * sb >= (128 << 10)) {
-                    moye_tensor ps = *src, pd = *dst;
-                    ps.rank = pd.rank = 2;
-                    ps.shape[0] = pd.shape[0] = src->shape[mi];
-                    ps.shape[1] = pd.shape[1] = src->shape[mj];
-                    ps.stride[0] = src->stride[mi]; ps.stride[1] = src->stride[mj];
-                    pd.stride[0] = dst->stride[mi]; pd.stride[1] = dst->stride[mj];
-                    int64_t idx[MOYE_MAX_RANK] = {0};
-                    for (int64_t b = 0; b < batch; ++b) {
-                        int64_t so = 0, dof = 0;
-                        for (int m = 0; m < r; ++m)
-                            if (m != mi && m != mj) { so += idx[m] * src->stride[m]; dof += idx[m] * dst->stride[m]; }
-                        ps.ptr = const_cast<char*>(s) + so * sb;
-                        pd.ptr = d + dof * sb;
-                        if (int32_t e = copy_if_dispatch(tc, &pd, &ps, nullptr, st)) return e;
-                        for (int m = 0; m < r; ++m) {  // next matrix, first mode fastest
-                            if (m == mi || m == mj) continue;
-                            if (++idx[m] < src->shape[m]) break;
-                            idx[m] = 0;
-                        }
-                    }
-                    return MOYE_OK;
-                }
-            }
-        }
-        // a pair the LDS-tiled op is meant for, but smaller than a patch or not 16-byte aligned: the general kernel moves it
+        TransposeArgs ta;
+        if (transpose_plan(*src, *dst, true, &ta))
+            return transpose_run(src->dtype, dst->dtype, true, tc && (tc->flags & MOYE_GEMM_NO_LDS_SWIZZLE), device_shape().xcds, ta, st);
+        // a pair the LDS-tiled op is meant for, but with too few elements along a side: the general kernel moves it
+        const bool lds_pair = sb <= 8 && src->rank == 2 && dst->rank == 2 && src->shape[0] == dst->shape[0] && src->shape[1] == dst->shape[1] &&
+                              ((src->stride[0] == 1 && dst->stride[1] == 1) || (src->stride[1] == 1 && dst->stride[0] == 1));
         if (tc && tc->op == MOYE_COPY_LDS_TILED && !lds_pair)
             return fail(MOYE_ERR_UNSUPPORTED,
                         "copyto!: the LDS-tiled copy takes rank-2 operands (or a batch of them) of 1-, 2- or 4-byte elements "
                         "with the unit stride on different modes");
     }
 
-    // (2c) a transpose that converts: a rank-2 pair of one shape, floating-point types that differ, the unit strides on
-    // different modes.  Whole aligned tiles through transpose_cvt_lds; other sizes as an interior of whole tiles plus two
-    // strips for the general kernel (8192^2 f32 -> f16: 294 us through the general kernel, which reads one side in single
-    // elements a pitch apart).
-    if (!same_bits && !mask && src->rank == 2 && dst->rank == 2 && src->shape[0] == dst->shape[0] && src->shape[1] == dst->shape[1] &&
-        is_float_dtype(src->dtype) && is_float_dtype(dst->dtype) && !(tc && tc->op == MOYE_COPY_LDS_TILED && (tc->tiler_mn[0] || tc->tiler_mn[1]))) {
-        int mi = -1;
-        if (src->stride[0] == 1 && dst->stride[1] == 1) mi = 0;
-        else if (src->stride[1] == 1 && dst->stride[0] == 1) mi = 1;
-        if (mi >= 0) {
-            const int mj = 1 - mi;
-            const int64_t ni = src->shape[mi], nj = src->shape[mj], lds_ = src->stride[mj], ldd = dst->stride[mi];
-            const int ti = cvt_tile_i(sb), tj = cvt_tile_j(db);
-            const bool lines = (lds_ * sb) % 16 == 0 && (ldd * db) % 16 == 0 && lds_ >= ni && ldd >= nj &&
-                               (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0;
-            if (lines && ni % ti == 0 && nj % tj == 0) return launch_transpose_cvt(src->dtype, dst->dtype, s, d, lds_, ldd, ni, nj, st, {0, 0, 0, 0, 1, 1});
-            const int64_t ni0 = ni / ti * ti, nj0 = nj / tj * tj;
-            if (lines && ni0 > 0 && nj0 > 0) {
-                auto part = [&](int64_t i0, int64_t ci, int64_t j0, int64_t cj) -> int32_t {
-                    if (ci == 0 || cj == 0) return MOYE_OK;
-                    moye_tensor ps = *src, pd = *dst;
-                    ps.ptr = static_cast<char*>(ps.ptr) + (i0 * ps.stride[mi] + j0 * ps.stride[mj]) * sb;
-                    pd.ptr = static_cast<char*>(pd.ptr) + (i0 * pd.stride[mi] + j0 * pd.stride[mj]) * db;
-                    ps.shape[mi] = pd.shape[mi] = ci;
-                    ps.shape[mj] = pd.shape[mj] = cj;
-                    return copy_if_dispatch(nullptr, &pd, &ps, nullptr, st);
-                };
-                if (int32_t e = part(0, ni0, 0, nj0)) return e;
-                if (int32_t e = part(ni0, ni - ni0, 0, nj)) return e;
-                return part(0, ni0, nj0, nj - nj0);
-            }
-        }
-    }
-
-    // (2d) a batch of such converting transposes, counted by one or two modes (NCHW f32 -> NHWC f16 after H and W have
-    // become one mode): whole aligned tiles, one launch
-    if (!same_bits && !mask && src->rank == dst->rank && src->rank > 2 && is_float_dtype(src->dtype) && is_float_dtype(dst->dtype) &&
-        !(tc && tc->op == MOYE_COPY_LDS_TILED && (tc->tiler_mn[0] || tc->tiler_mn[1]))) {
-        const int r = src->rank;
-        bool same = true;
-        int mi = -1, mj = -1;
-        for (int m = 0; m < r; ++m) {
-            same = same && src->shape[m] == dst->shape[m];
-            if (src->shape[m] > 1 && src->stride[m] == 1 && mi < 0) mi = m;
-            if (dst->shape[m] > 1 && dst->stride[m] == 1 && mj < 0) mj = m;
-        }
-        if (same && mi >= 0 && mj >= 0 && mi != mj) {
-            int bm[2] = {-1, -1}, nb = 0;
-            for (int m = 0; m < r; ++m)
-                if (m != mi && m != mj && src->shape[m] > 1) {
-                    if (nb < 2) bm[nb] = m;
-                    ++nb;
-                }
-            const int64_t ni = src->shape[mi], nj = src->shape[mj], lds_ = src->stride[mj], ldd = dst->stride[mi];
-            bool fits = (nb == 1 || nb == 2) && ni % cvt_tile_i(sb) == 0 && nj % cvt_tile_j(db) == 0 && (lds_ * sb) % 16 == 0 && (ldd * db) % 16 == 0 &&
-                        lds_ >= ni && ldd >= nj && (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0;
-            for (int b = 0; fits && b < nb; ++b)
-                fits = src->shape[bm[b]] <= 65535 && (src->stride[bm[b]] * sb) % 16 == 0 && (dst->stride[bm[b]] * db) % 16 == 0;
-            if (fits) {
-                const bool two = nb == 2;
-                return launch_transpose_cvt(src->dtype, dst->dtype, s, d, lds_, ldd, ni, nj, st,
-                                            {src->stride[bm[0]], dst->stride[bm[0]], two ? src->stride[bm[1]] : 0, two ? dst->stride[bm[1]] : 0,
-                                             src->shape[bm[0]], two ? src->shape[bm[1]] : 1});
-            }
-        }
+    // (2b) the same with a conversion on the way
+    if (!same_bits && !mask && !(tc && tc->op == MOYE_COPY_LDS_TILED && (tc->tiler_mn[0] || tc->tiler_mn[1]))) {
+        TransposeArgs ta;
+        if (transpose_plan(*src, *dst, false, &ta)) return transpose_run(src->dtype, dst->dtype, false, false, device_shape().xcds, ta, st);
     }
 
     // (3) generic

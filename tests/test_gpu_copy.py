@@ -1077,3 +1077,32 @@ def test_more_than_16_gib_in_one_call(mh):
     mh.copyto_(_tens(mh, h, [n], [1]), _tens(mh, xf, [n], [1]))
     torch.cuda.synchronize()
     assert bool((h.view(rows, cols) == (pat[None, :] % 1024).half()).all())
+
+
+@pytest.mark.parametrize("pair", ["uint8", "int16", "int32", "int64", "float32->bfloat16", "bfloat16->float32", "float32->float8_e4m3fn",
+                                  "bfloat16->float8_e4m3fn", "float8_e4m3fn->float16", "float64->float16", "float16->float64"])
+def test_transposes_at_the_edges_of_their_tiles(mh, pair):
+    """Extents around 16-byte pieces, tiles and the sizes where the tile changes; pitches and pointers that are aligned to
+    an element only; a mode that counts matrices.  Everything outside the destination's elements stays untouched."""
+    from moye_hip.torch_interop import tensor_of
+    sdt, ddt = [getattr(torch, x) for x in (pair.split("->") * 2)[:2]]
+    seen = 0
+    for ni, nj, batch, extra in [(32, 32, 1, 0), (33, 47, 3, 1), (63, 129, 2, 0), (64, 128, 2, 8), (65, 127, 1, 3), (129, 513, 2, 1), (257, 1025, 1, 0),
+                                 (49, 256, 5, 0), (256, 49, 5, 0), (1031, 33, 2, 5), (1601, 1603, 1, 2), (2304, 2048, 1, 0), (3001, 3003, 1, 1),
+                                 (4096, 2304, 1, 0)]:
+        lds, ldd, off = ni + extra, nj + extra, 1 if extra else 0
+        ns, nd = off + batch * nj * lds, off + batch * ni * ldd
+        g = torch.Generator(device="cuda").manual_seed(ni * 7 + nj)
+        if sdt.is_floating_point:
+            src = (torch.randn(ns, generator=g, device="cuda") * 8).to(sdt)
+        else:
+            src = torch.randint(0, 255, (ns * sdt.itemsize,), generator=g, device="cuda", dtype=torch.uint8).view(sdt)
+        dst = torch.full((nd * ddt.itemsize,), 0x5A, dtype=torch.uint8, device="cuda").view(ddt)
+        want = dst.clone()
+        want.as_strided((batch, ni, ldd), (ni * ldd, ldd, 1), off)[:, :, :nj] = \
+            src.as_strided((batch, nj, lds), (nj * lds, lds, 1), off)[:, :, :ni].transpose(1, 2).to(ddt)
+        mh.copyto_(tensor_of(dst[off:], (ni, nj, batch), (ldd, 1, ni * ldd)), tensor_of(src[off:], (ni, nj, batch), (1, lds, nj * lds)))
+        torch.cuda.synchronize()
+        assert torch.equal(dst.view(torch.uint8), want.view(torch.uint8)), (pair, ni, nj, batch, extra)
+        seen += 1
+    assert seen == 14
