@@ -164,8 +164,14 @@ struct ElF16 {
     typedef float compute;
     typedef _Float16 storage;
     static __device__ __forceinline__ float load(const _Float16* p) { return (float)*p; }
-    static __device__ __forceinline__ void store(_Float16* p, float v) { *p = (_Float16)v; }
-    static __device__ __forceinline__ float round(float v) { return (float)(_Float16)v; }
+    static __device__ __forceinline__ void store(_Float16* p, float v) { *p = narrow(v); }
+    static __device__ __forceinline__ float round(float v) { return (float)narrow(v); }
+    // (the value is made opaque first: a product the compiler can see goes through v_fma_mixlo_f16 with an addend of +0,
+    // which turns a product of -0 into +0)
+    static __device__ __forceinline__ _Float16 narrow(float v) {
+        asm("" : "+v"(v));
+        return (_Float16)v;
+    }
 };
 struct ElBF16 {
     typedef float compute;
@@ -250,74 +256,211 @@ __global__ __launch_bounds__(256) void fill_kernel(char* x, ELayout lx, int64_t 
 }
 
 // ---- dense fast path ------------------------------------------------------------------------------------------
-// When every array of a call is one run in logical order (compact column-major after dropping size-1 modes) and
-// 16-byte aligned, logical index = memory index on all sides: 16 bytes per lane, one access per operand and lane, one
-// workgroup per 4 KiB, no loop and no index arithmetic.  (Measured on 1 GiB arrays, a + b -> d: this form 6.4 TB/s with
-// non-temporal accesses, 6.0 without; workgroups that loop over chunks with four accesses of a lane in flight 5.5-6.1
-// whatever the grid; a fill 6.9 TB/s in this form with ordinary stores, 4.8-5.9 looping.)  The per-element arithmetic
-// is the same code as in the general kernels.
+// When every array of a call is one run in logical order (compact column-major after dropping size-1 modes), logical
+// index = memory index on all sides: 16 bytes per lane, one access per operand and lane, one workgroup per 4 KiB, no loop
+// and no index arithmetic; the lane behind the last whole piece takes what is left element by element.  (Measured on
+// 1 GiB arrays, a + b -> d: this form 6.4 TB/s with non-temporal accesses, 6.0 without; workgroups that loop over chunks
+// with four accesses of a lane in flight 5.5-6.1 whatever the grid; a fill 6.9 TB/s in this form with ordinary stores,
+// 4.8-5.9 looping.)  The per-element arithmetic gives the general kernels' bits, two elements at a time for the 16-bit
+// types, and the operation is a template argument: chosen once per element at run time, with a NaN test per bf16
+// rounding, a lane's eight elements were some 300 instructions and those set the pace beside memory.  bf16 4096 x 3000 (49 or
+// 74 MB), us before -> now: a vector added to every column 79.8 (the element-wise kernel: 64-bit divisions, 2-byte accesses)
+// -> 10.1, max with a scalar 11.9 -> 9.8, axpby! 14.6 -> 13.5; 1001 x 700, no whole number of pieces: map 7.1 -> 2.8, axpby! 6.3 -> 2.9.
 template <typename El>
 struct DenseVec {
     typedef typename El::storage S;
     static constexpr int N = 16 / (int)sizeof(S);
     typedef S type __attribute__((ext_vector_type(N)));
 };
+// a 16-byte access of an array that is only aligned to its elements
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 
-template <typename El>
-__global__ __launch_bounds__(256) void axpby_dense_kernel(typename El::compute a, const typename El::storage* x,
-                                                          typename El::compute b, typename El::storage* y, int64_t nvec,
-                                                          bool b_is_zero) {
-    typedef typename El::compute T;
-    typedef typename El::storage S;
-    typedef typename DenseVec<El>::type vec;
-    constexpr int N = DenseVec<El>::N;
-    const vec* xv = reinterpret_cast<const vec*>(x);
-    vec* yv = reinterpret_cast<vec*>(y);
-    auto one = [&](const vec& vx, const vec& vy) {
-        vec r;
+// 16 bytes <-> values of the compute type.  pack: rounded to T (a bf16 NaN that an operation made is quiet, and the
+// conversion keeps its bits as e_bf16_round does); pack_exact: values that are T's already.
+template <typename El> struct Piece;
+template <> struct Piece<ElF32> {
+    static __device__ __forceinline__ void unpack(const u32x4& w, float (&x)[4]) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            S ex = vx[k], ey = vy[k], er;
-            const T ax = El::round(a * El::load(&ex));
-            if (b_is_zero) El::store(&er, ax);
-            else El::store(&er, El::round(ax + El::round(b * El::load(&ey))));
-            r[k] = er;
+        for (int k = 0; k < 4; ++k) x[k] = __uint_as_float(w[k]);
+    }
+    static __device__ __forceinline__ u32x4 pack(const float (&x)[4]) {
+        return u32x4{__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]), __float_as_uint(x[3])};
+    }
+    static __device__ __forceinline__ u32x4 pack_exact(const float (&x)[4]) { return pack(x); }
+};
+template <> struct Piece<ElF64> {
+    static __device__ __forceinline__ void unpack(const u32x4& w, double (&x)[2]) { __builtin_memcpy(x, &w, 16); }
+    static __device__ __forceinline__ u32x4 pack(const double (&x)[2]) {
+        u32x4 w;
+        __builtin_memcpy(&w, x, 16);
+        return w;
+    }
+    static __device__ __forceinline__ u32x4 pack_exact(const double (&x)[2]) { return pack(x); }
+};
+template <> struct Piece<ElF16> {
+    static __device__ __forceinline__ void unpack(const u32x4& w, float (&x)[8]) {
+        const f16x8 h = (f16x8)w;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = (float)h[k];
+    }
+    static __device__ __forceinline__ u32x4 pack(const float (&x)[8]) {
+        f16x8 h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = ElF16::narrow(x[k]);
+        return (u32x4)h;
+    }
+    static __device__ __forceinline__ u32x4 pack_exact(const float (&x)[8]) { return pack(x); }
+};
+template <> struct Piece<ElBF16> {
+    static __device__ __forceinline__ void unpack(const u32x4& w, float (&x)[8]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[2 * k] = __uint_as_float(w[k] << 16);
+            x[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
         }
-        return r;
-    };
-    const int64_t i = flat_piece();
-    if (i >= nvec) return;
-    const vec vx = __builtin_nontemporal_load(xv + i);
-    __builtin_nontemporal_store(one(vx, b_is_zero ? vx : __builtin_nontemporal_load(yv + i)), yv + i);
+    }
+    static __device__ __forceinline__ u32x4 pack(const float (&x)[8]) {
+        bf16x8 h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = (__bf16)x[k];
+        return (u32x4)h;
+    }
+    static __device__ __forceinline__ u32x4 pack_exact(const float (&x)[8]) {
+        u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_perm(__float_as_uint(x[2 * k + 1]), __float_as_uint(x[2 * k]), 0x07060302u);
+        return w;
+    }
+};
+
+template <typename El, bool kZero /* b is zero: y is not read */>
+__global__ __launch_bounds__(256) void axpby_dense_kernel(typename El::compute a, const typename El::storage* x,
+                                                          typename El::compute b, typename El::storage* y, int64_t n) {
+    typedef typename El::compute T;
+    constexpr int N = DenseVec<El>::N;
+    const int64_t i = flat_piece() * N;
+    if (i + N <= n) {
+        T vx[N], vy[N];
+        u32x4_any* const py = reinterpret_cast<u32x4_any*>(y + i);
+        const u32x4 wx = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(x + i));
+        u32x4 wy;
+        if constexpr (!kZero) wy = __builtin_nontemporal_load(py);
+        __builtin_amdgcn_sched_barrier(0);  // both loads before the arithmetic of either
+        Piece<El>::unpack(wx, vx);
+#pragma unroll
+        for (int k = 0; k < N; ++k) vx[k] = a * vx[k];
+        u32x4 r = Piece<El>::pack(vx);
+        if constexpr (!kZero) {
+            Piece<El>::unpack(r, vx);
+            Piece<El>::unpack(wy, vy);
+#pragma unroll
+            for (int k = 0; k < N; ++k) vy[k] = b * vy[k];
+            Piece<El>::unpack(Piece<El>::pack(vy), vy);
+#pragma unroll
+            for (int k = 0; k < N; ++k) vx[k] = vx[k] + vy[k];
+            r = Piece<El>::pack(vx);
+        }
+        __builtin_nontemporal_store(r, py);
+        return;
+    }
+#pragma unroll 1
+    for (int64_t q = i; q < n; ++q) {
+        const T ax = El::round(a * El::load(x + q));
+        if constexpr (kZero) El::store(y + q, ax);
+        else El::store(y + q, El::round(ax + El::round(b * El::load(y + q))));
+    }
 }
 
-template <typename El>
-__global__ __launch_bounds__(256) void map_dense_kernel(int32_t op, typename El::storage* d, const typename El::storage* a,
-                                                        const typename El::storage* b, typename El::compute s, int64_t nvec) {
+// max / min of values without a NaN among a wave's: the instruction orders the zeros as Julia does (-0.0 < +0.0); with
+// one, Julia's rules spelled out
+template <int OP, typename T, int N>
+__device__ __forceinline__ void map_piece(T (&x)[N], const T (&y)[N]) {
+    if constexpr ((OP == MOYE_MAP_MAX || OP == MOYE_MAP_MIN) && sizeof(T) == 4) {
+        bool nan = false;
+#pragma unroll
+        for (int k = 0; k < N; ++k) nan |= __builtin_isunordered(x[k], y[k]);
+        if (__builtin_amdgcn_ballot_w64(nan) == 0) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) x[k] = OP == MOYE_MAP_MAX ? __builtin_fmaxf(x[k], y[k]) : __builtin_fminf(x[k], y[k]);
+            return;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) x[k] = map_op<T>(OP, x[k], y[k]);
+}
+// the second operand: a scalar (or none), an array like d, one of nb elements that repeats in whole pieces, or one of nb
+// elements that repeats anywhere
+enum { kScalar, kArray, kRepeatPieces, kRepeat };
+template <typename El, int OP, int kOperand>
+__global__ __launch_bounds__(256) void map_dense_kernel(typename El::storage* d, const typename El::storage* a,
+                                                        const typename El::storage* b, typename El::compute s, int64_t n, uint32_t nb) {
     typedef typename El::compute T;
-    typedef typename El::storage S;
-    typedef typename DenseVec<El>::type vec;
     constexpr int N = DenseVec<El>::N;
-    const vec* av = reinterpret_cast<const vec*>(a);
-    const vec* bv = reinterpret_cast<const vec*>(b);
-    vec* dv = reinterpret_cast<vec*>(d);
-    auto one = [&](const vec& va, const vec& vb) {
-        vec r;
+    const int64_t piece = flat_piece(), i = piece * N;
+    if (i + N <= n) {
+        // (d may be a or b: every lane reads its own piece before it writes it)
+        const u32x4 wa = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(a + i));
+        u32x4 wb;
+        typename El::storage eb[N];
+        if constexpr (kOperand == kArray) {
+            wb = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(b + i));
+        } else if constexpr (kOperand == kRepeatPieces) {
+            wb = *reinterpret_cast<const u32x4_any*>(b + (int64_t)((uint32_t)piece % (nb / N)) * N);
+        } else if constexpr (kOperand == kRepeat) {
+            uint32_t r = (uint32_t)i % nb;
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                eb[k] = b[r];
+                r = r + 1 == nb ? 0 : r + 1;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load before the arithmetic
+        T x[N], y[N];
+        if constexpr (kOperand == kArray || kOperand == kRepeatPieces) Piece<El>::unpack(wb, y);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            S ea = va[k], eb = vb[k], er;
-            const T x = El::load(&ea);
-            const T y = b ? El::load(&eb) : s;
-            El::store(&er, El::round(map_op(op, x, y)));
-            r[k] = er;
+            if constexpr (kOperand == kScalar) y[k] = s;
+            if constexpr (kOperand == kRepeat) y[k] = El::load(&eb[k]);
         }
-        return r;
-    };
-    const int64_t i = flat_piece();
-    if (i >= nvec) return;
-    // (d may be a or b: every lane reads its own piece before it writes it)
-    const vec va = __builtin_nontemporal_load(av + i);
-    __builtin_nontemporal_store(one(va, b ? __builtin_nontemporal_load(bv + i) : va), dv + i);
+        Piece<El>::unpack(wa, x);
+        map_piece<OP>(x, y);
+        constexpr bool exact = !(OP == MOYE_MAP_ADD || OP == MOYE_MAP_SUB || OP == MOYE_MAP_MUL || OP == MOYE_MAP_DIV);
+        __builtin_nontemporal_store(exact ? Piece<El>::pack_exact(x) : Piece<El>::pack(x), reinterpret_cast<u32x4_any*>(d + i));
+        return;
+    }
+#pragma unroll 1
+    for (int64_t q = i; q < n; ++q) {
+        const T y = kOperand == kScalar ? s : El::load(b + (kOperand == kArray ? q : q % nb));
+        El::store(d + q, El::round(map_op(OP, El::load(a + q), y)));
+    }
+}
+template <typename El, int OP>
+void launch_map_dense_op(typename El::storage* d, const typename El::storage* a, const typename El::storage* b, typename El::compute s, int64_t n,
+                         int64_t nb, hipStream_t st) {
+    constexpr int N = DenseVec<El>::N;
+    const dim3 grid = flat_grid((n + N - 1) / N);
+    constexpr bool unary = OP == MOYE_MAP_IDENTITY || OP == MOYE_MAP_NEG || OP == MOYE_MAP_ABS;
+    if constexpr (!unary) {
+        if (b && nb == n) { map_dense_kernel<El, OP, kArray><<<grid, 256, 0, st>>>(d, a, b, s, n, 0); return; }
+        if (b && nb % N == 0) { map_dense_kernel<El, OP, kRepeatPieces><<<grid, 256, 0, st>>>(d, a, b, s, n, (uint32_t)nb); return; }
+        if (b) { map_dense_kernel<El, OP, kRepeat><<<grid, 256, 0, st>>>(d, a, b, s, n, (uint32_t)nb); return; }
+    }
+    map_dense_kernel<El, OP, kScalar><<<grid, 256, 0, st>>>(d, a, b, s, n, 0);
+}
+template <typename El>
+void launch_map_dense(int32_t op, typename El::storage* d, const typename El::storage* a, const typename El::storage* b, typename El::compute s,
+                      int64_t n, int64_t nb, hipStream_t st) {
+    switch (op) {
+        case MOYE_MAP_ADD: launch_map_dense_op<El, MOYE_MAP_ADD>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_SUB: launch_map_dense_op<El, MOYE_MAP_SUB>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_MUL: launch_map_dense_op<El, MOYE_MAP_MUL>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_DIV: launch_map_dense_op<El, MOYE_MAP_DIV>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_MAX: launch_map_dense_op<El, MOYE_MAP_MAX>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_MIN: launch_map_dense_op<El, MOYE_MAP_MIN>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_NEG: launch_map_dense_op<El, MOYE_MAP_NEG>(d, a, b, s, n, nb, st); break;
+        case MOYE_MAP_ABS: launch_map_dense_op<El, MOYE_MAP_ABS>(d, a, b, s, n, nb, st); break;
+        default: launch_map_dense_op<El, MOYE_MAP_IDENTITY>(d, a, b, s, n, nb, st); break;
+    }
 }
 
 __global__ __launch_bounds__(256) void fill_dense_kernel(u32x4* x, int64_t nvec, u32x4 pattern) {
@@ -679,9 +822,9 @@ static void launch_axpby(typename El::compute a, const void* x, const ELayout& l
         return;
     }
     constexpr int N = DenseVec<El>::N;
-    const int64_t nvec = n / N, tail = n - nvec * N;
-    if (nvec) axpby_dense_kernel<El><<<flat_grid(nvec), 256, 0, st>>>(a, xs, b, ys, nvec, b0);
-    if (tail) axpby_kernel<El><<<1, 64, 0, st>>>(a, xs + nvec * N, run_layout(tail), b, ys + nvec * N, run_layout(tail), tail, b0);
+    const dim3 grid = flat_grid((n + N - 1) / N);
+    if (b0) axpby_dense_kernel<El, true><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
+    else axpby_dense_kernel<El, false><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
 }
 
 template <typename El>
@@ -705,12 +848,7 @@ static void launch_map(int32_t op, void* d, const ELayout& ld, const void* a, co
                                              same_modes_32(ld, la, n) && (!bs || (nb == n && same_modes_32(ld, lb, n))));
         return;
     }
-    constexpr int N = DenseVec<El>::N;
-    const int64_t nvec = n / N, tail = n - nvec * N;
-    if (nvec) map_dense_kernel<El><<<flat_grid(nvec), 256, 0, st>>>(op, ds, as, bs, s, nvec);
-    if (tail)
-        map_kernel<El><<<1, 64, 0, st>>>(op, ds + nvec * N, run_layout(tail), as + nvec * N, run_layout(tail), bs ? bs + nvec * N : nullptr,
-                                         run_layout(tail), tail, s, tail);
+    launch_map_dense<El>(op, ds, as, bs, s, n, nb, st);
 }
 
 int32_t axpby_dispatch(double a, const moye_tensor* X, double b, const moye_tensor* Y, hipStream_t st) {
@@ -721,14 +859,14 @@ int32_t axpby_dispatch(double a, const moye_tensor* X, double b, const moye_tens
     if (count(*Y) != n) return fail(MOYE_ERR_SHAPE, "axpby!: X holds %lld elements, Y %lld", (long long)n, (long long)count(*Y));
     if (n == 0) return MOYE_OK;
     ELayout lx = elayout_of(*X), ly = elayout_of(*Y);
-    bool fast = dense(*X) && dense(*Y) && aligned16(X->ptr) && aligned16(Y->ptr);
+    bool fast = dense(*X) && dense(*Y);
     bool rows = false, ordered = false;  // ordered: the layouts have one shape mode by mode and are sorted by Y's strides
     if (!fast) {
         ELayout* all[2] = {&ly, &lx};
         const void* ptrs[2] = {Y->ptr, X->ptr};
         if (order_modes_by_stride(all, 2)) {
             ordered = true;
-            if (dense_l(lx) && dense_l(ly) && aligned16(X->ptr) && aligned16(Y->ptr)) fast = true;  // one run each, in the same order
+            if (dense_l(lx) && dense_l(ly)) fast = true;  // one run each, in the same order
             else rows = recast_rows(all, ptrs, 2, 16 / dtype_bytes(X->dtype));
         }
     }
@@ -773,15 +911,15 @@ int32_t map_dispatch(int32_t op, const moye_tensor* D, const moye_tensor* A, con
     if (n == 0) return MOYE_OK;
     ELayout ld = elayout_of(*D), la = elayout_of(*A), lb = B ? elayout_of(*B) : ELayout{};
     const void* bp = B ? B->ptr : nullptr;
-    bool fast = dense(*D) && dense(*A) && aligned16(D->ptr) && aligned16(A->ptr) &&
-                (!B || (nb == n && dense(*B) && aligned16(B->ptr)));
+    // (a dense b that repeats over the trailing modes repeats over the run; its pieces are counted with 32 bits)
+    bool fast = dense(*D) && dense(*A) && (!B || (dense(*B) && (nb == n || n < ((int64_t)1 << 32))));
     bool rows = false, ordered = false;
     if (!fast && (!B || nb == n)) {  // (a b that is broadcast is tied to the leading modes of dst as the caller wrote them)
         ELayout* all[3] = {&ld, &la, &lb};
         const void* ptrs[3] = {D->ptr, A->ptr, bp};
         if (order_modes_by_stride(all, B ? 3 : 2)) {
             ordered = true;
-            if (dense_l(ld) && dense_l(la) && (!B || dense_l(lb)) && aligned16(D->ptr) && aligned16(A->ptr) && (!B || aligned16(B->ptr))) fast = true;
+            if (dense_l(ld) && dense_l(la) && (!B || dense_l(lb))) fast = true;
             else rows = recast_rows(all, ptrs, B ? 3 : 2, 16 / dtype_bytes(D->dtype));
         }
     }

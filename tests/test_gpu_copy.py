@@ -1106,3 +1106,55 @@ def test_transposes_at_the_edges_of_their_tiles(mh, pair):
         assert torch.equal(dst.view(torch.uint8), want.view(torch.uint8)), (pair, ni, nj, batch, extra)
         seen += 1
     assert seen == 14
+
+
+@pytest.mark.parametrize("dt", ["float32", "float64", "float16", "bfloat16"])
+def test_dense_maps_give_the_element_wise_kernels_bits(mh, dt):
+    """Arrays that are one run (any length, aligned to an element only; a second operand that is an array, a scalar or a
+    vector that repeats over the trailing mode) against the same values in rows an odd pitch apart, which go element by
+    element: the same bits, NaNs, infinities, signed zeros and subnormals among the values (which NaN an operation makes of
+    two is the instruction's business)."""
+    tdt = getattr(torch, dt)
+    itype = {2: torch.int16, 4: torch.int32, 8: torch.int64}[tdt.itemsize]
+    special = torch.tensor([float("nan"), -float("nan"), float("inf"), -float("inf"), 0.0, -0.0, 1e-40, -1e-40, 6e-8, 3.3895e38, 65504.0], dtype=torch.float64)
+
+    def same(x, y):
+        return bool(((x.view(itype) == y.view(itype)) | (torch.isnan(x) & torch.isnan(y))).all())
+
+    def values(rows, cols, seed, nans):
+        g = torch.Generator().manual_seed(seed)
+        v = torch.randn(cols, rows, generator=g, dtype=torch.float64) * 3
+        at = torch.randint(0, cols * rows, (max(1, cols * rows // 5),), generator=g)
+        v.view(-1)[at] = special[torch.arange(len(at)) % len(special)] if nans else special[4 + torch.arange(len(at)) % (len(special) - 4)]
+        return v.to(tdt).cuda()
+
+    for rows, cols, nans in [(1, 1, True), (7, 9, True), (8, 33, False), (24, 257, True), (1001, 65, False), (1024, 40, True), (3, 100003, False)]:
+        p = rows + 1 + rows % 2  # an odd pitch
+        a, b = values(rows, cols, rows, nans), values(rows, cols, cols, nans)
+        wide = lambda t: torch.nn.functional.pad(t, (0, p - rows))
+        aw, bw = wide(a), wide(b)
+        def dense(t):  # one element off alignment
+            u = torch.zeros(rows * cols + 1, dtype=tdt, device="cuda")
+            u[1:] = t.reshape(-1)
+            return u, _tens(mh, u[1:], (rows, cols), (1, rows))
+        ad, ta = dense(a)
+        bd, tb = dense(b)
+        pitched = lambda t: _tens(mh, t, (rows, cols), (1, p))
+        for op in ("add", "sub", "mul", "div", "max", "min", "neg", "abs", "identity"):
+            for second in ("array", "scalar", "repeat"):
+                dd, td = dense(torch.zeros_like(a))
+                dw = torch.zeros_like(aw)
+                s1 = {"array": tb, "scalar": None, "repeat": _tens(mh, bd[1:], (rows,), (1,))}[second]
+                s2 = {"array": pitched(bw), "scalar": None, "repeat": _tens(mh, bd[1:], (rows,), (1,))}[second]
+                mh.map_(op, td, ta, s1, -1.75)
+                mh.map_(op, pitched(dw), pitched(aw), s2, -1.75)
+                torch.cuda.synchronize()
+                assert same(dd[1:].view(cols, rows), dw[:, :rows].contiguous()), (dt, rows, cols, op, second)
+                assert int(dd[:1].view(itype)) == 0
+        for beta in (0.0, -1.25):
+            yd, ty = dense(b)
+            yw = bw.clone()
+            mh.axpby_(0.75, ta, beta, ty)
+            mh.axpby_(0.75, pitched(aw), beta, pitched(yw))
+            torch.cuda.synchronize()
+            assert same(yd[1:].view(cols, rows), yw[:, :rows].contiguous()), (dt, rows, cols, "axpby", beta)
