@@ -285,6 +285,8 @@ int32_t moye_layout_eval(const char* layout, const char* coord, int64_t* index);
  * went into it is, an Int32 when its dynamic inputs all are, an Int otherwise; Int32 arithmetic wraps modulo 2^32. */
 int32_t moye_layout_eval_typed(const char* layout, const char* coord, char* out, size_t cap);
 int32_t moye_layout_size(const char* layout, int64_t* size);                                 /* layout.jl:302-304 */
+/* flatten(layout) into a descriptor: rank, shape and stride; null pointer, dtype 0 (layout.jl:98-102) */
+int32_t moye_layout_descriptor(const char* layout, moye_tensor* out);
 int32_t moye_layout_cosize(const char* layout, int64_t* cosize);                             /* layout.jl:350-352 */
 int32_t moye_layout_rank_depth(const char* layout, int32_t* rank, int32_t* depth);           /* layout.jl:321-343 */
 int32_t moye_layout_flatten(const char* layout, char* out, size_t cap);                      /* layout.jl:292-294 */

@@ -203,10 +203,12 @@ GemmStep& GemmPlan::add_kernel(void (*kernel)(GemmArgs), const GemmArgs& a, unsi
     st.cap = cap;
     st.tile_m = tile_m; st.tile_n = tile_n; st.tile_k_bytes = tile_k_bytes;
     st.in_dt = in_dt; st.out_dt = out_dt;
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(st.name, sizeof st.name, fmt, ap);
-    va_end(ap);
+    if (named) {
+        va_list ap;
+        va_start(ap, fmt);
+        vsnprintf(st.name, sizeof st.name, fmt, ap);
+        va_end(ap);
+    }
     return st;
 }
 
@@ -318,7 +320,6 @@ static void plan_kmajor_copy(Mat* m, char* ws, GemmPlan& plan) {
     src.shape[0] = m->rows; src.shape[1] = m->cols; src.stride[0] = m->rs; src.stride[1] = m->cs;
     st.copy_dst = src;
     st.copy_dst.ptr = ws; st.copy_dst.stride[0] = pitch_e; st.copy_dst.stride[1] = 1;
-    snprintf(st.name, sizeof st.name, "kmajor_copy");
     m->ptr = ws; m->rs = pitch_e; m->cs = 1;
 }
 
@@ -397,7 +398,7 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         st.uargs = UArgs{A.ptr, B.ptr, tC ? C.ptr : nullptr, D.ptr, M, N, K, A.rs, A.cs, B.rs, B.cs,
                          C.rs, C.cs, D.rs, D.cs, alpha, A.dtype, B.dtype, tC ? C.dtype : D.dtype, D.dtype};
         st.ubm = bm; st.ubn = bn; st.ubk = bk;
-        snprintf(st.name, sizeof st.name, "gemm_universal<%d,%d,%d>", bm, bn, bk);
+        if (plan.named) snprintf(st.name, sizeof st.name, "gemm_universal<%d,%d,%d>", bm, bn, bk);
         return MOYE_OK;
     }
     const int32_t in_dt = atom_input_dtype(mma->atom);
@@ -501,7 +502,6 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         GemmStep& st = plan.steps.back();
         st.kind = GemmStep::kSplitKReduce;
         st.partials = P; st.split = split; st.args = r; st.out_dt = D.dtype; st.in_dt = MOYE_F32;
-        snprintf(st.name, sizeof st.name, "splitk_reduce");
         return MOYE_OK;
     }
     if (D.cs == 1) {  // row-major D
@@ -721,6 +721,7 @@ int32_t moye_gemm_explain(const moye_tiled_mma* mma, const moye_tensor* D, const
     if (!mma || !D || !A || !B || !out || cap == 0) return fail(MOYE_ERR_ARG, "moye_gemm_explain: null argument");
     out[0] = 0;
     GemmPlan plan;
+    plan.named = true;
     plan.shape = device_shape_for(compute_units);
     // the workspace of a plan that is only printed: an address nothing is read from or written to
     auto workspace = [](size_t, char** p) -> int32_t {

@@ -97,6 +97,7 @@ struct GemmPlan {
     DeviceShape shape{256, 8};
     size_t workspace_bytes = 0;  // what the steps use of the workspace (K-major operand copies, then split-K partial products)
     char* workspace = nullptr;   // where it is
+    bool named = false;          // fill in GemmStep::name (a plan that is printed; formatting costs as much as the rest of a plan)
     // appends a kernel launch; `name` is printf-style
     GemmStep& add_kernel(void (*kernel)(GemmArgs), const GemmArgs& a, unsigned grid_x, unsigned grid_y, unsigned block, int lds_bytes,
                          struct LdsCap* cap, int tile_m, int tile_n, int tile_k_bytes, int in_dt, int out_dt, const char* fmt, ...)

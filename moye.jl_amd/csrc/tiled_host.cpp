@@ -498,6 +498,25 @@ int32_t moye_layout_cosize(const char* layout, int64_t* n) {
         return (int32_t)MOYE_OK;
     });
 }
+int32_t moye_layout_descriptor(const char* layout, moye_tensor* out) {
+    MOYE_REQUIRE(layout && out);
+    return guarded([&] {
+        const Layout l = parse_layout(layout);
+        auto leaves = [](const IT& t) { return t.is_leaf() ? std::vector<IT>{t} : t.items; };
+        const std::vector<IT> shape = leaves(flatten(l.shape)), stride = leaves(flatten(l.stride));
+        std::memset(out, 0, sizeof *out);
+        if (shape.size() != stride.size()) throw Error(MOYE_ERR_RANK, "shape and stride must be congruent");
+        if (shape.empty() || shape.size() > MOYE_MAX_RANK)
+            throw Error(MOYE_ERR_RANK, "rank " + std::to_string(shape.size()) + " outside 1.." + std::to_string(MOYE_MAX_RANK));
+        out->rank = (int32_t)shape.size();
+        for (size_t i = 0; i < shape.size(); ++i) {
+            out->shape[i] = shape[i].leaf.v;
+            out->stride[i] = stride[i].leaf.v;
+        }
+        return (int32_t)MOYE_OK;
+    });
+}
+
 int32_t moye_layout_rank_depth(const char* layout, int32_t* r, int32_t* d) {
     MOYE_REQUIRE(layout && r && d);
     return guarded([&] {

@@ -87,6 +87,10 @@ def _declare(l):
         "moye_copy_if": [P(Tensor), P(Tensor), P(Tensor), vp],
         "moye_gemm": [P(TiledMMA), P(Tensor), P(Tensor), P(Tensor), P(Tensor), C.c_float, vp],
         "moye_gemm_ex": [P(TiledMMA), P(Tensor), P(Tensor), P(Tensor), P(Tensor), P(GemmEpilogue), vp, S, vp],
+        "moye_axpby": [C.c_double, P(Tensor), C.c_double, P(Tensor), vp],
+        "moye_fill": [P(Tensor), C.c_double, vp],
+        "moye_map": [I32, P(Tensor), P(Tensor), P(Tensor), C.c_double, vp],
+        "moye_layout_descriptor": [cs, P(Tensor)],
         "moye_gemm_release_workspace": [],
         "moye_gemm_noalloc": [P(TiledMMA), P(Tensor), P(Tensor), P(Tensor), P(Tensor), C.c_float, vp],
         "moye_gemm_workspace_size": [P(TiledMMA), P(Tensor), P(Tensor), P(Tensor), P(S)],

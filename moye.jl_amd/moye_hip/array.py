@@ -2,6 +2,7 @@
 src/array.jl, src/algorithm/array_algorithms.jl, src/atom/{mma,copy}.jl and
 src/algorithm/{copy,blas}.jl of the reference for arrays in device (global) memory."""
 import ctypes as C
+import functools
 
 from . import _lib, device
 from . import layout as L
@@ -45,8 +46,9 @@ class MoYeArray:
 
     def tensor(self):
         """The flattened moye_tensor descriptor handed to the HIP library."""
-        shape, stride = L.flat(self.layout)
-        return _lib.make_tensor(self.ptr, self.dtype, shape, stride, self.memspace)
+        t = _lib.Tensor.from_buffer_copy(self.layout.descriptor())
+        t.ptr, t.dtype, t.memspace = self.ptr, self.dtype, self.memspace
+        return t
 
     def _with(self, layout, offset=0):
         return MoYeArray(self.ptr + offset * self.elsize, self.dtype, layout, self.memspace, self._keep)
@@ -105,6 +107,14 @@ def _emit(text, file):
     return text
 
 
+@functools.lru_cache(maxsize=256)
+def _mma_descriptor(op, atom_layout, permutations):
+    """The bytes of the moye_tiled_mma that an atom, an atom layout and permutations (as text) come to."""
+    d = _lib.TiledMMA()
+    check(_l().moye_make_tiled_mma(op, _b(atom_layout), _b(permutations), C.byref(d)))
+    return bytes(d)
+
+
 class TiledMMA:
     """make_tiled_mma(op, atom_layout, permutations) (src/atom/mma.jl:193-233).  `op` is a
     moye_mma_atom number or an atom name (the reference's NVIDIA atoms exist by name, as data)."""
@@ -160,9 +170,8 @@ class TiledMMA:
         """moye_tiled_mma for the device call."""
         if not isinstance(self.op, int):
             raise MoyeError(_lib.ERR_UNSUPPORTED, "atom %s has no gfx950 kernel" % self.name)
-        d = _lib.TiledMMA()
         perm = "" if self.permutations is None else _tile_text(tuple(self.permutations))
-        check(_l().moye_make_tiled_mma(self.op, _b(self.atom_layout.text), _b(perm), C.byref(d)))
+        d = _lib.TiledMMA.from_buffer_copy(_mma_descriptor(self.op, self.atom_layout.text, perm))
         if self.cta_tile is not None:
             for i in range(3):
                 d.cta_tile_mnk[i] = self.cta_tile[i]
@@ -395,20 +404,22 @@ class ThrCopy:
 
 
 # ---- the algorithms --------------------------------------------------------------------------------
+def _t(x):
+    """The descriptor of an array; raw descriptors (and None) pass straight through."""
+    return x if x is None or isinstance(x, _lib.Tensor) else x.tensor()
+
+
 def copyto_(dst, src, tiled_copy=None, stream=None):
     """copyto!(dst, src) / copyto!(tiled_copy, dst, src) (src/algorithm/copy.jl:42-46,106-110); returns dst."""
     tc = tiled_copy.descriptor() if isinstance(tiled_copy, TiledCopy) else tiled_copy
-    d = dst if isinstance(dst, _lib.Tensor) else dst.tensor()   # raw descriptors pass straight through
-    s = src if isinstance(src, _lib.Tensor) else src.tensor()
-    device.copyto_(d, s, tc, stream)
+    device.copyto_(_t(dst), _t(src), tc, stream)
     return dst
 
 
 def copyto_if_(dst, src, mask, stream=None):
     """copyto_if!(dst, src, mask) (src/algorithm/copy.jl:4-16): element i moves where the mask's element i is true;
     the mask is a MoYeArray of bytes (Bool) with its own layout.  Returns dst."""
-    t = [x if isinstance(x, _lib.Tensor) else x.tensor() for x in (dst, src, mask)]
-    device.copyto_if_(t[0], t[1], t[2], stream)
+    device.copyto_if_(_t(dst), _t(src), _t(mask), stream)
     return dst
 
 
@@ -418,33 +429,25 @@ def gemm_(mma, D, A, B, C_=None, alpha=1.0, stream=None):
     if not isinstance(mma, (TiledMMA, _lib.TiledMMA)):  # gemm!(A, B, C): UniversalFMA
         A, B, C_, D = mma, D, A, A
         mma = TiledMMA(_lib.MMA_UNIVERSAL_FMA)
-    d = mma.descriptor() if isinstance(mma, TiledMMA) else mma
-
-    def t(x):
-        return x if x is None or isinstance(x, _lib.Tensor) else x.tensor()
-
-    device.gemm_(d, t(D), t(A), t(B), t(C_), alpha, stream)
+    device.gemm_(mma.descriptor() if isinstance(mma, TiledMMA) else mma, _t(D), _t(A), _t(B), _t(C_), alpha, stream)
 
 
 def axpby_(a, X, b, Y, stream=None):
     """axpby!(a, X, b, Y) (src/algorithm/blas.jl:1-9): Y = a*X + b*Y element by element; returns Y."""
-    x = X if isinstance(X, _lib.Tensor) else X.tensor()
-    y = Y if isinstance(Y, _lib.Tensor) else Y.tensor()
-    device.axpby_(a, x, b, y, stream)
+    device.axpby_(a, _t(X), b, _t(Y), stream)
     return Y
 
 
 def fill_(X, value, stream=None):
     """fill!(x, value) (src/algorithm/array_algorithms.jl:158-164); returns X."""
-    device.fill_(X if isinstance(X, _lib.Tensor) else X.tensor(), value, stream)
+    device.fill_(_t(X), value, stream)
     return X
 
 
 def map_(op, dst, A, B=None, scalar=0.0, stream=None):
     """dst .= op.(A, B) or op.(A, scalar) (src/broadcast.jl:5-41; map!, src/algorithm/array_algorithms.jl:192-210);
     op is one of "identity", "add", "sub", "mul", "div", "max", "min", "neg", "abs".  Returns dst."""
-    t = lambda x: x if isinstance(x, _lib.Tensor) else x.tensor()
-    device.map_(_lib.MAP_OPS[op] if isinstance(op, str) else op, t(dst), t(A), None if B is None else t(B), scalar, stream)
+    device.map_(_lib.MAP_OPS[op] if isinstance(op, str) else op, _t(dst), _t(A), _t(B), scalar, stream)
     return dst
 
 

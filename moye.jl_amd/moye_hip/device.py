@@ -169,22 +169,16 @@ def mma_atom_probe(atom, a_ptr, b_ptr, d_ptr, stream=None):
 
 def axpby_(a, x, b, y, stream=None):
     """axpby!(a, X, b, Y) on raw descriptors."""
-    f = lib().moye_axpby
-    f.argtypes = [C.c_double, C.c_void_p, C.c_double, C.c_void_p, C.c_void_p]
-    check(f(a, C.byref(x), b, C.byref(y), stream))
+    check(lib().moye_axpby(a, C.byref(x), b, C.byref(y), stream))
 
 
 def fill_(x, value, stream=None):
-    f = lib().moye_fill
-    f.argtypes = [C.c_void_p, C.c_double, C.c_void_p]
-    check(f(C.byref(x), value, stream))
+    check(lib().moye_fill(C.byref(x), value, stream))
 
 
 def map_(op, dst, a, b=None, scalar=0.0, stream=None):
     """dst .= op.(a, b) / op.(a, scalar) on raw descriptors (moye_map)."""
-    f = lib().moye_map
-    f.argtypes = [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double, C.c_void_p]
-    check(f(op, C.byref(dst), C.byref(a), C.byref(b) if b is not None else None, scalar, stream))
+    check(lib().moye_map(op, C.byref(dst), C.byref(a), C.byref(b) if b is not None else None, scalar, stream))
 
 
 def mfma_ceiling(in_dtype, random_operands=True, seconds=0.3, stream=None):

@@ -168,9 +168,10 @@ def _l():
 class Layout:
     """`Layout(shape, stride)` (src/layout.jl:48-59).  Immutable; `.text` is the canonical form."""
 
-    __slots__ = ("text",)
+    __slots__ = ("text", "_descriptor")
 
     def __init__(self, shape, stride=None):
+        self._descriptor = None
         if stride is None and isinstance(shape, str):
             self.text = _text_out(_l().moye_layout_normalize, _b(shape))
         elif stride is None:
@@ -195,6 +196,15 @@ class Layout:
     @property
     def stride(self):
         return parse_tuple(self._split()[1])
+
+    def descriptor(self):
+        """The bytes of a moye_tensor with this layout's rank, shape and stride (null pointer): flattened by the library
+        once, a layout never changes."""
+        if self._descriptor is None:
+            t = _lib.Tensor()
+            check(lib().moye_layout_descriptor(_b(self.text), C.byref(t)))
+            self._descriptor = bytes(t)
+        return self._descriptor
 
     def __repr__(self):
         return self.text

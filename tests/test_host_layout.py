@@ -427,7 +427,7 @@ def test_more_tuple_helpers_against_the_oracle():
     _same(ml.tuple_append(h, ml.StaticInt(1)), lo.append(t, S(1)))
     _same(ml.tuple_append(h, ml.StaticInt(1), 5), lo.append(t, S(1), 5))
     _same(ml.tuple_prepend(h, 9, 4), lo.prepend(t, 9, 4))
-    with pytest.raises(mh.MoyeError):
+    with pytest.raises(MoyeError):
         ml.tuple_append(h, 1, 2)
     z = (((1, 2), (3, 4)), ((5, 6), (7, 8)), (9, 10))
     _same(ml.zip2_by(ml.parse_tuple(_o2t(z)), ml.parse_tuple("((0,0),0)")), lo.zip2_by(z, ((0, 0), 0)))
@@ -572,3 +572,19 @@ def test_int32_random_differential():
                 assert repr(ml.index_to_coord(ml.Int32(i), a.shape, a.stride)) == repr(lo.index_to_coord(lo.I32(i), oa.shape, oa.stride))
         n += 1
     assert n == 300
+
+
+@pytest.mark.parametrize("shape,stride", [((384, 512), (512, 1)), (7, 3), (((2, 3), 4), ((1, 8), 2)), ((1, 1, (2, (3, 4)), 5, 6, 7), (0, 0, (1, (2, 6)), 24, 120, 720))])
+def test_array_descriptor_is_the_flattened_layout(shape, stride):
+    lay = ml.Layout(shape, stride)
+    x = mh.MoYeArray(1 << 20, mh.F16, lay)
+    for _ in range(2):
+        t = x.tensor()
+        s, d = ml.flat(lay)
+        assert (t.ptr, t.dtype, t.memspace, t.rank) == (1 << 20, mh.F16, 0, len(s))
+        assert list(t.shape)[:t.rank] == s and list(t.stride)[:t.rank] == d
+    t.shape[0] = 99  # a caller may edit its descriptor
+    assert x.tensor().shape[0] == s[0]
+    with pytest.raises(MoyeError) as e:
+        mh.MoYeArray(1 << 20, mh.F16, ml.Layout((2,) * 9)).tensor()
+    assert e.value.status == ERR_RANK
