@@ -121,30 +121,7 @@ __global__ __launch_bounds__(256) void gemm_universal_fma(UArgs p) {
         const int kmax = min(BK, p.K - k0);
         const bool more = k0 + BK < p.K;
         if (more) fetch(k0 + BK);  // in flight during the arithmetic below
-        if (kmax == BK && TM * TN <= 4) {
-            // a whole stage of a small thread tile: the fragments of eight k are read from LDS before the first product, so
-            // that one LDS latency is paid per eight k, not per k (there may be a single wave per SIMD to hide it)
-#pragma unroll
-            for (int kb = 0; kb < BK; kb += 8) {
-                float a[8][TM], b[8][TN];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) a[k][i] = sA[kb + k][tx + TX * i];
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) b[k][j] = sB[kb + k][ty + TY * j];
-                }
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            const float prod = round_in<kProd>(__fmul_rn(a[k][i], b[k][j]));
-                            acc[i][j] = round_in<kAcc>(__fadd_rn(prod, acc[i][j]));
-                        }
-            }
-        } else if (kmax == BK) {   // a whole stage: unrolled, so that the LDS reads of later k are in flight under the arithmetic
+        if (kmax == BK) {   // a whole stage: unrolled, so that the LDS reads of later k are in flight under the arithmetic
 #pragma unroll
             for (int k = 0; k < BK; ++k) k_step(k);
         } else {
@@ -171,6 +148,179 @@ __global__ __launch_bounds__(256) void gemm_universal_fma(UArgs p) {
                 u_store(p.D, m * p.sd_m + n * p.sd_n, p.d_dt, v);
             }
         }
+}
+
+// The form for few elements: tiles of 16 TM x 16 TN elements of D, TM x TN to a lane (rows 16 apart), so that a small problem
+// has a workgroup for every CU, and KB k to a stage.  Operands lie in LDS with k contiguous, rows KB + 4 floats apart: a lane's 128-bit read
+// brings four k, sixteen neighbouring lanes read sixteen rows in sixteen different groups of four banks, and the writes
+// (lanes along m or along k, whichever is contiguous in memory) spread over the banks.  Bound by latency at these sizes: a
+// launch, a memory round trip per stage (the next stage's is under way during the arithmetic), K dependent additions.
+// Against 32 x 32 tiles that read LDS value by value and told the types apart per element, us: fp32 256^3 17.4 -> 6.2, 64 x 64
+// x 768 44.9 -> 12.4, 512^3 35.0 -> 21.2, 768^3 63.7 -> 49.4, 1024^3 102 -> 80; fp16 256^3 25.5 -> 7.1, 768^3 111 -> 94.
+// The arithmetic is the kernel's above, element by element.
+// kAny: operands of different types, told apart at run time
+enum { kAny = -1 };
+template <int kDt> struct URaw { typedef float type; };
+template <> struct URaw<MOYE_F16> { typedef _Float16 type; };
+template <> struct URaw<MOYE_BF16> { typedef uint16_t type; };
+template <int kDt>
+__device__ __forceinline__ typename URaw<kDt>::type u_raw(const void* p, int64_t i, int dt) {
+    if constexpr (kDt == kAny) return u_load(p, i, dt);
+    else return static_cast<const typename URaw<kDt>::type*>(p)[i];
+}
+template <int kDt>
+__device__ __forceinline__ float u_widen(typename URaw<kDt>::type v) {
+    if constexpr (kDt == MOYE_BF16) return __uint_as_float((uint32_t)v << 16);
+    else return (float)v;
+}
+template <int TM, int TN, int KB, int kProd, int kAcc, int DA, int DB>
+__global__ __launch_bounds__(256) void gemm_universal_fma_small(UArgs p) {
+    constexpr int BM = 16 * TM, BN = 16 * TN, PITCH = KB + 4;
+    constexpr int DD = kAcc == 1 ? MOYE_F16 : kAcc == 2 ? MOYE_BF16 : MOYE_F32;  // C and D
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float sA[BM * PITCH];
+    __shared__ __align__(16) float sB[BN * PITCH];
+    const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
+    const bool a_kfast = p.sa_k == 1, b_kfast = p.sb_k == 1;
+    constexpr int LA = BM * KB / 256, LB = BN * KB / 256;
+    // element q of this lane in a stage: along k where that is the contiguous index, else along m (n)
+    auto place = [&](bool kfast, int rows, int q, int* row, int* k) {
+        const int idx = tid + 256 * q;
+        *row = kfast ? idx / KB : idx % rows;
+        *k = kfast ? idx % KB : idx / rows;
+    };
+    typename URaw<DA>::type ra[LA];
+    typename URaw<DB>::type rb[LB];
+    // (beyond M, N and K the last element is read again: what is computed from it is not stored or not added)
+    auto fetch = [&](int k0) {
+        const int klast = p.K - 1 - k0;
+#pragma unroll
+        for (int q = 0; q < LA; ++q) {
+            int m, k;
+            place(a_kfast, BM, q, &m, &k);
+            ra[q] = u_raw<DA>(p.A, (int64_t)min(m0 + m, p.M - 1) * p.sa_m + (int64_t)(k0 + min(k, klast)) * p.sa_k, p.a_dt);
+        }
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+            int n, k;
+            place(b_kfast, BN, q, &n, &k);
+            rb[q] = u_raw<DB>(p.B, (int64_t)min(n0 + n, p.N - 1) * p.sb_n + (int64_t)(k0 + min(k, klast)) * p.sb_k, p.b_dt);
+        }
+    };
+    float acc[TM][TN];
+    if (p.K > 0) fetch(0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int m = m0 + tx + 16 * i, n = n0 + ty + 16 * j;
+            acc[i][j] = (p.C && p.alpha == 1.0f && m < p.M && n < p.N) ? u_load(p.C, m * p.sc_m + n * p.sc_n, DD) : 0.0f;
+        }
+    auto fma = [&](const float (&a)[TM], const float (&b)[TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = round_in<kAcc>(__fadd_rn(round_in<kProd>(__fmul_rn(a[i], b[j])), acc[i][j]));
+    };
+    const float* const a0 = sA + tx * PITCH;
+    const float* const b0 = sB + ty * PITCH;
+    // G k-quads in one set of registers
+    constexpr int G = TM * TN == 1 ? 4 : TM * TN <= 4 ? 2 : 1;
+    struct Frag {
+        f32x4 a[G][TM], b[G][TN];
+    };
+    auto read = [&](Frag& f, int k) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) f.a[g][i] = *reinterpret_cast<const f32x4*>(a0 + 16 * i * PITCH + k + 4 * g);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) f.b[g][j] = *reinterpret_cast<const f32x4*>(b0 + 16 * j * PITCH + k + 4 * g);
+        }
+    };
+    auto work = [&](const Frag& f) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float a[TM], b[TN];
+#pragma unroll
+                for (int i = 0; i < TM; ++i) a[i] = f.a[g][i][e];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[j] = f.b[g][j][e];
+                fma(a, b);
+            }
+    };
+    for (int k0 = 0; k0 < p.K; k0 += KB) {
+        if (k0) __syncthreads();  // everybody is done reading the stage before this one
+#pragma unroll
+        for (int q = 0; q < LA; ++q) {
+            int m, k;
+            place(a_kfast, BM, q, &m, &k);
+            sA[m * PITCH + k] = u_widen<DA>(ra[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+            int n, k;
+            place(b_kfast, BN, q, &n, &k);
+            sB[n * PITCH + k] = u_widen<DB>(rb[q]);
+        }
+        __syncthreads();
+        if (k0 + KB < p.K) fetch(k0 + KB);  // in flight during the arithmetic below
+        const int kmax = min(KB, p.K - k0), whole = kmax / (8 * G) * (8 * G);
+        // two sets of fragments: one is read while the other is worked on
+        Frag f0, f1;
+        if (whole) read(f0, 0);
+#pragma unroll 1
+        for (int k = 0; k < whole; k += 8 * G) {
+            read(f1, k + 4 * G);
+            __builtin_amdgcn_sched_barrier(0);
+            work(f0);
+            if (k + 8 * G < whole) read(f0, k + 8 * G);
+            __builtin_amdgcn_sched_barrier(0);
+            work(f1);
+        }
+#pragma unroll 1
+        for (int k = whole; k < kmax; ++k) {
+            float a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[i] = a0[16 * i * PITCH + k];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[j] = b0[16 * j * PITCH + k];
+            fma(a, b);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int m = m0 + tx + 16 * i, n = n0 + ty + 16 * j;
+            if (m < p.M && n < p.N) {
+                float v = acc[i][j];
+                if (p.alpha != 1.0f) {
+                    v = __fmul_rn(p.alpha, v);
+                    if (p.C) v = __fadd_rn(v, u_load(p.C, m * p.sc_m + n * p.sc_n, DD));
+                }
+                u_store(p.D, m * p.sd_m + n * p.sd_n, DD, v);
+            }
+        }
+}
+
+template <int TM, int TN, int KB>
+static int32_t launch_small(const UArgs& a, int prod, int accT, hipStream_t st) {
+    const dim3 grid((a.M + 16 * TM - 1) / (16 * TM), (a.N + 16 * TN - 1) / (16 * TN));
+#define MOYE_U(P, Q, T) gemm_universal_fma_small<TM, TN, KB, P, Q, T, T><<<grid, 256, 0, st>>>(a)
+    if (prod == 0 && accT == 0 && a.a_dt == MOYE_F32 && a.b_dt == MOYE_F32) MOYE_U(0, 0, MOYE_F32);
+    else if (prod == 0 && accT == 0) MOYE_U(0, 0, kAny);
+    else if (prod == 1 && accT == 0) MOYE_U(1, 0, MOYE_F16);
+    else if (prod == 2 && accT == 0) MOYE_U(2, 0, MOYE_BF16);
+    else if (prod == 1 && accT == 1) MOYE_U(1, 1, MOYE_F16);
+    else if (prod == 2 && accT == 2) MOYE_U(2, 2, MOYE_BF16);
+    else return fail(MOYE_ERR_UNSUPPORTED, "gemm!: UniversalFMA has no kernel for this type combination");
+#undef MOYE_U
+    MOYE_HIP_CHECK(hipGetLastError());
+    return MOYE_OK;
 }
 
 template <int BM, int BN, int BK, int TM, int TN>
@@ -209,11 +359,18 @@ int32_t gemm_universal_dispatch(int bm, int bn, int bk, UArgs a, hipStream_t st)
         bm = bn = small ? 32 : 64;
     }
     if (bk == 0) bk = 8;
-    // bK of the caller's tile is how many k the reference's kernel stages per trip; the sum over k is strictly ascending
-    // whatever that number is, so the 32 x 32 tile, which small problems use with few waves per CU, stages 32 per trip (one
-    // global round trip and one barrier pair per 32 k: fp32 256^3 17 us instead of 20, 1024^3 102 instead of 112)
-    if (bm == 32 && bn == 32 && bk == 8) return launch_u<32, 32, 32, 2, 2>(a, prod, accT, st);
-    if (bm == 32 && bn == 32 && bk == 8) return launch_u<32, 32, 8, 2, 2>(a, prod, accT, st);
+    // bK of the caller's tile is how many k the reference's kernel stages per trip, and bM x bN what a workgroup computes; the
+    // sum over k is strictly ascending and no element depends on another whatever they are.  The 32 x 32 tile runs the form
+    // for few elements, on tiles of its own: the smaller, the more workgroups, the larger, the fewer LDS reads per product.
+    // fp32, us, 16 x 16 / 32 x 32 / 64 x 32: 256^3 6.2 / 11.9 / 18.0; 512^3 21.2 / 22.2 / 32.3; 640^3 39.2 / 32.1 / 40.1; 768^3
+    // 58.2 / 49.4 / 56.9; 1024^3 128.8 / 93.3 / 79.8.  From where 64 x 64 tiles of the kernel above fill the chip on, those.
+    if (bm == 32 && bn == 32 && bk == 8) {
+        const int64_t tiles = (int64_t)((a.M + 31) / 32) * ((a.N + 31) / 32), cus = device_shape().cus;
+        if (tiles <= cus) return launch_small<1, 1, 64>(a, prod, accT, st);
+        if (tiles <= 3 * cus) return launch_small<2, 2, 32>(a, prod, accT, st);
+        if (tiles <= 12 * cus) return launch_small<4, 2, 64>(a, prod, accT, st);
+        return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
+    }
     if (bm == 64 && bn == 64 && bk == 8) return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
     if (bm == 128 && bn == 128 && bk == 8) return launch_u<128, 128, 8, 8, 8>(a, prod, accT, st);
     return fail(MOYE_ERR_UNSUPPORTED, "gemm!: UniversalFMA CTA tile %dx%dx%d not built (32x32x8, 64x64x8, 128x128x8)", bm, bn, bk);

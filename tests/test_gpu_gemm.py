@@ -93,6 +93,39 @@ def test_universal_fma_ragged_bit_exact(mh, dt):
     assert np.array_equal(d.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("types", ["f32", "f16", "bf16", "f16->f16", "bf16->bf16", "f32*f16"])
+def test_universal_fma_small_tiles_give_the_same_bits(mh, types):
+    """The forms the 32 x 32 tile runs on (16 x 16, 32 x 32 and 64 x 32 elements, then the 64 x 64 kernel), around tiles and
+    stages, both majors of the operands, C and alpha: the bits of the 128 x 128 kernel, which is another kernel; f32
+    against the oracle as well.  D lies in a frame that must stay untouched."""
+    tdt = {"f32": (torch.float32,) * 3, "f16": (torch.float16, torch.float16, torch.float32), "bf16": (torch.bfloat16, torch.bfloat16, torch.float32),
+           "f16->f16": (torch.float16,) * 3, "bf16->bf16": (torch.bfloat16,) * 3, "f32*f16": (torch.float32, torch.float16, torch.float32)}[types]
+    for n, (M, N, K, a_k, b_k, alpha, with_c) in enumerate([
+            (1, 1, 1, 1, 1, 1.0, True), (15, 17, 63, 0, 1, 1.0, True), (16, 16, 64, 1, 0, 1.0, False), (17, 33, 65, 0, 0, 1.5, True),
+            (100, 31, 129, 1, 1, 1.0, True), (512, 512, 70, 0, 0, 1.0, True), (513, 512, 31, 1, 0, 1.0, True), (700, 601, 97, 0, 1, 1.0, True),
+            (1030, 900, 130, 1, 1, -0.5, True), (1800, 1793, 66, 0, 0, 1.0, True)]):
+        g = torch.Generator().manual_seed(n)
+        A, B = torch.randn(M, K, generator=g).to(tdt[0]), torch.randn(N, K, generator=g).to(tdt[1])
+        C0 = torch.randn(M, N, generator=g).to(tdt[2])
+        dev = lambda t, kfast: (t.cuda(), (t.shape[1], 1)) if kfast else (t.t().contiguous().cuda(), (1, t.shape[0]))
+        (a, sa), (b, sb) = dev(A, a_k), dev(B, b_k)
+        c = C0.cuda()
+        out = []
+        for tile in ((32, 32, 8), (128, 128, 8)):
+            d = torch.full((M + 2, N + 3), 7.0, device="cuda", dtype=tdt[2])
+            mh.gemm_(mh.tiled_mma_desc(mh.MMA_UNIVERSAL_FMA, cta_tile=tile), T(d[1:, 1:], (M, N), (N + 3, 1)), T(a, (M, K), sa), T(b, (N, K), sb),
+                     T(c) if with_c else None, alpha)
+            torch.cuda.synchronize()
+            out.append(d)
+        assert torch.equal(out[0], out[1]), (types, M, N, K)
+        frame = out[0].clone()
+        frame[1:M + 1, 1:N + 1] = 7.0
+        assert bool((frame == 7.0).all()), (types, M, N, K)
+        if types == "f32" and alpha == 1.0 and M * N * K < 3e7:
+            want = to.gemm_universal_fma(A.numpy(), B.numpy(), C0.numpy() if with_c else np.zeros((M, N), np.float32))
+            assert np.array_equal(out[0][1:M + 1, 1:N + 1].cpu().numpy(), want), (M, N, K)
+
+
 def test_universal_fma_matches_reference_device_test_shape(mh):
     """test/device/matmul.jl:75-81 — C = A*B' with A:(2048,256), B:(2048,256) column-major."""
     rng = np.random.default_rng(6)
