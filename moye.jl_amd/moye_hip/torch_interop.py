@@ -29,4 +29,6 @@ def tensor_of(t, shape=None, stride=None, dtype=None):
 
 
 def current_stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream as a raw handle (without building the torch.cuda.Stream object around it, which
+    takes as long as a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
