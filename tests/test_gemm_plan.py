@@ -404,3 +404,12 @@ def test_universal_fma_plan_and_errors():
     A, B, D = operands(256, 256, 256, mh.F16, mh.F32)
     st = _lib.lib().moye_gemm_explain(C.byref(mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16)), C.byref(D), C.byref(A), C.byref(B), None, None, 0, buf, 8)
     assert st == _lib.ERR_BUFFER
+
+
+@pytest.mark.parametrize("in_dt,K,lines", [(mh.F16, 504, False), (mh.F16, 512, True), (mh.F16, 520, True), (mh.F8E4M3, 1040, True), (mh.F32, 252, False), (mh.F32, 260, True)])
+def test_kmajor_copies_have_rows_of_whole_lines(in_dt, K, lines):
+    """Rows of 1 KiB and more of a K-major copy are padded to 128 bytes, shorter ones to 16 (run_case compares the
+    workspace with the query)."""
+    s = [s for s in run_case(in_dt, mh.F32, 200, 136, K, a_major="m", b_major="n", pad=(8, 24, 0))["steps"] if s["what"] == "kernel"][0]
+    piece = 128 if lines else 16
+    assert s["lda"] == s["ldb"] == -(-K * EB[in_dt] // piece) * piece // EB[in_dt], s

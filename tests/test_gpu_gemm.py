@@ -2325,3 +2325,21 @@ def test_operand_majors_native_random(mh):
         times[name] = mh.time_gemm(mma, T(d), ta, tb, None, 1.0, None, warmup=5, iters=100)
     print("fp16 2048^3 by operand major: " + ", ".join("%s %.1f us" % (k, v * 1e3) for k, v in times.items()))
     # (printed only; the 128x128 tile reads LDS near its limit already: about 1.4 x TN; with K-major copies about 1.3)
+
+
+@pytest.mark.parametrize("K", [8, 504, 512, 520, 1000])
+def test_kmajor_copies_with_padded_rows_exact_on_integers(mh, K):
+    """A M-major and B N-major on a problem of no whole tiles: both go through K-major copies whose rows are padded beyond
+    K; nothing of the padding reaches D."""
+    M, N = 200, 136
+    g = torch.Generator().manual_seed(K)
+    A = torch.randint(-4, 5, (K, M), generator=g).to(torch.float16).cuda()
+    B = torch.randint(-4, 5, (K, N), generator=g).to(torch.float16).cuda()
+    d = torch.full((M, N), 7.0, device="cuda")
+    ws = torch.full((1 << 20,), 0xff, dtype=torch.uint8, device="cuda")  # NaN in the padding
+    mma, ops = mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16), (T(d), T(A, (M, K), (1, M)), T(B, (N, K), (1, N)))
+    need = mh.gemm_workspace_size(mma, *ops, mh.gemm_epilogue())
+    assert 0 < need <= ws.numel()
+    mh.gemm_ex_(mma, *ops, None, mh.gemm_epilogue(), ws.data_ptr(), need)
+    torch.cuda.synchronize()
+    assert torch.equal(d.double(), A.double().t() @ B.double())
