@@ -336,6 +336,24 @@ static int32_t dispatch_atom32(int32_t in_dt, int32_t out_dt, int bm, int bn, in
     return launch_atom32<false>(in_dt, out_dt, a, plan);
 }
 
+// The part of a problem below its first m1 rows / to the right of its first n1 columns (bytes per element of the operands and of D)
+static GemmArgs rows_from(GemmArgs a, int64_t m1, int eb, int ob) {
+    a.M -= (int)m1;
+    a.A = static_cast<const char*>(a.A) + m1 * a.lda * eb;
+    a.D = static_cast<char*>(a.D) + m1 * a.ldd * ob;
+    if (a.C) a.C = static_cast<const char*>(a.C) + m1 * a.ldc_m * ob;
+    if (a.ep_x) a.ep_x = static_cast<const char*>(a.ep_x) + m1 * a.ep_xm * dtype_bytes(a.ep_xdt);
+    return a;
+}
+static GemmArgs columns_from(GemmArgs a, int64_t n1, int eb, int ob) {
+    a.N -= (int)n1;
+    a.B = static_cast<const char*>(a.B) + n1 * a.ldb * eb;
+    a.D = static_cast<char*>(a.D) + n1 * ob;
+    if (a.C) a.C = static_cast<const char*>(a.C) + n1 * a.ldc_n * ob;
+    if (a.ep_x) a.ep_x = static_cast<const char*>(a.ep_x) + n1 * a.ep_xn * dtype_bytes(a.ep_xdt);
+    return a;
+}
+
 // K-major A and B, N-contiguous D.  bk_elems = 0 picks the default K extent per tile.
 // `lib`: the tile (and K ranges) the host chose together with the split when everything was left to the library
 // (gemm_choose, gemm_plan.hpp); null where only the tile is open (a part of a larger problem, a split the caller named).
@@ -394,9 +412,57 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
         // (the hand-ordered kernel's guarded forms: K of whole 16-byte pieces)
         const bool hand_ordered_ragged = (eb == 2 || eb == 4 || in_dt == MOYE_F8E4M3) && ((int64_t)a.K * eb) % 16 == 0 &&
                                          stages < 2 && row_offsets_fit(a, 256, eb);
-        if ((!big || !aligned) && !thin && a.split <= 1 && bk_elems == 0 && aligned_ab && (in_dt != MOYE_F8E4M3 || hand_ordered_ragged) && ((int64_t)a.K * eb) % 16 == 0 &&
-            prefer256 && stages < 3 && (waves <= 1 || waves == 8) &&
-            !(a.flags & (MOYE_GEMM_WAVE4 | MOYE_GEMM_PINGPONG | kGemmAMajorM | kGemmBMajorN | kGemmAtom32))) {
+        const bool guarded_ok = (!big || !aligned) && !thin && a.split <= 1 && bk_elems == 0 && aligned_ab && (in_dt != MOYE_F8E4M3 || hand_ordered_ragged) &&
+                                ((int64_t)a.K * eb) % 16 == 0 && stages < 3 && (waves <= 1 || waves == 8) &&
+                                !(a.flags & (MOYE_GEMM_WAVE4 | MOYE_GEMM_PINGPONG | kGemmAMajorM | kGemmBMajorN | kGemmAtom32));
+        // The last round of ragged tiles leaves much of the chip idle: two launches, as for whole tiles below, the first
+        // on as many whole tile rows (or columns) as fill the rounds before it -- with N and K whole, those run unguarded
+        // --, the second on what the library would choose for the rest alone.  The guarded instance takes 1.03 times the
+        // whole one's time over several rounds, and 128 x 128 tiles that reach over the edge cost a full launch next to
+        // nothing (the 1.25 and 1.15 of the cost model hold for part-filled chips).  Rounds that fill the chip run at
+        // lower clocks than ones that do not, which the model does not know, so it has to see 8 %: bf16 6000 x 4096 x 14336
+        // (24 x 16 tiles, priced 0.89) 640 -> 572 us, but 6000 x 14336 x 4096 (24 x 56, priced 0.94) 598 in one launch and 597
+        // in two.  Also where 128 x 128 tiles would be cheaper than one launch of 256 x 256 ones: 3900 x 4608 x 3000
+        // 174.1 -> 127.5, 4000 x 5120 x 8192 317 -> 280, 4608 x 4800 x 4096 165 -> 145.5, 3700 x 5120 x 1536 64.0 -> 59.5,
+        // 4608 x 3960 x 2048 86.8 -> 79.8; f16 4100 x 4352 x 2048 93.3 -> 80.2, 3000 x 8192 x 8192 351 -> 334; fp8
+        // 3900 x 4608 x 6000 176.5 -> 128.5, 2500 x 14336 x 4096 153 -> 141.5.
+        if (guarded_ok && hand_ordered_ragged && waves <= 1 && stages == 0 && rtiles > cus && rtiles % cus) {
+            const bool k_tail = k_bytes_all % 128 != 0;
+            const double guarded = 1.03;
+            const int tm = (a.M + 255) / 256, tn = (a.N + 255) / 256;
+            auto alone = [&](int64_t m, int64_t n) {  // what the library would run the rest as, priced
+                double us = gemm_plan(m, n, k_bytes_all, eb == 4, m % 64 == 0 && n % 64 == 0 && !k_tail, 16, cus, 1).us;
+                if (m % 128 || n % 128 || k_tail) us /= 1.15;
+                if (gemm_short_m(m, n, k_bytes_all, eb == 4, cus)) gemm_short_m_ntw(m, n, k_bytes_all, cus, 1, &us);
+                return us;
+            };
+            double best_us = (eb == 4 ? 0.88 : 0.92) * (prefer256 ? guarded * gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, false, cus) : choice.us);
+            int64_t m1 = 0, n1 = 0;
+            for (const bool by_rows : {true, false}) {
+                const int other = by_rows ? tn : tm, nt = by_rows ? tm : tn;
+                for (int64_t rounds = rtiles / cus; rounds >= 1 && rounds + 1 >= rtiles / cus; --rounds) {
+                    const int64_t first = rounds * cus / other;
+                    if (first < 1 || first >= nt) continue;
+                    const int64_t m = by_rows ? first * 256 : a.M, n = by_rows ? a.N : first * 256;
+                    const bool whole = aligned && !k_tail && m % 256 == 0 && n % 256 == 0;
+                    const double us = (whole ? 1.0 : guarded) * gemm_plan_cost_256(m, n, k_bytes_all, eb == 4, false, cus) + 2.0 +
+                                      (by_rows ? alone(a.M - m, a.N) : alone(a.M, a.N - n));
+                    if (us < best_us) { best_us = us; m1 = m; n1 = n; }
+                }
+            }
+            if (m1 > 0) {
+                GemmArgs part = a;
+                part.M = (int)m1; part.N = (int)n1;
+                if (aligned && !k_tail && m1 % 256 == 0 && n1 % 256 == 0) {
+                    if (int32_t e = gemm_mfma_tn_dispatch(in_dt, out_dt, 256, 256, 128 / eb, 8, 0, part, plan)) return e;
+                } else {
+                    part.flags |= kGemmRagged;
+                    if (int32_t e = gemm_mfma_tn_256_w4_dispatch(in_dt, out_dt, part, 8, 128, false, plan)) return e;
+                }
+                return gemm_mfma_tn_dispatch(in_dt, out_dt, 0, 0, 0, 0, 0, m1 < a.M ? rows_from(a, m1, eb, ob0) : columns_from(a, n1, eb, ob0), plan);
+            }
+        }
+        if (guarded_ok && prefer256) {
             a.flags |= kGemmRagged;
             // the hand-ordered kernel's guarded forms (rows clamped, a K tail masked in registers; with a C or an
             // element-wise operation the instance whose epilogue is the general one)
@@ -471,22 +537,7 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
                 GemmArgs part = a;
                 (by_rows ? part.M : part.N) = first * 256;
                 if (int32_t e = gemm_mfma_tn_dispatch(in_dt, out_dt, 256, 256, 128 / eb, 8, 0, part, plan)) return e;
-                part = a;
-                if (by_rows) {
-                    const int64_t m1 = (int64_t)first * 256;
-                    part.M = a.M - (int)m1;
-                    part.A = static_cast<const char*>(a.A) + m1 * a.lda * eb;
-                    part.D = static_cast<char*>(a.D) + m1 * a.ldd * ob0;
-                    if (a.C) part.C = static_cast<const char*>(a.C) + m1 * a.ldc_m * ob0;
-                    if (a.ep_x) part.ep_x = static_cast<const char*>(a.ep_x) + m1 * a.ep_xm * dtype_bytes(a.ep_xdt);
-                } else {
-                    const int64_t n1 = (int64_t)first * 256;
-                    part.N = a.N - (int)n1;
-                    part.B = static_cast<const char*>(a.B) + n1 * a.ldb * eb;
-                    part.D = static_cast<char*>(a.D) + n1 * ob0;
-                    if (a.C) part.C = static_cast<const char*>(a.C) + n1 * a.ldc_n * ob0;
-                    if (a.ep_x) part.ep_x = static_cast<const char*>(a.ep_x) + n1 * a.ep_xn * dtype_bytes(a.ep_xdt);
-                }
+                part = by_rows ? rows_from(a, (int64_t)first * 256, eb, ob0) : columns_from(a, (int64_t)first * 256, eb, ob0);
                 return gemm_mfma_tn_dispatch(in_dt, out_dt, 0, 0, 0, 0, 0, part, plan);
             }
         }

@@ -413,3 +413,21 @@ def test_kmajor_copies_have_rows_of_whole_lines(in_dt, K, lines):
     s = [s for s in run_case(in_dt, mh.F32, 200, 136, K, a_major="m", b_major="n", pad=(8, 24, 0))["steps"] if s["what"] == "kernel"][0]
     piece = 128 if lines else 16
     assert s["lda"] == s["ldb"] == -(-K * EB[in_dt] // piece) * piece // EB[in_dt], s
+
+
+@pytest.mark.parametrize("M,N,K,first", [
+    (6000, 4096, 14336, (4096, 4096, False)),   # whole tile rows, unguarded
+    (3950, 4608, 3000, (3584, 4608, True)),     # a K tail: guarded, and 128 x 128 tiles would be chosen for one launch
+    (3950, 4608, 3072, (3584, 4608, False)),
+    (4608, 4000, 3072, (4608, 3584, False)),    # by columns
+])
+@pytest.mark.parametrize("d_major", ["n", "m"])
+def test_a_last_round_of_ragged_tiles_gets_a_launch_of_its_own(M, N, K, first, d_major):
+    """Two launches that cover D once (run_case), the first on 256 x 256 tiles; none for a problem in one round."""
+    if d_major == "m":
+        M, N, first = N, M, (first[1], first[0], first[2])
+    p = run_case(mh.BF16, mh.BF16, M, N, K, d_major=d_major, waves=(1, 1, 1))
+    s = [s for s in p["steps"] if s["what"] == "kernel"]
+    m, n = (s[0]["M"], s[0]["N"]) if d_major == "n" else (s[0]["N"], s[0]["M"])
+    assert len(s) == 2 and s[0]["tile"].startswith("256x256") and (m, n, "ragged" in s[0]["flags"]) == first, p["text"]
+    assert len(run_case(mh.BF16, mh.BF16, min(M, 4000), min(N, 4000), K, d_major=d_major, waves=(1, 1, 1))["steps"]) == 1

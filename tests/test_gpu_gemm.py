@@ -2343,3 +2343,33 @@ def test_kmajor_copies_with_padded_rows_exact_on_integers(mh, K):
     mh.gemm_ex_(mma, *ops, None, mh.gemm_epilogue(), ws.data_ptr(), need)
     torch.cuda.synchronize()
     assert torch.equal(d.double(), A.double().t() @ B.double())
+
+
+@pytest.mark.parametrize("M,N,K", [(3950, 4608, 2008), (3950, 4608, 2048), (4608, 3960, 2048)])
+@pytest.mark.parametrize("epilogue", ["plain", "bias", "c"])
+def test_ragged_problem_in_two_launches_exact_on_integers(mh, M, N, K, epilogue):
+    """A last round of ragged 256 x 256 tiles in a launch of its own, by rows and by columns: pointers of A, B, C, D and of the
+    epilogue's operand move along; the frame around D stays."""
+    from moye_hip import _lib
+    g = torch.Generator().manual_seed(M + K)
+    a = torch.randint(-4, 5, (M, K), generator=g).to(torch.float16).cuda()
+    b = torch.randint(-4, 5, (N, K), generator=g).to(torch.float16).cuda()
+    row, col, c = (torch.randint(-9, 10, s, generator=g).float().cuda() for s in ((M, 1), (1, N), (M, N)))
+    ref = a.double() @ b.double().t()
+    frame = torch.full((M + 2, N + 8), 77.0, device="cuda")
+    d = frame[1:M + 1, 4:N + 4]
+    mma = mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16)
+    calls = [(None, None, ref)]
+    if epilogue == "bias":
+        calls = [(mh.gemm_epilogue(op=_lib.MAP_ADD, operand=T(row, (M, N), (1, 0))), None, ref + row),
+                 (mh.gemm_epilogue(op=_lib.MAP_ADD, operand=T(col, (M, N), (0, 1))), None, ref + col)]
+    elif epilogue == "c":
+        calls = [(mh.gemm_epilogue(beta=2.0), c, ref + 2.0 * c)]
+    for ep, cc, want in calls:
+        assert len(kernels_of(mh, mma, T(d), T(a), T(b), None if cc is None else T(cc), ep)) == 2
+        mh.gemm_ex_(mma, T(d), T(a), T(b), None if cc is None else T(cc), ep)
+        torch.cuda.synchronize()
+        assert torch.equal(d.double(), want.double())
+        rest = frame.clone()
+        rest[1:M + 1, 4:N + 4] = 77.0
+        assert bool((rest == 77.0).all()), "stores outside D"
