@@ -34,7 +34,7 @@ TRAFFIC_CALIBRATION = ("copy_flat_b128", 524297.5, 1049490.6)     # the 1 GiB pl
 MEASURED_TRAFFIC = {
     # key: (kernel as the profile names it, FETCH_SIZE KiB, WRITE_SIZE KiB)
     "gemm_f16_4096_tile256": ("gemm_mfma_tn_256_w4<W4F16L, OutF16, 4, false, false, 256, 0, 0, false, false, false>", 98481.0, 32789.1),
-    "transpose_f32_16384": ("transpose_lds_b32_rows<4>", 524309.0, 1050103.0),
+    "transpose_f32_16384": ("transpose_blocks<7, 7, 4, 4, 16, 2, 512>", 524327.3, 1049961.1),
     "gemm_bf16_8192_tile256": ("gemm_mfma_tn_256_w4<W4BF16L, OutF32, 4, false, false, 256, 0, 0, false, false, true>", 827548.5, 263348.6),
     "gemm_f32_8192_tile256": ("gemm_mfma_tn_256_w4<W4F32L, OutF32, 4, false, false, 256, 0, 0, false, false, false>", 1653069.0, 262269.2),
     "gemm_fp8_8192_tile256": ("gemm_mfma_tn_256_w4<W4FP8L, OutBF16, 4, false, false, 256, 0, 0, false, false, true>", 395120.7, 132096.0),
