@@ -136,7 +136,7 @@ static int32_t scratch_of_current_device(char** out) {
 // Bytes from row to row of a K-major copy: whole 128-byte lines, so that each 128-byte piece of a row that a k-step loads is
 // one line and not parts of two; rows under 1 KiB, which that would lengthen by more than an eighth, keep 16-byte pieces.
 // (bf16 forward + both gradients of a linear layer, 6000 x 4096 -> 14336, 12000-byte rows in the weight's gradient: 2020 -> 1942 us,
-// that product 635 -> 540; 4104 x 4096 -> 11008 1079 -> 1013; f16 3000 x 2048 -> 8192 393 -> 369)
+// that product 635 -> 566; 4104 x 4096 -> 11008 1079 -> 1013; f16 3000 x 2048 -> 8192 393 -> 369)
 static int64_t kmajor_pitch(const Mat& m) {
     const int64_t row = m.cols * dtype_bytes(m.dtype), piece = row >= 1024 ? 128 : 16;
     return (row + piece - 1) / piece * piece;
