@@ -35,10 +35,14 @@ __device__ __forceinline__ void u_store(void* p, int64_t i, int dt, float v) {
 }
 
 // kProd / kAcc: 0 = fp32, 1 = fp16, 2 = bf16 — the type the product / the running sum is rounded in
+// (fp16: the value is made opaque first; a product the compiler can see is rounded by v_fma_mixlo_f16 with an addend of +0,
+// which turns a product of -0 into +0)
 template <int kT>
 __device__ __forceinline__ float round_in(float x) {
-    if constexpr (kT == 1) return (float)(_Float16)x;
-    else if constexpr (kT == 2) return u_bf16_round(x);
+    if constexpr (kT == 1) {
+        asm("" : "+v"(x));
+        return (float)(_Float16)x;
+    } else if constexpr (kT == 2) return u_bf16_round(x);
     else return x;
 }
 

@@ -126,6 +126,29 @@ def test_universal_fma_small_tiles_give_the_same_bits(mh, types):
             assert np.array_equal(out[0][1:M + 1, 1:N + 1].cpu().numpy(), want), (M, N, K)
 
 
+@pytest.mark.parametrize("tile", [(32, 32, 8), (64, 64, 8), (128, 128, 8)])
+@pytest.mark.parametrize("types", ["f32", "f16", "bf16", "f16->f16", "bf16->bf16"])
+def test_universal_fma_keeps_the_sign_of_zero(mh, types, tile):
+    """Products of -0 onto a C of -0: -0 where every product of an element is -0 and +0 where one is +0, sign bits against
+    the oracle (every value is a zero, so no accumulator type rounds)."""
+    ta, td = types.split("->") if "->" in types else (types, "f32")
+    dts = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    M, N, K = 37, 45, 70                                    # whole stages and a remainder in every kernel
+    rng = np.random.default_rng(3)
+    A = torch.from_numpy(np.where(rng.random((M, K)) < 0.5, 0.0, -0.0).astype(np.float32))
+    A[::2] = 0.0                                            # rows whose products with a negative column are all -0
+    B = torch.from_numpy(-np.abs(rng.standard_normal((N, K))).astype(np.float32) - 0.5)
+    B[::3] *= -1.0                                          # columns whose products with those rows are all +0
+    C0 = torch.full((M, N), -0.0)
+    a, b, c, d = A.to(dts[ta]).cuda(), B.to(dts[ta]).cuda(), C0.to(dts[td]).cuda(), torch.full((M, N), 7.0, device="cuda", dtype=dts[td])
+    mh.gemm_(mh.tiled_mma_desc(mh.MMA_UNIVERSAL_FMA, cta_tile=tile), T(d), T(a), T(b), T(c))
+    torch.cuda.synchronize()
+    want = to.gemm_universal_fma(A.numpy(), B.to(dts[ta]).float().numpy(), C0.numpy(), ta, ta)
+    assert (want == 0).all() and 0 < np.signbit(want).sum() < want.size
+    got = d.cpu().float().numpy()
+    assert (got == 0).all() and np.array_equal(np.signbit(got), np.signbit(want))
+
+
 def test_universal_fma_matches_reference_device_test_shape(mh):
     """test/device/matmul.jl:75-81 — C = A*B' with A:(2048,256), B:(2048,256) column-major."""
     rng = np.random.default_rng(6)
