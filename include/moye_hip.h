@@ -208,8 +208,11 @@ int32_t moye_map(int32_t op, const moye_tensor* dst, const moye_tensor* a, const
  *                 that needs one (a synchronous hipMalloc inside that call, so not under stream capture),
  *                 replaced by a larger one when a larger call comes, never freed inside a call.  Calls on
  *                 different streams do not share a buffer; calls on one stream are ordered by the stream.
- *   moye_gemm_ex  takes the workspace from the caller (256-byte aligned, at least the size reported here;
- *                 NULL when the call needs none) and never allocates, frees or synchronises.            */
+ *   moye_gemm_ex  takes the workspace from the caller (256-byte aligned, of the size reported here; NULL when the
+ *                 call needs none) and never allocates, frees or synchronises.
+ * The size counts the rows of a K-major copy in whole 128-byte lines where they have 1 KiB and more.  A workspace that
+ * holds the copies only with rows in 16-byte pieces (up to a ninth smaller) is taken too; the product is then slower,
+ * its bits are the same. */
 int32_t moye_gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor* D,
                                  const moye_tensor* A, const moye_tensor* B, size_t* bytes);
 /* waits for the devices that hold workspaces of moye_gemm and frees them all (no counterpart in the
@@ -265,7 +268,7 @@ int32_t moye_gemm_ex_workspace_size(const moye_tiled_mma* mma, const moye_tensor
  * that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results as moye_gemm, bit for bit;
  * the workspace (split-K partial products, K-major copies of operands that are not K-major) is a static device
  * array of MOYE_NOALLOC_SCRATCH_BYTES inside the library, one copy per GPU, held until the process ends.  A call
- * that needs more (moye_gemm_workspace_size) fails with MOYE_ERR_ARG before anything is launched.  Never calls
+ * that needs more, with the rows of its copies in 16-byte pieces, fails with MOYE_ERR_ARG before anything is launched.  Never calls
  * hipMalloc / hipFree or synchronises.  All calls on one GPU share that GPU's array: calls that overlap on one GPU
  * (different streams, or host threads that do not order their launches) race; calls on one stream are safe. */
 #define MOYE_NOALLOC_SCRATCH_BYTES (32u << 20)

@@ -132,16 +132,16 @@ static int32_t scratch_of_current_device(char** out) {
     return MOYE_OK;
 }
 
-// bytes of a K-major copy of an (rows x K) operand: row pitch rounded up to 16 bytes
-// Bytes from row to row of a K-major copy: whole 128-byte lines, so that each 128-byte piece of a row that a k-step loads is
-// one line and not parts of two; rows under 1 KiB, which that would lengthen by more than an eighth, keep 16-byte pieces.
+// Bytes from row to row of a K-major copy.  `lines`: whole 128-byte lines, so that each 128-byte piece of a row that a k-step
+// loads is one line and not parts of two; rows under 1 KiB, which that would lengthen by more than an eighth, keep 16-byte
+// pieces, and so do all rows of a call whose workspace holds the copies only that way (gemm_plan_build).
 // (bf16 forward + both gradients of a linear layer, 6000 x 4096 -> 14336, 12000-byte rows in the weight's gradient: 2020 -> 1942 us,
 // that product 635 -> 566; 4104 x 4096 -> 11008 1079 -> 1013; f16 3000 x 2048 -> 8192 393 -> 369)
-static int64_t kmajor_pitch(const Mat& m) {
-    const int64_t row = m.cols * dtype_bytes(m.dtype), piece = row >= 1024 ? 128 : 16;
+static int64_t kmajor_pitch(const Mat& m, bool lines) {
+    const int64_t row = m.cols * dtype_bytes(m.dtype), piece = lines && row >= 1024 ? 128 : 16;
     return (row + piece - 1) / piece * piece;
 }
-static size_t kmajor_bytes(const Mat& m) { return (size_t)(m.rows * kmajor_pitch(m) + 255) / 256 * 256; }
+static size_t kmajor_bytes(const Mat& m, bool lines) { return (size_t)(m.rows * kmajor_pitch(m, lines) + 255) / 256 * 256; }
 
 // K ranges for the short-M kernel that stages lines through LDS, when N is small and K long: N = 1024 puts 64 workgroups
 // of 16 rows of B on 256 CUs, and a workgroup streams its rows at about 64 GB/s whatever the others do.  The model of
@@ -298,23 +298,35 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
 }
 
 // K-major copies of A and B where needed, then the fp32 partial products of a split-K call
-static size_t gemm_workspace_bytes_impl(const moye_tiled_mma* mma, const Mat& A, const Mat& B, bool native, int cus) {
+static size_t gemm_workspace_bytes_impl(const moye_tiled_mma* mma, const Mat& A, const Mat& B, bool native, bool lines, int cus) {
     if (mma->atom == MOYE_MMA_UNIVERSAL_FMA) return 0;
     size_t n = 0;
-    if (!native && A.cs != 1 && A.cols > 1) n += kmajor_bytes(A);
-    if (!native && B.cs != 1 && B.cols > 1) n += kmajor_bytes(B);
+    if (!native && A.cs != 1 && A.cols > 1) n += kmajor_bytes(A, lines);
+    if (!native && B.cs != 1 && B.cols > 1) n += kmajor_bytes(B, lines);
     const int split = split_count(mma, A.rows, B.rows, A.cols, dtype_bytes(A.dtype), cus);
     if (split > 1) n += (size_t)split * (size_t)A.rows * (size_t)B.rows * sizeof(float);
     return n;
 }
 
-static size_t gemm_workspace_bytes(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep, int cus) {
-    return gemm_workspace_bytes_impl(mma, A, B, majors_run_natively(mma, A, B, D, ep, false, cus), cus);
+// The same from descriptors: what the fastest plan uses (`lines`), or the least the call can do with
+static int32_t gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor* D, const moye_tensor* A, const moye_tensor* B,
+                                   const moye_gemm_epilogue& ep, bool lines, size_t* bytes) {
+    *bytes = 0;
+    Mat a, b, d;
+    if (int32_t e = as_matrix(A, "A", &a)) return e;
+    if (int32_t e = as_matrix(B, "B", &b)) return e;
+    if (int32_t e = as_matrix(D, "D", &d)) return e;
+    for (Mat* x : {&a, &b, &d})
+        if (x->rows == 1 && x->cs == 1) x->rs = x->cols;
+    const int cus = device_shape().cus;
+    if (!(mma->flags & MOYE_GEMM_NO_WORKSPACE))
+        *bytes = gemm_workspace_bytes_impl(mma, a, b, majors_run_natively(mma, a, b, d, ep, false, cus), lines, cus);
+    return MOYE_OK;
 }
 
 // A step that transposes `m` (unit stride along its rows index) into ws as rows x K with K contiguous; rewrites `m`
-static void plan_kmajor_copy(Mat* m, char* ws, GemmPlan& plan) {
-    const int64_t pitch_e = kmajor_pitch(*m) / dtype_bytes(m->dtype);
+static void plan_kmajor_copy(Mat* m, char* ws, bool lines, GemmPlan& plan) {
+    const int64_t pitch_e = kmajor_pitch(*m, lines) / dtype_bytes(m->dtype);
     plan.steps.emplace_back();
     GemmStep& st = plan.steps.back();
     st.kind = GemmStep::kKMajorCopy;
@@ -356,9 +368,10 @@ static bool lane_op(const GemmArgs& g) {
 }
 
 // gemm!(mma, D, A, B, C) with the epilogue `ep` as a list of launches.  Pure host arithmetic on the descriptors: nothing
-// is launched, allocated or asked of a device (plan.shape says what the chip looks like).  `workspace(bytes, &ptr)` is
-// asked once, and only when the call needs a workspace, for `bytes` bytes: the caller's buffer, the library's own, the
-// static scratch array, or -- for moye_gemm_explain -- an address that is never dereferenced.
+// is launched, allocated or asked of a device (plan.shape says what the chip looks like).  `workspace(least, &bytes, &ptr)`
+// is asked once, and only when the call needs a workspace: for `bytes` bytes (the copies' rows in whole lines), which it may
+// lower to `least` (rows in 16-byte pieces) where there is no more room: the caller's buffer, the library's own, the static
+// scratch array, or -- for moye_gemm_explain -- an address that is never dereferenced.
 template <typename WorkspaceSource>
 static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD, const moye_tensor* tA, const moye_tensor* tB,
                                const moye_tensor* tC, const moye_gemm_epilogue& ep, WorkspaceSource&& workspace, GemmPlan& plan) {
@@ -422,21 +435,23 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         if (A.cs != 1 && A.cols > 1) { major_flags |= kGemmAMajorM; A.rs = A.cs; A.cs = 1; }  // Mat::rs now holds the pitch between consecutive k
         if (B.cs != 1 && B.cols > 1) { major_flags |= kGemmBMajorN; B.rs = B.cs; B.cs = 1; }
     }
-    plan.workspace_bytes = gemm_workspace_bytes_impl(mma, A, B, native_majors, cus);
+    plan.workspace_bytes = gemm_workspace_bytes_impl(mma, A, B, native_majors, true, cus);
     if (plan.workspace_bytes) {
         if (mma->flags & MOYE_GEMM_NO_WORKSPACE)
             return fail(MOYE_ERR_UNSUPPORTED, "gemm!: the MFMA kernels need K-major A and B (stride 1 along K, the 'TN' form), split_k needs room "
                                               "for its partial products, and MOYE_GEMM_NO_WORKSPACE forbids the use of a workspace");
-        if (int32_t e = workspace(plan.workspace_bytes, &ws)) return e;
+        const size_t wanted = plan.workspace_bytes;
+        if (int32_t e = workspace(gemm_workspace_bytes_impl(mma, A, B, native_majors, false, cus), &plan.workspace_bytes, &ws)) return e;
+        const bool lines = plan.workspace_bytes == wanted;
         plan.workspace = ws;
         if (!native_majors && A.cs != 1 && A.cols > 1) {
-            const size_t nb = kmajor_bytes(A);
-            plan_kmajor_copy(&A, ws, plan);
+            const size_t nb = kmajor_bytes(A, lines);
+            plan_kmajor_copy(&A, ws, lines, plan);
             ws += nb;
         }
         if (!native_majors && B.cs != 1 && B.cols > 1) {
-            const size_t nb = kmajor_bytes(B);
-            plan_kmajor_copy(&B, ws, plan);
+            const size_t nb = kmajor_bytes(B, lines);
+            plan_kmajor_copy(&B, ws, lines, plan);
             ws += nb;
         }
     }
@@ -560,25 +575,26 @@ static int32_t gemm_plan_run(const GemmPlan& plan, hipStream_t st) {
     return MOYE_OK;
 }
 
-// `caller_ws` / `caller_ws_bytes`: the workspace when the caller brings one (it must hold what moye_gemm_workspace_size
-// reports); with caller_brings_ws == false the library's own per-stream buffer is used.
+// `caller_ws` / `caller_ws_bytes`: the workspace when the caller brings one (what moye_gemm_workspace_size reports, or at
+// least what the call needs with rows of 16-byte pieces); with caller_brings_ws == false the library's own per-stream buffer is used.
 static int32_t gemm_impl(const moye_tiled_mma* mma, const moye_tensor* tD, const moye_tensor* tA,
                          const moye_tensor* tB, const moye_tensor* tC, const moye_gemm_epilogue& ep, bool caller_brings_ws, char* caller_ws,
                          size_t caller_ws_bytes, hipStream_t st) {
     std::unique_lock<std::mutex> ws_lock(g_ws_mutex, std::defer_lock);
     GemmPlan plan;
     plan.shape = device_shape();
-    auto workspace = [&](size_t bytes, char** out) -> int32_t {
+    auto workspace = [&](size_t least, size_t* bytes, char** out) -> int32_t {
         if (caller_brings_ws) {
-            if (bytes > caller_ws_bytes)
-                return fail(MOYE_ERR_ARG, "gemm!: this call needs a workspace of %zu bytes, the one passed holds %zu", bytes, caller_ws_bytes);
+            if (least > caller_ws_bytes)
+                return fail(MOYE_ERR_ARG, "gemm!: this call needs a workspace of %zu bytes, the one passed holds %zu", least, caller_ws_bytes);
+            if (*bytes > caller_ws_bytes) *bytes = least;
             if (reinterpret_cast<uintptr_t>(caller_ws) % 256)
                 return fail(MOYE_ERR_ALIGN, "gemm!: the workspace must start on a 256-byte boundary");
             *out = caller_ws;
             return MOYE_OK;
         }
         ws_lock.lock();  // until every kernel of this call is enqueued
-        return library_workspace(bytes, st, out);
+        return library_workspace(*bytes, st, out);
     };
     if (int32_t e = gemm_plan_build(mma, tD, tA, tB, tC, ep, workspace, plan)) return e;
     return gemm_plan_run(plan, st);
@@ -708,7 +724,7 @@ int32_t moye_gemm_noalloc(const moye_tiled_mma* mma, const moye_tensor* D, const
                           const moye_tensor* C, float alpha, void* stream) {
     if (!mma || !D || !A || !B) return fail(MOYE_ERR_ARG, "moye_gemm_noalloc: null argument");
     size_t need = 0;
-    if (int32_t e = moye_gemm_workspace_size(mma, D, A, B, &need)) return e;
+    if (int32_t e = gemm_workspace_size(mma, D, A, B, plain_epilogue(1.f), false, &need)) return e;
     if (need > kScratchBytes)
         return fail(MOYE_ERR_ARG, "moye_gemm_noalloc: this call needs %zu bytes of workspace, the static scratch array holds %zu; "
                                   "use moye_gemm_ex with a workspace of the caller's", need, kScratchBytes);
@@ -727,7 +743,7 @@ int32_t moye_gemm_explain(const moye_tiled_mma* mma, const moye_tensor* D, const
     plan.named = true;
     plan.shape = device_shape_for(compute_units);
     // the workspace of a plan that is only printed: an address nothing is read from or written to
-    auto workspace = [](size_t, char** p) -> int32_t {
+    auto workspace = [](size_t, size_t*, char** p) -> int32_t {
         *p = reinterpret_cast<char*>(uintptr_t(1) << 40);
         return MOYE_OK;
     };
@@ -789,15 +805,7 @@ int32_t moye_gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor* D
 int32_t moye_gemm_ex_workspace_size(const moye_tiled_mma* mma, const moye_tensor* D, const moye_tensor* A,
                                     const moye_tensor* B, const moye_gemm_epilogue* ep, size_t* bytes) {
     if (!mma || !D || !A || !B || !ep || !bytes) return fail(MOYE_ERR_ARG, "moye_gemm_workspace_size: null argument");
-    *bytes = 0;
-    Mat a, b, d;
-    if (int32_t e = as_matrix(A, "A", &a)) return e;
-    if (int32_t e = as_matrix(B, "B", &b)) return e;
-    if (int32_t e = as_matrix(D, "D", &d)) return e;
-    for (Mat* x : {&a, &b, &d})
-        if (x->rows == 1 && x->cs == 1) x->rs = x->cols;
-    if (!(mma->flags & MOYE_GEMM_NO_WORKSPACE)) *bytes = gemm_workspace_bytes(mma, a, b, d, *ep, device_shape().cus);
-    return MOYE_OK;
+    return gemm_workspace_size(mma, D, A, B, *ep, true, bytes);
 }
 
 int32_t moye_device_malloc(void** ptr, size_t bytes) {

@@ -104,3 +104,35 @@ def test_noalloc_plain_tn_and_limits(mh):
     with pytest.raises(mh.MoyeError) as e:
         mh.gemm_noalloc_(mma, T(big), T(ah), T(ah))
     assert e.value.status == _lib.ERR_ARG and "static scratch" in str(e.value)
+
+
+def test_a_workspace_that_holds_the_copies_only_in_16_byte_pieces_is_taken(mh):
+    """fp16 with K = 520, A M-major and B N-major: copies of 1040-byte rows take 30.4 MB, of 1152-byte ones, which
+    moye_gemm uses, 33.6 MB, more than the static array holds.  moye_gemm_noalloc and moye_gemm_ex with a buffer of the
+    smaller size give moye_gemm's bits and write nothing behind it; one byte less is refused."""
+    from moye_hip import _lib
+    M, N, K = 28000, 1208, 520
+    g = torch.Generator(device="cuda").manual_seed(31)
+    a = torch.randn(K, M, generator=g, device="cuda").mul_(K ** -0.5).half()
+    b = torch.randn(K, N, generator=g, device="cuda").half()
+    mma = mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16)
+    ta, tb = T(a, (M, K), (1, M)), T(b, (N, K), (1, N))
+    d = [torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3)]
+    least = sum((rows * 1040 + 255) // 256 * 256 for rows in (M, N))
+    wanted = mh.gemm_workspace_size(mma, T(d[0]), ta, tb)
+    assert least < mh.device.NOALLOC_SCRATCH_BYTES < wanted == sum((rows * 1152 + 255) // 256 * 256 for rows in (M, N))
+    mh.gemm_(mma, T(d[0]), ta, tb)
+    mh.gemm_noalloc_(mma, T(d[1]), ta, tb)
+    ws = torch.full((least + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert ws.data_ptr() % 256 == 0
+    mh.gemm_ex_(mma, T(d[2]), ta, tb, None, mh.gemm_epilogue(), ws.data_ptr(), least, None)
+    torch.cuda.synchronize()
+    assert bool((ws[least:] == 0xA5).all())
+    bits = [x.view(torch.int16) for x in d]
+    assert torch.equal(bits[0], bits[1]) and torch.equal(bits[0], bits[2])
+    rows = torch.arange(0, M, 997, device="cuda")
+    want = a[:, rows].double().t() @ b.double()
+    assert float((d[0][rows].double() - want).abs().max() / want.abs().max()) <= 1e-2   # fp16 inputs
+    with pytest.raises(mh.MoyeError) as e:
+        mh.gemm_ex_(mma, T(d[2]), ta, tb, None, mh.gemm_epilogue(), ws.data_ptr(), least - 1, None)
+    assert e.value.status == _lib.ERR_ARG and str(least) in str(e.value)
