@@ -200,11 +200,12 @@ class Layout:
     def descriptor(self):
         """The bytes of a moye_tensor with this layout's rank, shape and stride (null pointer): flattened by the library
         once, a layout never changes."""
-        if self._descriptor is None:
+        d = getattr(self, "_descriptor", None)  # (unset where a layout was made from its text alone, as an old pickle does)
+        if d is None:
             t = _lib.Tensor()
             check(lib().moye_layout_descriptor(_b(self.text), C.byref(t)))
-            self._descriptor = bytes(t)
-        return self._descriptor
+            d = self._descriptor = bytes(t)
+        return d
 
     def __repr__(self):
         return self.text

@@ -2,6 +2,8 @@
 the moye_hip Python mirror) against (1) the reference's own known answers and invariant helpers
 (tests/golden/layout_vectors.json) and (2) the independent Python oracle on seeded random cases.
 No GPU needed."""
+import copy
+import pickle
 import random
 
 import pytest
@@ -588,3 +590,12 @@ def test_array_descriptor_is_the_flattened_layout(shape, stride):
     with pytest.raises(MoyeError) as e:
         mh.MoYeArray(1 << 20, mh.F16, ml.Layout((2,) * 9)).tensor()
     assert e.value.status == ERR_RANK
+
+
+def test_a_layout_pickled_without_a_descriptor_still_makes_arrays():
+    """A pickle holds a layout's slots; one written before layouts kept their descriptor holds the text alone."""
+    lay = ml.Layout.__new__(ml.Layout)
+    lay.text = "(4,(2,3)):(6,(3,1))"
+    for x in (lay, pickle.loads(pickle.dumps(lay)), pickle.loads(pickle.dumps(ml.Layout("(4,(2,3)):(6,(3,1))"))), copy.deepcopy(lay)):
+        t = mh.MoYeArray(1 << 20, mh.F16, x).tensor()
+        assert (t.rank, list(t.shape)[:3], list(t.stride)[:3]) == (3, [4, 2, 3], [6, 3, 1])
