@@ -371,8 +371,8 @@ __global__ __launch_bounds__(256) void axpby_dense_kernel(typename El::compute a
     }
 }
 
-// max / min of values without a NaN among a wave's: the instruction orders the zeros as Julia does (-0.0 < +0.0); with
-// one, Julia's rules spelled out
+// max / min of values without a NaN among a wave's: IEEE 754's maximum / minimum, which order the zeros as Julia does
+// (-0.0 < +0.0; fmaxf / fminf may return either); with one, Julia's rules spelled out
 template <int OP, typename T, int N>
 __device__ __forceinline__ void map_piece(T (&x)[N], const T (&y)[N]) {
     if constexpr ((OP == MOYE_MAP_MAX || OP == MOYE_MAP_MIN) && sizeof(T) == 4) {
@@ -381,7 +381,7 @@ __device__ __forceinline__ void map_piece(T (&x)[N], const T (&y)[N]) {
         for (int k = 0; k < N; ++k) nan |= __builtin_isunordered(x[k], y[k]);
         if (__builtin_amdgcn_ballot_w64(nan) == 0) {
 #pragma unroll
-            for (int k = 0; k < N; ++k) x[k] = OP == MOYE_MAP_MAX ? __builtin_fmaxf(x[k], y[k]) : __builtin_fminf(x[k], y[k]);
+            for (int k = 0; k < N; ++k) x[k] = OP == MOYE_MAP_MAX ? __builtin_elementwise_maximum(x[k], y[k]) : __builtin_elementwise_minimum(x[k], y[k]);
             return;
         }
     }

@@ -1158,3 +1158,23 @@ def test_dense_maps_give_the_element_wise_kernels_bits(mh, dt):
             mh.axpby_(0.75, pitched(aw), beta, pitched(yw))
             torch.cuda.synchronize()
             assert same(yd[1:].view(cols, rows), yw[:, :rows].contiguous()), (dt, rows, cols, "axpby", beta)
+
+
+@pytest.mark.parametrize("dt", ["float32", "float64", "float16", "bfloat16"])
+def test_max_and_min_order_the_zeros(mh, dt):
+    """-0.0 < +0.0, as in Julia: a dense run of zeros of either sign against a scalar zero, an array and a vector that
+    repeats, by sign bits (map_piece where no value is a NaN)."""
+    tdt = getattr(torch, dt)
+    rows, cols = 24, 37
+    g = torch.Generator().manual_seed(4)
+    zeros = lambda n: torch.where(torch.rand(n, generator=g) < 0.5, 0.0, -0.0)
+    a, b, v = zeros(rows * cols), zeros(rows * cols), zeros(rows)
+    A, B, V, d = (x.to(tdt).cuda() for x in (a, b, v, torch.ones(rows * cols)))
+    t = lambda x: _tens(mh, x, (rows, cols), (1, rows))
+    for op in ("max", "min"):
+        for second, arr, scalar in ((b, t(B), 0.0), (v.repeat(cols), _tens(mh, V, (rows,), (1,)), 0.0), (torch.zeros(rows * cols), None, 0.0),
+                                    (-torch.zeros(rows * cols), None, -0.0)):
+            mh.map_(op, t(d), t(A), arr, scalar)
+            torch.cuda.synchronize()
+            neg = torch.signbit(a) & torch.signbit(second) if op == "max" else torch.signbit(a) | torch.signbit(second)
+            assert bool((d == 0).all()) and torch.equal(torch.signbit(d).cpu(), neg), (op, scalar, arr is None)
