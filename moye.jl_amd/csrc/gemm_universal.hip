@@ -367,13 +367,19 @@ int32_t gemm_universal_dispatch(int bm, int bn, int bk, UArgs a, hipStream_t st)
     // sum over k is strictly ascending and no element depends on another whatever they are.  The 32 x 32 tile runs the form
     // for few elements, on tiles of its own: the smaller, the more workgroups, the larger, the fewer LDS reads per product.
     // fp32, us, 16 x 16 / 32 x 32 / 64 x 32: 256^3 6.2 / 11.9 / 18.0; 512^3 21.2 / 22.2 / 32.3; 640^3 39.2 / 32.1 / 40.1; 768^3
-    // 58.2 / 49.4 / 56.9; 1024^3 128.8 / 93.3 / 79.8.  From where 64 x 64 tiles of the kernel above fill the chip on, those.
+    // 58.2 / 49.4 / 56.9; 1024^3 128.8 / 93.3 / 79.8; 30000 x 30 x 300 39.8 / 28.8 / 25.3.  64 x 32 and 64 x 64 (the kernel above) only
+    // where their tiles are full: two workgroups of 64 x 32 to a CU in one round, or seven eighths of more rounds (3000 x 1000
+    // x 500 180 / 113 / 106, but 1040 x 1000 x 200 31.9 / 22.8 / 30.0 and 64 x 64 39.0; 1500^2 x 300 86 / 55 / 61 / 67; 2048^2 x 200
+    // 113 / 65 / 67 / 53), and a side of at most 16 or 32 takes tiles no wider than that (16 x 100000 x 256 50 / 61 / 116 / 103;
+    // 32 x 32768 x 256 33.8 / 24.0 / 38.5 / 49.5).  A launch holds 65535 tiles along N.
     if (bm == 32 && bn == 32 && bk == 8) {
-        const int64_t tiles = (int64_t)((a.M + 31) / 32) * ((a.N + 31) / 32), cus = device_shape().cus;
-        if (tiles <= cus) return launch_small<1, 1, 64>(a, prod, accT, st);
-        if (tiles <= 3 * cus) return launch_small<2, 2, 32>(a, prod, accT, st);
-        if (tiles <= 12 * cus) return launch_small<4, 2, 64>(a, prod, accT, st);
-        return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
+        auto tiles = [&](int64_t tm, int64_t tn) { return ((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn); };
+        const int64_t cus = device_shape().cus, t32 = tiles(32, 32), rounds = (tiles(64, 32) + 2 * cus - 1) / (2 * cus);
+        auto full = [&](int64_t elements) { return 8 * (int64_t)a.M * a.N >= 7 * elements; };
+        if ((t32 <= cus || a.M <= 16 || a.N <= 16) && a.N <= 16 * 65535) return launch_small<1, 1, 64>(a, prod, accT, st);
+        if (a.N > 32 * 65535 || (t32 > 12 * cus && full(tiles(64, 64) * 64 * 64))) return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
+        if (t32 > 3 * cus && (rounds == 1 || full(rounds * 2 * cus * 64 * 32))) return launch_small<4, 2, 64>(a, prod, accT, st);
+        return launch_small<2, 2, 32>(a, prod, accT, st);
     }
     if (bm == 64 && bn == 64 && bk == 8) return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
     if (bm == 128 && bn == 128 && bk == 8) return launch_u<128, 128, 8, 8, 8>(a, prod, accT, st);

@@ -126,6 +126,24 @@ def test_universal_fma_small_tiles_give_the_same_bits(mh, types):
             assert np.array_equal(out[0][1:M + 1, 1:N + 1].cpu().numpy(), want), (M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1048576, 3), (1, 1048577, 3), (16, 30011, 70), (20003, 9, 65), (17, 70001, 33), (40001, 32, 40), (96, 16001, 66), (50000, 96, 30),
+                                   (1041, 1023, 40)])
+@pytest.mark.parametrize("dt", ["float32", "float16"])
+def test_universal_fma_thin_problems_give_the_same_bits(mh, dt, M, N, K):
+    """Many tiles and a short side, on either side of 16 and 32 and of what a launch holds along N: the bits of the
+    128 x 128 kernel, C included, and nothing beside D written."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, b = (torch.randn(n, K, generator=g, device="cuda").to(getattr(torch, dt)) for n in (M, N))
+    c = torch.randn(M, N, generator=g, device="cuda")
+    out = []
+    for tile in ((32, 32, 8), (128, 128, 8)):
+        d = torch.full((M * N + 64,), 7.0, device="cuda")
+        mh.gemm_(mh.tiled_mma_desc(mh.MMA_UNIVERSAL_FMA, cta_tile=tile), T(d[32:], (M, N), (N, 1)), T(a), T(b), T(c))
+        out.append(d)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1]) and bool((out[0][:32] == 7.0).all()) and bool((out[0][-32:] == 7.0).all())
+
+
 @pytest.mark.parametrize("tile", [(32, 32, 8), (64, 64, 8), (128, 128, 8)])
 @pytest.mark.parametrize("types", ["f32", "f16", "bf16", "f16->f16", "bf16->bf16"])
 def test_universal_fma_keeps_the_sign_of_zero(mh, types, tile):
