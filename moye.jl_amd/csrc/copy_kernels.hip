@@ -561,7 +561,8 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
                                 (long long)src->shape[m]);
         }
         TransposeArgs ta;
-        if (transpose_plan(*src, *dst, true, &ta))
+        const bool lds_batch = tc && tc->op == MOYE_COPY_LDS_TILED && src->rank > 2;  // (a batch has no other kernel under that op)
+        if (transpose_plan(*src, *dst, true, &ta) && (lds_batch || transpose_pays(src->dtype, dst->dtype, ta)))
             return transpose_run(src->dtype, dst->dtype, true, tc && (tc->flags & MOYE_GEMM_NO_LDS_SWIZZLE), device_shape().xcds, ta, st);
         // a pair the LDS-tiled op is meant for, but with too few elements along a side: the general kernel moves it
         const bool lds_pair = sb <= 8 && src->rank == 2 && dst->rank == 2 && src->shape[0] == dst->shape[0] && src->shape[1] == dst->shape[1] &&
@@ -575,7 +576,8 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
     // (2b) the same with a conversion on the way
     if (!same_bits && !mask && !(tc && tc->op == MOYE_COPY_LDS_TILED && (tc->tiler_mn[0] || tc->tiler_mn[1]))) {
         TransposeArgs ta;
-        if (transpose_plan(*src, *dst, false, &ta)) return transpose_run(src->dtype, dst->dtype, false, false, device_shape().xcds, ta, st);
+        if (transpose_plan(*src, *dst, false, &ta) && transpose_pays(src->dtype, dst->dtype, ta))
+            return transpose_run(src->dtype, dst->dtype, false, false, device_shape().xcds, ta, st);
     }
 
     // (3) generic

@@ -4,6 +4,7 @@
 // src(i, j) at i + j * lds (i is the source's contiguous index), dst(i, j) at i * ldd + j; further modes count matrices.
 // Any extents, pitches and element-aligned pointers: one launch, no strips.
 #include <algorithm>
+#include <initializer_list>
 
 #include "copy_convert.hpp"
 #include "copy_transpose.hpp"
@@ -32,8 +33,8 @@ __device__ __forceinline__ float element_f32(const u32x4& v, int e) {
     else if constexpr (kSrc == MOYE_BF16) return __uint_as_float(e % 2 ? v[e / 2] & 0xffff0000u : v[e / 2] << 16);
     else return f8e4m3_to_f32((uint8_t)(v[e / 4] >> (8 * (e % 4))));
 }
-// four bytes of results, rounded as store_from rounds them
-template <int kDst, int N>
+// four bytes of results, rounded as store_from rounds them; kFinite: none is a NaN
+template <int kDst, bool kFinite = false, int N>
 __device__ __forceinline__ uint32_t pack_f32(const float (&x)[N]) {
     if constexpr (kDst == MOYE_F32) {
         return __float_as_uint(x[0]);
@@ -44,11 +45,40 @@ __device__ __forceinline__ uint32_t pack_f32(const float (&x)[N]) {
         typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
         return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x[0], (__bf16)x[1]});
     } else {
-        // (the instruction gives every NaN the same sign: only where a lane holds one are the bytes made one by one)
-        const bool nan = __builtin_isunordered(x[0], x[1]) | __builtin_isunordered(x[2], x[3]);
-        if (__builtin_expect(nan, 0))
+        // (the instruction gives every NaN the same sign)
+        if constexpr (!kFinite)
             return f32_to_f8e4m3(x[0]) | ((uint32_t)f32_to_f8e4m3(x[1]) << 8) | ((uint32_t)f32_to_f8e4m3(x[2]) << 16) | ((uint32_t)f32_to_f8e4m3(x[3]) << 24);
         return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false), true);
+    }
+}
+
+// The first `left` elements of a piece, fewer than all: 8, 4, 2 and 1 bytes as they are needed (one store per element took a
+// byte matrix of 1000 x 300 from 4.2 to 7.8 us)
+template <int DB>
+__device__ __forceinline__ void store_first(char* p, u32x4 w, int left) {
+    const int bytes = left * DB;
+    if (bytes & 8) {
+        __builtin_memcpy(p, &w, 8);
+        p += 8;
+        w[0] = w[2];
+        w[1] = w[3];
+    }
+    if constexpr (DB <= 4) {
+        if (bytes & 4) {
+            __builtin_memcpy(p, &w, 4);
+            p += 4;
+            w[0] = w[1];
+        }
+    }
+    if constexpr (DB <= 2) {
+        if (bytes & 2) {
+            __builtin_memcpy(p, &w, 2);
+            p += 2;
+            w[0] >>= 16;
+        }
+    }
+    if constexpr (DB == 1) {
+        if (bytes & 1) *p = (char)w[0];
     }
 }
 
@@ -94,6 +124,49 @@ __device__ __forceinline__ void turn_block(const u32x4 (&v)[16 / DB], u32x4 (&o)
             __builtin_memcpy(&o[e], w, 16);
         }
     } else {
+        if constexpr (kDst == MOYE_F8E4M3) {  // (one test for a lane's block, not one for every four bytes of it)
+            bool nan = false;
+#pragma unroll
+            for (int e = 0; e < ES; ++e)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    float x[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) x[k] = element_f32<kSrc>(v[4 * w + k], e);
+                    nan |= __builtin_isunordered(x[0], x[1]) | __builtin_isunordered(x[2], x[3]);
+                    o[e][w] = pack_f32<kDst, true>(x);
+                }
+            if (__builtin_expect(!nan, 1)) return;
+        }
+        if constexpr (kSrc == MOYE_F8E4M3) {
+            // Two elements to an instruction (a lane's 128 conversions one by one were most of a small call: fp8 -> bf16 1024^2
+            // 5.9 us).  It makes every NaN negative: only a block with a positive one, 0x7f, goes the way below.
+            uint32_t found = 0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint32_t t = v[q][c] ^ 0x7f7f7f7fu;
+                    found |= (t - 0x01010101u) & ~t;  // bit 7 of the lowest byte that is zero
+                }
+            if (__builtin_expect((found & 0x80808080u) == 0, 1)) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        float x[4][4 / DB];
+#pragma unroll
+                        for (int k = 0; k < 4 / DB; ++k) {
+                            const int row = w * (4 / DB) + k;
+                            const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[row][c], false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[row][c], true);
+                            x[0][k] = lo[0]; x[1][k] = lo[1]; x[2][k] = hi[0]; x[3][k] = hi[1];
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[4 * c + e][w] = pack_f32<kDst>(x[e]);
+                    }
+                return;
+            }
+        }
 #pragma unroll
         for (int e = 0; e < ES; ++e)
 #pragma unroll
@@ -114,7 +187,7 @@ __device__ __forceinline__ void turn_block(const u32x4 (&v)[16 / DB], u32x4 (&o)
 //
 // Edges: a lane whose 16 bytes would reach beyond a source row's end reads the row's last 16 bytes instead (some
 // elements then come twice and are written to LDS twice, the same values); rows beyond nj are read from the last row and
-// not stored; the piece that crosses the end of a destination row goes out element by element.
+// not stored; the piece that crosses the end of a destination row goes out in halves.
 //
 // Bound by memory, and by lines that two workgroups share where a pitch is no multiple of 128 bytes.  Against the kernels
 // this one replaced (whole 64 x 64 patches; strips and unaligned pitches element by element), us before -> now:
@@ -211,13 +284,7 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
                 __builtin_nontemporal_store(slot(ES + r0 + RPP * p, jc), reinterpret_cast<u32x4_any*>(d + (int64_t)(RPP * p) * a.ldd * DB));
     } else if (left > 0) {
 #pragma unroll 1
-        for (int p = 0; r0 + RPP * p < min(iw, TI); ++p) {
-            const u32x4 w = slot(ES + r0 + RPP * p, jc);
-            char* const dr = d + (int64_t)(RPP * p) * a.ldd * DB;
-#pragma unroll
-            for (int q = 0; q < Q - 1; ++q)
-                if (q < left) __builtin_memcpy(dr + q * DB, reinterpret_cast<const char*>(&w) + q * DB, DB);
-        }
+        for (int p = 0; r0 + RPP * p < min(iw, TI); ++p) store_first<DB>(d + (int64_t)(RPP * p) * a.ldd * DB, slot(ES + r0 + RPP * p, jc), left);
     }
 }
 
@@ -242,58 +309,198 @@ static int32_t launch_blocks(TransposeArgs a, int lds_request, hipStream_t st) {
     return MOYE_OK;
 }
 
-// Which tile.  Few elements: small tiles, so that there are workgroups for every CU (f16 1024^2: 3.6 us on 64 x 128, 4.3 on
-// 64 x 256).  Rows that are whole 128-byte lines: tiles of 128-byte source runs, 512-byte destination runs (f16 8192^2 50.6
-// us, 55.7 on 128 x 512; f32 8192^2 96.6, 108 on 64 x 256).  Anything else, and arrays far beyond the caches: the longest
-// runs, whose ends are the smallest part of them (f16 10001 x 7003 77 us, 86 on 64 x 256).
+// The first of a list of tiles (its extents along i and j) that takes at most a quarter more than the tightest of them takes
+// over an array's edges.
+struct Tile {
+    int i, j;
+};
+static int first_that_fits(const TransposeArgs& a, std::initializer_list<Tile> tiles) {
+    auto padded = [&](const Tile& t) { return ((int64_t)a.ni + t.i - 1) / t.i * t.i * (((int64_t)a.nj + t.j - 1) / t.j * t.j); };
+    int64_t tightest = padded(*tiles.begin());
+    for (const Tile& t : tiles) tightest = std::min(tightest, padded(t));
+    int n = 0;
+    for (const Tile& t : tiles) {
+        if (4 * padded(t) <= 5 * tightest) return n;
+        ++n;
+    }
+    return 0;
+}
+
+// Which tile, and how the workgroups are spread.  Up to 2 Mi elements: small tiles, so that there are workgroups for every CU; up
+// to 8 Mi: medium ones.  Beyond, rows that are whole 128-byte lines on both sides take tiles whose runs are whole lines,
+// anything else the longest runs, whose ends are the smallest part of them.  In every class a matrix narrower than a tile
+// (batches of small matrices, long strips) takes a tile that it fills.
+//   Order: destination rows first where the source's contiguous extent is at least the destination's (writes are the side that
+// needs locality on this part: 16384^2 f32 341 us, 353 source rows first), else bands of 64 tile columns with the source's
+// index fastest, with whole lines from an extent of 4096 on (4096 x 32768 f32 196 us, 208 the other way; but bf16 -> f32
+// 64 x 1048576 71 and 86).  Neighbouring tiles go to one XCD (`run`), so that lines two of them share meet in one L2 (f32
+// 8192^2 102.8 -> 96.6 us, 16400 x 16392 ~420 -> 405), except where an even spread is worth more: few elements, and whole
+// lines below 64 MiB (f32 2048^2 8.3 -> 7.2).
+//   Measured with operands that are not cached, us, the kernels for whole 64 x 64 patches that this one replaced / one tile for
+// every extent / this rule: fp16 32768 x [64, 64] 85 / 400 / 85; 16384 x [128, 64] 85 / 235 / 87; 1048576 x 128 94 / 148 / 91; 4096^2
+// 15.8 / 14.8 / 12.6; fp32 2048^2 7.4 / 9.2 / 7.2; 16 x [512, 512] 7.2 / 8.6 / 7.1; 1048576 x 64 93 / 106 / 91; 100000 x [33, 33] 552 /
+// 1051 / 206; 4096 x 32768 196 / 209 / 197; bytes 2048^2 4.4 / 4.7 / 4.0, 262144 x 256 26 / 28 / 28; 8-byte elements 256 x 262144
+// 169 / 177 / 169, 8192 x [32, 32] 52 / 72 / 24; bf16 -> fp32 16384 x [64, 128] 139 / 216 / 136; fp8 -> bf16 64 x [1024, 1024] 34 / 40 / 36.
 template <int kSrc, int kDst, int SB, int DB>
 static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
+    constexpr int64_t Mi = 1 << 20;
     const int64_t n = (int64_t)a.ni * a.nj * a.batch, bytes = n * std::max(SB, DB);
     const bool lines = (a.lds * SB) % 128 == 0 && (a.ldd * DB) % 128 == 0;
-    const bool few = n <= (2 << 20), huge = bytes >= ((int64_t)256 << 20);
+    const bool few = n <= 2 * Mi, huge = bytes >= 256 * Mi, narrow = std::min(a.ni, a.nj) <= 512;
+    const bool medium = !few && lines && n <= 8 * Mi;
+    a.run = few || (lines && bytes < 64 * Mi) ? 1 : 4;
+    if (a.batch == 1 && a.ni < a.nj && (a.ni >= 4096 || !(few || lines))) a.band = 64;
+    auto fit = [&](std::initializer_list<Tile> tiles) { return first_that_fits(a, tiles); };
+#define MOYE_TILE(PI, NB, T, LDS) return launch_blocks<kSrc, kDst, SB, DB, PI, NB, T>(a, LDS, st)
     if constexpr (SB == 2 && DB == 2) {
-        if (few) return launch_blocks<kSrc, kDst, 2, 2, 8, 1, 128>(a, 0, st);
-        if (n <= (8 << 20)) return launch_blocks<kSrc, kDst, 2, 2, 16, 1, 256>(a, 0, st);
-        if (lines && !huge) return launch_blocks<kSrc, kDst, 2, 2, 8, 1, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 2, 2, 16, 2, 512>(a, 0, st);
+        if (few) switch (fit({{128, 64}, {64, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(16, 1, 128, 0);
+            case 1: MOYE_TILE(8, 1, 128, 0);
+            default: MOYE_TILE(8, 1, 64, 0);
+        }
+        if (n <= 8 * Mi) switch (fit({{128, 128}, {128, 64}, {64, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(16, 1, 256, 0);
+            case 1: MOYE_TILE(16, 1, 128, 0);
+            case 2: MOYE_TILE(8, 1, 128, 0);
+            default: MOYE_TILE(8, 1, 64, 0);
+        }
+        if (!lines || (n <= 16 * Mi && !narrow)) switch (fit({{128, 512}, {128, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(16, 2, 512, 0);
+            case 1: MOYE_TILE(16, 1, 256, 0);
+            default: MOYE_TILE(8, 1, 64, 0);
+        }
+        if (huge) switch (fit({{128, 256}, {128, 128}, {128, 64}})) {
+            case 0: MOYE_TILE(16, 2, 256, 0);
+            case 1: MOYE_TILE(16, 1, 256, 0);
+            default: MOYE_TILE(16, 1, 128, 0);
+        }
+        if (!narrow && a.batch == 1) MOYE_TILE(8, 1, 256, 0);
+        switch (fit({{256, 64}, {64, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(32, 1, 256, 0);
+            case 1: MOYE_TILE(8, 1, 128, 0);
+            default: MOYE_TILE(8, 1, 64, 0);
+        }
     } else if constexpr (SB == 4 && DB == 4) {
-        // (one workgroup per CU, for which the LDS request sees, where the array is far beyond the caches: 16384^2 341 us
-        // against 344; and the tiles in plain order then: 341 against 357)
-        const bool far = bytes >= ((int64_t)600 << 20);
-        if (far && lines && a.band == 0) a.run = 1;
-        if (far || (!lines && bytes >= ((int64_t)32 << 20))) return launch_blocks<kSrc, kDst, 4, 4, 16, 2, 512>(a, 96 * 1024, st);
-        if (few || lines) return launch_blocks<kSrc, kDst, 4, 4, 8, 1, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 4, 4, 16, 2, 256>(a, 0, st);
+        constexpr int kAlone = 96 * 1024;  // one workgroup per CU, where the arrays are far beyond the caches
+        if (few) { if (fit({{32, 64}, {64, 64}}) == 0) MOYE_TILE(8, 1, 128, 0); else MOYE_TILE(16, 2, 128, 0); }
+        if (medium) { if (fit({{128, 64}, {64, 64}}) == 0) MOYE_TILE(32, 2, 256, 0); else MOYE_TILE(16, 2, 128, 0); }
+        if (!lines) switch (bytes >= 32 * Mi ? fit({{64, 256}, {128, 128}, {64, 64}}) : 3 + fit({{64, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(16, 2, 512, kAlone);
+            case 1: MOYE_TILE(32, 4, 256, 0);
+            case 3: MOYE_TILE(16, 2, 256, 0);
+            default: MOYE_TILE(16, 2, 128, 0);
+        }
+        if (a.ni <= 128) MOYE_TILE(32, 2, 256, 0);
+        if (narrow) { if (fit({{64, 128}, {64, 64}}) == 0) MOYE_TILE(16, 2, 256, 0); else MOYE_TILE(16, 1, 256, 0); }
+        if (bytes >= 600 * Mi) {  // (the tiles in plain order: 16384^2 341 us against 357)
+            if (a.band == 0) a.run = 1;
+            MOYE_TILE(16, 2, 512, kAlone);
+        }
+        if (a.band) MOYE_TILE(32, 4, 256, 0);
+        MOYE_TILE(8, 1, 256, 0);
     } else if constexpr (SB == 1 && DB == 1) {
-        if (n <= (6 << 20)) return launch_blocks<kSrc, kDst, 1, 1, 4, 1, 64>(a, 0, st);
-        if (n <= (64 << 20)) return launch_blocks<kSrc, kDst, 1, 1, 16, 1, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 1, 1, 8, 1, 256>(a, 0, st);
+        if (n <= 6 * Mi || medium) switch (fit({{256, 64}, {128, 128}, {64, 256}})) {
+            case 0: MOYE_TILE(16, 1, 64, 0);
+            case 1: MOYE_TILE(8, 1, 64, 0);
+            default: MOYE_TILE(4, 1, 64, 0);
+        }
+        if (!lines && n <= 8 * Mi) { if (fit({{256, 128}, {256, 64}}) == 0) MOYE_TILE(16, 1, 128, 0); else MOYE_TILE(16, 1, 64, 0); }
+        switch (n > 64 * Mi                         ? 1 + fit({{128, 512}, {256, 128}, {256, 64}})
+                : !lines                            ? fit({{256, 256}, {128, 512}, {256, 128}, {256, 64}})
+                : a.batch == 1                      ? 4 + fit({{256, 256}, {256, 128}, {128, 256}, {256, 64}})
+                                                    : 5 + fit({{256, 128}, {128, 256}, {256, 64}})) {
+            case 0: case 4: MOYE_TILE(16, 1, 256, 0);
+            case 1: MOYE_TILE(8, 1, 256, 0);
+            case 2: case 5: MOYE_TILE(16, 1, 128, 0);
+            case 6: MOYE_TILE(8, 1, 128, 0);
+            default: MOYE_TILE(16, 1, 64, 0);
+        }
     } else if constexpr (SB == 8 && DB == 8) {
-        if (bytes < ((int64_t)24 << 20)) return launch_blocks<kSrc, kDst, 8, 8, 16, 4, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 8, 8, 32, 4, 512>(a, 96 * 1024, st);
+        if (few) { if (fit({{32, 64}, {32, 32}}) == 0) MOYE_TILE(16, 4, 128, 0); else MOYE_TILE(16, 2, 128, 0); }
+        if (medium) { if (fit({{64, 64}, {32, 32}}) == 0) MOYE_TILE(32, 4, 256, 0); else MOYE_TILE(16, 2, 128, 0); }
+        if (!lines) switch (fit({{64, 128}, {64, 64}, {32, 32}})) {
+            case 0: MOYE_TILE(32, 4, 512, bytes >= 24 * Mi ? 96 * 1024 : 0);
+            case 1: MOYE_TILE(32, 4, 256, 0);
+            default: MOYE_TILE(16, 2, 128, 0);
+        }
+        if (huge && a.nj > 128 && fit({{64, 128}, {64, 64}}) == 0) {  // (plain order from 1 GiB: 16384^2 699 us against 774, 8192^2 185 and 180)
+            if (bytes >= 1024 * Mi || a.ni < a.nj) a.run = 1;
+            a.band = 0;
+            MOYE_TILE(32, 4, 512, 96 * 1024);
+        }
+        MOYE_TILE(32, 2, 512, 0);
     } else if constexpr (SB == 4 && DB == 2) {
-        if (few) return launch_blocks<kSrc, kDst, 4, 2, 8, 1, 128>(a, 0, st);
-        if (lines) return launch_blocks<kSrc, kDst, 4, 2, 16, 1, 512>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 4, 2, 16, 2, 512>(a, 0, st);
+        if (few) { if (fit({{32, 64}, {64, 64}}) == 0) MOYE_TILE(8, 1, 64, 0); else MOYE_TILE(16, 1, 128, 0); }
+        if (medium) MOYE_TILE(16, 1, 128, 0);
+        if (!lines) {
+            const int t = fit({{64, 512}, {128, 128}, {64, 64}});
+            if (t == 0) MOYE_TILE(16, 2, 512, 0);
+            if (t == 1) MOYE_TILE(32, 1, 512, 0); else MOYE_TILE(16, 1, 128, 0);
+        }
+        if (narrow || a.batch > 1) switch (fit({{128, 128}, {64, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(32, 1, 512, 0);
+            case 1: MOYE_TILE(16, 1, 256, 0);
+            default: MOYE_TILE(16, 1, 128, 0);
+        }
+        if (n <= 16 * Mi) MOYE_TILE(32, 1, 256, 0);
+        MOYE_TILE(16, 1, 512, 0);
     } else if constexpr (SB == 2 && DB == 4) {
-        if (few) return launch_blocks<kSrc, kDst, 2, 4, 8, 1, 128>(a, 0, st);
-        if (lines && !huge) return launch_blocks<kSrc, kDst, 2, 4, 8, 1, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 2, 4, 16, 2, 512>(a, 0, st);
+        if (few) MOYE_TILE(8, 1, 128, 0);
+        if (!lines) switch (fit({{128, 256}, {128, 128}, {64, 64}})) {
+            case 0: MOYE_TILE(16, 2, 512, 0);
+            case 1: MOYE_TILE(16, 2, 256, 0);
+            default: MOYE_TILE(8, 1, 128, 0);
+        }
+        if (medium || std::min(a.ni, a.nj) <= 128 || (narrow && a.batch > 1)) {
+            if (fit({{128, 64}, {64, 64}}) == 0) MOYE_TILE(16, 1, 256, 0); else MOYE_TILE(8, 1, 128, 0);
+        }
+        if (huge) MOYE_TILE(16, 2, 256, 0);
+        MOYE_TILE(8, 1, 256, 0);
     } else if constexpr (SB == 4 && DB == 1) {
-        if (few) return launch_blocks<kSrc, kDst, 4, 1, 8, 1, 128>(a, 0, st);
-        if (n <= (8 << 20)) return launch_blocks<kSrc, kDst, 4, 1, 16, 1, 256>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 4, 1, 16, 1, 512>(a, 0, st);
+        if (few) MOYE_TILE(16, 1, 64, 0);
+        if (medium) { if (fit({{128, 64}, {64, 64}}) == 0) MOYE_TILE(32, 1, 128, 0); else MOYE_TILE(16, 1, 64, 0); }
+        switch (!lines && n <= 8 * Mi ? 1 + fit({{64, 256}, {64, 64}})
+                : lines && huge       ? 3 + fit({{128, 128}, {64, 256}, {64, 64}})
+                                      : 6 + fit({{64, 512}, {64, 256}, {128, 64}, {64, 64}})) {
+            case 1: case 4: case 7: MOYE_TILE(16, 1, 256, 0);
+            case 3: MOYE_TILE(32, 1, 256, 0);
+            case 6: MOYE_TILE(16, 1, 512, 0);
+            case 8: MOYE_TILE(32, 1, 128, 0);
+            default: MOYE_TILE(16, 1, 64, 0);
+        }
     } else if constexpr (SB == 2 && DB == 1) {
-        if (n <= (8 << 20)) return launch_blocks<kSrc, kDst, 2, 1, 8, 1, 128>(a, 0, st);
-        return launch_blocks<kSrc, kDst, 2, 1, 16, 1, 256>(a, 0, st);
-    } else if constexpr (SB == 1) {  // runs of 64 or 128 bytes in, 512 or 1024 out
-        return launch_blocks<kSrc, kDst, 1, DB, DB == 8 ? 4 : 8, 1, 256>(a, 0, st);
+        if (few || medium) { if (fit({{64, 128}, {128, 64}}) == 0) MOYE_TILE(8, 1, 64, 0); else MOYE_TILE(16, 1, 64, 0); }
+        switch (fit({{128, 256}, {128, 128}, {64, 256}, {128, 64}})) {
+            case 0: MOYE_TILE(16, 1, 256, 0);
+            case 1: MOYE_TILE(16, 1, 128, 0);
+            case 2: MOYE_TILE(8, 1, 128, 0);
+            default: MOYE_TILE(16, 1, 64, 0);
+        }
+    } else if constexpr (SB == 1 && DB == 2) {
+        if (few) { if (fit({{128, 64}, {64, 128}}) == 0) MOYE_TILE(8, 1, 64, 0); else MOYE_TILE(4, 1, 64, 0); }
+        switch (medium   ? 1 + fit({{128, 128}, {128, 64}})
+                : !lines ? fit({{128, 256}, {128, 128}, {128, 64}})
+                         : 3 + fit({{256, 128}, {256, 64}, {128, 64}})) {
+            case 0: MOYE_TILE(8, 1, 256, 0);
+            case 1: MOYE_TILE(8, 1, 128, 0);
+            case 3: MOYE_TILE(16, 1, 256, 0);
+            case 4: MOYE_TILE(16, 1, 128, 0);
+            default: MOYE_TILE(8, 1, 64, 0);
+        }
+    } else if constexpr (SB == 1 && DB == 4) {
+        if (few || medium) MOYE_TILE(4, 1, 64, 0);
+        if (!lines) { if (fit({{128, 128}, {64, 64}}) == 0) MOYE_TILE(8, 1, 256, 0); else MOYE_TILE(4, 1, 64, 0); }
+        if (fit({{128, 64}, {64, 64}}) == 0) MOYE_TILE(8, 1, 128, 0); else MOYE_TILE(4, 1, 64, 0);
+    } else if constexpr (SB == 1) {
+        static_assert(DB == 8, "every pair of sizes");
+        MOYE_TILE(4, 1, 256, 0);
     } else if constexpr (SB == 8) {
-        return launch_blocks<kSrc, kDst, 8, DB, 16, DB == 4 ? 2 : 1, 256>(a, 0, st);
+        MOYE_TILE(16, DB == 4 ? 2 : 1, 256, 0);
     } else {
         static_assert(DB == 8, "every pair of sizes");
-        return launch_blocks<kSrc, kDst, SB, 8, SB == 4 ? 16 : 8, SB == 4 ? 4 : 2, 256>(a, 0, st);
+        MOYE_TILE(SB == 4 ? 16 : 8, SB == 4 ? 4 : 2, 256, 0);
     }
+#undef MOYE_TILE
 }
 
 template <int kSrc, int SB>
@@ -344,14 +551,25 @@ bool transpose_plan(const moye_tensor& src, const moye_tensor& dst, bool same_bi
     return true;
 }
 
-// Which order.  Destination rows first where the source's contiguous extent is at least the destination's: writes are the
-// side that needs locality on this part (16384^2 f32: 341 us, 353 source rows first), else bands of 64 tile columns with
-// the source's index fastest (4096 x 32768 f32 192 us, 202 the other way).  Four neighbouring tiles to an XCD, so that
-// lines two of them share meet in one L2 (f32 8192^2 102.8 -> 96.6 us, 16400 x 16392 ~420 -> 405).
+// Few elements, of one or two bytes, are a chain of latencies in a lane's block (16 loads and 256 bytes to turn for bytes), the
+// longer one where destination rows end inside a piece; the general kernel has a wave for every 64 elements.  us, that one / this one:
+// bytes 201 x 303 3.5 / 5.6, 700 x 500 4.9 / 5.8, 1001 x 700 6.9 / 6.8, 256 x 256 3.5 / 3.0; bf16 -> fp8 256 x 256 3.2 / 4.1, 700 x
+// 500 4.5 / 5.5; fp16 128 x 128 2.5 / 2.2, 500 x 300 4.0 / 4.4, 700 x 500 4.9 / 4.4; fp8 -> fp32 201 x 303 3.4 / 5.4, 500 x 300 3.8 / 4.2; bf16 -> fp32 201 x 303
+// 3.1 / 4.0, 128 x 128 3.0 / 2.4; fp32 201 x 303 3.6 / 3.5, 128 x 128 3.0 / 2.3.
+bool transpose_pays(int32_t src_dt, int32_t dst_dt, const TransposeArgs& a) {
+    const int sb = dtype_bytes(src_dt), db = dtype_bytes(dst_dt), lo = std::min(sb, db), hi = std::max(sb, db);
+    const bool whole = a.nj % (16 / db) == 0;
+    const int64_t n = (int64_t)a.ni * a.nj * a.batch;
+    if (hi == 8 || lo == 4) return true;
+    if (lo == 1 && hi <= 2) return n > (!whole ? 512 << 10 : hi == 2 ? 64 << 10 : 12 << 10);
+    if (lo == 2 && hi == 2) return n > (whole ? 8 << 10 : 160 << 10);
+    if (lo == 1) return whole || n > (160 << 10);
+    return whole || n > (64 << 10);
+}
+
 int32_t transpose_run(int32_t src_dt, int32_t dst_dt, bool same_bits, bool linear_lds, int xcds, TransposeArgs a, hipStream_t st) {
-    a.band = a.ni >= a.nj || a.batch > 1 ? 0 : 64;
+    a.band = 0;  // (the tile's choice may set both)
     a.xcds = xcds;
-    a.run = 4;
     a.linear = linear_lds;
     if (same_bits) {
         switch (dtype_bytes(src_dt)) {

@@ -22,6 +22,8 @@ struct TransposeArgs {
 
 // Is this copy one (arrays of one shape, mode by mode, the unit strides on different modes of 32 and more elements)?
 bool transpose_plan(const moye_tensor& src, const moye_tensor& dst, bool same_bits, TransposeArgs* a);
+// Does it pay (against the general kernel, element by element)?
+bool transpose_pays(int32_t src_dt, int32_t dst_dt, const TransposeArgs& a);
 int32_t transpose_run(int32_t src_dt, int32_t dst_dt, bool same_bits, bool linear_lds, int xcds, TransposeArgs a, hipStream_t st);
 
 }  // namespace moye

@@ -1178,3 +1178,33 @@ def test_max_and_min_order_the_zeros(mh, dt):
             torch.cuda.synchronize()
             neg = torch.signbit(a) & torch.signbit(second) if op == "max" else torch.signbit(a) | torch.signbit(second)
             assert bool((d == 0).all()) and torch.equal(torch.signbit(d).cpu(), neg), (op, scalar, arr is None)
+
+
+@pytest.mark.parametrize("pair", [("float32", "float32"), ("float16", "float16"), ("uint8", "uint8"), ("float32", "bfloat16"), ("float8_e4m3fn", "float16")])
+def test_batches_of_ragged_transposes_in_one_launch(mh, pair):
+    """More matrices than one grid dimension takes (32768), and three modes that count them in an order of their own on
+    either side; odd extents, pitches and pointers, nothing written beside dst."""
+    ts, td = (getattr(torch, t) for t in pair)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32}
+    for logical, s_order, s_pad, d_order, d_pad in [
+        ((33, 35, 40000), (2, 1, 0), 0, (2, 0, 1), 0),
+        ((33, 41, 3, 5, 7), (3, 2, 1, 4, 0), 2, (4, 2, 0, 3, 1), 3),
+        ((130, 67, 2, 3, 2), (4, 1, 2, 3, 0), 1, (2, 3, 4, 0, 1), 0),
+    ]:
+        def storage(order, pad, dtype, fill):   # a buffer one element off alignment, its innermost mode padded
+            sizes = [logical[m] for m in order]
+            sizes[-1] += pad
+            n = int(np.prod(sizes))
+            buf = torch.full((n + 2,), fill, dtype=torch.uint8 if dtype.itemsize == 1 else dtype, device="cuda")
+            view = buf.view(dtype)[1:1 + n].view(sizes)
+            return buf, view[..., :logical[order[-1]]].permute([order.index(m) for m in range(len(order))])
+        sbuf, src = storage(s_order, s_pad, ts, 0)
+        vals = torch.randint(0, 100, (sbuf.numel(),), generator=g, device="cuda")
+        sbuf.copy_(vals if ts.itemsize == 1 else vals.to(ts) - 50)        # (as an fp8, a byte below 100 is finite)
+        dbuf, dst = storage(d_order, d_pad, td, 77)
+        want, expect = storage(d_order, d_pad, td, 77)
+        expect.copy_(src.float().to(td) if ts != td else src)
+        mh.copyto_(_tens(mh, dst, tuple(dst.shape), tuple(dst.stride())), _tens(mh, src, tuple(src.shape), tuple(src.stride())))
+        torch.cuda.synchronize()
+        assert torch.equal(dbuf.view(bits[td.itemsize]), want.view(bits[td.itemsize])), (pair, logical)
