@@ -430,13 +430,39 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
             const bool k_tail = k_bytes_all % 128 != 0;
             const double guarded = 1.03;
             const int tm = (a.M + 255) / 256, tn = (a.N + 255) / 256;
-            auto alone = [&](int64_t m, int64_t n) {  // what the library would run the rest as, priced
-                double us = gemm_plan(m, n, k_bytes_all, eb == 4, m % 64 == 0 && n % 64 == 0 && !k_tail, 16, cus, 1).us;
-                if (m % 128 || n % 128 || k_tail) us /= 1.15;
-                if (gemm_short_m(m, n, k_bytes_all, eb == 4, cus)) gemm_short_m_ntw(m, n, k_bytes_all, cus, 1, &us);
-                return us;
+            // What the dispatcher runs the rest on, priced.  The 1.15 comes off where 128 x 128 tiles carry it.  64 x 64 tiles have
+            // no ragged form: two or three of them on a CU take about as much less than their price, one takes all of it (f16
+            // 4992 x 3200 x 8320, 156 workgroups for the rest, 265 us in one launch, 286 in two), and of the price of four only
+            // the launch, which is counted below, can come off (bf16 2240 x 8640 x 5248, 945 for 448 rows, 219 and 228, 198
+            // by columns; fp8 16320 x 1280 x 9856, 1020, 208 either way, 192 by columns).
+            bool on64 = false;
+            auto alone = [&](int64_t m, int64_t n) {
+                double us;
+                on64 = false;
+                if (gemm_short_m(m, n, k_bytes_all, eb == 4, cus)) {
+                    gemm_short_m_ntw(m, n, k_bytes_all, cus, 1, &us);
+                    return us;
+                }
+                const TileChoice t = gemm_plan(m, n, k_bytes_all, eb == 4, aligned && m % 64 == 0 && n % 64 == 0 && !k_tail, 16, cus, 1);
+                const bool whole128 = m % 128 == 0 && n % 128 == 0 && !k_tail, whole256 = whole128 && m % 256 == 0 && n % 256 == 0;
+                // (256 x 256 tiles: their 1.25 for ragged ones is too much where they fill most of the chip)
+                const double on256 = gemm_plan_cost_256(m, n, k_bytes_all, eb == 4, !whole256, cus);
+                const bool takes256 = ((m + 255) / 256) * ((n + 255) / 256) >= cus / 4 && on256 <= t.us;
+                on64 = t.tile == 64 && !takes256;
+                const int64_t tiles64 = m / 64 * (n / 64);
+                us = (t.tile == 128 && whole128) || (on64 && eb != 4 && tiles64 <= cus) ? t.us : t.us / 1.15;
+                if (on64 && tiles64 > 3 * (int64_t)cus) us = std::max(us, t.us - 3.0);
+                return takes256 ? std::min(on256, us) : us;
             };
-            double best_us = (eb == 4 ? 0.88 : 0.92) * (prefer256 ? guarded * gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, false, cus) : choice.us);
+            // One launch.  Its 128 x 128 tiles do not carry the 1.15 where they fill two rounds of two to a CU and lose half a tile along
+            // one edge; against a rest on 64 x 64 tiles that decides (bf16 5056 x 3200 x 1920 62 us in one launch, 76 in two; fp8
+            // 7552 x 2112 x 4608 79 and 88; but bf16 1088 x 13952 x 2304, 64 rows left for the short-M kernel, 92 and 82).
+            const bool half_tile = eb != 4 && choice.tile == 128 && !k_tail && a.M % 64 == 0 && a.N % 64 == 0 && (a.M % 128 == 0) != (a.N % 128 == 0) &&
+                                   (((int64_t)a.M + 127) / 128) * (((int64_t)a.N + 127) / 128) <= 4 * (int64_t)cus;
+            const double one_us = prefer256 ? guarded * gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, false, cus) : choice.us;
+            // (fp32: 12 %, but 6 against one launch of 64 x 64 tiles, whose price holds: 5440 x 4544 x 768 338 -> 314 us)
+            const double margin = eb != 4 ? 0.92 : !prefer256 && choice.tile == 64 ? 0.94 : 0.88;
+            double best_us = margin * one_us;
             int64_t m1 = 0, n1 = 0;
             for (const bool by_rows : {true, false}) {
                 const int other = by_rows ? tn : tm, nt = by_rows ? tm : tn;
@@ -445,9 +471,9 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
                     if (first < 1 || first >= nt) continue;
                     const int64_t m = by_rows ? first * 256 : a.M, n = by_rows ? a.N : first * 256;
                     const bool whole = aligned && !k_tail && m % 256 == 0 && n % 256 == 0;
-                    const double us = (whole ? 1.0 : guarded) * gemm_plan_cost_256(m, n, k_bytes_all, eb == 4, false, cus) + 2.0 +
-                                      (by_rows ? alone(a.M - m, a.N) : alone(a.M, a.N - n));
-                    if (us < best_us) { best_us = us; m1 = m; n1 = n; }
+                    const double rest = by_rows ? alone(a.M - m, a.N) : alone(a.M, a.N - n);
+                    const double us = (whole ? 1.0 : guarded) * gemm_plan_cost_256(m, n, k_bytes_all, eb == 4, false, cus) + 2.0 + rest;
+                    if (us < best_us && !(on64 && half_tile && !prefer256 && us >= margin * one_us / 1.15)) { best_us = us; m1 = m; n1 = n; }
                 }
             }
             if (m1 > 0) {

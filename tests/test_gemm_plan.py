@@ -431,3 +431,22 @@ def test_a_last_round_of_ragged_tiles_gets_a_launch_of_its_own(M, N, K, first, d
     m, n = (s[0]["M"], s[0]["N"]) if d_major == "n" else (s[0]["N"], s[0]["M"])
     assert len(s) == 2 and s[0]["tile"].startswith("256x256") and (m, n, "ragged" in s[0]["flags"]) == first, p["text"]
     assert len(run_case(mh.BF16, mh.BF16, min(M, 4000), min(N, 4000), K, d_major=d_major, waves=(1, 1, 1))["steps"]) == 1
+
+
+@pytest.mark.parametrize("in_dt,M,N,K,launches", [
+    (mh.BF16, 5056, 3200, 1920, 1),      # two rounds of 128 x 128 tiles against 240 + 158 workgroups
+    (mh.F8E4M3, 7552, 2112, 4608, 1),
+    (mh.F16, 4992, 3200, 8320, 1),       # 64 x 64 tiles with a CU to themselves cost what they are priced at
+    (mh.F16, 7360, 15872, 5248, 2),
+    (mh.BF16, 1088, 13952, 2304, 2),     # a rest for the short-M kernel
+    (mh.BF16, 5440, 8320, 720, 2),       # a rest on 256 x 256 tiles
+    (mh.BF16, 2240, 8640, 5248, 2),
+    (mh.F8E4M3, 16320, 1280, 9856, 2),
+    (mh.F32, 5440, 4544, 768, 2),
+])
+def test_the_rest_of_a_ragged_problem_is_priced_as_what_runs(in_dt, M, N, K, launches):
+    """One or two launches where both were timed; no 16-bit or fp8 rest goes to four 64 x 64 tiles on a CU over a long K."""
+    p = run_case(in_dt, mh.F32 if in_dt == mh.F32 else mh.BF16, M, N, K, waves=(1, 1, 1))
+    s = [s for s in p["steps"] if s["what"] == "kernel"]
+    assert len(s) == launches, p["text"]
+    assert in_dt == mh.F32 or K < 5000 or not (s[-1]["tile"].startswith("64x64") and s[-1]["M"] * s[-1]["N"] > 3 * 256 * 64 * 64), p["text"]
