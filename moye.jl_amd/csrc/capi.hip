@@ -413,8 +413,8 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         st.kind = GemmStep::kUniversal;
         st.uargs = UArgs{A.ptr, B.ptr, tC ? C.ptr : nullptr, D.ptr, M, N, K, A.rs, A.cs, B.rs, B.cs,
                          C.rs, C.cs, D.rs, D.cs, alpha, A.dtype, B.dtype, tC ? C.dtype : D.dtype, D.dtype};
-        st.ubm = bm; st.ubn = bn; st.ubk = bk;
-        if (plan.named) snprintf(st.name, sizeof st.name, "gemm_universal<%d,%d,%d>", bm, bn, bk);
+        if (int32_t e = gemm_universal_choose(bm, bn, bk, st.uargs, cus, &st.utile)) return e;
+        if (plan.named) snprintf(st.name, sizeof st.name, "%s", gemm_universal_name(st.utile));
         return MOYE_OK;
     }
     const int32_t in_dt = atom_input_dtype(mma->atom);
@@ -568,7 +568,7 @@ static int32_t gemm_plan_run(const GemmPlan& plan, hipStream_t st) {
                 if (int32_t e = splitk_reduce_dispatch(s.partials, s.split, s.args.M, s.args.N, s.args, s.out_dt, st)) return e;
                 break;
             case GemmStep::kUniversal:
-                if (int32_t e = gemm_universal_dispatch(s.ubm, s.ubn, s.ubk, s.uargs, st)) return e;
+                if (int32_t e = gemm_universal_dispatch(s.utile, s.uargs, st)) return e;
                 break;
         }
     }

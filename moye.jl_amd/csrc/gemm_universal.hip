@@ -344,15 +344,16 @@ static int32_t launch_u(const UArgs& a, int prod, int accT, hipStream_t st) {
 
 static int type_class(int dt) { return dt == MOYE_F16 ? 1 : dt == MOYE_BF16 ? 2 : 0; }
 
-int32_t gemm_universal_dispatch(int bm, int bn, int bk, UArgs a, hipStream_t st) {
+// the type of the product, promote_type(TA, TB): the narrow one only when both operands have it
+static int product_class(const UArgs& a) { return type_class(a.a_dt) == type_class(a.b_dt) ? type_class(a.a_dt) : 0; }
+
+int32_t gemm_universal_choose(int bm, int bn, int bk, const UArgs& a, int cus, UniversalTile* tile) {
     for (int dt : {a.a_dt, a.b_dt, a.d_dt, a.C ? a.c_dt : MOYE_F32})
         if (dt != MOYE_F32 && dt != MOYE_F16 && dt != MOYE_BF16)
             return fail(MOYE_ERR_UNSUPPORTED, "gemm!: UniversalFMA kernels take f32, f16 or bf16, not %s", dtype_name(dt));
-    // promote_type(TA, TB): the narrow type only when both operands have it
-    const int prod = type_class(a.a_dt) == type_class(a.b_dt) ? type_class(a.a_dt) : 0;
     // the running sum lives in the accumulator type TC == TD
     const int accT = type_class(a.d_dt);
-    if (accT != 0 && accT != prod)
+    if (accT != 0 && accT != product_class(a))
         return fail(MOYE_ERR_UNSUPPORTED, "gemm!: a %s accumulator needs %s operands", dtype_name(a.d_dt), dtype_name(a.d_dt));
     if (a.C && a.c_dt != a.d_dt)
         return fail(MOYE_ERR_UNSUPPORTED, "gemm!: C and D must have the same element type");
@@ -374,16 +375,39 @@ int32_t gemm_universal_dispatch(int bm, int bn, int bk, UArgs a, hipStream_t st)
     // 32 x 32768 x 256 33.8 / 24.0 / 38.5 / 49.5).  A launch holds 65535 tiles along N.
     if (bm == 32 && bn == 32 && bk == 8) {
         auto tiles = [&](int64_t tm, int64_t tn) { return ((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn); };
-        const int64_t cus = device_shape().cus, t32 = tiles(32, 32), rounds = (tiles(64, 32) + 2 * cus - 1) / (2 * cus);
+        const int64_t t32 = tiles(32, 32), rounds = (tiles(64, 32) + 2 * cus - 1) / (2 * cus);
         auto full = [&](int64_t elements) { return 8 * (int64_t)a.M * a.N >= 7 * elements; };
-        if ((t32 <= cus || a.M <= 16 || a.N <= 16) && a.N <= 16 * 65535) return launch_small<1, 1, 64>(a, prod, accT, st);
-        if (a.N > 32 * 65535 || (t32 > 12 * cus && full(tiles(64, 64) * 64 * 64))) return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
-        if (t32 > 3 * cus && (rounds == 1 || full(rounds * 2 * cus * 64 * 32))) return launch_small<4, 2, 64>(a, prod, accT, st);
-        return launch_small<2, 2, 32>(a, prod, accT, st);
+        if ((t32 <= cus || a.M <= 16 || a.N <= 16) && a.N <= 16 * 65535) *tile = UniversalTile::k16x16;
+        else if (a.N > 32 * 65535 || (t32 > 12 * cus && full(tiles(64, 64) * 64 * 64))) *tile = UniversalTile::k64x64;
+        else if (t32 > 3 * cus && (rounds == 1 || full(rounds * 2 * cus * 64 * 32))) *tile = UniversalTile::k64x32;
+        else *tile = UniversalTile::k32x32;
+        return MOYE_OK;
     }
-    if (bm == 64 && bn == 64 && bk == 8) return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
-    if (bm == 128 && bn == 128 && bk == 8) return launch_u<128, 128, 8, 8, 8>(a, prod, accT, st);
-    return fail(MOYE_ERR_UNSUPPORTED, "gemm!: UniversalFMA CTA tile %dx%dx%d not built (32x32x8, 64x64x8, 128x128x8)", bm, bn, bk);
+    if (bm == 64 && bn == 64 && bk == 8) *tile = UniversalTile::k64x64;
+    else if (bm == 128 && bn == 128 && bk == 8) *tile = UniversalTile::k128x128;
+    else return fail(MOYE_ERR_UNSUPPORTED, "gemm!: UniversalFMA CTA tile %dx%dx%d not built (32x32x8, 64x64x8, 128x128x8)", bm, bn, bk);
+    return MOYE_OK;
+}
+
+const char* gemm_universal_name(UniversalTile tile) {
+    switch (tile) {
+        case UniversalTile::k16x16: return "gemm_universal_fma_small<16,16,64>";
+        case UniversalTile::k32x32: return "gemm_universal_fma_small<32,32,32>";
+        case UniversalTile::k64x32: return "gemm_universal_fma_small<64,32,64>";
+        case UniversalTile::k64x64: return "gemm_universal_fma<64,64,8>";
+        default: return "gemm_universal_fma<128,128,8>";
+    }
+}
+
+int32_t gemm_universal_dispatch(UniversalTile tile, const UArgs& a, hipStream_t st) {
+    const int prod = product_class(a), accT = type_class(a.d_dt);
+    switch (tile) {
+        case UniversalTile::k16x16: return launch_small<1, 1, 64>(a, prod, accT, st);
+        case UniversalTile::k32x32: return launch_small<2, 2, 32>(a, prod, accT, st);
+        case UniversalTile::k64x32: return launch_small<4, 2, 64>(a, prod, accT, st);
+        case UniversalTile::k64x64: return launch_u<64, 64, 8, 4, 4>(a, prod, accT, st);
+        default: return launch_u<128, 128, 8, 8, 8>(a, prod, accT, st);
+    }
 }
 
 }  // namespace moye

@@ -72,6 +72,8 @@ inline bool row_offsets_fit(const GemmArgs& a, int rows, int elem_bytes) {
 // The host code that chooses kernels (capi.hip: gemm_plan_build; gemm_mfma.hip and the kernel files' dispatch functions)
 // launches nothing: it appends steps to a GemmPlan.  gemm_plan_run (capi.hip) then enqueues them on a stream, and
 // moye_gemm_explain prints them.  Building a plan touches no device, so it runs, and is tested, on hosts without one.
+// The UniversalFMA kernels' instances: elements of D per workgroup (gemm_universal.hip)
+enum class UniversalTile { k16x16, k32x32, k64x32, k64x64, k128x128 };
 struct GemmStep {
     enum Kind { kKernel, kKMajorCopy, kSplitKReduce, kUniversal } kind = kKernel;
     // kKernel: one launch of an MFMA kernel instance
@@ -88,9 +90,9 @@ struct GemmStep {
     // kSplitKReduce: sums `split` fp32 partial products of M x N in args.D's place (P) and applies the epilogue of `args`
     const float* partials = nullptr;
     int split = 0;
-    // kUniversal: the UniversalFMA kernel on CTA tile (ubm, ubn, ubk)
+    // kUniversal: the UniversalFMA kernel
     UArgs uargs{};
-    int ubm = 0, ubn = 0, ubk = 0;
+    UniversalTile utile = UniversalTile::k32x32;
 };
 struct GemmPlan {
     std::vector<GemmStep> steps;
@@ -127,6 +129,9 @@ int32_t map_dispatch(int32_t op, const moye_tensor* D, const moye_tensor* A, con
 // C with strides ldc_m / ldc_n; D with strides ldd / ldd_n), M x N elements
 int32_t splitk_reduce_dispatch(const float* P, int split, int64_t M, int64_t N, const GemmArgs& e, int32_t out_dt, hipStream_t st);
 int32_t mfma_ceiling(int32_t in_dt, int32_t random_operands, float seconds, float* tflops, float* clock_ghz, hipStream_t st);
-int32_t gemm_universal_dispatch(int bm, int bn, int bk, UArgs a, hipStream_t st);
+// the instance for a CTA tile (0: left to the library) on a chip of `cus` compute units; its name; its launch
+int32_t gemm_universal_choose(int bm, int bn, int bk, const UArgs& a, int cus, UniversalTile* tile);
+const char* gemm_universal_name(UniversalTile tile);
+int32_t gemm_universal_dispatch(UniversalTile tile, const UArgs& a, hipStream_t st);
 
 }  // namespace moye

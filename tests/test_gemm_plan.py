@@ -395,7 +395,7 @@ def test_every_branch_of_the_dispatcher_is_reached():
 def test_universal_fma_plan_and_errors():
     A, B, D = operands(256, 256, 256, mh.F32, mh.F32, "m", "k")
     p = mh.gemm_explain(mh.tiled_mma_desc(mh.MMA_UNIVERSAL_FMA, cta_tile=(32, 32, 8)), D, A, B)
-    assert p["steps"][0]["name"] == "gemm_universal<32,32,8>" and p["workspace"] == 0
+    assert p["steps"][0]["name"] == "gemm_universal_fma_small<16,16,64>" and p["workspace"] == 0
     with pytest.raises(mh.MoyeError):           # K of A and B differ
         mh.gemm_explain(mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16), tensor(PD, mh.F32, (64, 64), (64, 1)),
                         tensor(PA, mh.F16, (64, 32), (32, 1)), tensor(PB, mh.F16, (64, 64), (64, 1)))
@@ -404,6 +404,28 @@ def test_universal_fma_plan_and_errors():
     A, B, D = operands(256, 256, 256, mh.F16, mh.F32)
     st = _lib.lib().moye_gemm_explain(C.byref(mh.tiled_mma_desc(mh.MFMA_F32_16x16x32_F16)), C.byref(D), C.byref(A), C.byref(B), None, None, 0, buf, 8)
     assert st == _lib.ERR_BUFFER
+
+
+@pytest.mark.parametrize("cus", [256, 64])
+def test_universal_fma_plan_names_the_instance_that_runs(cus):
+    """The instance behind the 32 x 32 tile and the open one, on either side of every line of the rule (in 32 x 32 tiles: one
+    and three to a CU, two workgroups of 64 x 32 to a CU, twelve to a CU; sides of 16; 65535 tiles along N)."""
+    S, W = "gemm_universal_fma_small<%d,%d,%d>", "gemm_universal_fma<%d,%d,8>"
+    k16, k32, k64x32, k64, k128 = S % (16, 16, 64), S % (32, 32, 32), S % (64, 32, 64), W % (64, 64), W % (128, 128)
+
+    def name(M, N, tile=(32, 32, 8)):
+        A, B, D = operands(M, N, 8, mh.F32, mh.F32, "m", "k")
+        return mh.gemm_explain(mh.tiled_mma_desc(mh.MMA_UNIVERSAL_FMA, cta_tile=tile), D, A, B, compute_units=cus)["steps"][0]["name"]
+
+    t = 32 * cus
+    assert [name(32, t), name(32, t + 1), name(96, t), name(64, 2 * t - 1), name(64, 2 * t), name(64, 2 * t + 1)] == [k16, k32, k32, k64x32, k64x32, k32]
+    assert [name(96, 3 * t), name(384, t), name(384, t + 1), name(350, t + 64), name(384, t + 64), name(200, 4 * t)] == [k32, k64x32, k64, k32, k64, k32]
+    assert [name(16, 40 * t), name(17, 40 * t), name(40 * t, 16), name(40 * t, 17)] == [k16, k32, k16, k32]
+    assert [name(1, 16 * 65535), name(1, 16 * 65535 + 1), name(1, 32 * 65535), name(1, 32 * 65535 + 1)] == [k16, k32, k32, k64]
+    assert [name(64, 64, (0, 0, 0)), name(1024, 1024, (0, 0, 0)), name(1024, 1025, (0, 0, 0)), name(64, 64, (64, 64, 8)), name(64, 64, (128, 128, 8))] == \
+        [k16, k64x32 if cus == 256 else k64, k64, k64, k128]
+    with pytest.raises(mh.MoyeError):
+        name(64, 64, (48, 64, 8))
 
 
 @pytest.mark.parametrize("in_dt,K,lines", [(mh.F16, 504, False), (mh.F16, 512, True), (mh.F16, 520, True), (mh.F8E4M3, 1040, True), (mh.F32, 252, False), (mh.F32, 260, True)])
