@@ -29,6 +29,7 @@ def tensor_of(t, shape=None, stride=None, dtype=None):
 
 
 def current_stream():
-    """The current device's current stream as a raw handle (without building the torch.cuda.Stream object around it, which
-    takes as long as a launch)."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    """The current device's current stream as a raw handle (where torch has a function for that, without building the
+    torch.cuda.Stream object around it, which takes as long as a launch)."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return torch.cuda.current_stream().cuda_stream if raw is None else raw(torch.cuda.current_device())
