@@ -41,7 +41,7 @@ def _rand_bits(n, seed, device="cuda"):
 
 @pytest.mark.parametrize("M,N", [(64, 64), (128, 256), (192, 64), (1024, 2048)])
 def test_transpose_matches_oracle_and_closed_form(mh, M, N):
-    """config-2 shape family: column-major src -> row-major dst through the 64x64 LDS tile."""
+    """config-2 shape family: column-major src -> row-major dst through the LDS tiles."""
     src = _rand_bits(M * N, 1002)
     dst = torch.zeros(M * N, dtype=torch.int32, device="cuda")
     tc = mh.tiled_copy_desc(op=mh.COPY_LDS_TILED, vec_bits=128, tiler=(64, 64))
@@ -68,9 +68,8 @@ def test_transpose_other_orientation_and_pitch(mh):
 
 @pytest.mark.parametrize("dt", ["float32", "float16"])
 @pytest.mark.parametrize("M,N", [(1000, 1032), (72, 4104), (8200, 136), (64, 64 + 8)])
-def test_ragged_transpose_interior_and_strips(mh, M, N, dt):
-    """Sizes that are not multiples of the 64 x 64 tile: the interior goes through the LDS tiles, the strips through the
-    general kernel; together they are the transpose, bit for bit, and nothing outside dst is written."""
+def test_ragged_transpose_writes_dst_alone(mh, M, N, dt):
+    """Sizes that are not multiples of a tile: the transpose, bit for bit, and nothing outside dst is written."""
     tdt = getattr(torch, dt)
     bits = _rand_bits(M * N, 5).view(torch.int32)
     src = (bits.view(torch.float32) if dt == "float32" else bits.to(torch.int16).view(torch.float16)).clone()   # any bit pattern
@@ -86,7 +85,7 @@ def test_ragged_transpose_interior_and_strips(mh, M, N, dt):
 
 @pytest.mark.parametrize("dt", ["float32", "float16"])
 def test_ragged_transpose_with_padded_pitches(mh, dt):
-    """Sizes that are not even whole 16-byte pieces, inside aligned pitches: the strips go through the general kernel."""
+    """Sizes that are not even whole 16-byte pieces, inside aligned pitches."""
     tdt = getattr(torch, dt)
     M, N, PM, PN = 1002, 205, 1008, 208
     it = torch.int32 if dt == "float32" else torch.int16
@@ -706,10 +705,8 @@ def test_transpose_two_byte_elements(mh, M, N):
 @pytest.mark.parametrize("M,N", [(64, 256), (128, 512), (192, 256), (256, 1024), (512, 256), (768, 1280), (4096, 4096), (8192, 2048), (200, 300), (1088, 784),
                                  (16384, 12288)])
 def test_transpose_one_byte_elements(mh, M, N):
-    """fp8 matrices / bytes through the 1-byte LDS tiles (256 x 256 bytes in whole 256-byte runs where M is a multiple of 256,
-    else 64 x 256 with 1 or 2 sub-tiles per workgroup), sizes
-    that are not multiples of the tile through interior + strips or the general kernel: both orientations, padded pitches,
-    compared as bytes; the oracle on the small cases."""
+    """fp8 matrices / bytes through the LDS tiles, whole and ragged, or the general kernel (few elements): both orientations,
+    padded pitches, compared as bytes; the oracle on the small cases."""
     g = torch.Generator().manual_seed(M + N)
     src = torch.randint(0, 256, (M * N,), dtype=torch.uint8, generator=g).cuda()
     dst = torch.zeros(M * N, dtype=torch.uint8, device="cuda")
@@ -738,8 +735,7 @@ def test_transpose_one_byte_elements(mh, M, N):
 
 @pytest.mark.parametrize("M,N", [(64, 128), (128, 256), (192, 384), (4096, 2048), (200, 300), (1088, 896), (8192, 4096)])
 def test_transpose_eight_byte_elements(mh, M, N):
-    """Float64 / Int64 matrices through the 8-byte LDS tile (64 x 128 elements, destination rows first), sizes that are not
-    multiples of the tile through interior + strips or the general kernel: both orientations, padded pitches, a batch of
+    """Float64 / Int64 matrices through the LDS tiles, whole and ragged: both orientations, padded pitches, a batch of
     matrices in one launch; compared as bits; the oracle on the small cases."""
     g = torch.Generator().manual_seed(M * 3 + N)
     src = torch.randint(-2 ** 62, 2 ** 62, (M * N,), dtype=torch.int64, generator=g).cuda()
@@ -773,8 +769,8 @@ def test_transpose_eight_byte_elements(mh, M, N):
 @pytest.mark.parametrize("pair", ["float32->float16", "float16->float32", "float32->bfloat16", "bfloat16->float16", "float16->float8_e4m3fn",
                                   "float8_e4m3fn->float32", "float64->float16", "float32->float64", "float64->float8_e4m3fn", "float8_e4m3fn->bfloat16"])
 def test_transpose_that_converts(mh, pair):
-    """copyto! between matrices of different floating-point types whose unit strides lie on different modes: whole tiles
-    through the LDS kernel that converts on the way, other sizes as interior + strips, both orientations, padded pitches.
+    """copyto! between matrices of different floating-point types whose unit strides lie on different modes: through the
+    LDS kernel that converts on the way, whole tiles and ragged ones, both orientations, padded pitches.
     Bit for bit what the library's dense conversion makes of the transposed source (that conversion is pinned against the
     oracle elsewhere), values that round differently in every target among them; the frame of the destination untouched."""
     sname, dname = pair.split("->")
@@ -999,8 +995,8 @@ def test_batches_of_transposes(mh, dt):
 @pytest.mark.parametrize("tiler", [(32, 32), (64, 64), (16, 128), (8, 8), (0, 0)])
 def test_lds_tiled_copy_takes_any_tiler_that_divides(mh, tiler):
     """The reference's own transpose kernel tiles 32 x 32 with 256 threads (test/host/copy_async.jl:51-76): the tiler
-    of the descriptor only has to divide the array; closed form dst[j, i] == src[i, j] bit for bit, for sizes that are
-    whole 64 x 64 patches, sizes that leave strips, and an array smaller than a patch."""
+    of the descriptor only has to divide the array; closed form dst[j, i] == src[i, j] bit for bit, for sizes of
+    whole tiles, ragged ones, and an array smaller than a tile."""
     for (M, N) in ((2048, 4096), (4096, 2048), (96, 160), (32, 32), (2048 + 32, 2048)):
         if tiler[0] and (M % tiler[0] or N % tiler[1]):
             continue
@@ -1189,8 +1185,8 @@ def test_batches_of_ragged_transposes_in_one_launch(mh, pair):
     bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32}
     for logical, s_order, s_pad, d_order, d_pad in [
         ((33, 35, 40000), (2, 1, 0), 0, (2, 0, 1), 0),
-        ((33, 41, 3, 5, 7), (3, 2, 1, 4, 0), 2, (4, 2, 0, 3, 1), 3),
-        ((130, 67, 2, 3, 2), (4, 1, 2, 3, 0), 1, (2, 3, 4, 0, 1), 0),
+        ((33, 41, 6, 10, 14), (3, 2, 1, 4, 0), 2, (4, 2, 0, 3, 1), 3),
+        ((130, 67, 4, 6, 5), (4, 1, 2, 3, 0), 1, (2, 3, 4, 0, 1), 0),
     ]:
         def storage(order, pad, dtype, fill):   # a buffer one element off alignment, its innermost mode padded
             sizes = [logical[m] for m in order]
@@ -1208,3 +1204,37 @@ def test_batches_of_ragged_transposes_in_one_launch(mh, pair):
         mh.copyto_(_tens(mh, dst, tuple(dst.shape), tuple(dst.stride())), _tens(mh, src, tuple(src.shape), tuple(src.stride())))
         torch.cuda.synchronize()
         assert torch.equal(dbuf.view(bits[td.itemsize]), want.view(bits[td.itemsize])), (pair, logical)
+
+
+@pytest.mark.parametrize("pair", ["uint8", "int16", "int32", "int64", "float32->bfloat16", "bfloat16->float32", "float32->float8_e4m3fn",
+                                  "bfloat16->float8_e4m3fn", "float8_e4m3fn->bfloat16", "float8_e4m3fn->float32", "float64->float16"])
+def test_every_tile_of_the_transposes(mh, pair):
+    """Sizes from either side of the lines of the tile's choice (2, 6, 8 and 16 Mi elements, 64 and 256 MiB, whole lines or
+    not, matrices narrower than a tile along either side) with ragged edges, pitches and pointers; now and then a NaN, an infinity or any
+    other bits among the values.  Against torch's transpose of what the library's dense copy (pinned against the oracle
+    elsewhere) makes of the source; everything outside the destination's elements stays untouched."""
+    from moye_hip.torch_interop import tensor_of
+    sdt, ddt = [getattr(torch, x) for x in (pair.split("->") * 2)[:2]]
+    bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32, 8: torch.int64}
+    for ni, nj, batch, extra in [(33, 47, 400, 1), (65, 127, 70, 3), (129, 513, 9, 1), (200, 96, 40, 0), (128, 128, 40, 0),
+                                 (70, 1001, 40, 1), (1001, 70, 50, 0), (128, 128, 300, 0), (256, 128, 130, 0), (128, 384, 100, 0), (1001, 6007, 1, 0),
+                                 (33, 35, 8000, 0), (130, 67, 1200, 1), (67, 130, 1200, 3), (128, 128, 700, 0), (384, 256, 110, 0), (3001, 3203, 1, 1),
+                                 (3203, 3001, 1, 0), (3200, 3072, 1, 0), (256, 40000, 1, 0), (40000, 256, 1, 0), (700, 13001, 1, 0), (13001, 700, 1, 0),
+                                 (8192, 8320, 1, 0), (4160, 16384, 1, 0), (4101, 16501, 1, 0)]:
+        lds, ldd, off = ni + extra, nj + extra, 1 if extra else 0
+        ns, nd = off + batch * nj * lds, off + batch * ni * ldd
+        g = torch.Generator(device="cuda").manual_seed(ni * 7 + nj)
+        raw = torch.randint(0, 256, (ns * sdt.itemsize,), generator=g, device="cuda", dtype=torch.uint8).view(bits[sdt.itemsize])
+        if sdt.is_floating_point:
+            any_bits = torch.rand(ns, generator=g, device="cuda") < 3e-4
+            raw = torch.where(any_bits, raw, (torch.randn(ns, generator=g, device="cuda") * 8).to(sdt).view(bits[sdt.itemsize]))
+            del any_bits
+        src, dense = raw.view(sdt), torch.empty(ns, dtype=bits[ddt.itemsize], device="cuda")
+        mh.copyto_(tensor_of(dense.view(ddt)), tensor_of(src))
+        dst = torch.full((nd * ddt.itemsize,), 0x5A, dtype=torch.uint8, device="cuda").view(bits[ddt.itemsize])
+        want = dst.clone()
+        want.as_strided((batch, ni, ldd), (ni * ldd, ldd, 1), off)[:, :, :nj] = dense.as_strided((batch, nj, lds), (nj * lds, lds, 1), off)[:, :, :ni].transpose(1, 2)
+        mh.copyto_(tensor_of(dst.view(ddt)[off:], (ni, nj, batch), (ldd, 1, ni * ldd)), tensor_of(src[off:], (ni, nj, batch), (1, lds, nj * lds)))
+        torch.cuda.synchronize()
+        assert torch.equal(dst, want), (pair, ni, nj, batch, extra)
+        del raw, src, dense, dst, want
