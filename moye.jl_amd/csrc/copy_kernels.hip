@@ -569,7 +569,7 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
                               ((src->stride[0] == 1 && dst->stride[1] == 1) || (src->stride[1] == 1 && dst->stride[0] == 1));
         if (tc && tc->op == MOYE_COPY_LDS_TILED && !lds_pair)
             return fail(MOYE_ERR_UNSUPPORTED,
-                        "copyto!: the LDS-tiled copy takes rank-2 operands (or a batch of them) of 1-, 2- or 4-byte elements "
+                        "copyto!: the LDS-tiled copy takes rank-2 operands (or a batch of them) of 1- to 8-byte elements "
                         "with the unit stride on different modes");
     }
 

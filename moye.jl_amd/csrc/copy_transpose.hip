@@ -52,8 +52,8 @@ __device__ __forceinline__ uint32_t pack_f32(const float (&x)[N]) {
     }
 }
 
-// The first `left` elements of a piece, fewer than all: 8, 4, 2 and 1 bytes as they are needed (one store per element took a
-// byte matrix of 1000 x 300 from 4.2 to 7.8 us)
+// The first `left` elements of a piece, fewer than all: 8, 4, 2 and 1 bytes as they are needed (with one store per element bytes
+// 1000 x 300 took 8.1 us, with these 6.8)
 template <int DB>
 __device__ __forceinline__ void store_first(char* p, u32x4 w, int left) {
     const int bytes = left * DB;
@@ -140,7 +140,7 @@ __device__ __forceinline__ void turn_block(const u32x4 (&v)[16 / DB], u32x4 (&o)
         }
         if constexpr (kSrc == MOYE_F8E4M3) {
             // Two elements to an instruction (a lane's 128 conversions one by one were most of a small call: fp8 -> bf16 1024^2
-            // 5.9 us).  It makes every NaN negative: only a block with a positive one, 0x7f, goes the way below.
+            // 5.9 -> 3.6 us).  It makes every NaN negative: only a block with a positive one, 0x7f, goes the way below.
             uint32_t found = 0;
 #pragma unroll
             for (int q = 0; q < Q; ++q)
@@ -335,12 +335,12 @@ static int first_that_fits(const TransposeArgs& a, std::initializer_list<Tile> t
 // index fastest, with whole lines from an extent of 4096 on (4096 x 32768 f32 196 us, 208 the other way; but bf16 -> f32
 // 64 x 1048576 71 and 86).  Neighbouring tiles go to one XCD (`run`), so that lines two of them share meet in one L2 (f32
 // 8192^2 102.8 -> 96.6 us, 16400 x 16392 ~420 -> 405), except where an even spread is worth more: few elements, and whole
-// lines below 64 MiB (f32 2048^2 8.3 -> 7.2).
+// lines below 64 MiB (128 x 128 tiles, fp16 2048^2 5.2 -> 4.6, bf16 -> fp32 4096 x 1024 6.0 -> 5.2).
 //   Measured with operands that are not cached, us, the kernels for whole 64 x 64 patches that this one replaced / one tile for
-// every extent / this rule: fp16 32768 x [64, 64] 85 / 400 / 85; 16384 x [128, 64] 85 / 235 / 87; 1048576 x 128 94 / 148 / 91; 4096^2
-// 15.8 / 14.8 / 12.6; fp32 2048^2 7.4 / 9.2 / 7.2; 16 x [512, 512] 7.2 / 8.6 / 7.1; 1048576 x 64 93 / 106 / 91; 100000 x [33, 33] 552 /
-// 1051 / 206; 4096 x 32768 196 / 209 / 197; bytes 2048^2 4.4 / 4.7 / 4.0, 262144 x 256 26 / 28 / 28; 8-byte elements 256 x 262144
-// 169 / 177 / 169, 8192 x [32, 32] 52 / 72 / 24; bf16 -> fp32 16384 x [64, 128] 139 / 216 / 136; fp8 -> bf16 64 x [1024, 1024] 34 / 40 / 36.
+// every extent / this rule: fp16 32768 x [64, 64] 85 / 400 / 85; 16384 x [128, 64] 85 / 235 / 87; 1048576 x 128 93 / 148 / 89; 4096^2
+// 15.8 / 14.8 / 12.6; fp32 2048^2 7.4 / 9.2 / 7.0; 16 x [512, 512] 7.2 / 8.6 / 7.0; 1048576 x 64 93 / 106 / 90; 100000 x [33, 33] 552 /
+// 1051 / 206; 4096 x 32768 196 / 209 / 196; bytes 2048^2 4.4 / 4.7 / 4.0, 262144 x 256 26 / 28 / 28; 8-byte elements 256 x 262144
+// 169 / 177 / 169, 8192 x [32, 32] 52 / 72 / 24; bf16 -> fp32 16384 x [64, 128] 138 / 216 / 135; fp8 -> bf16 64 x [1024, 1024] 34 / 40 / 36.
 template <int kSrc, int kDst, int SB, int DB>
 static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
     constexpr int64_t Mi = 1 << 20;

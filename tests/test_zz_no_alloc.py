@@ -40,7 +40,7 @@ def _case(mh, M, N, K, split, seed, out_dt=torch.float16, cta=(128, 128, 32), wa
     need = C.c_size_t()
     _lib.check(lib.moye_gemm_workspace_size(C.byref(mma), C.byref(T(c)), C.byref(ta), C.byref(T(b)), C.byref(need)))
     # the call does use the scratch: the partial products of every K range and the K-major copy of A, whose rows are
-    # rounded up to 16 bytes and whose size to 256; and the plan it runs uses exactly what the query says
+    # rounded up to 16 bytes at least and whose size to 256; and the plan it runs uses exactly what the query says
     plan = mh.gemm_explain(mma, T(c), ta, T(b), T(c))
     ranges = max(s["split"] for s in plan["steps"] if s["what"] == "kernel")       # (split = -1: the library's own choice)
     assert ranges == split or split == -1
