@@ -149,6 +149,8 @@ typedef struct {
  * Base.copyto!(tiled_copy, dst, src) (src/algorithm/copy.jl:106-130): logical element i of
  * src goes to logical element i of dst through both layouts; bit-exact when the dtypes
  * agree, round-to-nearest-even conversion otherwise (src/arch/copy/copy.jl:38-43).
+ * An element of dst may lie on the same element of src (a conversion between types of one width
+ * in place); where it lies on another one, the result is undefined.
  * `tc` may be NULL (plain copyto!). */
 int32_t moye_copy(const moye_tiled_copy* tc, const moye_tensor* dst, const moye_tensor* src,
                   void* stream);

@@ -147,7 +147,8 @@ __global__ __launch_bounds__(256) void copy_generic_cvt(const char* __restrict__
 // The same element loops, V elements per lane: for arrays whose first mode (once the modes are ordered by stride) is a
 // run of unit stride and one length of at least V on every side -- pitched matrices, slices of larger arrays -- whatever its
 // length, the pitches and the alignment.  The last group of a run is moved back to end with it: what two lanes then move
-// twice is the same (under a mask too: both write the elements it names, and leave or write back the others).
+// twice is the same (under a mask too: both write the elements it names, and leave or write back the others) -- unless a
+// conversion's source is its destination, where one lane may read what another has converted: launch_groups refuses that.
 // The vectorisation the reference computes with max_common_vector
 // (src/layout.jl:752-761) and leaves unused (src/algorithm/copy.jl:53-58), here also for converting copies (the wider
 // side moves 16 bytes per lane) and for copyto_if! (the mask is read V bytes at a time; a group whose mask is all true
@@ -436,16 +437,33 @@ static bool launch_groups_dst(int32_t dd, const char* s, char* d, const FlatLayo
         default: return false;
     }
 }
+// Do the bytes between the first and the last element of two arrays overlap?
+static bool share_memory(const moye_tensor& x, const moye_tensor& y) {
+    const char *first[2], *last[2];
+    const moye_tensor* both[2] = {&x, &y};
+    for (int i = 0; i < 2; ++i) {
+        int64_t lo = 0, hi = 0;
+        for (int m = 0; m < both[i]->rank; ++m) {
+            const int64_t span = (both[i]->shape[m] - 1) * both[i]->stride[m];
+            (span < 0 ? lo : hi) += span;
+        }
+        first[i] = static_cast<const char*>(both[i]->ptr) + lo * dtype_bytes(both[i]->dtype);
+        last[i] = static_cast<const char*>(both[i]->ptr) + (hi + 1) * dtype_bytes(both[i]->dtype);
+    }
+    return first[0] < last[1] && first[1] < last[0];
+}
+
 // Groups of V = 16 / (the wider element) elements along the first mode, when every layout of the call (the modes already
 // ordered by stride) has it as a run of unit stride and one length of V and more.  `same_bits`: a copy of bits (with a mask:
-// copyto_if!).  Returns false, having launched nothing, when the call does not qualify.
-static bool launch_groups(int32_t src_dt, int32_t dst_dt, const char* s, char* d, FlatLayout ls, FlatLayout ld, Mask mk, bool same_bits, int64_t n,
-                          hipStream_t st) {
+// copyto_if!); `in_place`: a conversion whose two sides share memory, which takes groups only where they end with the run, so that
+// every element has one lane.  Returns false, having launched nothing, when the call does not qualify.
+static bool launch_groups(int32_t src_dt, int32_t dst_dt, const char* s, char* d, FlatLayout ls, FlatLayout ld, Mask mk, bool same_bits, bool in_place,
+                          int64_t n, hipStream_t st) {
     const int sb = dtype_bytes(src_dt), db = dtype_bytes(dst_dt);
     const int V = 16 / std::max(sb, db);
     if (V < 2 || ls.rank < 1 || ld.rank != ls.rank) return false;
     const int64_t run = ls.shape[0];
-    if (run < V || ld.shape[0] != run || ls.stride[0] != 1 || ld.stride[0] != 1) return false;
+    if (run < V || (in_place && run % V) || ld.shape[0] != run || ls.stride[0] != 1 || ld.stride[0] != 1) return false;
     if (mk.ptr && (mk.l.rank != ls.rank || mk.l.shape[0] != run || mk.l.stride[0] != 1)) return false;
     const int64_t groups = (run + V - 1) / V, ng = n / run * groups;
     ls.shape[0] = ld.shape[0] = mk.l.shape[0] = groups;
@@ -624,7 +642,7 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
             width /= 2;
         }
         // (under 8 bytes at a time: runs in groups that need no alignment, where the layouts have runs)
-        if (sb * width < 8 && launch_groups(src->dtype, dst->dtype, s, d, ls, ld, mk, true, n, st)) {
+        if (sb * width < 8 && launch_groups(src->dtype, dst->dtype, s, d, ls, ld, mk, true, false, n, st)) {
             MOYE_HIP_CHECK(hipGetLastError());
             return MOYE_OK;
         }
@@ -658,7 +676,8 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
     // (up to 64 MiB a run that does not end with a group: in groups below, which leave no rest for a second launch; f32 -> bf16 1301 x 1333 6.3 ->
     // 3.9 us)
     const int64_t per_lane = 16 / std::min(sb, db);
-    if (!same_bits && !mask && one_run_each(*src, *dst) && (n % per_lane == 0 || n * std::max(sb, db) > ((int64_t)64 << 20)) &&
+    const bool in_place = !same_bits && share_memory(*src, *dst);
+    if (!same_bits && !mask && one_run_each(*src, *dst) && (n % per_lane == 0 || in_place || n * std::max(sb, db) > ((int64_t)64 << 20)) &&
         (reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) % 16 == 0) {
         // both sides one aligned run: 16-byte accesses for all whole groups, the general kernel for what is left
         const int64_t done = launch_cvt_dense(src->dtype, dst->dtype, s, d, n, st);
@@ -678,7 +697,7 @@ int32_t copy_if_dispatch(const moye_tiled_copy* tc, const moye_tensor* dst, cons
     }
     // converting copies between pitched arrays, and copyto_if!: groups of elements along the first mode where the layouts allow
     // (a plain copy of bits has had its turn above)
-    if ((!same_bits || mask) && launch_groups(src->dtype, dst->dtype, s, d, ls, ld, mk, same_bits, n, st)) {
+    if ((!same_bits || mask) && launch_groups(src->dtype, dst->dtype, s, d, ls, ld, mk, same_bits, in_place, n, st)) {
         MOYE_HIP_CHECK(hipGetLastError());
         return MOYE_OK;
     }

@@ -1311,3 +1311,28 @@ def test_runs_of_any_length_and_alignment(mh, src_dt, dst_dt, L):
                 mh.copyto_(tensor_of(d), tensor_of(s))
             torch.cuda.synchronize()
             assert torch.equal(fd.cpu(), want.cpu()), (rows, pad_s, pad_d, off, masked)
+
+
+@pytest.mark.parametrize("src_dt,dst_dt", [(torch.float16, torch.bfloat16), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("L", [7, 8, 9, 513, 4096, 70001])
+def test_conversions_in_place(mh, src_dt, dst_dt, L):
+    """The destination on the source's own memory, runs that do and do not end with a group of eight, dense and pitched, off
+    16-byte boundaries, with and without a mask: every element is converted once."""
+    from moye_hip.torch_interop import tensor_of
+    g = torch.Generator().manual_seed(L)
+    for rows, pad, off in ((1, 0, 0), (1, 0, 1), (3, 0, 0), (9, 5, 0), (9, 8, 3)):
+        for masked in (False, True):
+            mem = (torch.randn(off + rows * (L + pad), generator=g) * 20).to(src_dt).cuda()
+            want = mem.clone().view(dst_dt)
+            s = mem.clone().as_strided((rows, L), (L + pad, 1), off)
+            w = want.as_strided((rows, L), (L + pad, 1), off)
+            d = mem.view(dst_dt).as_strided((rows, L), (L + pad, 1), off)
+            if masked:
+                m = (torch.rand((rows, L), generator=g) < 0.6).to(torch.uint8).cuda()
+                w.copy_(torch.where(m.bool(), s.to(dst_dt), w))
+                mh.copyto_if_(tensor_of(d), tensor_of(mem.as_strided((rows, L), (L + pad, 1), off)), tensor_of(m))
+            else:
+                w.copy_(s)
+                mh.copyto_(tensor_of(d), tensor_of(mem.as_strided((rows, L), (L + pad, 1), off)))
+            torch.cuda.synchronize()
+            assert torch.equal(mem.view(torch.int16).cpu(), want.view(torch.int16).cpu()), (rows, pad, off, masked)
