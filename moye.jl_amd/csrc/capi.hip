@@ -229,7 +229,9 @@ static bool rows_in_16_bytes(const Mat& m) {
     if (m.cs != 1 && m.cols > 1) return 256 * kmajor_pitch(m, true) < ((int64_t)1 << 32);
     return reinterpret_cast<uintptr_t>(m.ptr) % 16 == 0 && pitch % 16 == 0 && 256 * pitch < ((int64_t)1 << 32);
 }
-static LibraryChoice library_choice(const moye_tiled_mma* mma, const Mat& A, const Mat& B, int cus) {
+// D with its unit stride along M: the kernels compute D' = B A', row-major
+static bool column_major(const Mat& D) { return D.cs != 1 && D.rs == 1; }
+static LibraryChoice library_choice(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, int cus) {
     const int64_t M = A.rows, N = B.rows, K = A.cols;
     const int eb = dtype_bytes(A.dtype);
     LibraryChoice c;
@@ -240,7 +242,7 @@ static LibraryChoice library_choice(const moye_tiled_mma* mma, const Mat& A, con
                         mma->atom == MOYE_MFMA_F32_16x16x4_F32;
     const bool forms = atom16 && mma->stages == 0 && mma->atom_layout_mnk[0] * mma->atom_layout_mnk[1] <= 1 &&
                        !(mma->flags & (MOYE_GEMM_PINGPONG | MOYE_GEMM_WAVE4)) && rows_in_16_bytes(A) && rows_in_16_bytes(B);
-    c.tile = gemm_choose(M, N, K * eb, eb, (mma->flags & MOYE_GEMM_NO_WORKSPACE) ? 1 : 16, cus, forms);
+    c.tile = gemm_choose(M, N, K * eb, eb, (mma->flags & MOYE_GEMM_NO_WORKSPACE) ? 1 : 16, cus, forms, column_major(D));
     return c;
 }
 
@@ -248,7 +250,7 @@ static LibraryChoice library_choice(const moye_tiled_mma* mma, const Mat& A, con
 // what the cost model of gemm_plan.hpp finds cheapest together with the tile (none where 256 x 256 tiles come out
 // cheapest); with a named tile, none when the problem's 128 x 128 tiles fill half the chip,
 // else the largest count up to cus / tiles that cuts K into equal ranges of whole 128-byte pieces of at least 512 bytes.
-static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, int cus) {
+static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, int cus) {
     const int64_t M = A.rows, N = B.rows, K = A.cols;
     const int eb = dtype_bytes(A.dtype);
     if (mma->split_k >= 0) return mma->split_k > 1 ? mma->split_k : 1;
@@ -258,7 +260,7 @@ static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, in
         // 30.4 us against 41.3 with two ranges and the second pass); K ranges are whole lines
         return skinny_lines_split(M, N, K * eb, cus);
     }
-    if (const LibraryChoice c = library_choice(mma, A, B, cus); c.open) return c.tile.split;
+    if (const LibraryChoice c = library_choice(mma, A, B, D, cus); c.open) return c.tile.split;
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
     if (tiles <= 0 || tiles >= cus / 2) return 1;
     for (int64_t s = std::min<int64_t>(cus / tiles, K); s >= 2; --s)
@@ -312,12 +314,12 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
 }
 
 // K-major copies of A and B where needed, then the fp32 partial products of a split-K call
-static size_t gemm_workspace_bytes_impl(const moye_tiled_mma* mma, const Mat& A, const Mat& B, bool native, bool lines, int cus) {
+static size_t gemm_workspace_bytes_impl(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, bool native, bool lines, int cus) {
     if (mma->atom == MOYE_MMA_UNIVERSAL_FMA) return 0;
     size_t n = 0;
     if (!native && A.cs != 1 && A.cols > 1) n += kmajor_bytes(A, lines);
     if (!native && B.cs != 1 && B.cols > 1) n += kmajor_bytes(B, lines);
-    const int split = split_count(mma, A, B, cus);
+    const int split = split_count(mma, A, B, D, cus);
     if (split > 1) n += (size_t)split * (size_t)A.rows * (size_t)B.rows * sizeof(float);
     return n;
 }
@@ -334,7 +336,7 @@ static int32_t gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor*
         if (x->rows == 1 && x->cs == 1) x->rs = x->cols;
     const int cus = device_shape().cus;
     if (!(mma->flags & MOYE_GEMM_NO_WORKSPACE))
-        *bytes = gemm_workspace_bytes_impl(mma, a, b, majors_run_natively(mma, a, b, d, ep, false, cus), lines, cus);
+        *bytes = gemm_workspace_bytes_impl(mma, a, b, d, majors_run_natively(mma, a, b, d, ep, false, cus), lines, cus);
     return MOYE_OK;
 }
 
@@ -449,13 +451,13 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         if (A.cs != 1 && A.cols > 1) { major_flags |= kGemmAMajorM; A.rs = A.cs; A.cs = 1; }  // Mat::rs now holds the pitch between consecutive k
         if (B.cs != 1 && B.cols > 1) { major_flags |= kGemmBMajorN; B.rs = B.cs; B.cs = 1; }
     }
-    plan.workspace_bytes = gemm_workspace_bytes_impl(mma, A, B, native_majors, true, cus);
+    plan.workspace_bytes = gemm_workspace_bytes_impl(mma, A, B, D, native_majors, true, cus);
     if (plan.workspace_bytes) {
         if (mma->flags & MOYE_GEMM_NO_WORKSPACE)
             return fail(MOYE_ERR_UNSUPPORTED, "gemm!: the MFMA kernels need K-major A and B (stride 1 along K, the 'TN' form), split_k needs room "
                                               "for its partial products, and MOYE_GEMM_NO_WORKSPACE forbids the use of a workspace");
         const size_t wanted = plan.workspace_bytes;
-        if (int32_t e = workspace(gemm_workspace_bytes_impl(mma, A, B, native_majors, false, cus), &plan.workspace_bytes, &ws)) return e;
+        if (int32_t e = workspace(gemm_workspace_bytes_impl(mma, A, B, D, native_majors, false, cus), &plan.workspace_bytes, &ws)) return e;
         const bool lines = plan.workspace_bytes == wanted;
         plan.workspace = ws;
         if (!native_majors && A.cs != 1 && A.cols > 1) {
@@ -510,9 +512,9 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
     g.flags = !(mma->flags & MOYE_GEMM_NO_XCD_SWIZZLE) | (mma->flags & 0xff00) | (atom32 ? kGemmAtom32 : 0) | (rotate_k ? kGemmRotateK : 0) |
               (stream_d ? kGemmStreamD : 0) | major_flags;
     // tile and K ranges, where both are left to the library, are one decision (gemm_choose)
-    const LibraryChoice lib = library_choice(mma, A, B, cus);
+    const LibraryChoice lib = library_choice(mma, A, B, D, cus);
     const TileChoice* lib_tile = lib.open ? &lib.tile : nullptr;
-    if (const int split = split_count(mma, A, B, cus); split > 1) {
+    if (const int split = split_count(mma, A, B, D, cus); split > 1) {
         // K is cut into `split` equal ranges, all in one launch (gridDim.y); each range writes its fp32 product, compact and
         // row-major, into the workspace; a second pass sums the ranges in ascending order, applies alpha and C and converts
         const int eb = dtype_bytes(in_dt);
@@ -550,7 +552,7 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         g.C = tC ? C.ptr : nullptr; g.ldc_m = C.rs; g.ldc_n = C.cs; g.D = D.ptr;
         return gemm_mfma_skinny_dispatch(in_dt, D.dtype, g, plan);
     }
-    if (D.rs == 1) {  // column-major D: D' = B * A' is row-major
+    if (column_major(D)) {  // D' = B * A' is row-major
         g.A = B.ptr; g.B = A.ptr; g.M = N; g.N = M; g.lda = B.rs; g.ldb = A.rs; g.ldd = D.cs;
         g.C = tC ? C.ptr : nullptr; g.ldc_m = C.cs; g.ldc_n = C.rs; g.D = D.ptr;
         std::swap(g.ep_xm, g.ep_xn);  // the kernel's m is the caller's n
@@ -559,7 +561,7 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
         if (rows_in_16_byte_pieces(g.C, g.ldc_m, g.ldc_n, D.dtype)) g.flags |= kGemmRowC;
         if (operand_rows_in_16_byte_pieces(g)) g.flags |= kGemmEpiRowX;
         if (lane_op(g)) g.flags |= kGemmEpiLaneOp;
-        // (the library's choice was priced for (M, N); the cost model is symmetric in them)
+        // (the library's choice was priced for this orientation)
         return gemm_mfma_tn_dispatch(in_dt, D.dtype, bn, bm, bk, waves, mma->stages, g, plan, lib_tile);
     }
     return fail(MOYE_ERR_UNSUPPORTED, "gemm!: D needs a unit stride along M or N");

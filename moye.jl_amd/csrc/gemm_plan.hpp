@@ -158,8 +158,10 @@ inline GemmForm gemm_form_choose(int64_t M, int64_t N, int64_t k_bytes, int elem
 // Everything left to the library (tile, waves, K ranges): the cheapest of 64 x 64 / 128 x 128 tiles with 1 .. max_split K
 // ranges and of unsplit 256 x 256 tiles, which are considered from a quarter of the CUs' worth of tiles on.  The one
 // place where tile and K ranges are chosen together: the workspace sizing and the dispatcher both take their answer
-// from here.
-inline TileChoice gemm_choose(int64_t M, int64_t N, int64_t k_bytes, int elem_bytes, int max_split, int cus, bool forms) {
+// from here.  `transposed`: the kernels run N x M (a column-major D), and the forms, some with two different sides, are priced for
+// that.  bf16, B not cached, us as M x N / as N x M: 1000 x 6144 x 4096 80 on 288 tiles of 128 x 192 / 52-59 on 256 of 192 x 128, 2048 x
+// 3072 x 4096 79.5 / 52.5, 639 x 9216 x 1152 36.5 / 29.5 (with a row-major D 54, 52 and 29.5).
+inline TileChoice gemm_choose(int64_t M, int64_t N, int64_t k_bytes, int elem_bytes, int max_split, int cus, bool forms, bool transposed) {
     const bool f32_in = elem_bytes == 4;
     TileChoice best = gemm_plan(M, N, k_bytes, f32_in, M % 64 == 0 && N % 64 == 0 && k_bytes % 128 == 0, max_split, cus);
     const bool ragged = M % 256 || N % 256 || k_bytes % 128;
@@ -180,7 +182,7 @@ inline TileChoice gemm_choose(int64_t M, int64_t N, int64_t k_bytes, int elem_by
     }
     if (forms) {
         double us;
-        const GemmForm form = gemm_form_choose(M, N, k_bytes, elem_bytes, cus, best.us, &us);
+        const GemmForm form = gemm_form_choose(transposed ? N : M, transposed ? M : N, k_bytes, elem_bytes, cus, best.us, &us);
         if (form != GemmForm::kOther) best = TileChoice{0, 1, us, form};
     }
     return best;
