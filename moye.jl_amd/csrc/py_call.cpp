@@ -10,6 +10,7 @@
 #include "../../include/moye_hip.h"
 
 static PyTypeObject *g_array, *g_tensor, *g_mma, *g_copy, *g_epilogue;  // MoYeArray and the ctypes structures
+static PyObject* g_layout;                                              // Layout, where MoYeArray's module has it
 static PyObject *s_ptr, *s_dtype, *s_memspace, *s_layout, *s_descriptor_, *s_descriptor;
 static decltype(&moye_gemm) f_gemm;
 static decltype(&moye_gemm_ex) f_gemm_ex;
@@ -42,14 +43,15 @@ static bool integer(PyObject* o, PyObject* name, unsigned long long* out) {
 }
 
 // the descriptor of an array: a moye_tensor, a MoYeArray (its layout's flattened form with the pointer, element type and memory
-// space filled in, as MoYeArray.tensor() does), or None
+// space filled in, as MoYeArray.tensor() does), or None.  A subclass of either class may have methods of its own: a MoYeArray's
+// goes through ctypes, which asks tensor(), a Layout's is asked for its descriptor().
 static bool tensor(PyObject* o, moye_tensor* store, const moye_tensor** out) {
-    if (!PyObject_TypeCheck(o, g_array)) return structure(o, g_tensor, out);
+    if (Py_TYPE(o) != g_array) return structure(o, g_tensor, out);
     unsigned long long ptr, dtype, memspace;
     if (!integer(o, s_ptr, &ptr) || !integer(o, s_dtype, &dtype) || !integer(o, s_memspace, &memspace)) return false;
     PyObject* layout = PyObject_GetAttr(o, s_layout);
     if (!layout) return false;
-    PyObject* flat = PyObject_GetAttr(layout, s_descriptor_);
+    PyObject* flat = reinterpret_cast<PyObject*>(Py_TYPE(layout)) == g_layout ? PyObject_GetAttr(layout, s_descriptor_) : nullptr;
     if (!flat || !PyBytes_CheckExact(flat)) {
         PyErr_Clear();
         Py_XDECREF(flat);
@@ -177,6 +179,15 @@ static PyObject* bind(PyObject*, PyObject* args) {
         Py_INCREF(ty[i]);
         *slots[i] = reinterpret_cast<PyTypeObject*>(ty[i]);
     }
+    Py_CLEAR(g_layout);
+    if (PyObject* name = PyObject_GetAttrString(ty[0], "__module__")) {
+        if (PyObject* module = PyImport_Import(name)) {
+            g_layout = PyObject_GetAttrString(module, "Layout");
+            Py_DECREF(module);
+        }
+        Py_DECREF(name);
+    }
+    PyErr_Clear();
     f_gemm = reinterpret_cast<decltype(f_gemm)>(f[0]);
     f_gemm_ex = reinterpret_cast<decltype(f_gemm_ex)>(f[1]);
     f_copy = reinterpret_cast<decltype(f_copy)>(f[2]);

@@ -78,6 +78,34 @@ def test_arrays_and_descriptors_arrive_as_ctypes_hands_them_over(recorder):
     assert recorder.seen[-1][2] == bytes(A.tensor()) != bytes(raw[1])
 
 
+def test_an_array_s_own_descriptor_is_asked_for(recorder, monkeypatch):
+    """A subclass of MoYeArray that says what its descriptor is (it takes ctypes), and a subclass of Layout that does."""
+    class Library:
+        @staticmethod
+        def moye_copy(tc, dst, src, stream):
+            recorder.seen.append([tc, bytes(dst._obj), bytes(src._obj), stream])
+            return 0
+    monkeypatch.setattr(device, "lib", Library)
+
+    class Shifted(mh.MoYeArray):
+        def tensor(self):
+            t = super().tensor()
+            t.ptr += 128
+            return t
+
+    class Halved(mh.Layout):
+        def descriptor(self):
+            return mh.Layout((4, 4), (8, 1)).descriptor()
+
+    D, A = array(4, 4), Shifted(PTR, mh.F16, mh.Layout((4, 4), (4, 1)))
+    mh.copyto_(D, A)
+    assert recorder.seen[-1][2] == bytes(A.tensor()) != bytes(array(4, 4).tensor())
+    B = mh.MoYeArray(PTR, mh.F16, Halved((8, 4), (4, 1)))
+    B.layout._descriptor = mh.Layout((8, 4), (4, 1)).descriptor()
+    mh.copyto_(D, B)
+    assert recorder.seen[-1][2] == bytes(B.tensor())
+
+
 @pytest.mark.parametrize("bad", [None, object(), 3.5, "x"])
 def test_what_ctypes_refuses_stays_refused(recorder, bad):
     D, A = array(8, 4), array(8, 4)
