@@ -9,7 +9,6 @@ import re
 import subprocess
 import sys
 import sysconfig
-import sys
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -188,19 +187,27 @@ def asm_mfma_hazards(lines, name="asm"):
 
 
 def _build_python_calls(force):
-    """moye_hip/_call: the calls of a program's loop without ctypes.  A Python without its headers goes without it."""
+    """moye_hip/_call: the calls of a program's loop without ctypes.  Optional: without Python's headers or a host compiler, or where it
+    does not compile, the package calls the library through ctypes, and no module of an earlier build is left to be loaded."""
     src = os.path.join(CSRC, "py_call.cpp")
     out = os.path.join(HERE, "moye_hip", "_call" + sysconfig.get_config_var("EXT_SUFFIX"))
     inc = sysconfig.get_paths()["include"]
-    if not os.path.exists(os.path.join(inc, "Python.h")):
-        print("no Python.h: moye_hip calls the library through ctypes")
-        return
-    if not force and not _stale(out, [src, os.path.join(HERE, "..", "include", "moye_hip.h")]):
-        return
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", inc, src, "-o", out]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError("g++ failed for py_call.cpp:\n" + r.stdout + r.stderr)
+    if os.path.exists(os.path.join(inc, "Python.h")):
+        if not force and not _stale(out, [src, os.path.join(HERE, "..", "include", "moye_hip.h")]):
+            return
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", inc, src, "-o", out]
+        try:
+            r = subprocess.run(cmd, capture_output=True, text=True)
+            if r.returncode == 0:
+                return
+            why = "g++ failed for py_call.cpp:\n" + r.stdout + r.stderr
+        except OSError as e:
+            why = "no host compiler (%s)" % e
+    else:
+        why = "no Python.h"
+    if os.path.exists(out):
+        os.remove(out)
+    print("%s: moye_hip calls the library through ctypes" % why)
 
 
 def build(force=False, verbose=True):

@@ -2,7 +2,11 @@
 asm_mfma_hazards): the compiler does not know that those results are still in flight, so nothing of its own may name an
 accumulator or a fragment register between the MFMAs.  Synthetic listings: what must pass and what must be caught."""
 import os
+import shutil
 import sys
+import sysconfig
+
+import pytest
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "moye.jl_amd"))
 import build  # noqa: E402
@@ -67,3 +71,28 @@ def test_the_shipped_listing_is_checked_at_build_time():
         assert "v_mfma" in f.read()
     users = [s for s in build.SOURCES if s.endswith(".hip") and "gemm_mfma_w4_kernel.hpp" in open(os.path.join(build.CSRC, s)).read()]
     assert users and set(users) == set(build.ASM_MFMA_SOURCES)
+
+
+@pytest.mark.parametrize("why", ["no compiler", "an error", "no headers"])
+def test_the_calls_without_ctypes_are_optional(monkeypatch, tmp_path, capsys, why):
+    """Whatever keeps moye_hip/_call from being built, the build goes on and a module of an earlier one does not stay."""
+    def run(cmd, **kw):
+        if why == "no compiler":
+            raise FileNotFoundError(2, "No such file or directory", cmd[0])
+        return build.subprocess.CompletedProcess(cmd, 1, "", "error: expected")
+
+    old = tmp_path / "moye_hip" / ("_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    old.parent.mkdir()
+    old.write_bytes(b"of an earlier build")
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build.subprocess, "run", run)
+    if why == "no headers":
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    build._build_python_calls(True)
+    assert not old.exists() and "ctypes" in capsys.readouterr().out
+
+
+@pytest.mark.skipif(not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")) or shutil.which("g++") is None, reason="no headers or no compiler")
+def test_the_calls_without_ctypes_are_built_where_they_can_be():
+    import moye_hip
+    assert moye_hip._lib.calls is not None
