@@ -331,6 +331,8 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     static_assert(BAR >= 0 && BAR < A0, "the next k-step's stage is known to be there before its first read");
     // per wave and stage: RWA rows of A and RWB of B, LDA and LDB load-to-LDS instructions
     constexpr int RWA = BM / NW, RWB = BN / NW, LDA = RWA / RPI, LDB = RWB / RPI, ND = LDA + LDB;
+    static_assert(!kMid || NPOS - BAR - 1 >= ND, "dma_index_after: a group of its own for every load of a stage, none is left out");
+    static_assert(NI > 2 || BAR < H, "two columns: B1 is read last, and the barrier's wait for every read has to come before its first use");
     typedef typename In::frag frag;
     typedef std::conditional_t<In::kBytes == 4, W4TrFrag32, W4TrFrag> frag_t;
     typedef std::conditional_t<AMAJ != 0, frag_t, frag> frag_a;
@@ -603,7 +605,8 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
             constexpr int i = MOYE_I(P), j = MOYE_J(P);
             // B0 is followed by NI + 1 fragment reads, B1 by NI; a stricter count costs nothing where the
             // older reads are hundreds of clocks old (fp8: two reads per fragment, 32-clock MFMAs)
-            // (in reads: B1 .. B(NI-1) and the last two A fragments follow B0)
+            // (in reads: B1 .. B(NI-1) and the last two A fragments follow B0; NI == 2: nothing follows B1, which the wait at P == H
+            // does not cover then -- the barrier's, for every read, does: BAR < H)
             constexpr int after_b0 = (NI - 1) * RPB + 2 * RPA, after_b1 = (NI - 2) * RPB + 2 * RPA;
             if (P == 0) __builtin_amdgcn_s_waitcnt(0xC07F | ((after_b0 < 12 ? after_b0 : 12) << 8));
             if (P == H) __builtin_amdgcn_s_waitcnt(0xC07F | ((after_b1 < 12 ? after_b1 : 12) << 8));
