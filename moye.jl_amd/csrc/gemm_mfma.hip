@@ -375,30 +375,6 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
         const int ranges = a.split > 1 ? a.split : 1;
         const int64_t k_bytes_all = (int64_t)a.K * eb * ranges;
         const bool whole256 = a.M % 256 == 0 && a.N % 256 == 0 && a.K % (128 / eb) == 0;
-        // few elements, or few tiles: the forms that gemm_form_choose prices (operands in 16-byte pieces, any D, any epilogue)
-        const bool form_open = ranges == 1 && bk_elems == 0 && waves <= 1 && stages == 0 && ((int64_t)a.K * eb) % 16 == 0 &&
-                               !(a.flags & (MOYE_GEMM_PINGPONG | MOYE_GEMM_WAVE4 | kGemmAMajorM | kGemmBMajorN)) && (a.lda * eb) % 16 == 0 &&
-                               (a.ldb * eb) % 16 == 0 && (reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.B)) % 16 == 0 && row_offsets_fit(a, 256, eb);
-        const bool tiles_in_rings = form_open && eb <= 2;  // (what is left of a larger problem may run on those of the forms)
-        if (form_open) {
-            GemmForm form = lib ? lib->form : GemmForm::kOther;
-            if (!lib) {
-                const TileChoice c = gemm_plan(a.M, a.N, k_bytes_all, eb == 4, a.M % 64 == 0 && a.N % 64 == 0 && k_bytes_all % 128 == 0, 16, cus, 1);
-                double us = rtiles >= cus / 4 ? std::min(c.us, gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, !whole256, cus)) : c.us;
-                form = gemm_form_choose(a.M, a.N, k_bytes_all, eb, cus, us, &us, part);
-            }
-            if (form >= GemmForm::kTile128x64) return gemm_mfma_w4_tiles_dispatch(in_dt, out_dt, form, a, plan);
-            if (form != GemmForm::kOther) return gemm_mfma_blocks_dispatch(in_dt, out_dt, form, a, plan);
-        }
-        const TileChoice choice = lib && lib->tile != 256 ? *lib
-                                  : gemm_plan(a.M, a.N, k_bytes_all, eb == 4, a.M % 64 == 0 && a.N % 64 == 0 && ((int64_t)a.K * eb) % 128 == 0, 16, cus, ranges);
-        // (operands that were left M- or N-major: the host made sure of whole 128 x 128 tiles, an aligned D and no K ranges;
-        // such a call takes whole 256 x 256 or 128 x 128 tiles, never 64 x 64 ones, ragged ones or fringes)
-        const bool majors = a.flags & (kGemmAMajorM | kGemmBMajorN);
-        const bool prefer256 = lib ? lib->tile == 256
-                               : ranges > 1 ? rtiles >= cus / 2
-                                            : rtiles >= cus / 4 && gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, !whole256, cus) <= choice.us;
-        const bool big = whole256 && prefer256;
         // A large problem whose M or N is not a multiple of 256: the interior runs on 256x256 tiles, the fringe to the
         // right (all interior rows, the last N % 256 columns) and the fringe below (the last M % 256 rows, all columns)
         // on the kernels that take residue tiles.  Three launches on the same stream, disjoint parts of D.
@@ -420,11 +396,43 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
         const bool guarded_takes_interior = in_dt != MOYE_F8E4M3 && stages < 3 && (waves <= 1 || waves == 8) &&
                                             !(a.flags & (MOYE_GEMM_WAVE4 | MOYE_GEMM_PINGPONG | kGemmAMajorM | kGemmBMajorN | kGemmAtom32));
         const bool thin_shape = (fr_m > 0 || fr_n > 0) && fr_m <= 64 && fr_n <= 64 && a.K % (128 / eb) == 0 && aligned_ab && ranges == 1 &&
-                                (aligned || guarded_takes_interior);
+                                (aligned || guarded_takes_interior) && (int64_t)(M0 / 256) * (N0 / 256) >= cus / 4;
         const double fringe_us = (fr_n > 0 ? 4.5 + (double)(M0 + fr_n) * (double)k_bytes_all / 6.0e6 : 0.0) +
                                  (fr_m > 0 ? 4.5 + (double)(a.N + fr_m) * (double)k_bytes_all / 6.0e6 : 0.0);
-        const bool thin = thin_shape && (int64_t)(M0 / 256) * (N0 / 256) >= cus / 4 &&
-                          gemm_plan_cost_256(M0, N0, k_bytes_all, eb == 4, false, cus) + fringe_us <= choice.us;
+        // few elements, or few tiles: the forms that gemm_form_choose prices (operands in 16-byte pieces, any D, any epilogue)
+        const bool form_open = ranges == 1 && bk_elems == 0 && waves <= 1 && stages == 0 && ((int64_t)a.K * eb) % 16 == 0 &&
+                               !(a.flags & (MOYE_GEMM_PINGPONG | MOYE_GEMM_WAVE4 | kGemmAMajorM | kGemmBMajorN)) && (a.lda * eb) % 16 == 0 &&
+                               (a.ldb * eb) % 16 == 0 && (reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.B)) % 16 == 0 && row_offsets_fit(a, 256, eb);
+        const bool tiles_in_rings = form_open && eb <= 2;  // (what is left of a larger problem may run on those of the forms)
+        bool thin_forms = false;
+        if (form_open) {
+            GemmForm form = lib ? lib->form : GemmForm::kOther;
+            double us = lib ? lib->us : 0.0;
+            if (!lib) {
+                const TileChoice c = gemm_plan(a.M, a.N, k_bytes_all, eb == 4, a.M % 64 == 0 && a.N % 64 == 0 && k_bytes_all % 128 == 0, 16, cus, 1);
+                us = rtiles >= cus / 4 ? std::min(c.us, gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, !whole256, cus)) : c.us;
+                form = gemm_form_choose(a.M, a.N, k_bytes_all, eb, cus, us, &us, part);
+            }
+            // (thin fringes in launches of their own leave an interior that may have a cheaper form; 5 % for the two launches more.  bf16, B
+            // not cached, us: 2049 x 4097 x 8192 195 on 363 tiles of 192 x 128, 144 as 256 of 128 x 256 and two fringes; 4099 x 2050 x 4096
+            // 100 and 82, 2049 x 4097 x 2048 69 and 55; but 2048 x 3088 x 6144 84 either way, cached 73 and 79)
+            if (double interior; thin_shape && form >= GemmForm::kTile128x64) {
+                gemm_form_choose(M0, N0, k_bytes_all, eb, cus, 1e30, &interior, true);
+                thin_forms = interior + fringe_us < 0.95 * us;
+            }
+            if (form >= GemmForm::kTile128x64 && !thin_forms) return gemm_mfma_w4_tiles_dispatch(in_dt, out_dt, form, a, plan);
+            if (form != GemmForm::kOther && !thin_forms) return gemm_mfma_blocks_dispatch(in_dt, out_dt, form, a, plan);
+        }
+        const TileChoice choice = lib && lib->tile != 256 ? *lib
+                                  : gemm_plan(a.M, a.N, k_bytes_all, eb == 4, a.M % 64 == 0 && a.N % 64 == 0 && ((int64_t)a.K * eb) % 128 == 0, 16, cus, ranges);
+        // (operands that were left M- or N-major: the host made sure of whole 128 x 128 tiles, an aligned D and no K ranges;
+        // such a call takes whole 256 x 256 or 128 x 128 tiles, never 64 x 64 ones, ragged ones or fringes)
+        const bool majors = a.flags & (kGemmAMajorM | kGemmBMajorN);
+        const bool prefer256 = lib ? lib->tile == 256
+                               : ranges > 1 ? rtiles >= cus / 2
+                                            : rtiles >= cus / 4 && gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, !whole256, cus) <= choice.us;
+        const bool big = whole256 && prefer256;
+        const bool thin = thin_shape && (thin_forms || gemm_plan_cost_256(M0, N0, k_bytes_all, eb == 4, false, cus) + fringe_us <= choice.us);
         // (the hand-ordered kernel's guarded forms: K of whole 16-byte pieces)
         const bool hand_ordered_ragged = (eb == 2 || eb == 4 || in_dt == MOYE_F8E4M3) && ((int64_t)a.K * eb) % 16 == 0 &&
                                          stages < 2 && row_offsets_fit(a, 256, eb);
