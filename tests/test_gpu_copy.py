@@ -1336,3 +1336,20 @@ def test_conversions_in_place(mh, src_dt, dst_dt, L):
                 mh.copyto_(tensor_of(d), tensor_of(mem.as_strided((rows, L), (L + pad, 1), off)))
             torch.cuda.synchronize()
             assert torch.equal(mem.view(torch.int16).cpu(), want.view(torch.int16).cpu()), (rows, pad, off, masked)
+
+
+@pytest.mark.parametrize("pair,ni,nj", [("uint8", 4104, 4096), ("uint8", 4104, 4080), ("uint8", 4097, 4224), ("bfloat16->float8_e4m3fn", 4104, 4224), ("float32->float8_e4m3fn", 8200, 2176),
+                                        ("int32", 8192, 8200), ("int32", 9216, 9000), ("float32->bfloat16", 10240, 10300), ("int16", 16384, 10001)])
+def test_transposes_with_one_ragged_pitch(mh, pair, ni, nj):
+    """Rows of whole lines on one side only, either side of the lines of the choice between hinted and ordinary accesses (16 Mi
+    elements of bytes, 300 MiB of the source)."""
+    sdt, ddt = [getattr(torch, x) for x in (pair.split("->") * 2)[:2]]
+    bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32}
+    g = torch.Generator(device="cuda").manual_seed(ni + nj)
+    raw = torch.randint(0, 256, (ni * nj * sdt.itemsize,), generator=g, device="cuda", dtype=torch.uint8)
+    src = (raw[:ni * nj].float() - 128).to(sdt) if sdt != ddt else raw.view(sdt)
+    dst = torch.full((ni * nj + 64,), 0x5A, dtype=bits[ddt.itemsize], device="cuda")
+    mh.copyto_(_tens(mh, dst[:ni * nj].view(ddt), (ni, nj), (nj, 1)), _tens(mh, src, (ni, nj), (1, ni)))
+    torch.cuda.synchronize()
+    want = src.to(ddt).view(bits[ddt.itemsize]).view(nj, ni).t()
+    assert torch.equal(dst[:ni * nj].view(ni, nj), want) and bool((dst[ni * nj:] == 0x5A).all()), (pair, ni, nj)
