@@ -373,12 +373,12 @@ static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
     if (a.batch == 1 && a.ni < a.nj && (a.ni >= 4096 || !(few || lines))) a.band = 64;
     // Which accesses go without the non-temporal hint.  Lines of the source that two tiles share (a pitch that is no whole lines), or a
     // call of which the 256 MiB memory-side cache holds a good part: ordinary loads.  Bytes whose destination has such a pitch, from 16 Mi
-    // elements on: ordinary stores instead.  us with operands that are not cached, hinted / loads / stores (/ both): f32 3000^2 18.3 / 17.0 / 19.0 /
+    // elements on: ordinary stores instead.  us, hinted / loads / stores (/ both): f32 3000^2 18.3 / 17.0 / 19.0 /
     // 18.4, 10001 x 7003 134.6 / 118.8 / 146 / 125, 4096^2 24.3 / 20.4 / 24.2 / 28.6, but 16384 x 2048 47.7 / 51.2 / 51.1 / 56.0, 8192^2 94.8 / 101 / 102 / 109
     // and 2796 x 693 5.6 / 6.2 / 5.8 / 6.0; f32 -> bf16 4096^2 18.5 / 15.7 / 18.8 / 19.4, 5000 x 3000 19.1 / 16.1 / 18.6 / 18.0; fp16 10001 x 7003 75.3 /
     // 70.2 / 80.4 / 73.7; bytes 5000 x 7003 26.7 / 27.2 / 21.7 / 21.7, but 1968 x 6271 9.2 / 9.8 / 10.3 / 10.4; bf16 -> fp8 9001 x 7003 61.4 / 57.8 / 46.0 / 53.0.
     //   Only the destination's pitch ragged, the source's lines read once each: ordinary loads while the cache holds most of the source, up to
-    // 300 MiB (f32 5760 x 12408 120.7 / 102.1, 8192 x 8200 101.5 / 104.2 and cached 99.9 / 80.2), hinted ones beyond (f32 9216 x 9000 126.6 / 135.0,
+    // 300 MiB (f32 8192 x 8200 101.5 / 104.2 but cached 99.9 / 80.2, 5760 x 12408 121.5 / 123.3 but cached 120.5 / 105), hinted ones beyond (f32 9216 x 9000 126.6 / 135.0,
     // 16000 x 16010 445 / 471; f32 -> bf16 9216 x 9000 94.8 / 100.9, 14336 x 7000 114.9 / 121.4, 7168 x 14003 127.3 / 129.5; fp16 20480 x 10000
     // 156.3 / 165.3).  Only the source's, bytes: loads (12408 x 5760 40.4 / 35.1 / 42.3, 10000 x 20480 99.4 / 87.4 / 99.9; bf16 -> fp8 7000 x 7168 33.1 /
     // 31.2 / 36.2).

@@ -456,9 +456,11 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
             const int tm = (a.M + 255) / 256, tn = (a.N + 255) / 256;
             // What the dispatcher runs the rest on, priced.  The 1.15 comes off where 128 x 128 tiles carry it.  64 x 64 tiles have
             // no ragged form: two or three of them on a CU take about as much less than their price, one takes all of it (f16
-            // 4992 x 3200 x 8320, 156 workgroups for the rest, 265 us in one launch, 286 in two), and of the price of four only
+            // 4992 x 3200 x 8320: 274 us in one launch, 286 with 156 workgroups of them for the rest; on 78 tiles of 128 x 64 in a ring,
+            // which it takes now, 252), and of the price of four only
             // the launch, which is counted below, can come off (bf16 2240 x 8640 x 5248, 945 for 448 rows, 219 and 228, 198
             // by columns; fp8 16320 x 1280 x 9856, 1020, 208 either way, 192 by columns).
+            // (on64: the choice apart from the tiles in deep rings is 64 x 64 ones)
             bool on64 = false;
             auto alone = [&](int64_t m, int64_t n) {
                 double us;
@@ -483,8 +485,10 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
                 return takes256 ? std::min(on256, us) : us;
             };
             // One launch.  Its 128 x 128 tiles do not carry the 1.15 where they fill two rounds of two to a CU and lose half a tile along
-            // one edge; against a rest on 64 x 64 tiles that decides (bf16 5056 x 3200 x 1920 62 us in one launch, 76 in two; fp8
-            // 7552 x 2112 x 4608 79 and 88; but bf16 1088 x 13952 x 2304, 64 rows left for the short-M kernel, 92 and 82).
+            // one edge; against a rest of on64 that decides (bf16 5056 x 3200 x 1920 62 us in one launch, 76 in two with the rest on
+            // 64 x 64 tiles; but bf16 1088 x 13952 x 2304, 64 rows left for the short-M kernel, 92 and 82).  Where deep rings would
+            // carry that rest it stays one launch as well, which is not the faster of the two: over fourteen such problems two
+            // take 0.90 to 0.99 of its time (bf16 5056 x 3200 x 1920 70.5 / 68.7, 1152 x 14016 x 1920 85 / 76; fp8 8512 x 1920 x 3456 64.4 / 60.2).
             const bool half_tile = eb != 4 && choice.tile == 128 && !k_tail && a.M % 64 == 0 && a.N % 64 == 0 && (a.M % 128 == 0) != (a.N % 128 == 0) &&
                                    (((int64_t)a.M + 127) / 128) * (((int64_t)a.N + 127) / 128) <= 4 * (int64_t)cus;
             const double one_us = prefer256 ? guarded * gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, false, cus) : choice.us;

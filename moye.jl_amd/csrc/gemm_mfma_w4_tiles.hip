@@ -1,7 +1,10 @@
 // The hand-ordered kernel (gemm_mfma_w4_kernel.hpp) on tiles between 128 x 64 and 128 x 256, whole-line stages in rings of three
 // to five, one workgroup per CU: problems of few tiles, where 128 x 128 and 256 x 256 ones in two stages leave CUs idle or
 // every k-step waits for the loads of the step before (two stages: a k-step takes a load's latency, 0.85 us for 128 x 128 tiles
-// with a CU each; in a ring of four 0.4-0.54, which is the LDS: 768 cycles of fragment reads and stage writes for 512 of MFMAs).
+// with a CU each; in a ring of four 0.4-0.54).  What bounds them then is neither pipe alone.  Cycles of a k-step, of which the MFMAs /
+// the LDS's reads, by counters, bf16, K = 4096 or 8192: 128 x 128 1100, 512 / 395; 128 x 192 1500, 768 / 480; 192 x 128 1320, 768 / 540; 128 x 256
+// 2060, 1024 / 530; bank conflicts 1 % of them.  A wave waits for loads, reads or the barrier for 24 to 29 % of its time, and for its turn
+// to issue, with the other wave of its SIMD in the matrix pipe, for 42 to 50 %.
 // The ring is what fits beside nothing else in 160 KiB; four stages where three would do made no difference (128 x 192
 // 50.3 / 51.0 us at 1000 x 6144 x 4096).  Eight waves against four: 128 x 128 a twelfth faster where operands are cached,
 // 128 x 256 a twentieth, 128 x 192 the same; 128 x 64 has room for four.  Always the guarded form (ragged tiles, any D, a K tail):

@@ -17,6 +17,7 @@
 // of gemm_form_choose, whose formula and prices are their own.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 #include <initializer_list>
 
@@ -27,7 +28,7 @@ namespace moye {
 enum class GemmForm { kOther, kBlock32x32, kBlock64x32, kBlock64x64, kTile128x64, kTile128x128, kTile128x192, kTile192x128, kTile128x256 };
 
 struct TileChoice {
-    int tile;   // 64 or 128
+    int tile;   // 64, 128 or 256; 0 where `form` says what runs
     int split;  // K ranges
     double us;
     GemmForm form = GemmForm::kOther;
