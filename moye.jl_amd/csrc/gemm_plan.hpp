@@ -243,4 +243,11 @@ inline int gemm_short_m_ntw(int64_t M, int64_t N, int64_t k_bytes, int cus, int 
     return best;
 }
 
+// The hardware deals consecutive workgroups to the XCDs in turn.  Which of `n` tiles workgroup `bid` takes, so that each XCD gets one
+// run of neighbouring tiles, the first n % xcds of them a tile more than the others.
+constexpr int tile_in_xcd_runs(int bid, int n, int xcds) {
+    const int xcd = bid % xcds, rest = n % xcds;
+    return xcd * (n / xcds) + (xcd < rest ? xcd : rest) + bid / xcds;
+}
+
 }  // namespace moye

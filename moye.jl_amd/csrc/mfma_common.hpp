@@ -1,6 +1,7 @@
 // Element traits, LDS swizzle and tile mapping shared by the MFMA GEMM kernels.
 #pragma once
 
+#include "gemm_plan.hpp"
 #include "kernels.hpp"
 
 namespace moye {
@@ -186,15 +187,19 @@ __device__ __forceinline__ void store_d_chunk(const GemmArgs& p, char* d, const 
 }
 
 // blockIdx -> (tile_m, tile_n).  Hardware deals consecutive workgroup ids round-robin to the 8
-// XCDs; remapping id -> (id % 8) * (n / 8) + id / 8 hands each XCD one contiguous run of tiles,
+// XCDs; tile_in_xcd_runs hands each XCD one contiguous run of tiles,
 // and inside a run tiles are walked in bands of 8 tile-rows so that the A and B panels an
 // XCD's L2 holds are reused by the workgroups that follow.
 // (`bid` of `n` tiles: a persistent kernel walks bid = blockIdx.x, blockIdx.x + gridDim.x, ... with gridDim.x a multiple of
 // the number of XCDs, so every tile of a workgroup comes from its own XCD's run)
+// Tile counts that the XCDs do not divide get runs too: bf16 1352 x 6912 x 6528 (11 x 36 tiles of 128 x 192) 167 us in the order they are
+// dealt, 144 in runs, 1340 x 7232 x 8000 (7 x 57) 190 / 173, fp8 850 x 7424 x 4288 (7 x 29, cached) 43 / 34.  Not several bands of fewer
+// than 8 columns: dealt in order, each XCD has one tile-row of every band, and no other reads its rows of A (fp8 5567 x 560 x 2112, 44 x 5
+// tiles, cached 13.2 / 14.8).
 __device__ __forceinline__ void tile_of_index(int tiles_m, int tiles_n, int xcds, int flags, int bid, int n, int* tm, int* tn) {
     const int x = xcds;
-    if ((flags & 1) && x > 1 && (n % x) == 0) bid = (bid % x) * (n / x) + bid / x;
     constexpr int kGroup = 8;
+    if ((flags & 1) && x > 1 && (n % x == 0 || tiles_m < kGroup || tiles_n >= kGroup)) bid = tile_in_xcd_runs(bid, n, x);
     const int per_group = kGroup * tiles_n;
     const int g = bid / per_group;
     const int first_m = g * kGroup;
