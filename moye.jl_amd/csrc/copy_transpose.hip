@@ -380,12 +380,13 @@ static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
     //   Only the destination's pitch ragged, the source's lines read once each: ordinary loads while the cache holds most of the source, up to
     // 300 MiB (f32 8192 x 8200 101.5 / 104.2 but cached 99.9 / 80.2, 5760 x 12408 121.5 / 123.3 but cached 120.5 / 105), hinted ones beyond (f32 9216 x 9000 126.6 / 135.0,
     // 16000 x 16010 445 / 471; f32 -> bf16 9216 x 9000 94.8 / 100.9, 14336 x 7000 114.9 / 121.4, 7168 x 14003 127.3 / 129.5; fp16 20480 x 10000
-    // 156.3 / 165.3).  Only the source's, bytes: loads (12408 x 5760 40.4 / 35.1 / 42.3, 10000 x 20480 99.4 / 87.4 / 99.9; bf16 -> fp8 7000 x 7168 33.1 /
+    // 156.3 / 165.3) and for few elements (up to 4 Mi, of 16-bit sources 8, over 45 sizes 0.96 of the time with loads, cached 1.02: f32 512 x 4792
+    // 6.36 / 6.84, cached 5.32 / 5.19; f32 -> bf16 768 x 4128 7.02 / 7.40, 5.06 / 4.83; fp16 5760 x 963 6.88 / 7.11, 5.74 / 5.79).  Only the source's, bytes: loads (12408 x 5760 40.4 / 35.1 / 42.3, 10000 x 20480 99.4 / 87.4 / 99.9; bf16 -> fp8 7000 x 7168 33.1 /
     // 31.2 / 36.2).
     const int keep = few || (lines && DB == 1 && n <= 4 * Mi) ? 0
                      : lines                                  ? (n * (SB + DB) <= 160 * Mi ? 1 : 0)
                      : DB == 1                                ? (n < 16 * Mi ? 0 : dst_lines ? 1 : 2)
-                                                              : (src_lines && n * SB > 300 * Mi ? 0 : 1);
+                                                              : (src_lines && (n * SB > 300 * Mi || n <= (SB == 2 ? 8 : 4) * Mi) ? 0 : 1);
     auto fit = [&](std::initializer_list<Tile> tiles) { return first_that_fits(a, tiles); };
 #define MOYE_TILE(PI, NB, T, LDS) return launch_blocks<kSrc, kDst, SB, DB, PI, NB, T>(a, keep, LDS, st)
     if constexpr (SB == 2 && DB == 2) {

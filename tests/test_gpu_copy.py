@@ -1339,10 +1339,11 @@ def test_conversions_in_place(mh, src_dt, dst_dt, L):
 
 
 @pytest.mark.parametrize("pair,ni,nj", [("uint8", 4104, 4096), ("uint8", 4104, 4080), ("uint8", 4097, 4224), ("bfloat16->float8_e4m3fn", 4104, 4224), ("float32->float8_e4m3fn", 8200, 2176),
-                                        ("int32", 8192, 8200), ("int32", 9216, 9000), ("float32->bfloat16", 10240, 10300), ("int16", 16384, 10001)])
+                                        ("int32", 8192, 8200), ("int32", 9216, 9000), ("float32->bfloat16", 10240, 10300), ("int16", 16384, 10001),
+                                        ("int16", 4096, 2040), ("int16", 4096, 2056), ("int32", 2048, 2040), ("int32", 2048, 2056), ("float32->bfloat16", 2048, 2040)])
 def test_transposes_with_one_ragged_pitch(mh, pair, ni, nj):
     """Rows of whole lines on one side only, either side of the lines of the choice between hinted and ordinary accesses (16 Mi
-    elements of bytes, 300 MiB of the source)."""
+    elements of bytes, 300 MiB of the source, 8 Mi elements of 16 bits and 4 Mi of 32)."""
     sdt, ddt = [getattr(torch, x) for x in (pair.split("->") * 2)[:2]]
     bits = {1: torch.uint8, 2: torch.int16, 4: torch.int32}
     g = torch.Generator(device="cuda").manual_seed(ni + nj)
