@@ -414,8 +414,8 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
                 form = gemm_form_choose(a.M, a.N, k_bytes_all, eb, cus, us, &us, part);
             }
             // (thin fringes in launches of their own leave an interior that may have a cheaper form; 5 % for the two launches more.  bf16, B
-            // not cached, us: 2049 x 4097 x 8192 195 on 363 tiles of 192 x 128, 144 as 256 of 128 x 256 and two fringes; 4099 x 2050 x 4096
-            // 100 and 82, 2049 x 4097 x 2048 69 and 55; but 2048 x 3088 x 6144 84 either way, cached 73 and 79)
+            // not cached, us: 2049 x 4097 x 8192 175 on 363 tiles of 192 x 128, 145 as 256 of 128 x 256 and two fringes; 4099 x 2050 x 4096
+            // 90 and 77, 2049 x 4097 x 2048 61 and 51; but 2048 x 3088 x 6144 81 either way, cached 69 and 78)
             if (double interior; thin_shape && form >= GemmForm::kTile128x64) {
                 gemm_form_choose(M0, N0, k_bytes_all, eb, cus, 1e30, &interior, true);
                 thin_forms = interior + fringe_us < 0.95 * us;
@@ -487,8 +487,8 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
             // One launch.  Its 128 x 128 tiles do not carry the 1.15 where they fill two rounds of two to a CU and lose half a tile along
             // one edge; against a rest of on64 that decides (bf16 5056 x 3200 x 1920 62 us in one launch, 76 in two with the rest on
             // 64 x 64 tiles; but bf16 1088 x 13952 x 2304, 64 rows left for the short-M kernel, 92 and 82).  Where deep rings would
-            // carry that rest it stays one launch as well, which is not the faster of the two: over fourteen such problems two
-            // take 0.90 to 0.99 of its time (bf16 5056 x 3200 x 1920 70.5 / 68.7, 1152 x 14016 x 1920 85 / 76; fp8 8512 x 1920 x 3456 64.4 / 60.2).
+            // carry that rest it stays one launch as well: over fourteen such problems two take 0.98 of its time (B not cached, bf16 5056 x
+            // 3200 x 1920 65.7 / 66.9, 1152 x 14016 x 1920 73.9 / 65.5; fp8 8512 x 1920 x 3456 55.2 / 55.3).
             const bool half_tile = eb != 4 && choice.tile == 128 && !k_tail && a.M % 64 == 0 && a.N % 64 == 0 && (a.M % 128 == 0) != (a.N % 128 == 0) &&
                                    (((int64_t)a.M + 127) / 128) * (((int64_t)a.N + 127) / 128) <= 4 * (int64_t)cus;
             const double one_us = prefer256 ? guarded * gemm_plan_cost_256(a.M, a.N, k_bytes_all, eb == 4, false, cus) : choice.us;

@@ -11,7 +11,7 @@
 // a round of tiles or two, where its 3 % are less than a second set of instances is worth.  The barrier sits before the last
 // column's reads of the next stage (BAR < A0).
 // us before / now, operands not cached, bf16: 1000 x 6144 x 4096 69.9 / 49.9 (cached 49.5 / 43.0), 512 x 8192 x 8192 unsplit 109.9 / 72.6,
-// 300 x 7168 x 4096 59.8 / 32.8, 742 x 10496 x 5888 110.8 / 84.4, 1080 x 4352 x 1664 31.9 / 22.3.
+// 300 x 7168 x 4096 59.8 / 32.8, 742 x 10496 x 5888 110.8 / 89.6, 1080 x 4352 x 1664 31.9 / 22.3.
 #include "gemm_mfma_w4_kernel.hpp"
 #include "gemm_plan.hpp"
 
