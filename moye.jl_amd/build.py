@@ -35,6 +35,8 @@ SOURCES = {
     "gemm_mfma256w4_ops.hip": ["-ffp-contract=off"],
     "gemm_mfma256w4_persist.hip": ["-ffp-contract=off"],
     "gemm_mfma_w4_tiles.hip": ["-ffp-contract=off"],
+    "gemm_mfma_w4_majors_f16.hip": ["-ffp-contract=off"],
+    "gemm_mfma_w4_majors_bf16.hip": ["-ffp-contract=off"],
     "gemm_mfma128w4.hip": ["-ffp-contract=off"],
     "gemm_mfma128w4_majors.hip": ["-ffp-contract=off"],
     "gemm_mfma_skinny.hip": ["-ffp-contract=off"],
@@ -76,7 +78,8 @@ def _compile(item, force):
 # Kernels whose MFMAs are inline assembly: the compiler does not know how long their results take, so any
 # instruction of its own that touches an accumulator register next to them (a copy made by the register
 # allocator, an epilogue read scheduled upwards) would read a value that is not there yet, silently.
-ASM_MFMA_SOURCES = ["gemm_mfma256w4.hip", "gemm_mfma256w4_majors.hip", "gemm_mfma256w4_ops.hip", "gemm_mfma256w4_persist.hip", "gemm_mfma128w4.hip", "gemm_mfma128w4_majors.hip", "gemm_mfma_w4_tiles.hip"]
+ASM_MFMA_SOURCES = ["gemm_mfma256w4.hip", "gemm_mfma256w4_majors.hip", "gemm_mfma256w4_ops.hip", "gemm_mfma256w4_persist.hip", "gemm_mfma128w4.hip", "gemm_mfma128w4_majors.hip", "gemm_mfma_w4_tiles.hip",
+                    "gemm_mfma_w4_majors_f16.hip", "gemm_mfma_w4_majors_bf16.hip"]
 
 
 def check_accumulator_hazards(src, force=False):

@@ -274,8 +274,9 @@ static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, co
 // (named, or the library's own choice for a problem of whole 128 x 128 tiles with more than 64 rows), the two-stage
 // schedule, no K ranges; fp8 and fp32 on the hand-ordered kernel's whole 256 x 256 or 128 x 128 tiles with 128 bytes of K
 // per k-step (named so, or left to the library: 256 x 256 tiles when the problem has at least 128 of them), plain calls; the operand dense
-// along its rows with a pitch of whole 16-byte pieces, and D 16-byte aligned (the guarded instances, which take any D,
-// read K-major operands only).
+// along its rows with a pitch of whole 16-byte pieces, and D 16-byte aligned; or on the guarded tiles of majors_on_guarded_tiles, 16-bit types
+// and any D.
+static bool majors_on_guarded_tiles(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep, int cus);
 static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep,
                                 bool has_c, int cus) {
     const bool b16 = mma->atom == MOYE_MFMA_F32_16x16x32_F16 || mma->atom == MOYE_MFMA_F32_16x16x32_BF16;
@@ -286,11 +287,15 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
     const int64_t M = A.rows, N = B.rows, K = A.cols;
     const int eb = dtype_bytes(A.dtype);
     const int bm = mma->cta_tile_mnk[0], bn = mma->cta_tile_mnk[1], bk = mma->cta_tile_mnk[2];
-    if ((K * eb) % 128) return false;
+    const bool whole_lines = (K * eb) % 128 == 0;
+    const int64_t d_pitch = D.cs == 1 ? D.rs : D.cs;
+    const bool whole_d = (D.cs == 1 || D.rs == 1) && (d_pitch * dtype_bytes(D.dtype)) % 16 == 0 && reinterpret_cast<uintptr_t>(D.ptr) % 16 == 0;
     const bool four_waves = mma->atom_layout_mnk[0] * mma->atom_layout_mnk[1] == 4;
     const bool named256 = bm == 256 && bn == 256 && (b16 ? (bk == 0 || bk == 64) : bk * eb == 128) && !four_waves && M % 256 == 0 && N % 256 == 0;
     const bool named128 = bm == 128 && bn == 128 && bk * eb == 128 && M % 128 == 0 && N % 128 == 0;
-    const bool chosen = bm == 0 && bn == 0 && bk == 0 && M > 64 && M % 128 == 0 && N % 128 == 0;
+    const bool chosen = bm == 0 && bn == 0 && bk == 0 && M > 64 && M % 128 == 0 && N % 128 == 0 && whole_lines && whole_d;
+    if (!named256 && !named128 && !chosen && majors_on_guarded_tiles(mma, A, B, D, ep, cus)) return true;
+    if (!whole_lines || !whole_d) return false;
     if (wide) {
         // (the hand-ordered kernel reads such operands in plain calls only, and fp32 and fp8 have no other kernel that does)
         if (ep.op != MOYE_MAP_IDENTITY || mma->stages >= 2) return false;
@@ -303,14 +308,39 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
         return false;
     }
     (void)has_c;
-    const int64_t d_pitch = D.cs == 1 ? D.rs : D.cs;
-    if ((D.cs != 1 && D.rs != 1) || (d_pitch * dtype_bytes(D.dtype)) % 16 || reinterpret_cast<uintptr_t>(D.ptr) % 16) return false;
     for (const Mat* x : {&A, &B}) {
         if (x->cs == 1 || x->cols == 1) continue;  // K-major already
         if (x->rs != 1 || (x->cs * eb) % 16 || reinterpret_cast<uintptr_t>(x->ptr) % 16 || x->cs < x->rows) return false;
         if (wide && 256 * x->cs * eb >= ((int64_t)1 << 32)) return false;  // (the kernel's 32-bit lane offsets)
     }
     return true;
+}
+
+// ... and f16 / bf16 operands, tile left to the library, whose problem is no whole number of tiles: the guarded tiles that read such
+// operands (gemm_mfma_w4_majors.hpp).  Rows along M and N and K in whole 16-byte pieces (a K-major operand's row count is free), K of a
+// stage and more, any D, a C but no operation; unless copies and a K-major form cost less (gemm_majors_copies_pay).
+static bool majors_on_guarded_tiles(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep, int cus) {
+    GemmArgs g{};
+    g.ep_op = ep.op;
+    g.flags = mma->flags & 0xff00;
+    const int32_t in_dt = atom_input_dtype(mma->atom);
+    const bool atom16 = mma->atom == MOYE_MFMA_F32_16x16x32_F16 || mma->atom == MOYE_MFMA_F32_16x16x32_BF16;
+    const int waves = mma->atom_layout_mnk[0] * mma->atom_layout_mnk[1];
+    if (!atom16 || mma->cta_tile_mnk[0] || mma->cta_tile_mnk[1] || !majors_take_any_tile(in_dt, D.dtype, mma->cta_tile_mnk[2], waves, mma->stages, g)) return false;
+    if (A.cols % 8 || A.cols < 64 || A.rows <= 64 || B.rows <= 64 || (D.cs != 1 && D.rs != 1)) return false;
+    int64_t copied = 0;
+    int launches = 0;
+    for (const Mat* x : {&A, &B}) {
+        const bool kmajor = x->cs == 1 || x->cols == 1;
+        const int64_t pitch = kmajor ? x->rs : x->cs;
+        if (pitch % 8 || reinterpret_cast<uintptr_t>(x->ptr) % 16 || 256 * pitch * 2 >= ((int64_t)1 << 32)) return false;
+        if (kmajor) continue;
+        if (x->rs != 1 || x->rows % 8 || pitch < x->rows) return false;
+        copied += x->rows * x->cols;
+        ++launches;
+    }
+    const bool swap = column_major(D);
+    return !gemm_majors_copies_pay(swap ? B.rows : A.rows, swap ? A.rows : B.rows, A.cols * 2, copied, launches, cus);
 }
 
 // K-major copies of A and B where needed, then the fp32 partial products of a split-K call

@@ -336,10 +336,11 @@ static int32_t dispatch_atom32(int32_t in_dt, int32_t out_dt, int bm, int bn, in
     return launch_atom32<false>(in_dt, out_dt, a, plan);
 }
 
-// The part of a problem below its first m1 rows / to the right of its first n1 columns (bytes per element of the operands and of D)
+// The part of a problem below its first m1 rows / to the right of its first n1 columns (bytes per element of the operands and of D;
+// an operand that is not K-major has its rows next to each other)
 static GemmArgs rows_from(GemmArgs a, int64_t m1, int eb, int ob) {
     a.M -= (int)m1;
-    a.A = static_cast<const char*>(a.A) + m1 * a.lda * eb;
+    a.A = static_cast<const char*>(a.A) + m1 * (a.flags & kGemmAMajorM ? 1 : a.lda) * eb;
     a.D = static_cast<char*>(a.D) + m1 * a.ldd * ob;
     if (a.C) a.C = static_cast<const char*>(a.C) + m1 * a.ldc_m * ob;
     if (a.ep_x) a.ep_x = static_cast<const char*>(a.ep_x) + m1 * a.ep_xm * dtype_bytes(a.ep_xdt);
@@ -347,11 +348,69 @@ static GemmArgs rows_from(GemmArgs a, int64_t m1, int eb, int ob) {
 }
 static GemmArgs columns_from(GemmArgs a, int64_t n1, int eb, int ob) {
     a.N -= (int)n1;
-    a.B = static_cast<const char*>(a.B) + n1 * a.ldb * eb;
+    a.B = static_cast<const char*>(a.B) + n1 * (a.flags & kGemmBMajorN ? 1 : a.ldb) * eb;
     a.D = static_cast<char*>(a.D) + n1 * ob;
     if (a.C) a.C = static_cast<const char*>(a.C) + n1 * a.ldc_n * ob;
     if (a.ep_x) a.ep_x = static_cast<const char*>(a.ep_x) + n1 * a.ep_xn * dtype_bytes(a.ep_xdt);
     return a;
+}
+
+// Operands that keep their M- / N-major form, 16-bit types, tile left to the library: guarded tiles of 256 x 256 and in deep rings
+// (gemm_mfma_w4_majors.hpp), whole 256 x 256 and 128 x 128 ones in two stages (what calls on whole tiles also run with an epilogue
+// operation, gemm_mfma_tn_dispatch).  One launch of the cheapest of them by the prices of K-major operands; more 256 x 256 tiles than CUs:
+// also in two launches, whole rounds of them and the rest on what is cheapest for it alone, as K-major operands have it there.  bf16, operands
+// not cached, us before (K-major copies, or whole 256 x 256 / 128 x 128 tiles in one launch) / now: 6000 x 4096 x 14336 with B N-major 570 / 524,
+// 14336 x 4096 x 6000 with both the other way round 573 / 526, 7424 x 1152 x 3600 109 / 84, 3840 x 2048 x 1240 42 / 27; whole 14336 x 4096 x 4096
+// 376 / 364, 2048 x 4096 x 4096 73.7 / 62.4, 256 x 4096 x 4096 with B N-major 52.9 / 36.5.  A linear layer's forward and two gradients, 6000 x
+// 4096 -> 14336: 1690 / 1590; 1240 x 2048 -> 3840: 111 / 91.
+static int32_t dispatch_majors(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan) {
+    const int eb = 2, ob = dtype_bytes(out_dt), cus = plan.shape.cus;
+    const int64_t k_bytes = (int64_t)a.K * eb;
+    const bool aligned_d = !((a.ldd * ob) % 16 || reinterpret_cast<uintptr_t>(a.D) % 16);
+    auto whole = [&](int64_t m, int64_t n, int tile) { return m % tile == 0 && n % tile == 0 && k_bytes % 128 == 0 && aligned_d; };
+    struct Part { int64_t m, n; GemmForm form; int tile; double us; };  // (tile: 256 or 128 in two stages where form is kOther)
+    auto one = [&](int64_t m, int64_t n) {
+        const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
+        double us;
+        const FormPrice* f = gemm_majors_form(m, n, k_bytes, cus, !a.C || whole(m, n, 256), tiles256 <= cus && whole(m, n, 128), &us);
+        Part best{m, n, f->form, f->tm, us};
+        if (tiles256 > cus && (!a.C || whole(m, n, 256)))  // (the prices of several rounds do not compare: gemm_form_choose)
+            best = Part{m, n, GemmForm::kOther, 256, (whole(m, n, 256) ? 1.0 : 1.03) * gemm_plan_cost_256(m, n, k_bytes, false, false, cus)};
+        return best;
+    };
+    auto run = [&](const Part& t, GemmArgs g) {
+        g.M = (int)t.m; g.N = (int)t.n;
+        if (t.form == GemmForm::kOther && whole(t.m, t.n, t.tile))
+            return t.tile == 256 ? gemm_mfma_tn_256_w4_dispatch(in_dt, out_dt, g, 8, 128, false, plan)
+                                 : (g.tiles_m = g.M / 128, g.tiles_n = g.N / 128, gemm_mfma_tn_128_w4_dispatch(in_dt, out_dt, g, plan));
+        g.flags |= kGemmRagged;
+        return in_dt == MOYE_F16 ? gemm_mfma_w4_majors_f16(out_dt, t.form, g, plan) : gemm_mfma_w4_majors_bf16(out_dt, t.form, g, plan);
+    };
+    const Part all = one(a.M, a.N);
+    Part first{0, 0, GemmForm::kOther, 256, 0.0}, rest = first;
+    const int tm = (a.M + 255) / 256, tn = (a.N + 255) / 256;
+    const int64_t tiles = (int64_t)tm * tn;
+    if (tiles > cus && tiles % cus && !a.C) {
+        double best_us = 0.96 * all.us;
+        for (const bool by_rows : {true, false}) {
+            const int other = by_rows ? tn : tm, nt = by_rows ? tm : tn;
+            for (int64_t rounds = tiles / cus; rounds >= 1 && rounds + 1 >= tiles / cus; --rounds) {
+                const int64_t rows = rounds * cus / other;
+                if (rows < 1 || rows >= nt) continue;
+                const int64_t m = by_rows ? rows * 256 : a.M, n = by_rows ? a.N : rows * 256;
+                const double us1 = (whole(m, n, 256) ? 1.0 : 1.03) * gemm_plan_cost_256(m, n, k_bytes, false, false, cus);
+                const Part left = by_rows ? one(a.M - m, a.N) : one(a.M, a.N - n);
+                if (us1 + 2.0 + left.us < best_us) {
+                    best_us = us1 + 2.0 + left.us;
+                    first = Part{m, n, GemmForm::kOther, 256, us1};
+                    rest = left;
+                }
+            }
+        }
+    }
+    if (first.m == 0) return run(all, a);
+    if (int32_t e = run(first, a)) return e;
+    return run(rest, first.m < a.M ? rows_from(a, first.m, eb, ob) : columns_from(a, first.n, eb, ob));
 }
 
 // K-major A and B, N-contiguous D.  bk_elems = 0 picks the default K extent per tile.
@@ -367,6 +426,9 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
     if ((bm == 0 && bn == 0 && gemm_short_m(a.M, a.N, (int64_t)a.K * eb * (a.split > 1 ? a.split : 1), eb == 4, cus)) || (bm == a.M && bm <= 64 && bn == 16))
         return gemm_mfma_skinny_dispatch(in_dt, out_dt, a, plan);
     const bool chosen_here = bm == 0 && bn == 0;
+    if (chosen_here && (a.flags & (kGemmAMajorM | kGemmBMajorN)) && majors_take_any_tile(in_dt, out_dt, bk_elems, waves, stages, a) && row_offsets_fit(a, 256, eb) &&
+        !((a.lda * eb) % 16 || (a.ldb * eb) % 16 || (reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.B)) % 16))
+        return dispatch_majors(in_dt, out_dt, a, plan);
     if (bm == 0 && bn == 0) {
         // the library chooses: 256 x 256 tiles, one per CU, where the cost model of gemm_plan.hpp prices them below
         // 128 x 128 and 64 x 64 tiles (they need not fill the chip: fp16 4096 x 2304 x 4096, 144 tiles, 73 us against 93;

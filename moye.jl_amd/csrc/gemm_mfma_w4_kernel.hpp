@@ -307,12 +307,21 @@ struct W4F32L {
 // k-rows 4 g + e and 16 + 4 g + e (k-rows of 1 KiB, 32 per stage; the 64-byte piece index XORed with (row / 4) % 2, so
 // that the two k-rows the 32 lanes of a pass read lie in different halves of the banks).  Whole-line stages, plain calls
 // on whole tiles: the 256 x 256 tile with eight waves, the 128 x 128 tile with four (k-rows of 128 operand rows).
+// AMAJ / BMAJ = 2: the same for guarded tiles of any side that 64 divides, 16-bit types (gemm_mfma_w4_majors_{f16,bf16}.hip).
+// The operand's half of a stage is blocks of 64 operand rows, 64 k-rows of one 128-byte line each, so that a load-to-LDS
+// instruction reads eight whole lines as for a K-major operand.  A line's four 32-byte granules are XORed with
+// (row / 2) % 2 | 2 ((row / 8) % 2): the k-rows 0-3 and 8-11 (16-19, 24-27) that the 32 lanes of a pass read then lie in eight bank
+// groups, two lines to a sweep of the banks.  Pieces beyond the operand's last row are read from its last piece.  A K that
+// ends inside a stage: the last stage holds the last 64 k all the same, those that the stage before has brought as zeros.
 template <typename In, typename Out, int WGN, bool kBias = false, bool kRagged = false, int TILE = 256, int AMAJ = 0, int BMAJ = 0, bool kOps = false, bool kNoC = false, bool kPersist = false, int TILE_N = TILE>
 __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRing * In::kRow <= 256 ? 2 : 1) void gemm_mfma_tn_256_w4(GemmArgs p) {
     constexpr bool kMid = TILE != TILE_N || TILE == 192 || (TILE == 128 && In::kRow == 128 && In::kRing > 2);
-    static_assert(!(AMAJ || BMAJ) || (In::kRow == 128 && ((TILE == 256 && WGN == 4) || (TILE == 128 && WGN == 2)) && !kBias && !kRagged),
+    constexpr bool kBlocks64 = AMAJ == 2 || BMAJ == 2;
+    static_assert(!(AMAJ == 1 || BMAJ == 1) || (In::kRow == 128 && ((TILE == 256 && WGN == 4) || (TILE == 128 && WGN == 2)) && !kBias && !kRagged && !kBlocks64),
                   "operands that are not K-major: whole-line stages, eight waves, plain whole tiles");
-    static_assert(!kRagged || (!kBias && In::kRow == 128 && !AMAJ && !BMAJ), "ragged tiles: the plain whole-line form, K-major operands");
+    static_assert(!kBlocks64 || (In::kRow == 128 && In::kBytes == 2 && WGN == 4 && kRagged && TILE % 64 == 0 && TILE_N % 64 == 0),
+                  "... in blocks of 64 rows: 16-bit types, whole-line stages, eight waves, guarded tiles");
+    static_assert(!kRagged || (!kBias && In::kRow == 128 && AMAJ != 1 && BMAJ != 1), "ragged tiles: the plain whole-line form");
     static_assert(!kOps || (In::kRow == 128 && TILE == 256 && WGN == 4 && !kBias && !AMAJ && !BMAJ), "epilogue operations: whole-line stages, eight waves, K-major operands");
     static_assert(!kPersist || (In::kRow == 128 && TILE == 256 && WGN == 4 && !kRagged && !kOps && !AMAJ && !BMAJ),
                   "the persistent form: whole-line stages, eight waves, whole tiles, K-major operands (its C patches lie beside the stages)");
@@ -340,13 +349,14 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     constexpr int RPT = In::kBytes == 4 ? 8 : 4;                    // LDS reads per fragment of a transposed operand
     constexpr int RPA = AMAJ ? RPT : RPF, RPB = BMAJ ? RPT : RPF;  // LDS reads per fragment of A and of B
     // transposed operand halves of a stage: k-rows of TROW bytes, a swizzle granule of 16 operand rows (GB bytes)
-    constexpr int TROW = TILE * In::kBytes, TKROWS = 128 / In::kBytes, TLPR = TROW / 16, TRPI = 64 / TLPR, GB = 16 * In::kBytes;
+    constexpr int TROW = kBlocks64 ? 128 : TILE * In::kBytes, TKROWS = 128 / In::kBytes, TLPR = TROW / 16, TRPI = 64 / TLPR, GB = 16 * In::kBytes;
     // (bytes: the 32 lanes of a pass read k-rows 0-7 and 16-23.  On the 256 x 256 tile a k-row has sixteen 16-byte granules
     // and bit 4 of the row picks the half of them; on the 128 x 128 tile it has eight, a k-row is half a sweep of the
     // banks, and the k-rows whose bit 4 is set are stored with their neighbour's place instead (tr_place), so that rows
     // j and 16 + j lie in different halves.  Without either, every such read took two more cycles.)
     auto tr_swz = [](int krow) {
-        return In::kBytes == 2   ? ((krow & 3) | (((krow >> 3) & 1) << 2))
+        return kBlocks64         ? (((krow >> 1) & 1) | (((krow >> 3) & 1) << 1))
+               : In::kBytes == 2 ? ((krow & 3) | (((krow >> 3) & 1) << 2))
                : In::kBytes == 1 ? ((krow & 7) | (TROW >= 256 ? ((krow >> 4) & 1) << 3 : 0))
                                  : ((krow >> 2) & 1);
     };
@@ -418,10 +428,18 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     [[maybe_unused]] const int last_a = p.M - 1 - tm * BM, last_b = p.N - 1 - tn * BN;  // ragged: the last row of the operand, counted from the tile's first
     // an M-major (N-major) operand: its instruction qi of wave w brings k-rows 8 w + 2 qi + lane / 32 of the stage,
     // lane l the 16-byte piece that belongs in physical slot l % 32 of its k-row
-    static_assert(!(AMAJ || BMAJ) || (TKROWS / NW == TRPI * LDA && LDA == LDB), "a wave's k-rows of a transposed operand: LDA instructions");
+    static_assert(!(AMAJ == 1 || BMAJ == 1) || (TKROWS / NW == TRPI * LDA && LDA == LDB), "a wave's k-rows of a transposed operand: LDA instructions");
 #pragma unroll
     for (int q = 0; q < ND; ++q) {
         const int qi = q < LDA ? q : q - LDA;
+        if ((q < LDA && AMAJ == 2) || (q >= LDA && BMAJ == 2)) {
+            // instruction t of the operand's half: k-rows 8 (t % 8) .. + 7 of its block t / 8 of 64 operand rows
+            const int t = wave * (q < LDA ? LDA : LDB) + qi, krow = (t & 7) * 8 + lane / 8;
+            const int col = (t >> 3) * 64 + (((lane & 7) >> 1) ^ tr_swz(krow)) * 16 + (lane & 1) * 8;
+            // (the operand's rows are whole pieces of eight: the last piece that has them)
+            voff[q] = (uint32_t)(krow * (q < LDA ? pitch_a : pitch_b) + (int64_t)min(col, (q < LDA ? last_a : last_b) - 7) * 2);
+            continue;
+        }
         if ((q < LDA && AMAJ) || (q >= LDA && BMAJ)) {
             // (the k-row whose place in the stage this lane fills)
             const int krow = tr_place(wave * (TKROWS / NW) + TRPI * qi + lane / TLPR), p16 = lane % TLPR;
@@ -438,17 +456,20 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     // the last in time as well
     const int g0 = ((p.flags & kGemmRotateK) && !tail_pieces) ? (int)((int64_t)(blockIdx.x % p.xcds) * nsteps / p.xcds) * SPS : 0;
     // what a lane whose piece lies beyond K in the last stage subtracts from its offset to land on the row's first piece
-    [[maybe_unused]] const uint32_t tail_cut = (kRagged && tail_pieces && lch >= tail_pieces) ? (uint32_t)lch * 16 : 0;
+    [[maybe_unused]] const uint32_t tail_cut = (kRagged && !kBlocks64 && tail_pieces && lch >= tail_pieces) ? (uint32_t)lch * 16 : 0;
+    // ... and how many pieces (of 16 bytes of K) early the last stage starts where operands lie in blocks of 64 rows (K is a stage or more)
+    [[maybe_unused]] const int tail_back = kBlocks64 && tail_pieces ? 8 - tail_pieces : 0;
     auto dma1 = [&](int g, int ring_slot, auto qc) __attribute__((always_inline)) {
         constexpr int Q = decltype(qc)::value;
         const int gr = g + g0 >= nstages ? g + g0 - nstages : g + g0;
         // (stage gr of a K-major operand starts kRow bytes further along every row, of an M-major one 64 k-rows further down)
-        const char* const base = uniform_ptr(Q < LDA ? a_tile + (AMAJ ? (int64_t)gr * TKROWS * pitch_a : (int64_t)gr * kRow)
-                                                    : b_tile + (BMAJ ? (int64_t)gr * TKROWS * pitch_b : (int64_t)gr * kRow));
+        const int64_t back = kBlocks64 && gr == nstages - 1 ? tail_back : 0;
+        const char* const base = uniform_ptr(Q < LDA ? a_tile + (AMAJ ? ((int64_t)gr * TKROWS - back * 8) * pitch_a : (int64_t)gr * kRow - back * 16)
+                                                    : b_tile + (BMAJ ? ((int64_t)gr * TKROWS - back * 8) * pitch_b : (int64_t)gr * kRow - back * 16));
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + ring_slot * kStageBytes + (Q < LDA ? 0 : kATileBytes) +
                                                             (uint32_t)(Q < LDA ? wave * RWA + RPI * Q : wave * RWB + RPI * (Q - LDA)) * kRow);
         uint32_t lane_off = voff[Q];  // (a captured array element cannot be an asm operand of a generic lambda)
-        if constexpr (kRagged) lane_off -= gr == nstages - 1 ? tail_cut : 0u;  // (a uniform choice; tail_cut is zero without a tail)
+        if constexpr (kRagged && !kBlocks64) lane_off -= gr == nstages - 1 ? tail_cut : 0u;  // (a uniform choice; tail_cut is zero without a tail)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(base), "s"(dst)
                      : "memory");
     };
@@ -477,11 +498,24 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     // nor the bits the swizzle looks at change)
     [[maybe_unused]] const uint32_t ta_byte = lds0 + (uint32_t)(tr_place(tr_row0) * TROW + ((wm0 / 16) ^ tr_fx) * GB + tr_in);
     [[maybe_unused]] const uint32_t tb_byte = lds0 + kATileBytes + (uint32_t)(tr_place(tr_row0) * TROW + ((wn0 / 16) ^ tr_fx) * GB + tr_in);
+    // Blocks of 64 operand rows: the address of a wave's first 16-row block's first read; block BLK XORs (BLK % 4) granules into
+    // it and lies BLK / 4 blocks of 64 rows further where the wave tile starts on whole blocks of 64 rows (of 32, if it is 32 rows
+    // long); in wave tiles of 96 and 48 rows every 16-row block has an address of its own.
+    constexpr bool kOwnA = (BM / 2) % 64 != 0, kOwnB = WN % 64 != 0 && WN != 32;
+    [[maybe_unused]] uint32_t ta_at[AMAJ == 2 && kOwnA ? MI : 1], tb_at[BMAJ == 2 && kOwnB ? NI : 1];
+    if constexpr (kBlocks64) {
+        auto at64 = [&](int g16) { return (uint32_t)((g16 >> 2) * 64 * TROW + tr_row0 * TROW + ((g16 & 3) ^ tr_fx) * GB + tr_in); };
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof ta_at / sizeof *ta_at); ++i) ta_at[i] = lds0 + at64(wm0 / 16 + i);
+#pragma unroll
+        for (int j = 0; j < (int)(sizeof tb_at / sizeof *tb_at); ++j) tb_at[j] = lds0 + kATileBytes + at64(wn0 / 16 + j);
+    }
     // the fragment of 16-row block BLK for the k-step whose stages start at byte offsets o0 (, o1)
     auto load_frag = [&](auto& f, uint32_t base, auto blk_c, uint32_t o0, uint32_t o1) __attribute__((always_inline)) {
         constexpr int OFF = 16 * kRow * decltype(blk_c)::value;
         if constexpr (std::is_same_v<std::remove_reference_t<decltype(f)>, W4TrFrag>) {
-            const uint32_t at = (base ^ (uint32_t)(decltype(blk_c)::value * GB)) + o0;  // (stage offsets are multiples of 64 KiB)
+            // (stage offsets are multiples of 64 KiB; blocks of 64 rows: `base` is the 16-row block's own address)
+            const uint32_t at = (kBlocks64 ? base : base ^ (uint32_t)(decltype(blk_c)::value * GB)) + o0;
             if constexpr (In::kBytes == 2) {
                 f.q0 = lds_read_tr8<0>(at);
                 f.q1 = lds_read_tr8<4 * TROW>(at);
@@ -513,6 +547,17 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
             f.hi = lds_read16<OFF>(base + o1);
         }
     };
+    // the address load_frag starts from for 16-row block i (j) of the wave tile
+    auto fa_base = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (AMAJ == 2) return kOwnA ? ta_at[kOwnA ? i : 0] : (ta_at[0] ^ (uint32_t)((i & 3) * GB)) + (uint32_t)((i >> 2) * 64 * TROW);
+        else return AMAJ ? ta_byte : fa_byte;
+    };
+    auto fb_base = [&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+        if constexpr (BMAJ == 2) return kOwnB ? tb_at[kOwnB ? j : 0] : (tb_at[0] ^ (uint32_t)((j & 3) * GB)) + (uint32_t)((j >> 2) * 64 * TROW);
+        else return BMAJ ? tb_byte : fb_byte;
+    };
 #define MOYE_BLK(N) std::integral_constant<int, (N)> {}
 
     // prologue: all stages of the ring requested, wait for the first k-step's
@@ -541,11 +586,11 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     else __builtin_amdgcn_s_waitcnt(0x0F70);
     MOYE_BARRIER()
     static_for<MI>([&](auto ic) __attribute__((always_inline)) {
-        load_frag(fa[decltype(ic)::value], AMAJ ? ta_byte : fa_byte, ic, 0, kStageBytes);
+        load_frag(fa[decltype(ic)::value], fa_base(ic), ic, 0, kStageBytes);
         if ((decltype(ic)::value + 1) % (12 / RPA < 4 ? 12 / RPA : 4) == 0) __builtin_amdgcn_s_waitcnt(0xC07F);  // at most 15 reads in flight
     });
     static_for<NI>([&](auto jc) __attribute__((always_inline)) {
-        load_frag(fb[decltype(jc)::value], BMAJ ? tb_byte : fb_byte, jc, 0, kStageBytes);
+        load_frag(fb[decltype(jc)::value], fb_base(jc), jc, 0, kStageBytes);
         if ((decltype(jc)::value + 1) % (12 / RPB < 4 ? 12 / RPB : 4) == 0) __builtin_amdgcn_s_waitcnt(0xC07F);
     });
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -579,11 +624,17 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
             // are pieces kq and kq + 4 of its row).  In a block of its own, after every fragment read has returned.
             if (tail_pieces) {
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                const bool cut_lo = kq >= tail_pieces, cut_hi = kq + 4 >= tail_pieces;
+                const bool cut_lo = kBlocks64 ? kq < tail_back : kq >= tail_pieces, cut_hi = kBlocks64 ? kq + 4 < tail_back : kq + 4 >= tail_pieces;
                 auto cut = [&](auto& f) __attribute__((always_inline)) {
-                    // (only the two-piece fragments of the whole-line forms exist in ragged instances; the test keeps
+                    // (only two-piece fragments and transposed 16-bit ones exist in ragged instances; the tests keep
                     // the other instantiations of this lambda well-formed)
-                    if constexpr (std::is_class_v<std::remove_reference_t<decltype(f)>>) {
+                    if constexpr (std::is_same_v<std::remove_reference_t<decltype(f)>, W4TrFrag>) {
+                        const u32x2 zero = {0u, 0u};
+                        f.q0 = cut_lo ? zero : f.q0;
+                        f.q1 = cut_lo ? zero : f.q1;
+                        f.q2 = cut_hi ? zero : f.q2;
+                        f.q3 = cut_hi ? zero : f.q3;
+                    } else if constexpr (std::is_same_v<std::remove_reference_t<decltype(f)>, frag> && std::is_class_v<frag>) {
                         const u32x4 zero = {0u, 0u, 0u, 0u};
                         f.lo = cut_lo ? zero : f.lo;
                         f.hi = cut_hi ? zero : f.hi;
@@ -668,11 +719,10 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
             }
             if (MORE) {
                 constexpr int B0 = (MI - 2) * NI;
-                const uint32_t fa_at = AMAJ ? ta_byte : fa_byte, fb_at = BMAJ ? tb_byte : fb_byte;
-                if constexpr (P >= A0 && P < A0 + H) load_frag(fa[i], fa_at, MOYE_BLK(i), o0, o1);  // the rows of the first phase: last use
-                if constexpr (P >= H * NI && P < B0 && (P + 1) % NI == 0) load_frag(fa[i], fa_at, MOYE_BLK(i), o0, o1);  // a whole row: its end
-                if constexpr (P >= NPOS - 2) load_frag(fa[i], fa_at, MOYE_BLK(i), o0, o1);          // the last two rows: last use
-                if constexpr (P >= B0 && ((P - B0) & 1)) load_frag(fb[(P - B0) / 2], fb_at, MOYE_BLK((P - B0) / 2), o0, o1);
+                if constexpr (P >= A0 && P < A0 + H) load_frag(fa[i], fa_base(MOYE_BLK(i)), MOYE_BLK(i), o0, o1);  // the rows of the first phase: last use
+                if constexpr (P >= H * NI && P < B0 && (P + 1) % NI == 0) load_frag(fa[i], fa_base(MOYE_BLK(i)), MOYE_BLK(i), o0, o1);  // a whole row: its end
+                if constexpr (P >= NPOS - 2) load_frag(fa[i], fa_base(MOYE_BLK(i)), MOYE_BLK(i), o0, o1);          // the last two rows: last use
+                if constexpr (P >= B0 && ((P - B0) & 1)) load_frag(fb[(P - B0) / 2], fb_base(MOYE_BLK((P - B0) / 2)), MOYE_BLK((P - B0) / 2), o0, o1);
             }
         });
         slot = slot_n;
@@ -755,11 +805,12 @@ static int32_t launch256_w4(const GemmArgs& a, GemmPlan& plan) {
     return MOYE_OK;
 }
 
-// The instances live in seven translation units (so that they compile side by side): gemm_mfma256w4.hip (the 256 x 256
+// The instances live in nine translation units (so that they compile side by side): gemm_mfma256w4.hip (the 256 x 256
 // tile with K-major operands), gemm_mfma256w4_majors.hip (operands that keep their M- / N-major form),
 // gemm_mfma256w4_ops.hip (an element-wise operation in the epilogue), gemm_mfma256w4_persist.hip (one workgroup per CU
 // that walks over the tiles), gemm_mfma128w4.hip (the 128 x 128 tile), gemm_mfma128w4_majors.hip (the 128 x 128 tile with
-// M- / N-major operands), gemm_mfma_w4_tiles.hip (128 x 64 to 128 x 256 tiles in deeper rings).
+// M- / N-major operands), gemm_mfma_w4_tiles.hip (128 x 64 to 128 x 256 tiles in deeper rings), gemm_mfma_w4_majors_f16.hip and
+// ..._bf16.hip (guarded tiles with M- / N-major operands).
 int32_t launch256_w4_majors_dispatch(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan);
 int32_t launch256_w4_ops_dispatch(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan);
 int32_t launch128_w4_majors_dispatch(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan);

@@ -110,6 +110,13 @@ struct FormPrice {
     int tm, tn, slots, waves_k;
     double start, more, each, filled;
 };
+inline constexpr FormPrice kFormPrices16[] = {
+    {GemmForm::kOther, 256, 256, 1, 1, 7.6, 8.4, 1.09, 0.385},       {GemmForm::kOther, 128, 128, 2, 1, 4.73, 3.13, 0.544, 0.502},
+    {GemmForm::kBlock32x32, 32, 32, 2, 4, 3.40, 0.75, 0.19, 0.64},   {GemmForm::kBlock64x32, 64, 32, 1, 4, 3.63, 1.63, 0.47, 0.23},
+    {GemmForm::kBlock64x64, 64, 64, 1, 4, 4.24, 2.73, 0.77, 0.12},
+    {GemmForm::kTile128x64, 128, 64, 1, 1, 4.30, 2.91, 0.277, 0.063}, {GemmForm::kTile128x128, 128, 128, 1, 1, 4.33, 2.93, 0.385, 0.152},
+    {GemmForm::kTile128x192, 128, 192, 1, 1, 5.61, 4.91, 0.464, 0.235}, {GemmForm::kTile192x128, 192, 128, 1, 1, 5.11, 4.30, 0.511, 0.168},
+    {GemmForm::kTile128x256, 128, 256, 1, 1, 6.03, 4.83, 0.585, 0.269}};
 inline double gemm_form_us(const FormPrice& f, int64_t M, int64_t N, int64_t k_bytes, int cus) {
     const int64_t wgs = ((M + f.tm - 1) / f.tm) * ((N + f.tn - 1) / f.tn), per = (int64_t)cus * f.slots, full = wgs / per, rest = wgs % per;
     const int64_t lines = (k_bytes + 127) / 128, kt = (lines + f.waves_k - 1) / f.waves_k;
@@ -119,13 +126,6 @@ inline double gemm_form_us(const FormPrice& f, int64_t M, int64_t N, int64_t k_b
 // `part`: what is left of a larger problem, for which the blocks are not looked at (a round of tiles wide or long, it has too many
 // elements for them).  The cheapest form of the table, or kOther where one of the other two, or what `limit_us` stands for, is no dearer.
 inline GemmForm gemm_form_choose(int64_t M, int64_t N, int64_t k_bytes, int elem_bytes, int cus, double limit_us, double* us, bool part = false) {
-    static const FormPrice bits16[] = {
-        {GemmForm::kOther, 256, 256, 1, 1, 7.6, 8.4, 1.09, 0.385},       {GemmForm::kOther, 128, 128, 2, 1, 4.73, 3.13, 0.544, 0.502},
-        {GemmForm::kBlock32x32, 32, 32, 2, 4, 3.40, 0.75, 0.19, 0.64},   {GemmForm::kBlock64x32, 64, 32, 1, 4, 3.63, 1.63, 0.47, 0.23},
-        {GemmForm::kBlock64x64, 64, 64, 1, 4, 4.24, 2.73, 0.77, 0.12},
-        {GemmForm::kTile128x64, 128, 64, 1, 1, 4.30, 2.91, 0.277, 0.063}, {GemmForm::kTile128x128, 128, 128, 1, 1, 4.33, 2.93, 0.385, 0.152},
-        {GemmForm::kTile128x192, 128, 192, 1, 1, 5.61, 4.91, 0.464, 0.235}, {GemmForm::kTile192x128, 192, 128, 1, 1, 5.11, 4.30, 0.511, 0.168},
-        {GemmForm::kTile128x256, 128, 256, 1, 1, 6.03, 4.83, 0.585, 0.269}};
     static const FormPrice bits8[] = {
         {GemmForm::kOther, 256, 256, 1, 1, 7.7, 6.5, 1.04, 0.5},         {GemmForm::kOther, 128, 128, 2, 1, 4.76, 2.76, 0.514, 0.619},
         {GemmForm::kBlock32x32, 32, 32, 2, 4, 3.32, 0.79, 0.23, 0.67},   {GemmForm::kBlock64x32, 64, 32, 1, 4, 3.49, 1.61, 0.51, 0.38},
@@ -150,10 +150,43 @@ inline GemmForm gemm_form_choose(int64_t M, int64_t N, int64_t k_bytes, int elem
             if (t < *us) { *us = t; best = f[i].form; }
         }
     };
-    if (elem_bytes == 2) look(bits16, sizeof bits16 / sizeof *bits16);
+    if (elem_bytes == 2) look(kFormPrices16, sizeof kFormPrices16 / sizeof *kFormPrices16);
     else if (elem_bytes == 1) look(bits8, sizeof bits8 / sizeof *bits8);
     else look(bits32, sizeof bits32 / sizeof *bits32);
     return best;
+}
+
+// 16-bit operands that are not K-major on tiles that read them as they lie, in one launch: the cheapest of the tiles in deep rings and of
+// 256 x 256 ones (guarded or whole, `two_stages`: 128 x 128 ones in two stages too, which take whole tiles only; `tile256`: 256 x 256 ones
+// where there are no more of them than CUs).  Prices of K-major operands, which the transposing reads miss by little: bf16, operands not
+// cached, us K-major / B N-major / A M-major / both: 2048 x 4096 x 4096 on 128 x 256 tiles 57.5 / 59.4 / 60.0 / 62.4, 1000 x 6144 x 4096 on
+// 128 x 192 49.6 / 53.2 / 55.5 / 54.8, 1536 x 3072 x 4096 on 192 x 128 45.7 / 45.2 / - / 45.7.
+inline const FormPrice* gemm_majors_form(int64_t M, int64_t N, int64_t k_bytes, int cus, bool tile256, bool two_stages, double* us) {
+    const FormPrice* best = nullptr;
+    *us = 1e30;
+    for (const FormPrice& f : kFormPrices16) {
+        if (f.waves_k > 1 || f.form == GemmForm::kTile128x64) continue;
+        if (f.form == GemmForm::kOther && (f.tm == 256 ? !tile256 || ((M + 255) / 256) * ((N + 255) / 256) > cus : !two_stages)) continue;
+        // (whole tiles in two stages run unguarded: they keep what is a tenth dearer)
+        const double t = (f.form == GemmForm::kOther && f.tm == 128 ? 0.9 : 1.0) * gemm_form_us(f, M, N, k_bytes, cus);
+        if (t < *us) { *us = t; best = &f; }
+    }
+    return best;
+}
+// Are K-major copies (`copied` elements of operands in all, one launch for each operand) and the cheapest K-major form the better plan?  The
+// blocks, which divide K among four waves, have no form that reads operands otherwise: few elements (bf16 264 x 1024 x 1088, B N-major:
+// 10.3 us with a copy and blocks, tiles 10.6 at 256 x 1024 x 1024).  Beyond that copies are 5 us and twice the operands' bytes: 1000 x 6144 x
+// 4096 69.2 with a copy of B, 53.2 as it lies, both operands 76.8 / 54.8; 1088 x 1024 x 264 both 15.8 / 8.3.  Two kinds of call keep their
+// copies without a look at prices, because callers size buffers for them by the query and get the launches they sized them for: fewer than
+// 8 tiles of 128 x 128 (200 x 136 x 504 12.7 us, eight tiles as they lie 9.1) and more than 16384 rows with a short K (28000 x 1208 x 520 81
+// and 62).
+inline bool gemm_majors_copies_pay(int64_t M, int64_t N, int64_t k_bytes, int64_t copied, int launches, int cus) {
+    if (((M + 127) / 128) * ((N + 127) / 128) * 32 < cus) return true;
+    if ((M > 16384 || N > 16384) && k_bytes < 2048) return true;
+    double native, kmajor;
+    gemm_majors_form(M, N, k_bytes, cus, true, false, &native);
+    gemm_form_choose(M, N, k_bytes, 2, cus, 1e30, &kmajor);
+    return kmajor + 2.5 * launches + 4.0 * (double)copied / 5.0e6 < native;
 }
 
 // Everything left to the library (tile, waves, K ranges): the cheapest of 64 x 64 / 128 x 128 tiles with 1 .. max_split K

@@ -121,6 +121,14 @@ int32_t gemm_mfma_tn_256_w4_dispatch(int32_t in_dt, int32_t out_dt, GemmArgs a, 
 int32_t gemm_mfma_tn_128_dispatch(int32_t in_dt, int32_t out_dt, GemmArgs a, GemmPlan& plan);
 int32_t gemm_mfma_blocks_dispatch(int32_t in_dt, int32_t out_dt, GemmForm form, const GemmArgs& a, GemmPlan& plan);
 int32_t gemm_mfma_w4_tiles_dispatch(int32_t in_dt, int32_t out_dt, GemmForm form, GemmArgs a, GemmPlan& plan);
+int32_t gemm_mfma_w4_majors_f16(int32_t out_dt, GemmForm form, const GemmArgs& a, GemmPlan& plan);
+int32_t gemm_mfma_w4_majors_bf16(int32_t out_dt, GemmForm form, const GemmArgs& a, GemmPlan& plan);
+// Does a call with M- / N-major operands and its tile left to the library run on the guarded tiles that take them (gemm_mfma_w4_majors.hpp)
+// as far as everything but the operands' own pointers, pitches and extents goes?
+inline bool majors_take_any_tile(int32_t in_dt, int32_t out_dt, int bk_elems, int waves, int stages, const GemmArgs& a) {
+    return (in_dt == MOYE_F16 || in_dt == MOYE_BF16) && (out_dt == in_dt || out_dt == MOYE_F32) && bk_elems == 0 && waves <= 1 && stages == 0 && a.split <= 1 &&
+           a.ep_op == MOYE_MAP_IDENTITY && !(a.flags & (MOYE_GEMM_PINGPONG | MOYE_GEMM_WAVE4 | kGemmAtom32));
+}
 int32_t gemm_mfma_skinny_dispatch(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan);
 // The short-M kernel stages whole 128-byte lines of K through LDS, four waves with a K range each, when K is this many
 // bytes or a multiple of it (else every lane loads its own 16-byte pieces).
