@@ -153,14 +153,14 @@ static size_t kmajor_bytes(const Mat& m, bool lines) { return (size_t)(m.rows * 
 static int skinny_lines_split(int64_t M, int64_t N, int64_t k_bytes, int cus) {
     if ((N + 31) / 32 >= cus) return 1;  // 32 rows of B per workgroup and every CU has one
     double t1;
-    gemm_short_m_ntw(M, N, k_bytes, cus, 1, &t1);
+    gemm_short_m_rows(M, N, k_bytes, cus, 1, &t1);
     double t[9];
     double best = t1;
     const int max_split = M > 32 ? 2 : 8;
     for (int sp = 2; sp <= max_split; ++sp) {
         t[sp] = 1e30;
         if (k_bytes % ((int64_t)sp * kSkinnyLineBytes) || k_bytes / sp < 2048) continue;
-        gemm_short_m_ntw(M, N, k_bytes, cus, sp, &t[sp]);
+        gemm_short_m_rows(M, N, k_bytes, cus, sp, &t[sp]);
         best = std::min(best, t[sp]);
     }
     if (best > 0.9 * t1) return 1;

@@ -528,7 +528,7 @@ int32_t gemm_mfma_tn_dispatch(int32_t in_dt, int32_t out_dt, int bm, int bn, int
                 double us;
                 on64 = false;
                 if (gemm_short_m(m, n, k_bytes_all, eb == 4, cus)) {
-                    gemm_short_m_ntw(m, n, k_bytes_all, cus, 1, &us);
+                    gemm_short_m_rows(m, n, k_bytes_all, cus, 1, &us);
                     return us;
                 }
                 const TileChoice t = gemm_plan(m, n, k_bytes_all, eb == 4, aligned && m % 64 == 0 && n % 64 == 0 && !k_tail, 16, cus, 1);

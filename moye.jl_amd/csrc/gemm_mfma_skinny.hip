@@ -37,7 +37,9 @@ __device__ __forceinline__ void short_m_body(GemmArgs& p) {
     extern __shared__ u32x4 smem[];
     split_of_block(p);
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r16 = lane % 16, kq = lane / 16;
-    int n0 = blockIdx.x * 16 * NTW, walk = blockIdx.x / (unsigned)p.xcds;
+    // rows of B of a workgroup: whole blocks of 16, or eight less (p.tiles_n)
+    const int rows = kBlocks ? 16 * NTW : p.tiles_n;
+    int n0 = blockIdx.x * rows, walk = blockIdx.x / (unsigned)p.xcds;
     if constexpr (kBlocks) {
         // several blocks of 16 MT rows of A: each XCD takes one run of the blocks, those that share rows of B one after the other
         const int q = blockIdx.x / (unsigned)p.xcds, t = blockIdx.x % (unsigned)p.xcds * (gridDim.x / (unsigned)p.xcds) + q, tm = t % p.tiles_m;
@@ -88,6 +90,8 @@ __device__ __forceinline__ void short_m_body(GemmArgs& p) {
     // read where A ends before them (what a buffer holds there reaches only rows of D that are not stored): bf16
     // 64 x 14336 x 4096 25.9 us before, 24.9 with the order, 50 rows 24.4 / 23.6
     const bool full_a = kBlocks || p.M > 16 * MT - 8;
+    // (the same of B's last block where the workgroup has half of it)
+    const bool full_b = rows == 16 * NTW;
 #define MOYE_WAIT_VM(N) __builtin_amdgcn_s_waitcnt(((N) & 0xF) | (((N) >> 4) << 14) | 0x0F70);
 #define MOYE_STAGE_LOAD(T)                                                                                      \
     {                                                                                                           \
@@ -96,8 +100,9 @@ __device__ __forceinline__ void short_m_body(GemmArgs& p) {
         _Pragma("unroll") for (int j = 2 * NTW; j < LD - 1; ++j)                                                \
             __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + off_), (lptr_t)(dst_ + 64 * j), 16, 0, 0);       \
         if (full_a) __builtin_amdgcn_global_load_lds((gptr_t)(src[LD - 1] + off_), (lptr_t)(dst_ + 64 * (LD - 1)), 16, 0, 0); \
-        _Pragma("unroll") for (int j = 0; j < 2 * NTW; ++j)                                                     \
+        _Pragma("unroll") for (int j = 0; j < 2 * NTW - 1; ++j)                                                 \
             __builtin_amdgcn_global_load_lds((gptr_t)(src[j] + off_), (lptr_t)(dst_ + 64 * j), 16, 0, kAuxB);   \
+        if (full_b) __builtin_amdgcn_global_load_lds((gptr_t)(src[2 * NTW - 1] + off_), (lptr_t)(dst_ + 64 * (2 * NTW - 1)), 16, 0, kAuxB); \
     }
 #pragma unroll
     for (int t = 0; t < kStages - 1; ++t)
@@ -106,7 +111,9 @@ __device__ __forceinline__ void short_m_body(GemmArgs& p) {
         if (t + kStages - 1 < len) {
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragment reads of trip t - 1 are out of the buffer refilled now
             MOYE_STAGE_LOAD(t + kStages - 1)
-            if (full_a) MOYE_WAIT_VM((kStages - 1) * LD) else MOYE_WAIT_VM((kStages - 1) * (LD - 1))
+            if (full_a && full_b) MOYE_WAIT_VM((kStages - 1) * LD)
+            else if (full_a || full_b) MOYE_WAIT_VM((kStages - 1) * (LD - 1))
+            else MOYE_WAIT_VM((kStages - 1) * (LD - 2))
         } else {
             // the tail: fewer stages are behind this one; waiting for all of them costs little over so few trips
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -173,7 +180,7 @@ __device__ __forceinline__ void short_m_body(GemmArgs& p) {
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) v += part[w * MT * NTW * 64 + unit];
         const int m = 16 * (it / NTW) + l % 16, n = n0 + 16 * (it % NTW) + 4 * (l / 16);
-        if (m >= p.M) continue;
+        if (m >= p.M || n - n0 >= rows) continue;
         const int64_t sn = p.ldd_n ? p.ldd_n : 1;  // D may have its unit stride along m
         OutT* d = static_cast<OutT*>(p.D) + (int64_t)m * p.ldd + (int64_t)n * sn;
         if (sn == 1 && n + 3 < p.N && !p.C && p.ep_op == MOYE_MAP_IDENTITY && reinterpret_cast<uintptr_t>(d) % (4 * sizeof(OutT)) == 0) {
@@ -215,11 +222,12 @@ __global__ __launch_bounds__(256) void gemm_mfma_blocks(GemmArgs p) {
 constexpr int kSkinnyLdsWaves = 4;
 static_assert(kSkinnyLineBytes == 128, "the host decides about K ranges by this");
 template <typename In, typename Out, int MT, int W, int NTW, int S, int AUX>
-static int32_t launch_skinny_lds_v(const GemmArgs& a, GemmPlan& plan) {
+static int32_t launch_skinny_lds_v(GemmArgs a, int rows, GemmPlan& plan) {
+    a.tiles_n = rows;
     constexpr int kLds = W * S * (16 * NTW + 16 * MT) * 128;
     static LdsCap cap;
-    plan.add_kernel(gemm_mfma_skinny_lds<In, Out, MT, NTW, W, S, AUX>, a, (unsigned)((a.N + 16 * NTW - 1) / (16 * NTW)), (unsigned)(a.split > 1 ? a.split : 1),
-                    W * 64, kLds, &cap, 0, 16 * NTW, 128, In::kDt, Out::kDt, "gemm_mfma_skinny_lds<%s,%s,mt=%d,ntw=%d,waves=%d,stages=%d>", In::kName, Out::kName,
+    plan.add_kernel(gemm_mfma_skinny_lds<In, Out, MT, NTW, W, S, AUX>, a, (unsigned)((a.N + rows - 1) / rows), (unsigned)(a.split > 1 ? a.split : 1),
+                    W * 64, kLds, &cap, 0, rows, 128, In::kDt, Out::kDt, "gemm_mfma_skinny_lds<%s,%s,mt=%d,ntw=%d,waves=%d,stages=%d>", In::kName, Out::kName,
                     MT, NTW, W, S);
     return MOYE_OK;
 }
@@ -231,41 +239,41 @@ static int32_t launch_skinny_lds(const GemmArgs& a, GemmPlan& plan) {
     // B without the non-temporal hint 23.6.  As with the transposes, less in flight is faster on this part, down to what
     // covers the latency.  32 rows per workgroup once that gives every CU one (bf16, K = 8192: N = 16384 40.1 us against
     // 45.3 with 16 rows; N = 4096 17.9 against 13.5).
-    // (which of them: gemm_short_m_ntw, gemm_plan.hpp -- the rounds the workgroups of a launch need on the CUs decide)
+    // (which of them: gemm_short_m_rows, gemm_plan.hpp -- the rounds the workgroups of a launch need on the CUs decide)
     const int ranges = a.split > 1 ? a.split : 1;
-    const int ntw = gemm_short_m_ntw(a.M, a.N, (int64_t)a.K * In::kBytes * ranges, plan.shape.cus, ranges);
+    const int rows = gemm_short_m_rows(a.M, a.N, (int64_t)a.K * In::kBytes * ranges, plan.shape.cus, ranges), ntw = (rows + 15) / 16;
     // (64 rows, and 48 against more than 32 rows of A: two buffers instead of three, for the LDS or because a third gave
     // nothing: bf16 32 x 14336 x 4096 20.9 us with either.  48 rows: the one round of 8193 <= N <= 12288 and the second up
     // to 24576)
     if (ntw == 4) {
         switch ((a.M + 15) / 16) {
-            case 1: return launch_skinny_lds_v<In, Out, 1, W, 4, 2, 2>(a, plan);
-            case 2: return launch_skinny_lds_v<In, Out, 2, W, 4, 2, 2>(a, plan);
-            case 3: return launch_skinny_lds_v<In, Out, 3, W, 4, 2, 2>(a, plan);
-            default: return launch_skinny_lds_v<In, Out, 4, W, 4, 2, 2>(a, plan);
+            case 1: return launch_skinny_lds_v<In, Out, 1, W, 4, 2, 2>(a, rows, plan);
+            case 2: return launch_skinny_lds_v<In, Out, 2, W, 4, 2, 2>(a, rows, plan);
+            case 3: return launch_skinny_lds_v<In, Out, 3, W, 4, 2, 2>(a, rows, plan);
+            default: return launch_skinny_lds_v<In, Out, 4, W, 4, 2, 2>(a, rows, plan);
         }
     }
     if (ntw == 3) {
         switch ((a.M + 15) / 16) {
-            case 1: return launch_skinny_lds_v<In, Out, 1, W, 3, 3, 2>(a, plan);
-            case 2: return launch_skinny_lds_v<In, Out, 2, W, 3, 3, 2>(a, plan);
-            case 3: return launch_skinny_lds_v<In, Out, 3, W, 3, 2, 2>(a, plan);
-            default: return launch_skinny_lds_v<In, Out, 4, W, 3, 2, 2>(a, plan);
+            case 1: return launch_skinny_lds_v<In, Out, 1, W, 3, 3, 2>(a, rows, plan);
+            case 2: return launch_skinny_lds_v<In, Out, 2, W, 3, 3, 2>(a, rows, plan);
+            case 3: return launch_skinny_lds_v<In, Out, 3, W, 3, 2, 2>(a, rows, plan);
+            default: return launch_skinny_lds_v<In, Out, 4, W, 3, 2, 2>(a, rows, plan);
         }
     }
     if (ntw == 2) {
         switch ((a.M + 15) / 16) {
-            case 1: return launch_skinny_lds_v<In, Out, 1, W, 2, 3, 2>(a, plan);
-            case 2: return launch_skinny_lds_v<In, Out, 2, W, 2, 3, 2>(a, plan);
-            case 3: return launch_skinny_lds_v<In, Out, 3, W, 2, 3, 2>(a, plan);
-            default: return launch_skinny_lds_v<In, Out, 4, W, 2, 3, 2>(a, plan);
+            case 1: return launch_skinny_lds_v<In, Out, 1, W, 2, 3, 2>(a, rows, plan);
+            case 2: return launch_skinny_lds_v<In, Out, 2, W, 2, 3, 2>(a, rows, plan);
+            case 3: return launch_skinny_lds_v<In, Out, 3, W, 2, 3, 2>(a, rows, plan);
+            default: return launch_skinny_lds_v<In, Out, 4, W, 2, 3, 2>(a, rows, plan);
         }
     }
     switch ((a.M + 15) / 16) {
-        case 1: return launch_skinny_lds_v<In, Out, 1, W, 1, 3, 2>(a, plan);
-        case 2: return launch_skinny_lds_v<In, Out, 2, W, 1, 3, 2>(a, plan);
-        case 3: return launch_skinny_lds_v<In, Out, 3, W, 1, 3, 2>(a, plan);
-        default: return launch_skinny_lds_v<In, Out, 4, W, 1, 3, 2>(a, plan);
+        case 1: return launch_skinny_lds_v<In, Out, 1, W, 1, 3, 2>(a, rows, plan);
+        case 2: return launch_skinny_lds_v<In, Out, 2, W, 1, 3, 2>(a, rows, plan);
+        case 3: return launch_skinny_lds_v<In, Out, 3, W, 1, 3, 2>(a, rows, plan);
+        default: return launch_skinny_lds_v<In, Out, 4, W, 1, 3, 2>(a, rows, plan);
     }
 }
 

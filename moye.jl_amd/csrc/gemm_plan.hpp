@@ -251,28 +251,49 @@ inline bool gemm_short_m(int64_t M, int64_t N, int64_t k_bytes, bool f32_in, int
 // 64 x 4096 x 14336 42.0 unsplit on 256 workgroups of 16 rows, 47.0 in two K ranges on 512.  In microseconds:
 // 4.5 (two launches of a split: 7.5, and never under 10.7) + the longer of all bytes at 6 TB/s and rounds x a workgroup's
 // bytes at its rate.
-inline double gemm_short_m_us(int64_t M, int64_t N, int64_t k_bytes, int cus, int ntw, int split) {
+inline double gemm_short_m_us(int64_t M, int64_t N, int64_t k_bytes, int cus, int rows, int split) {
     const int mt = (int)((M + 15) / 16);
-    const int64_t wgs = (N + 16 * ntw - 1) / (16 * ntw) * split, rounds = (wgs + cus - 1) / cus;
-    const double wg_us = (double)(16 * ntw + 16 * mt) * ((double)k_bytes / split) / (ntw > 2 ? 56.0e3 : 64.0e3);
+    const int64_t wgs = (N + rows - 1) / rows * split, rounds = (wgs + cus - 1) / cus;
+    const double wg_us = (double)(rows + 16 * mt) * ((double)k_bytes / split) / (rows > 32 ? 56.0e3 : 64.0e3);
     const double floor_us = (double)(N + M) * (double)k_bytes / 6.0e6;
     const double t = floor_us > (double)rounds * wg_us ? floor_us : (double)rounds * wg_us;
     if (split > 1) return 7.5 + t > 10.7 ? 7.5 + t : 10.7;
     return 4.5 + t;
 }
-// 16-row blocks of B per workgroup for a launch in `split` K ranges: the fewest rows of A and B that a CU reads in all its
+// Rows of B per workgroup for a launch in `split` K ranges: the fewest rows of A and B that a CU reads in all its
 // rounds, more rows at once on a tie.  (A is read in groups of eight rows.  Up to 16 rows of A two workgroups of 32 rows of B
 // share a CU, which is worth 15 % from a second round on: 5 x 14336 x 8192 36.4 us against 38.5 with 64 rows; from a fifth
-// on 22 %: 16 x 40960 x 4096 49.7 / 52.9, fp8 15 x 34304 x 4096 24.6 against 26.4 with 48.)
-inline int gemm_short_m_ntw(int64_t M, int64_t N, int64_t k_bytes, int cus, int split, double* us = nullptr) {
-    int best = 1;
-    double best_rows = 1e30;
-    for (int ntw : {1, 2, 3, 4}) {
-        const int64_t wgs = (N + 16 * ntw - 1) / (16 * ntw) * split, rounds = (wgs + cus - 1) / cus;
-        const double rows = (double)(rounds * (16 * ntw + (M + 7) / 8 * 8)) * (ntw > 2 || M > 16 || rounds == 1 ? 1.0 : rounds < 5 ? 0.85 : 0.78);
-        if (rows <= best_rows) { best_rows = rows; best = ntw; }
+// on 22 %: 16 x 40960 x 4096 49.7 / 52.9, fp8 15 x 34304 x 4096 24.6 against 26.4 with 48.)  Whole MFMA blocks of 16 rows, or one of
+// them half empty, its last eight rows neither read nor stored, where that leaves a CU 6 % less to read: bf16, not cached, us whole /
+// half: 50 x 14336 x 4096 23.5 (64 rows) / 22.7 (56), 16 x 6144 x 8192 19.3 (32) / 17.2 (24), 40 x 10240 x 8192 32.6 (48) / 30.2 (40), 50 x 2048 x 4096
+// 11.8 (16) / 10.5 (8), 16 x 20480 x 4096 29.1 / 27.7, 64 x 28672 x 8192 92.8 / 88.3.  Not with a few rows of A and long rows, which run at
+// the memory's rate as they are (1 x 6144 x 16384 30.6 / 33.7, 1 x 5120 x 16384 28.2 / 28.9; but 1 x 5000 x 12288 22.1 / 20.1), nor
+// 40 and 56 rows with rows under 4 KiB, in several rounds up to that (1 x 9600 x 1024 5.7 / 5.9, 40 x 28672 x 2048 24.6 / 25.0).  Eight rows in
+// unsplit launches only.  `us` is the price with whole blocks, which the model was fitted to: on it K ranges are decided (16 x 2048 x 16384
+// 22.2 unsplit with 16 rows, 19.9 with 8, 17.1 in two ranges).
+inline int gemm_short_m_rows(int64_t M, int64_t N, int64_t k_bytes, int cus, int split, double* us = nullptr) {
+    // (the host's time for a call of a few microseconds counts: no division where one round holds the workgroups)
+    const int m8 = (int)((M + 7) / 8 * 8);
+    auto rounds_of = [&](int r) {
+        const int64_t wgs = (int64_t)(((uint32_t)N + (uint32_t)r - 1) / (uint32_t)r) * split;
+        return wgs <= cus ? 1 : (wgs + cus - 1) / cus;
+    };
+    auto cost = [&](int r, int64_t rounds) { return (double)(rounds * (r + m8)) * (r > 32 || M > 16 || rounds == 1 ? 1.0 : rounds < 5 ? 0.85 : 0.78); };
+    int best = 16;
+    double least = cost(16, rounds_of(16));
+    for (int r : {32, 48, 64}) {
+        const double c = cost(r, rounds_of(r));
+        if (c <= least) { best = r; least = c; }
     }
     if (us) *us = gemm_short_m_us(M, N, k_bytes, cus, best, split);
+    least *= 0.94;
+    for (int r : {8, 24, 40, 56}) {
+        if (r == 8 ? split > 1 : M <= 8 && k_bytes >= 28 * 1024) continue;
+        const int64_t rounds = rounds_of(r);
+        if (r >= 40 && k_bytes < (rounds > 1 ? 4097 : 4096)) continue;
+        const double c = cost(r, rounds);
+        if (c <= least) { best = r; least = c; }
+    }
     return best;
 }
 
