@@ -1354,3 +1354,25 @@ def test_transposes_with_one_ragged_pitch(mh, pair, ni, nj):
     torch.cuda.synchronize()
     want = src.to(ddt).view(bits[ddt.itemsize]).view(nj, ni).t()
     assert torch.equal(dst[:ni * nj].view(ni, nj), want) and bool((dst[ni * nj:] == 0x5A).all()), (pair, ni, nj)
+
+
+@pytest.mark.parametrize("n", [8 << 20, (8 << 20) + 1, (8 << 20) + 7])
+@pytest.mark.parametrize("start", [0, 1])
+def test_results_on_either_side_of_what_the_l2s_hold(mh, n, start):
+    """Dense map! and axpby! whose result is 32 MiB (ordinary stores) and one element or more beyond it (hinted ones), from an aligned
+    and an odd address: in place, with an array, with a vector that repeats, with a scalar."""
+    from moye_hip.torch_interop import tensor_of
+    g = torch.Generator(device="cuda").manual_seed(n + start)
+    x, y, v = (torch.randn(k + 1, generator=g, device="cuda")[start:start + k] for k in (n, n, 1024))
+    d = torch.full((n + 2,), 77.0, device="cuda")
+    td = tensor_of(d[1:-1])
+    for got, want in ((lambda: mh.map_("add", td, tensor_of(x), tensor_of(y)), x + y), (lambda: mh.map_("max", td, td, scalar=0.25), (x + y).clamp_min(0.25)),
+                      (lambda: mh.axpby_(0.5, tensor_of(x), 2.0, td), 0.5 * x + 2.0 * (x + y).clamp_min(0.25)), (lambda: mh.axpby_(3.0, tensor_of(x), 0.0, td), 3.0 * x)):
+        got()
+        torch.cuda.synchronize()
+        assert torch.equal(d[1:-1], want) and float(d[0]) == float(d[-1]) == 77.0
+    if n % 1024 == 0:
+        columns = ((1024, n // 1024), (1, 1024))
+        mh.map_("add", tensor_of(d[1:-1], *columns), tensor_of(x, *columns), tensor_of(v))
+        torch.cuda.synchronize()
+        assert torch.equal(d[1:-1].view(-1, 1024), x.view(-1, 1024) + v)
