@@ -195,14 +195,19 @@ __device__ __forceinline__ void turn_block(const u32x4 (&v)[16 / DB], u32x4 (&o)
 // f16 16384^2 192 -> 187, 6000 x 4096 24.1 -> 19.3, 10001 x 7003 1042 -> 75; [4,2000,32,128] -> [4,32,128,2000] 937 -> 28.4;
 // NCHW -> NHWC 32 x 256 x 28 x 28 234 -> 7.5; bytes 16384^2 121 -> 103; 8-byte elements 8192^2 188 -> 180;
 // f32 -> bf16 5000 x 3000 32.1 -> 21.3, 8192^2 80.8 -> 72.2.
+// kSkew: destination rows whose pitch is no whole lines: a workgroup's part of a row starts and ends on the row's own 128-byte
+// boundaries, up to 127 bytes behind those of the tile, so that no line but a row's first and last is written by two
+// workgroups, and every store is aligned.  1: pitches and addresses of whole pieces, 2: any.  It reads eight pieces' worth of source rows more, which its neighbour reads as well (skew_of: where, and what it measured).
 // kKeep: bit 0: the source is read, bit 1: the destination is written through the caches in the ordinary way instead of with the
 // non-temporal hint (launch_shape decides).
-template <int kSrc, int kDst, int SB, int DB, int PI, int NB, int T, int kKeep>
+template <int kSrc, int kDst, int SB, int DB, int PI, int NB, int T, int kKeep, int kSkew>
 __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
     constexpr int ES = 16 / SB, Q = 16 / DB, NJ = T / PI, TI = PI * ES, JC = NJ * NB, TJ = JC * Q;
+    constexpr int JX = kSkew ? 8 : 0, JL = JC + JX;  // pieces of an LDS row
+    static_assert(!kSkew || (NJ >= JX && JC % 8 == 0), "the pieces more come from one more block of the first lanes, and are swizzled among themselves");
     const int sw = a.linear ? 0 : JC < 8 ? JC - 1 : 7;
     static_assert(T % JC == 0 && TI % (T / JC) == 0, "whole rows per pass");
-    extern __shared__ u32x4 tile[];  // ES rows that are never read (see below), then TI rows, of JC pieces
+    extern __shared__ u32x4 tile[];  // ES rows that are never read (see below), then TI rows, of JL pieces
     const char* src = a.src;
     char* dst = a.dst;
     {
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
     const int jc = threadIdx.x % JC, r0 = threadIdx.x / JC;
     const int iw = a.ni - ti * TI, jw = a.nj - tj * TJ;  // what is left of the two extents here
     // LDS rows are counted from ES on: a lane that was shifted back may write rows that belong to the tile before this one
-    auto slot = [&](int row, int piece) -> u32x4& { return tile[row * JC + (piece ^ ((row / ES) & sw))]; };
+    auto slot = [&](int row, int piece) -> u32x4& { return tile[row * JL + (piece ^ ((row / ES) & sw))]; };
     auto load = [](const char* p) -> u32x4 {
         if constexpr (kKeep & 1) return *reinterpret_cast<const u32x4_any*>(p);
         else return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
@@ -257,7 +262,39 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
         }
     };
     char* const d = dst + ((int64_t)(ti * TI + r0) * a.ldd + tj * TJ + Q * jc) * DB;
-    if (iw >= TI && jw >= TJ) {
+    auto put1 = [&](int row0, const u32x4 (&v)[Q]) {  // the block behind the tile's (kSkew)
+        u32x4 o[ES];
+        turn_block<kSrc, kDst, SB, DB>(v, o);
+#pragma unroll
+        for (int e = 0; e < ES; ++e) slot(row0 + e, JC + jr) = o[e];
+    };
+    // bytes from the tile's start in row p of this lane's pass to the row's next whole line (the lanes of a wave share a row)
+    static_assert(!kSkew || JC % 64 == 0, "a wave has one row");
+    auto shift = [&](int p) { return kSkew ? __builtin_amdgcn_readfirstlane((int)(-reinterpret_cast<uintptr_t>(d + (int64_t)(RPP * p) * a.ldd * DB - 16 * jc) & 127)) : 0; };
+    // 16 bytes of an LDS row that start `by` bytes behind this lane's piece
+    auto bytes_from = [&](int row, int by) -> u32x4 {
+        const u32x4 lo = slot(row, jc + by / 16);
+        const int sh = by % 16;
+        if (kSkew == 1 || sh == 0) return lo;
+        const u32x4 hi = slot(row, jc + by / 16 + 1);
+        auto five = [&](uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3, uint32_t x4) {
+            return u32x4{__builtin_amdgcn_alignbyte(x1, x0, sh & 3), __builtin_amdgcn_alignbyte(x2, x1, sh & 3), __builtin_amdgcn_alignbyte(x3, x2, sh & 3),
+                         __builtin_amdgcn_alignbyte(x4, x3, sh & 3)};
+        };
+        switch (sh >> 2) {
+            case 0: return five(lo[0], lo[1], lo[2], lo[3], hi[0]);
+            case 1: return five(lo[1], lo[2], lo[3], hi[0], hi[1]);
+            case 2: return five(lo[2], lo[3], hi[0], hi[1], hi[2]);
+            default: return five(lo[3], hi[0], hi[1], hi[2], hi[3]);
+        }
+    };
+    // what lies before the first whole line of a row, in its first tile
+    auto row_start = [&](int row, char* to, int sh) {
+        const int left = min(sh / DB, jw) - Q * jc;
+        if (left >= Q) store(slot(row, jc), to);
+        else if (left > 0) store_first<DB>(to, slot(row, jc), left);
+    };
+    if (iw >= TI && jw >= TJ + JX * Q) {
         const char* const s = src + ((int64_t)(tj * TJ + Q * jr) * a.lds + ti * TI + pi * ES) * SB;
         u32x4 v[NB][Q];
 #pragma unroll
@@ -265,11 +302,27 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
 #pragma unroll
             for (int q = 0; q < Q; ++q)
                 v[b][q] = load(s + (int64_t)(Q * NJ * b + q) * a.lds * SB);
+        if constexpr (kSkew) {
+            if (jr < JX) {
+                u32x4 x[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) x[q] = load(s + (int64_t)(TJ + q) * a.lds * SB);
+                put1(ES + pi * ES, x);
+            }
+        }
         put(ES + pi * ES, v);
         __syncthreads();
 #pragma unroll
-        for (int p = 0; p < TI / RPP; ++p)
-            store(slot(ES + r0 + RPP * p, jc), d + (int64_t)(RPP * p) * a.ldd * DB);
+        for (int p = 0; p < TI / RPP; ++p) {
+            const int sh = shift(p);
+            char* const to = d + (int64_t)(RPP * p) * a.ldd * DB;
+            if constexpr (kSkew) {
+                store(bytes_from(ES + r0 + RPP * p, sh), to + sh);
+                if (tj == 0) row_start(ES + r0 + RPP * p, to, sh);
+            } else {
+                store(slot(ES + r0 + RPP * p, jc), to);
+            }
+        }
         return;
     }
     if (pi * ES < iw) {
@@ -284,8 +337,28 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
                 v[b][q] = load(s + (int64_t)j * a.lds * SB);
             }
         put(ES + il, v);
+        if constexpr (kSkew) {
+            if (jr < JX) {
+                u32x4 x[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) x[q] = load(s + (int64_t)min(Q * (JC + jr) + q, jw - 1) * a.lds * SB);
+                put1(ES + il, x);
+            }
+        }
     }
     __syncthreads();
+    if constexpr (kSkew) {
+#pragma unroll 1
+        for (int p = 0; r0 + RPP * p < min(iw, TI); ++p) {
+            const int sh = shift(p), row = ES + r0 + RPP * p;
+            char* const to = d + (int64_t)(RPP * p) * a.ldd * DB;
+            const int left = jw - Q * jc - sh / DB;
+            if (left >= Q) store(bytes_from(row, sh), to + sh);
+            else if (left > 0) store_first<DB>(to + sh, bytes_from(row, sh), left);
+            if (tj == 0) row_start(row, to, sh);
+        }
+        return;
+    }
     const int left = jw - Q * jc;
     if (left >= Q) {
 #pragma unroll
@@ -298,12 +371,12 @@ __global__ __launch_bounds__(T) void transpose_blocks(TransposeArgs a) {
     }
 }
 
-template <int kSrc, int kDst, int SB, int DB, int PI, int NB, int T, int kKeep>
+template <int kSrc, int kDst, int SB, int DB, int PI, int NB, int T, int kKeep, int kSkew = 0>
 static int32_t launch_kept(TransposeArgs a, int lds_request, hipStream_t st) {
-    constexpr int ES = 16 / SB, Q = 16 / DB, NJ = T / PI, TI = PI * ES, TJ = NJ * NB * Q, kLds = (TI + ES) * TJ * DB;
+    constexpr int ES = 16 / SB, Q = 16 / DB, NJ = T / PI, TI = PI * ES, TJ = NJ * NB * Q, kLds = (TI + ES) * (TJ * DB + (kSkew ? 128 : 0));
     constexpr int kCap = 160 * 1024;  // all of a CU's LDS
     static_assert(kLds <= kCap, "the tile fits");
-    auto kern = transpose_blocks<kSrc, kDst, SB, DB, PI, NB, T, kKeep>;
+    auto kern = transpose_blocks<kSrc, kDst, SB, DB, PI, NB, T, kKeep, kSkew>;
     const int lds = std::max(kLds, lds_request);
     if (lds > 48 * 1024) {
         static LdsCap cap;
@@ -317,6 +390,33 @@ static int32_t launch_kept(TransposeArgs a, int lds_request, hipStream_t st) {
     kern<<<dim3((unsigned)tiles, gy, gz), T, lds, st>>>(a);
     MOYE_HIP_CHECK(hipGetLastError());
     return MOYE_OK;
+}
+
+// Which form of the destination's rows (kSkew), for tiles of 1 KiB of a row: 0 where their pitch is whole lines, or where the tiles more that the shift
+// costs are worth more than the lines.  us without / with, operands not cached: fp16 into rows of whole pieces from 4000 bytes on,
+// 4864 x 5992 28.0 / 23.1, 16000 x 16008 230 / 207, [1,3000,32,128] -> [1,32,128,3000] 10.7 / 10.1, but 12345 x 1400 18.1 / 19.3; f32 from 20 KiB and 48 MiB
+// on, 4860 x 5992 50.3 / 47.5, 16000 x 16008 446 / 405, but 13361 x 3728 76.6 / 78.4, 3004 x 2996 15.7 / 16.3; fp16 into any rows of one matrix
+// from 5888 elements on, 4861 x 5993 29.6 / 27.1, 16001 x 16011 254 / 216, 1033 x 14001 14.3 / 13.6, but 10001 x 4099 39.0 / 41.8, 4000 x 4499 20.8 / 21.8 and
+// in batches [4,2001,32,128] 31.7 / 33.2; f32 into any rows 115.3 / 119.1 (10001 x 7003); f32 -> bf16 18.5 / 18.5 (5000 x 3000).
+// Not 16-bit tiles, one to a CU, of which a second round has less than half a round's (1329 x 13256 18.2 / 18.8, 1691 x 11920 19.1 / 19.7).
+static int skew_of(const TransposeArgs& a, int db, bool dst_lines) {
+    constexpr int64_t Mi = 1 << 20;
+    const int64_t row = (int64_t)a.nj * db;
+    if (dst_lines || row < (db == 2 ? 4000 : 20480) || (db == 4 && row * a.ni * a.batch < 48 * Mi)) return 0;
+    const int64_t tiles = ((int64_t)a.ni + 127) / 128 * ((a.nj + 511) / 512) * a.batch, cus = 32 * a.xcds;
+    if (db == 2 && tiles > cus && 2 * tiles < 3 * cus) return 0;
+    int64_t all = reinterpret_cast<uintptr_t>(a.dst) | a.ldd * db;
+    for (int m = 0; m < a.modes; ++m) all |= a.d_stride[m] * db;
+    if (all % 16 == 0) return 1;
+    return db == 2 && a.batch == 1 && a.nj >= 5888 ? 2 : 0;
+}
+template <int kSrc, int kDst, int SB, int DB>
+static int32_t launch_skewed(const TransposeArgs& a, int skew, int keep, int lds_request, hipStream_t st) {
+    if constexpr (DB == 2) {
+        if (skew == 2)
+            return keep == 1 ? launch_kept<kSrc, kDst, SB, DB, 16, 2, 512, 1, 2>(a, lds_request, st) : launch_kept<kSrc, kDst, SB, DB, 16, 2, 512, 0, 2>(a, lds_request, st);
+    }
+    return keep == 1 ? launch_kept<kSrc, kDst, SB, DB, 16, 2, 512, 1, 1>(a, lds_request, st) : launch_kept<kSrc, kDst, SB, DB, 16, 2, 512, 0, 1>(a, lds_request, st);
 }
 
 template <int kSrc, int kDst, int SB, int DB, int PI, int NB, int T>
@@ -402,7 +502,9 @@ static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
             default: MOYE_TILE(8, 1, 64, 0);
         }
         if (!lines || (n <= 16 * Mi && !narrow)) switch (fit({{128, 512}, {128, 128}, {64, 64}})) {
-            case 0: MOYE_TILE(16, 2, 512, 0);
+            case 0:
+                if (const int skew = skew_of(a, DB, dst_lines)) return launch_skewed<kSrc, kDst, SB, DB>(a, skew, keep, 0, st);
+                MOYE_TILE(16, 2, 512, 0);
             case 1: MOYE_TILE(16, 1, 256, 0);
             default: MOYE_TILE(8, 1, 64, 0);
         }
@@ -422,7 +524,9 @@ static int32_t launch_shape(TransposeArgs a, hipStream_t st) {
         if (few) { if (fit({{32, 64}, {64, 64}}) == 0) MOYE_TILE(8, 1, 128, 0); else MOYE_TILE(16, 2, 128, 0); }
         if (medium) { if (fit({{128, 64}, {64, 64}}) == 0) MOYE_TILE(32, 2, 256, 0); else MOYE_TILE(16, 2, 128, 0); }
         if (!lines) switch (bytes >= 32 * Mi ? fit({{64, 256}, {128, 128}, {64, 64}}) : 3 + fit({{64, 128}, {64, 64}})) {
-            case 0: MOYE_TILE(16, 2, 512, kAlone);
+            case 0:
+                if (const int skew = skew_of(a, DB, dst_lines)) return launch_skewed<kSrc, kDst, SB, DB>(a, skew, keep, kAlone, st);
+                MOYE_TILE(16, 2, 512, kAlone);
             case 1: MOYE_TILE(32, 4, 256, 0);
             case 3: MOYE_TILE(16, 2, 256, 0);
             default: MOYE_TILE(16, 2, 128, 0);

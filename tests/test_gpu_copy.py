@@ -1376,3 +1376,29 @@ def test_results_on_either_side_of_what_the_l2s_hold(mh, n, start):
         mh.map_("add", tensor_of(d[1:-1], *columns), tensor_of(x, *columns), tensor_of(v))
         torch.cuda.synchronize()
         assert torch.equal(d[1:-1].view(-1, 1024), x.view(-1, 1024) + v)
+
+
+@pytest.mark.parametrize("dt", [torch.int16, torch.int32])
+@pytest.mark.parametrize("ni,nj,batch,off,pad", [
+    (4100, 3080, 1, 0, 0),      # rows of 16-byte pieces: a shift of its own for each of eight rows
+    (2101, 6001, 1, 1, 0), (1500, 6145, 1, 3, 2),   # odd rows from an odd element
+    (131, 3080, 40, 8, 0),      # matrices that tiles do not fill, a base in the middle of a line
+    (128, 2568, 40, 24, 40),    # tiles in whole and a part that the shift empties for some rows; padded rows
+    (4099, 3077, 1, 16, 11),    # rows that end inside a piece
+    (2500, 6013, 1, 17, 0),     # ... at any address
+    (2796, 4632, 1, 56, 0), (257, 2072, 64, 0, 0), (2460, 5148, 1, 4, 0), (131, 5141, 19, 8, 3)])
+def test_transposes_into_rows_of_no_whole_lines(mh, dt, ni, nj, batch, off, pad):
+    """Destination rows whose pitch is no multiple of 128 bytes: every workgroup's part of a row runs from one of the row's
+    own lines to another; frames and padding stay."""
+    from moye_hip.torch_interop import tensor_of
+    g = torch.Generator(device="cuda").manual_seed(ni + nj)
+    n = ni * nj * batch
+    src = torch.randint(-30000, 30000, (n,), generator=g, device="cuda").to(dt)
+    pitch = nj + pad
+    dst = torch.full((off + batch * ni * pitch + 8,), 77, device="cuda").to(dt)
+    assert (pitch * dt.itemsize) % 128
+    mh.copyto_(tensor_of(dst[off:], (ni, nj, batch), (pitch, 1, ni * pitch)), tensor_of(src, (ni, nj, batch), (1, ni, ni * nj)))
+    torch.cuda.synchronize()
+    body = dst[off:off + batch * ni * pitch].view(batch, ni, pitch)
+    assert torch.equal(body[:, :, :nj], src.view(batch, nj, ni).transpose(1, 2))
+    assert bool((dst[:off] == 77).all()) and bool((body[:, :, nj:] == 77).all()) and bool((dst[off + batch * ni * pitch:] == 77).all())
