@@ -361,8 +361,8 @@ static GemmArgs columns_from(GemmArgs a, int64_t n1, int eb, int ob) {
 // also in two launches, whole rounds of them and the rest on what is cheapest for it alone, as K-major operands have it there.  bf16, operands
 // not cached, us before (K-major copies, or whole 256 x 256 / 128 x 128 tiles in one launch) / now: 6000 x 4096 x 14336 with B N-major 570 / 524,
 // 14336 x 4096 x 6000 with both the other way round 573 / 526, 7424 x 1152 x 3600 109 / 84, 3840 x 2048 x 1240 42 / 27; whole 14336 x 4096 x 4096
-// 376 / 364, 2048 x 4096 x 4096 73.7 / 62.4, 256 x 4096 x 4096 with B N-major 52.9 / 36.5.  A linear layer's forward and two gradients, 6000 x
-// 4096 -> 14336: 1690 / 1590; 1240 x 2048 -> 3840: 111 / 91.
+// 376 / 364, 2048 x 4096 x 4096 73.7 / 62.4, 256 x 4096 x 4096 with B N-major 52.9 / 28.3 (128 x 64 tiles; 36.5 on 128 x 128 ones).  A linear layer's
+// forward and two gradients, 6000 x 4096 -> 14336: 1690 / 1590; 1240 x 2048 -> 3840: 111 / 92; 256 x 1024 -> 14336: 181 / 105.
 static int32_t dispatch_majors(int32_t in_dt, int32_t out_dt, const GemmArgs& a, GemmPlan& plan) {
     const int eb = 2, ob = dtype_bytes(out_dt), cus = plan.shape.cus;
     const int64_t k_bytes = (int64_t)a.K * eb;

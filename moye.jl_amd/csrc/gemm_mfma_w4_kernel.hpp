@@ -319,8 +319,8 @@ __global__ __launch_bounds__(128 * WGN, TILE == 128 && TILE_N == 128 && In::kRin
     constexpr bool kBlocks64 = AMAJ == 2 || BMAJ == 2;
     static_assert(!(AMAJ == 1 || BMAJ == 1) || (In::kRow == 128 && ((TILE == 256 && WGN == 4) || (TILE == 128 && WGN == 2)) && !kBias && !kRagged && !kBlocks64),
                   "operands that are not K-major: whole-line stages, eight waves, plain whole tiles");
-    static_assert(!kBlocks64 || (In::kRow == 128 && In::kBytes == 2 && WGN == 4 && kRagged && TILE % 64 == 0 && TILE_N % 64 == 0),
-                  "... in blocks of 64 rows: 16-bit types, whole-line stages, eight waves, guarded tiles");
+    static_assert(!kBlocks64 || (In::kRow == 128 && In::kBytes == 2 && kRagged && TILE % 64 == 0 && TILE_N % 64 == 0),
+                  "... in blocks of 64 rows: 16-bit types, whole-line stages, guarded tiles");
     static_assert(!kRagged || (!kBias && In::kRow == 128 && AMAJ != 1 && BMAJ != 1), "ragged tiles: the plain whole-line form");
     static_assert(!kOps || (In::kRow == 128 && TILE == 256 && WGN == 4 && !kBias && !AMAJ && !BMAJ), "epilogue operations: whole-line stages, eight waves, K-major operands");
     static_assert(!kPersist || (In::kRow == 128 && TILE == 256 && WGN == 4 && !kRagged && !kOps && !AMAJ && !BMAJ),

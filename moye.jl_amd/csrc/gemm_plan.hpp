@@ -165,7 +165,7 @@ inline const FormPrice* gemm_majors_form(int64_t M, int64_t N, int64_t k_bytes, 
     const FormPrice* best = nullptr;
     *us = 1e30;
     for (const FormPrice& f : kFormPrices16) {
-        if (f.waves_k > 1 || f.form == GemmForm::kTile128x64) continue;
+        if (f.waves_k > 1) continue;
         if (f.form == GemmForm::kOther && (f.tm == 256 ? !tile256 || ((M + 255) / 256) * ((N + 255) / 256) > cus : !two_stages)) continue;
         // (whole tiles in two stages run unguarded: they keep what is a tenth dearer)
         const double t = (f.form == GemmForm::kOther && f.tm == 128 ? 0.9 : 1.0) * gemm_form_us(f, M, N, k_bytes, cus);
@@ -174,9 +174,10 @@ inline const FormPrice* gemm_majors_form(int64_t M, int64_t N, int64_t k_bytes, 
     return best;
 }
 // Are K-major copies (`copied` elements of operands in all, one launch for each operand) and the cheapest K-major form the better plan?  The
-// blocks, which divide K among four waves, have no form that reads operands otherwise: few elements (bf16 264 x 1024 x 1088, B N-major:
-// 10.3 us with a copy and blocks, tiles 10.6 at 256 x 1024 x 1024).  Beyond that copies are 5 us and twice the operands' bytes: 1000 x 6144 x
-// 4096 69.2 with a copy of B, 53.2 as it lies, both operands 76.8 / 54.8; 1088 x 1024 x 264 both 15.8 / 8.3.  Two kinds of call keep their
+// blocks, which divide K among four waves, have no form that reads operands otherwise: few elements and a long K (bf16 500 x 1000 x 1992, A
+// M-major, 14.8 us so).  Beyond that copies are 5 us and twice the operands' bytes: 264 x 1024 x 1088 with B N-major 10.5 with a copy and blocks,
+// 9.0 as it lies, 1000 x 6144 x 4096 69.2 / 53.2, both operands 76.8 / 54.8; 1088 x 1024 x 264 both 15.8 / 7.5.  A K that ends inside a stage costs the
+// tiles 2 us (1000 x 520 x 1984 / 1992 15.5 / 17.3; 1992 with B N-major 18.2 with a copy, 19.2 as it lies).  Two kinds of call keep their
 // copies without a look at prices, because callers size buffers for them by the query and get the launches they sized them for: fewer than
 // 8 tiles of 128 x 128 (200 x 136 x 504 12.7 us, eight tiles as they lie 9.1) and more than 16384 rows with a short K (28000 x 1208 x 520 81
 // and 62).
@@ -186,6 +187,7 @@ inline bool gemm_majors_copies_pay(int64_t M, int64_t N, int64_t k_bytes, int64_
     double native, kmajor;
     gemm_majors_form(M, N, k_bytes, cus, true, false, &native);
     gemm_form_choose(M, N, k_bytes, 2, cus, 1e30, &kmajor);
+    if (k_bytes % 128) native += 2.0;
     return kmajor + 2.5 * launches + 4.0 * (double)copied / 5.0e6 < native;
 }
 
