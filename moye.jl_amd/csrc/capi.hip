@@ -330,17 +330,21 @@ static bool majors_on_guarded_tiles(const moye_tiled_mma* mma, const Mat& A, con
     if (A.cols % 8 || A.cols < 64 || A.rows <= 64 || B.rows <= 64 || (D.cs != 1 && D.rs != 1)) return false;
     int64_t copied = 0;
     int launches = 0;
+    bool ragged_rows = false;
     for (const Mat* x : {&A, &B}) {
         const bool kmajor = x->cs == 1 || x->cols == 1;
         const int64_t pitch = kmajor ? x->rs : x->cs;
         if (pitch % 8 || reinterpret_cast<uintptr_t>(x->ptr) % 16 || 256 * pitch * 2 >= ((int64_t)1 << 32)) return false;
-        if (kmajor) continue;
+        if (kmajor) {
+            ragged_rows = pitch * 2 % 128 != 0;
+            continue;
+        }
         if (x->rs != 1 || x->rows % 8 || pitch < x->rows) return false;
         copied += x->rows * x->cols;
         ++launches;
     }
     const bool swap = column_major(D);
-    return !gemm_majors_copies_pay(swap ? B.rows : A.rows, swap ? A.rows : B.rows, A.cols * 2, copied, launches, cus);
+    return !gemm_majors_copies_pay(swap ? B.rows : A.rows, swap ? A.rows : B.rows, A.cols * 2, copied, launches, ragged_rows, cus);
 }
 
 // K-major copies of A and B where needed, then the fp32 partial products of a split-K call
