@@ -16,7 +16,9 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "moye_hip", "libmoye_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
+# (align-mismatch: a wide access of an array that is only aligned to its elements goes through a type that says so; a template
+# parameter deduced from such a pointer has lost that, and with it the reason the access is allowed)
+COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Werror=align-mismatch",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # source -> extra flags
 SOURCES = {

@@ -339,8 +339,8 @@ template <> struct Piece<ElBF16> {
 // 4096 (64) 117.5 / 117.8; one call alone, bf16, 24 MiB: a + b 13.6 / 13.6, max with a scalar 9.8 / 10.1, axpby! 13.6 / 13.4; 64 MiB: 33.9 / 36.6,
 // 23.3 / 24.4, 34.0 / 33.7; f32 128 MiB 65 / 69, 44 / 47, 66 / 75.
 constexpr int64_t kKeptResult = (int64_t)32 << 20;
-template <bool kKeep, typename P>
-__device__ __forceinline__ void store_result(const u32x4& w, P* p) {
+template <bool kKeep>
+__device__ __forceinline__ void store_result(const u32x4& w, u32x4_any* p) {
     if constexpr (kKeep) *p = w;
     else __builtin_nontemporal_store(w, p);
 }

@@ -73,6 +73,17 @@ def test_the_shipped_listing_is_checked_at_build_time():
     assert users and set(users) == set(build.ASM_MFMA_SOURCES)
 
 
+@pytest.mark.skipif(shutil.which(build.HIPCC) is None, reason="no compiler")
+@pytest.mark.parametrize("src", ["elementwise.hip", "copy_kernels.hip", "copy_transpose.hip"])
+def test_wide_accesses_of_arrays_of_any_alignment_say_so(src):
+    """Dense arrays start at any element: their 16-byte accesses go through a type without an alignment, and no helper on the
+    way takes them for aligned ones.  The build refuses a source that does (the host pass sees every instance)."""
+    assert "-Werror=align-mismatch" in build.COMMON
+    cmd = [build.HIPCC] + build.COMMON + build.SOURCES[src] + ["-fsyntax-only", "--cuda-host-only", os.path.join(build.CSRC, src)]
+    r = build.subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 @pytest.mark.parametrize("why", ["no compiler", "an error", "no headers"])
 def test_the_calls_without_ctypes_are_optional(monkeypatch, tmp_path, capsys, why):
     """Whatever keeps moye_hip/_call from being built, the build goes on and a module of an earlier one does not stay."""
