@@ -206,6 +206,10 @@ int32_t moye_map(int32_t op, const moye_tensor* dst, const moye_tensor* a, const
  * that run on whole 256x256x64 or 128x128x64 tiles without K ranges, and for fp8 / fp32 operands of any major on whole
  * 256x256 tiles with 128 bytes of K per k-step (named so, or left to the library on problems of at least 128 such
  * tiles) -- all read where they lie.  Assumes the plain epilogue of moye_gemm (see moye_gemm_ex_workspace_size).
+ *   Most plain calls on f16 / bf16 operands that are not K-major read them where they lie also on problems of no whole number of
+ * tiles (tile and K ranges left open; their rows in whole 16-byte pieces, K of 64 and more).  Their copies are counted all the same: such a
+ * call takes nothing of the workspace and may be given none (moye_gemm_explain tells), while the same problem with an operation in the
+ * epilogue, with an operand off a 16-byte boundary or with fewer rows may need it, and has room in a buffer of this size.
  *   moye_gemm     keeps a workspace of its own per (device, stream): allocated by the first call on that stream
  *                 that needs one (a synchronous hipMalloc inside that call, so not under stream capture),
  *                 replaced by a larger one when a larger call comes, never freed inside a call.  Calls on
@@ -247,7 +251,7 @@ int32_t moye_gemm_ex(const moye_tiled_mma* mma, const moye_tensor* D, const moye
  * caller -- and this library's tests -- see what the dispatcher decided.  `ep` may be NULL (the plain epilogue of
  * moye_gemm).  `compute_units`: plan for a chip of that many CUs (32 to an XCD); 0 = the current device, or 256 CUs in 8
  * XCDs when there is none.  One line per step:
- *   plan: <n> step(s), workspace <bytes> bytes, <cus> CUs in <xcds> XCDs
+ *   plan: <n> step(s), workspace <bytes> bytes, <cus> CUs in <xcds> XCDs       (what these steps use)
  *   step <i>: kernel <function<template arguments>> grid=<x>x<y> block=<lanes> lds=<bytes> tile=<m>x<n>x<k bytes>B
  *             in=<dtype> out=<dtype> M= N= K= lda= ldb= ldd= ldd_n= A=<where> B= D= C= a16= b16= d16= split= alpha=
  *             beta= op= flags=<names joined by |>

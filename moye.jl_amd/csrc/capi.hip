@@ -274,11 +274,13 @@ static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, co
 // (named, or the library's own choice for a problem of whole 128 x 128 tiles with more than 64 rows), the two-stage
 // schedule, no K ranges; fp8 and fp32 on the hand-ordered kernel's whole 256 x 256 or 128 x 128 tiles with 128 bytes of K
 // per k-step (named so, or left to the library: 256 x 256 tiles when the problem has at least 128 of them), plain calls; the operand dense
-// along its rows with a pitch of whole 16-byte pieces, and D 16-byte aligned; or on the guarded tiles of majors_on_guarded_tiles, 16-bit types
-// and any D.
+// along its rows with a pitch of whole 16-byte pieces, and D 16-byte aligned; or (`guarded`) on the guarded tiles of
+// majors_on_guarded_tiles, 16-bit types and any D.
+//   The sizing functions ask without the guarded tiles and count the copies: whether a call runs on them hangs on its epilogue, its
+// row count and its operands' addresses, and a buffer of the size reported serves the same problem with others of them.
 static bool majors_on_guarded_tiles(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep, int cus);
 static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep,
-                                bool has_c, int cus) {
+                                bool guarded, int cus) {
     const bool b16 = mma->atom == MOYE_MFMA_F32_16x16x32_F16 || mma->atom == MOYE_MFMA_F32_16x16x32_BF16;
     const bool wide = mma->atom == MOYE_MFMA_F32_16x16x32_FP8 || mma->atom == MOYE_MFMA_F32_16x16x4_F32;  // hand-ordered kernel only
     if (!b16 && !wide) return false;
@@ -294,7 +296,7 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
     const bool named256 = bm == 256 && bn == 256 && (b16 ? (bk == 0 || bk == 64) : bk * eb == 128) && !four_waves && M % 256 == 0 && N % 256 == 0;
     const bool named128 = bm == 128 && bn == 128 && bk * eb == 128 && M % 128 == 0 && N % 128 == 0;
     const bool chosen = bm == 0 && bn == 0 && bk == 0 && M > 64 && M % 128 == 0 && N % 128 == 0 && whole_lines && whole_d;
-    if (!named256 && !named128 && !chosen && majors_on_guarded_tiles(mma, A, B, D, ep, cus)) return true;
+    if (guarded && !named256 && !named128 && !chosen && majors_on_guarded_tiles(mma, A, B, D, ep, cus)) return true;
     if (!whole_lines || !whole_d) return false;
     if (wide) {
         // (the hand-ordered kernel reads such operands in plain calls only, and fp32 and fp8 have no other kernel that does)
@@ -307,7 +309,6 @@ static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const M
     } else if (!named256 && !named128 && !chosen) {
         return false;
     }
-    (void)has_c;
     for (const Mat* x : {&A, &B}) {
         if (x->cs == 1 || x->cols == 1) continue;  // K-major already
         if (x->rs != 1 || (x->cs * eb) % 16 || reinterpret_cast<uintptr_t>(x->ptr) % 16 || x->cs < x->rows) return false;
@@ -358,9 +359,10 @@ static size_t gemm_workspace_bytes_impl(const moye_tiled_mma* mma, const Mat& A,
     return n;
 }
 
-// The same from descriptors: what the fastest plan uses (`lines`), or the least the call can do with
+// The same from descriptors: what callers are told, enough for the fastest plan of every such call (`any_call`), or the least that this
+// one can do with
 static int32_t gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor* D, const moye_tensor* A, const moye_tensor* B,
-                                   const moye_gemm_epilogue& ep, bool lines, size_t* bytes) {
+                                   const moye_gemm_epilogue& ep, bool any_call, size_t* bytes) {
     *bytes = 0;
     Mat a, b, d;
     if (int32_t e = as_matrix(A, "A", &a)) return e;
@@ -370,7 +372,7 @@ static int32_t gemm_workspace_size(const moye_tiled_mma* mma, const moye_tensor*
         if (x->rows == 1 && x->cs == 1) x->rs = x->cols;
     const int cus = device_shape().cus;
     if (!(mma->flags & MOYE_GEMM_NO_WORKSPACE))
-        *bytes = gemm_workspace_bytes_impl(mma, a, b, d, majors_run_natively(mma, a, b, d, ep, false, cus), lines, cus);
+        *bytes = gemm_workspace_bytes_impl(mma, a, b, d, majors_run_natively(mma, a, b, d, ep, !any_call, cus), any_call, cus);
     return MOYE_OK;
 }
 
@@ -479,7 +481,7 @@ static int32_t gemm_plan_build(const moye_tiled_mma* mma, const moye_tensor* tD,
     // NN / NT / TT (the naming of src/arch/mma/make_mma_ops.jl:253-265): operands whose unit stride is not
     // along K are brought to the K-major form the kernels read (one tiled transpose each)
     char* ws = nullptr;
-    const bool native_majors = majors_run_natively(mma, A, B, D, ep, tC != nullptr, plan.shape.cus);
+    const bool native_majors = majors_run_natively(mma, A, B, D, ep, true, plan.shape.cus);
     int major_flags = 0;  // which of the kernel's operands keep their M- (N-) major form
     if (native_majors) {
         if (A.cs != 1 && A.cols > 1) { major_flags |= kGemmAMajorM; A.rs = A.cs; A.cs = 1; }  // Mat::rs now holds the pitch between consecutive k

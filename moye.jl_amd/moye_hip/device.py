@@ -120,9 +120,10 @@ def gemm_release_workspace():
 
 
 def gemm_workspace_size(mma, D, A, B, epilogue=None):
-    """Bytes of library-owned device workspace this gemm! call needs (K-major copies of operands that are not K-major,
-    partial products of a split-K call); 0 for a plain TN call.  With `epilogue` (a moye_gemm_epilogue): for the
-    moye_gemm_ex call with that epilogue."""
+    """Bytes of device workspace this gemm! call needs (K-major copies of operands that are not K-major, partial products of
+    a split-K call); 0 for a plain TN call.  f16 / bf16 operands of ragged problems count with their copies also where this very
+    call reads them as they lie: the same problem with an operation, at other addresses or with fewer rows has room in a buffer
+    of this size.  With `epilogue` (a moye_gemm_epilogue): for the moye_gemm_ex call with that epilogue."""
     n = C.c_size_t()
     if epilogue is None:
         check(lib().moye_gemm_workspace_size(C.byref(mma), C.byref(D), C.byref(A), C.byref(B), C.byref(n)))
