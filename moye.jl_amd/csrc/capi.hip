@@ -281,6 +281,8 @@ static int split_count(const moye_tiled_mma* mma, const Mat& A, const Mat& B, co
 static bool majors_on_guarded_tiles(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep, int cus);
 static bool majors_run_natively(const moye_tiled_mma* mma, const Mat& A, const Mat& B, const Mat& D, const moye_gemm_epilogue& ep,
                                 bool guarded, int cus) {
+    // (nothing to copy, and nothing below changes that: calls of a few microseconds wait for the host)
+    if ((A.cs == 1 || A.cols == 1) && (B.cs == 1 || B.cols == 1)) return true;
     const bool b16 = mma->atom == MOYE_MFMA_F32_16x16x32_F16 || mma->atom == MOYE_MFMA_F32_16x16x32_BF16;
     const bool wide = mma->atom == MOYE_MFMA_F32_16x16x32_FP8 || mma->atom == MOYE_MFMA_F32_16x16x4_F32;  // hand-ordered kernel only
     if (!b16 && !wide) return false;
