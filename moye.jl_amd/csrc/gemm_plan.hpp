@@ -178,13 +178,11 @@ inline const FormPrice* gemm_majors_form(int64_t M, int64_t N, int64_t k_bytes, 
 // M-major, 14.8 us so).  Beyond that copies are 5 us and twice the operands' bytes: 264 x 1024 x 1088 with B N-major 10.5 with a copy and blocks,
 // 9.0 as it lies, 1000 x 6144 x 4096 69.2 / 53.2, both operands 76.8 / 54.8; 1088 x 1024 x 264 both 15.8 / 7.5.  `ragged_rows`: the other
 // operand is K-major with a pitch of no whole lines, which costs the tiles 2 us more than the blocks (A M-major, 1000 x 520 x 1984 / 1992 15.5 /
-// 17.3; 1992 with B N-major 18.2 with a copy, 19.2 as it lies).  Two kinds of call keep their
-// copies without a look at prices, because callers size buffers for them by the query and get the launches they sized them for: fewer than
-// 8 tiles of 128 x 128 (200 x 136 x 504 12.7 us, eight tiles as they lie 9.1) and more than 16384 rows with a short K (28000 x 1208 x 520 81
-// and 62).
+// 17.3; 1992 with B N-major 18.2 with a copy, 19.2 as it lies).  Few tiles and long problems with a short K follow the prices like any other: both
+// operands, copies / as they lie, 200 x 136 x 504 11.2 / 8.0, 408 x 96 x 1280 12.7 / 11.7, 28000 x 1208 x 520 81.9 / 66.0, 208 x 37432 x 960 63.9 / 32.4;
+// of 66 such problems the one that prices send the slower way as it lies is 16848 x 3280 x 152 with A M-major, 57.4 / 59.5, and of fewer than 8 tiles of
+// 128 x 128 with one operand to copy and a K under 500 they copy where that takes 0.3 to 2 us more (136 x 160 x 144 6.7 / 4.8).
 inline bool gemm_majors_copies_pay(int64_t M, int64_t N, int64_t k_bytes, int64_t copied, int launches, bool ragged_rows, int cus) {
-    if (((M + 127) / 128) * ((N + 127) / 128) * 32 < cus) return true;
-    if ((M > 16384 || N > 16384) && k_bytes < 2048) return true;
     double native, kmajor;
     gemm_majors_form(M, N, k_bytes, cus, true, false, &native);
     gemm_form_choose(M, N, k_bytes, 2, cus, 1e30, &kmajor);

@@ -107,11 +107,11 @@ def test_noalloc_plain_tn_and_limits(mh):
 
 
 def test_a_workspace_that_holds_the_copies_only_in_16_byte_pieces_is_taken(mh):
-    """fp16 with K = 520, A M-major and B N-major: copies of 1040-byte rows take 30.4 MB, of 1152-byte ones, which
-    moye_gemm uses, 33.6 MB, more than the static array holds.  moye_gemm_noalloc and moye_gemm_ex with a buffer of the
+    """fp16 with K = 520, A M-major (an odd number of rows: no kernel reads it as it lies) and B N-major: copies of 1040-byte rows take
+    30.4 MB, of 1152-byte ones, which moye_gemm uses, 33.6 MB, more than the static array holds.  moye_gemm_noalloc and moye_gemm_ex with a buffer of the
     smaller size give moye_gemm's bits and write nothing behind it; one byte less is refused."""
     from moye_hip import _lib
-    M, N, K = 28000, 1208, 520
+    M, N, K = 28001, 1208, 520
     g = torch.Generator(device="cuda").manual_seed(31)
     a = torch.randn(K, M, generator=g, device="cuda").mul_(K ** -0.5).half()
     b = torch.randn(K, N, generator=g, device="cuda").half()
