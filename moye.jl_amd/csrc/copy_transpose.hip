@@ -393,16 +393,19 @@ static int32_t launch_kept(TransposeArgs a, int lds_request, hipStream_t st) {
 }
 
 // Which form of the destination's rows (kSkew), for tiles of 1 KiB of a row: 0 where their pitch is whole lines, or where the tiles more that the shift
-// costs are worth more than the lines.  us without / with, operands not cached: fp16 into rows of whole pieces from 4000 bytes on,
-// 4864 x 5992 28.0 / 23.1, 16000 x 16008 230 / 207, [1,3000,32,128] -> [1,32,128,3000] 10.7 / 10.1, but 12345 x 1400 18.1 / 19.3; f32 from 20 KiB and 48 MiB
+// costs are worth more than the lines.  us without / with, operands not cached: fp16 into rows of whole pieces from four tiles to a row on,
+// 4864 x 5992 28.0 / 23.1, 16000 x 16008 230 / 207, [1,3000,32,128] -> [1,32,128,3000] 10.7 / 10.1, [4,1672,32,128] 25.2 / 22.6, 14336 x 1640 21.9 / 21.6,
+// 24704 x 1640 37.8 / 36.8, 22392 x 1992 40.3 / 37.9; three tiles to a row gain as often as they lose (21852 x 1288 25.7 / 26.3, 34908 x 1288 39.7 / 41.0,
+// 38400 x 1288 43.7 / 42.2, 22004 x 1464 30.7 / 32.4), two as well (128 matrices 128 x 776 11.8 / 12.3, 128 x 904 14.1 / 13.4); f32 from 20 KiB and 48 MiB
 // on, 4860 x 5992 50.3 / 47.5, 16000 x 16008 446 / 405, but 13361 x 3728 76.6 / 78.4, 3004 x 2996 15.7 / 16.3; fp16 into any rows of one matrix
 // from 5888 elements on, 4861 x 5993 29.6 / 27.1, 16001 x 16011 254 / 216, 1033 x 14001 14.3 / 13.6, but 10001 x 4099 39.0 / 41.8, 4000 x 4499 20.8 / 21.8 and
 // in batches [4,2001,32,128] 31.7 / 33.2; f32 into any rows 115.3 / 119.1 (10001 x 7003); f32 -> bf16 18.5 / 18.5 (5000 x 3000).
-// Not 16-bit tiles, one to a CU, of which a second round has less than half a round's (1329 x 13256 18.2 / 18.8, 1691 x 11920 19.1 / 19.7).
+// Not 16-bit tiles, one to a CU, of which a second round has less than half a round's (1329 x 13256 18.2 / 18.8, 1691 x 11920 19.1 / 19.7, 8448 x 1640 16.1 / 16.4,
+// 4216 x 4000 17.9 / 20.3).
 static int skew_of(const TransposeArgs& a, int db, bool dst_lines) {
     constexpr int64_t Mi = 1 << 20;
     const int64_t row = (int64_t)a.nj * db;
-    if (dst_lines || row < (db == 2 ? 4000 : 20480) || (db == 4 && row * a.ni * a.batch < 48 * Mi)) return 0;
+    if (dst_lines || (db == 2 ? a.nj <= 3 * 512 : row < 20480) || (db == 4 && row * a.ni * a.batch < 48 * Mi)) return 0;
     const int64_t tiles = ((int64_t)a.ni + 127) / 128 * ((a.nj + 511) / 512) * a.batch, cus = 32 * a.xcds;
     if (db == 2 && tiles > cus && 2 * tiles < 3 * cus) return 0;
     int64_t all = reinterpret_cast<uintptr_t>(a.dst) | a.ldd * db;

@@ -1386,6 +1386,7 @@ def test_results_on_either_side_of_what_the_l2s_hold(mh, n, start):
     (128, 2568, 40, 24, 40),    # tiles in whole and a part that the shift empties for some rows; padded rows
     (4099, 3077, 1, 16, 11),    # rows that end inside a piece
     (2500, 6013, 1, 17, 0),     # ... at any address
+    (5500, 1640, 1, 0, 0), (250, 1928, 64, 8, 8),   # four tiles to a row, the fewest in 16 bits
     (2796, 4632, 1, 56, 0), (257, 2072, 64, 0, 0), (2460, 5148, 1, 4, 0), (131, 5141, 19, 8, 3)])
 def test_transposes_into_rows_of_no_whole_lines(mh, dt, ni, nj, batch, off, pad):
     """Destination rows whose pitch is no multiple of 128 bytes: every workgroup's part of a row runs from one of the row's
