@@ -1,6 +1,6 @@
 // MFMA GEMM for a short A: at most 64 rows against a long B (N x K), K-major operands.
 // The work is streaming B from HBM once, so the kernel is laid out for bandwidth, not for the matrix pipe: one workgroup
-// owns 16 to 64 rows of B (that many output columns) and all of A; its four waves split K into contiguous ranges of
+// owns 8 to 64 rows of B, in eights (that many output columns) and all of A; its four waves split K into contiguous ranges of
 // whole 128-byte lines, both operands go through LDS by load-to-LDS instructions that read whole lines, and the per-wave
 // partial accumulators are summed through LDS in wave order, which makes the result independent of timing.  A (at most
 // 64 x K) is re-read by every workgroup and lives in L2.  bf16 16 x 8192 x 8192: 21.0 us (0.80 of the HBM peak); a

@@ -243,7 +243,7 @@ inline bool gemm_short_m(int64_t M, int64_t N, int64_t k_bytes, bool f32_in, int
     return !(4 * tiles >= 3 * (int64_t)cus && k_bytes <= 2048);
 }
 
-// The short-M kernel's workgroups take 16, 32, 48 or 64 rows of B and all of A, one workgroup on a CU at a time (its rings
+// The short-M kernel's workgroups take 8 to 64 rows of B, in eights, and all of A, one workgroup on a CU at a time (its rings
 // fill the LDS), and a workgroup streams its rows at about 64 GB/s whatever the others do (56 with 48 and 64 rows of B,
 // measured with long K).  A launch therefore takes as many rounds as its workgroups -- times the K ranges of a split -- need
 // on the CUs: bf16, us with 32 / 48 / 64 rows: 64 x 12288 x 8192 59.0 / 39.2 / 44.1; 64 x 14336 x 4096 33.0 / 37.9 / 24.9;
@@ -269,8 +269,12 @@ inline double gemm_short_m_us(int64_t M, int64_t N, int64_t k_bytes, int cus, in
 // half: 50 x 14336 x 4096 23.5 (64 rows) / 22.7 (56), 16 x 6144 x 8192 19.3 (32) / 17.2 (24), 40 x 10240 x 8192 32.6 (48) / 30.2 (40), 50 x 2048 x 4096
 // 11.8 (16) / 10.5 (8), 16 x 20480 x 4096 29.1 / 27.7, 64 x 28672 x 8192 92.8 / 88.3.  Not with a few rows of A and long rows, which run at
 // the memory's rate as they are (1 x 6144 x 16384 30.6 / 33.7, 1 x 5120 x 16384 28.2 / 28.9; but 1 x 5000 x 12288 22.1 / 20.1), nor
-// 40 and 56 rows with rows under 4 KiB, in several rounds up to that (1 x 9600 x 1024 5.7 / 5.9, 40 x 28672 x 2048 24.6 / 25.0).  Eight rows in
-// unsplit launches only.  `us` is the price with whole blocks, which the model was fitted to: on it K ranges are decided (16 x 2048 x 16384
+// 40 and 56 rows with rows under 2 KiB, where they win as often as they lose (40 x 14336 x 256 5.4 / 5.6, x 512 6.9 / 6.6, x 768 7.8 / 7.8; from 2 KiB
+// on 40 x 9600 x 1536 9.6 / 9.3, 24 x 20480 x 2048 18.5 / 17.7, 24 x 14336 x 2040 19.5 / 19.1), or up to 4 KiB where two workgroups of 32 share a CU
+// (12 x 19456 x 1536 12.7 / 13.5, x 2048 15.3 / 15.8, x 2056 24.9 / 24.3, x 2304 17.1 / 17.2, x 2560 20.1 / 19.2), nor 56 rows in several rounds beside more than 32 rows of A where rows are 4 KiB, more
+// than 40 where they are 8 KiB: their lines at one k lie in few memory channels (N = 28672, M = 40 / 56 / 64: K = 2048 24.2 / 24.9, 26.4 / 27.6, 27.2 / 28.4,
+// K = 4096 41.2 / 41.0, 44.9 / 45.8, 46.7 / 47.8; but K = 1536 21.3 / 20.8, 23.5 / 23.3, 24.2 / 24.2, 3072 35.7 / 34.8, 39.1 / 39.1, 40.5 / 40.5, 6144 64.1 / 63.6,
+// 71.7 / 71.2, 75.0 / 73.8, 8192 76.1 / 75.9, 86.1 / 82.8, 90.5 / 84.6).  Eight rows in unsplit launches only.  `us` is the price with whole blocks, which the model was fitted to: on it K ranges are decided (16 x 2048 x 16384
 // 22.2 unsplit with 16 rows, 19.9 with 8, 17.1 in two ranges).
 inline int gemm_short_m_rows(int64_t M, int64_t N, int64_t k_bytes, int cus, int split, double* us = nullptr) {
     // (the host's time for a call of a few microseconds counts: no division where one round holds the workgroups)
@@ -288,10 +292,12 @@ inline int gemm_short_m_rows(int64_t M, int64_t N, int64_t k_bytes, int cus, int
     }
     if (us) *us = gemm_short_m_us(M, N, k_bytes, cus, best, split);
     least *= 0.94;
+    const int whole = best;
     for (int r : {8, 24, 40, 56}) {
         if (r == 8 ? split > 1 : M <= 8 && k_bytes >= 28 * 1024) continue;
         const int64_t rounds = rounds_of(r);
-        if (r >= 40 && k_bytes < (rounds > 1 ? 4097 : 4096)) continue;
+        if (r >= 40 && (k_bytes < 2048 || (whole == 32 && k_bytes <= 4096))) continue;
+        if (r == 56 && rounds > 1 && ((M > 32 && k_bytes == 4096) || (M > 40 && k_bytes == 8192))) continue;
         const double c = cost(r, rounds);
         if (c <= least) { best = r; least = c; }
     }
