@@ -334,16 +334,13 @@ template <> struct Piece<ElBF16> {
 };
 
 // How a result goes out.  Ordinary stores (kKeep) leave it in the L2s for the call that reads it next, as far as they hold it: results of
-// up to 32 MiB, the eight XCDs' L2s together.  Beyond that, and for a result that nothing reads soon, the non-temporal hint is better.  us, hinted
-// / ordinary, operands not cached: bias, ReLU, residual and mask on bf16 4096 x 1500 (12 MiB an array) 30.2 / 28.2, 4096 x 3000 (23) 50.5 / 47.1, 8192 x
-// 4096 (64) 117.5 / 117.8; one call alone, bf16, 24 MiB: a + b 13.6 / 13.6, max with a scalar 9.8 / 10.1, axpby! 13.6 / 13.4; 64 MiB: 33.9 / 36.6,
-// 23.3 / 24.4, 34.0 / 33.7; f32 128 MiB 65 / 69, 44 / 47, 66 / 75.
+// up to 32 MiB, the eight XCDs' L2s together, of map! on two arrays, up to 24 MiB of axpby! with both terms.  Everything else goes out with the
+// non-temporal hint.  us for bias, ReLU, residual and mask on bf16, hinted throughout / so / ordinary stores throughout: 4096 x 1500 (12 MiB an array)
+// 27.3 / 26.8 / 27.0, 4096 x 3000 (23) 49.3 / 46.1 / 45.8, 4096 x 4000 (31) 62.8 / 59.3 / 60.6, f32 4096 x 2000 (31) 61.4 / 57.4 / 59.6; 8192 x 4096 (64) 117.5
+// hinted, 117.8 ordinary.  One call alone, whose result nothing reads, bf16, hinted / ordinary: a + b 16 MiB 9.8 / 9.5, 23 MiB 13.4 / 13.6, 31 MiB 17.1 / 18.1 (in
+// place 17.1 / 17.1), a + bias 23 MiB 9.9 / 10.3, axpby! 16 MiB 9.5 / 9.2, 23 MiB 13.4 / 13.1, 31 MiB 17.2 / 17.2; what is hinted at every size, 23 MiB: max with a
+// scalar 9.6 / 10.1, -a 9.7 / 10.1, axpby! with b = 0 9.7 / 10.1.
 constexpr int64_t kKeptResult = (int64_t)32 << 20;
-template <bool kKeep>
-__device__ __forceinline__ void store_result(const u32x4& w, u32x4_any* p) {
-    if constexpr (kKeep) *p = w;
-    else __builtin_nontemporal_store(w, p);
-}
 
 template <typename El, bool kZero /* b is zero: y is not read */, bool kKeep>
 __global__ __launch_bounds__(256) void axpby_dense_kernel(typename El::compute a, const typename El::storage* x,
@@ -372,7 +369,8 @@ __global__ __launch_bounds__(256) void axpby_dense_kernel(typename El::compute a
             for (int k = 0; k < N; ++k) vx[k] = vx[k] + vy[k];
             r = Piece<El>::pack(vx);
         }
-        store_result<kKeep>(r, py);
+        if constexpr (kKeep) *py = r;
+        else __builtin_nontemporal_store(r, py);
         return;
     }
 #pragma unroll 1
@@ -437,7 +435,10 @@ __global__ __launch_bounds__(256) void map_dense_kernel(typename El::storage* d,
         Piece<El>::unpack(wa, x);
         map_piece<OP>(x, y);
         constexpr bool exact = !(OP == MOYE_MAP_ADD || OP == MOYE_MAP_SUB || OP == MOYE_MAP_MUL || OP == MOYE_MAP_DIV);
-        store_result<kKeep>(exact ? Piece<El>::pack_exact(x) : Piece<El>::pack(x), reinterpret_cast<u32x4_any*>(d + i));
+        const u32x4 r = exact ? Piece<El>::pack_exact(x) : Piece<El>::pack(x);
+        u32x4_any* const pd = reinterpret_cast<u32x4_any*>(d + i);
+        if constexpr (kKeep) *pd = r;
+        else __builtin_nontemporal_store(r, pd);
         return;
     }
 #pragma unroll 1
@@ -457,13 +458,16 @@ void launch_map_dense_kept(typename El::storage* d, const typename El::storage* 
         if (b && nb % N == 0) { map_dense_kernel<El, OP, kRepeatPieces, kKeep><<<grid, 256, 0, st>>>(d, a, b, s, n, (uint32_t)nb); return; }
         if (b) { map_dense_kernel<El, OP, kRepeat, kKeep><<<grid, 256, 0, st>>>(d, a, b, s, n, (uint32_t)nb); return; }
     }
-    map_dense_kernel<El, OP, kScalar, kKeep><<<grid, 256, 0, st>>>(d, a, b, s, n, 0);
+    if constexpr (!kKeep) map_dense_kernel<El, OP, kScalar, false><<<grid, 256, 0, st>>>(d, a, b, s, n, 0);
 }
 template <typename El, int OP>
 void launch_map_dense_op(typename El::storage* d, const typename El::storage* a, const typename El::storage* b, typename El::compute s, int64_t n,
                          int64_t nb, hipStream_t st) {
-    if (n * (int64_t)sizeof(*d) <= kKeptResult) launch_map_dense_kept<El, OP, true>(d, a, b, s, n, nb, st);
-    else launch_map_dense_kept<El, OP, false>(d, a, b, s, n, nb, st);
+    constexpr bool unary = OP == MOYE_MAP_IDENTITY || OP == MOYE_MAP_NEG || OP == MOYE_MAP_ABS;
+    if constexpr (!unary) {
+        if (b && n * (int64_t)sizeof(*d) <= kKeptResult) { launch_map_dense_kept<El, OP, true>(d, a, b, s, n, nb, st); return; }
+    }
+    launch_map_dense_kept<El, OP, false>(d, a, b, s, n, nb, st);
 }
 template <typename El>
 void launch_map_dense(int32_t op, typename El::storage* d, const typename El::storage* a, const typename El::storage* b, typename El::compute s,
@@ -841,9 +845,9 @@ static void launch_axpby(typename El::compute a, const void* x, const ELayout& l
     }
     constexpr int N = DenseVec<El>::N;
     const dim3 grid = flat_grid((n + N - 1) / N);
-    const bool keep = n * (int64_t)sizeof(*ys) <= kKeptResult;
-    if (b0) (keep ? axpby_dense_kernel<El, true, true> : axpby_dense_kernel<El, true, false>)<<<grid, 256, 0, st>>>(a, xs, b, ys, n);
-    else (keep ? axpby_dense_kernel<El, false, true> : axpby_dense_kernel<El, false, false>)<<<grid, 256, 0, st>>>(a, xs, b, ys, n);
+    if (b0) axpby_dense_kernel<El, true, false><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
+    else if (n * (int64_t)sizeof(*ys) <= kKeptResult / 4 * 3) axpby_dense_kernel<El, false, true><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
+    else axpby_dense_kernel<El, false, false><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
 }
 
 template <typename El>
