@@ -1380,17 +1380,24 @@ def test_results_on_either_side_of_what_the_l2s_hold(mh, n, start):
 
 @pytest.mark.parametrize("dt", [torch.int16, torch.int32])
 @pytest.mark.parametrize("ni,nj,batch,off,pad", [
-    (4100, 3080, 1, 0, 0),      # rows of 16-byte pieces: a shift of its own for each of eight rows
-    (2101, 6001, 1, 1, 0), (1500, 6145, 1, 3, 2),   # odd rows from an odd element
-    (131, 3080, 40, 8, 0),      # matrices that tiles do not fill, a base in the middle of a line
+    # tiles that end on the rows' own lines, 16 bits, a source of at most 300 MiB: rows of 16-byte pieces
+    (4100, 3080, 1, 0, 0),      # a shift of its own for each of eight rows
+    (250, 3080, 40, 8, 0),      # matrices that tiles do not fill, a base in the middle of a line
     (128, 2568, 40, 24, 40),    # tiles in whole and a part that the shift empties for some rows; padded rows
     (4099, 3077, 1, 16, 11),    # rows that end inside a piece
-    (2500, 6013, 1, 17, 0),     # ... at any address
-    (5500, 1640, 1, 0, 0), (250, 1928, 64, 8, 8),   # four tiles to a row, the fewest in 16 bits
-    (2796, 4632, 1, 56, 0), (257, 2072, 64, 0, 0), (2460, 5148, 1, 4, 0), (131, 5141, 19, 8, 3)])
+    (5500, 1640, 1, 0, 0), (250, 1928, 64, 8, 8),   # four tiles to a row, the fewest
+    (2796, 4632, 1, 56, 0),
+    # ... rows at any address
+    (2101, 6001, 1, 1, 0), (1500, 6145, 1, 3, 2), (2500, 6013, 1, 17, 0),
+    # ... 32 bits
+    (2460, 5148, 1, 4, 0), (131, 5141, 19, 8, 3), (250, 5140, 10, 4, 4),
+    # a source of whole lines beyond 300 MiB, read once with the hint: 16 and 32 bits; 16 bits at any address; 32 bits
+    (12800, 12296, 1, 8, 0), (12800, 12301, 1, 3, 0), (9216, 8712, 1, 4, 0),
+    # other tiles, beside the rule: matrices that these would not fill, rows with fewer tiles
+    (131, 3080, 40, 8, 0), (257, 2072, 64, 0, 0), (7000, 1336, 1, 8, 0)])
 def test_transposes_into_rows_of_no_whole_lines(mh, dt, ni, nj, batch, off, pad):
-    """Destination rows whose pitch is no multiple of 128 bytes: every workgroup's part of a row runs from one of the row's
-    own lines to another; frames and padding stay."""
+    """Destination rows whose pitch is no multiple of 128 bytes: where there are enough of them, every workgroup's part of a row runs from one
+    of the row's own lines to another; frames and padding stay."""
     from moye_hip.torch_interop import tensor_of
     g = torch.Generator(device="cuda").manual_seed(ni + nj)
     n = ni * nj * batch
@@ -1403,3 +1410,17 @@ def test_transposes_into_rows_of_no_whole_lines(mh, dt, ni, nj, batch, off, pad)
     body = dst[off:off + batch * ni * pitch].view(batch, ni, pitch)
     assert torch.equal(body[:, :, :nj], src.view(batch, nj, ni).transpose(1, 2))
     assert bool((dst[:off] == 77).all()) and bool((body[:, :, nj:] == 77).all()) and bool((dst[off + batch * ni * pitch:] == 77).all())
+
+
+@pytest.mark.parametrize("sdt,ddt", [(torch.float16, torch.bfloat16), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("ni,nj,off", [(4100, 3080, 8), (2101, 6001, 1)])
+def test_converting_transposes_into_rows_of_no_whole_lines(mh, sdt, ddt, ni, nj, off):
+    """The same tiles where 16-bit elements change their type on the way: rows of 16-byte pieces, rows at any address."""
+    from moye_hip.torch_interop import tensor_of
+    g = torch.Generator(device="cuda").manual_seed(ni)
+    src = torch.randn(nj, ni, generator=g, device="cuda").to(sdt)
+    dst = torch.full((off + ni * nj + 8,), 77.0, device="cuda").to(ddt)
+    mh.copyto_(tensor_of(dst[off:], (ni, nj), (nj, 1)), tensor_of(src, (ni, nj), (1, ni)))
+    torch.cuda.synchronize()
+    assert torch.equal(dst[off:off + ni * nj].view(ni, nj), src.t().to(ddt))
+    assert bool((dst[:off] == 77.0).all()) and bool((dst[off + ni * nj:] == 77.0).all())
