@@ -334,11 +334,11 @@ template <> struct Piece<ElBF16> {
 };
 
 // How a result goes out.  Ordinary stores (kKeep) leave it in the L2s for the call that reads it next, as far as they hold it: results of
-// up to 32 MiB, the eight XCDs' L2s together, of map! on two arrays, up to 24 MiB of axpby! with both terms.  Everything else goes out with the
+// up to 32 MiB, the eight XCDs' L2s together, of map! on two arrays, up to half of that of axpby! with both terms.  Everything else goes out with the
 // non-temporal hint.  us for bias, ReLU, residual and mask on bf16, hinted throughout / so / ordinary stores throughout: 4096 x 1500 (12 MiB an array)
-// 27.3 / 26.8 / 27.0, 4096 x 3000 (23) 49.3 / 46.1 / 45.8, 4096 x 4000 (31) 62.8 / 59.3 / 60.6, f32 4096 x 2000 (31) 61.4 / 57.4 / 59.6; 8192 x 4096 (64) 117.5
+// 27.3 / 26.8 / 27.0, 4096 x 3000 (23) 48.6 / 45.7 / 46.1 (axpby! ordinary too 46.5), 4096 x 4000 (31) 62.8 / 59.3 / 60.6, f32 4096 x 2000 (31) 61.4 / 57.4 / 59.6; 8192 x 4096 (64) 117.5
 // hinted, 117.8 ordinary.  One call alone, whose result nothing reads, bf16, hinted / ordinary: a + b 16 MiB 9.8 / 9.5, 23 MiB 13.4 / 13.6, 31 MiB 17.1 / 18.1 (in
-// place 17.1 / 17.1), a + bias 23 MiB 9.9 / 10.3, axpby! 16 MiB 9.5 / 9.2, 23 MiB 13.4 / 13.1, 31 MiB 17.2 / 17.2; what is hinted at every size, 23 MiB: max with a
+// place 17.1 / 17.1), a + bias 23 MiB 9.9 / 10.3, axpby! 16 MiB 9.5 / 9.2, 23 MiB 13.4 / 13.1 (0.3 that the chain gives back twice), 31 MiB 17.2 / 17.2; what is hinted at every size, 23 MiB: max with a
 // scalar 9.6 / 10.1, -a 9.7 / 10.1, axpby! with b = 0 9.7 / 10.1.
 constexpr int64_t kKeptResult = (int64_t)32 << 20;
 
@@ -846,7 +846,7 @@ static void launch_axpby(typename El::compute a, const void* x, const ELayout& l
     constexpr int N = DenseVec<El>::N;
     const dim3 grid = flat_grid((n + N - 1) / N);
     if (b0) axpby_dense_kernel<El, true, false><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
-    else if (n * (int64_t)sizeof(*ys) <= kKeptResult / 4 * 3) axpby_dense_kernel<El, false, true><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
+    else if (n * (int64_t)sizeof(*ys) <= kKeptResult / 2) axpby_dense_kernel<El, false, true><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
     else axpby_dense_kernel<El, false, false><<<grid, 256, 0, st>>>(a, xs, b, ys, n);
 }
 
