@@ -4,9 +4,10 @@
 // with a CU each; in a ring of four 0.4-0.54).  What bounds them then is neither pipe alone.  Cycles of a k-step, of which the MFMAs /
 // the LDS's reads, by counters, bf16, K = 4096 or 8192: 128 x 128 1100, 512 / 395; 128 x 192 1500, 768 / 480; 192 x 128 1320, 768 / 540; 128 x 256
 // 2060, 1024 / 530; bank conflicts 1 % of them.  A wave waits for loads, reads or the barrier for 24 to 29 % of its time, and for its turn
-// to issue, with the other wave of its SIMD in the matrix pipe, for 42 to 50 %.  With operands that are cached the power limit sets the pace
-// (1000 x 6144 x 4096 45.2 us, on all-zero operands 36.6; without loads 34.3, without MFMAs 30.8), with a B that is not, its lines out of
-// memory (49.7, on zeros 47.9, without MFMAs 44.1, all workgroups on one panel of B 30.1).
+// to issue, with the other wave of its SIMD in the matrix pipe, for 42 to 50 %.  The schedule and the clock both cost.  1000 x 6144 x 4096, call after
+// call, operands cached: 1168 cycles of a k-step, 768 of them MFMAs, at 1.87 GHz, 45.0 us; all-zero operands take the same cycles (1181) at 2.38 GHz, 37.6 us; with
+// a B that is not cached 1316 cycles at 1.93 GHz, 49.1 us, 148 cycles more for its lines out of memory.  2048 x 4096 x 4096 on 128 x 256 tiles 1412 cycles (1024)
+// at 1.85 GHz, zeros 1430 at 2.36, not cached 1489 at 1.81; 1536 x 3072 x 4096 on 192 x 128, 192 workgroups, 1187 (768) at 2.32, 1434 at 2.28 not cached.
 // The ring is what fits beside nothing else in 160 KiB; four stages where three would do made no difference (128 x 192
 // 50.3 / 51.0 us at 1000 x 6144 x 4096).  Eight waves against four: 128 x 128 a twelfth faster where operands are cached,
 // 128 x 256 a twentieth, 128 x 192 the same; 128 x 64 has room for four.  Always the guarded form (ragged tiles, any D, a K tail):
